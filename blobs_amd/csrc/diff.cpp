@@ -3,6 +3,7 @@
 // segment-by-segment adjoint.
 #include "diff.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 #include <hip/hip_runtime.h>
@@ -23,6 +24,8 @@ namespace bg {
     } while (0)
 
 namespace {
+
+constexpr uint64_t kTapeBytes = 2ull << 30;  // tape memory beyond which segments are recomputed one at a time
 
 template <class T>
 hipError_t dalloc(T** p, size_t n) {
@@ -157,6 +160,10 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
     if (hipGetDeviceCount(&dev_n) != hipSuccess || dev_n == 0)
         return fail(BG_ERR_NO_DEVICE, "no HIP device available: the rollout has no CPU fallback");
     ck_every_ = checkpoint_every;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+        cus_ = (uint32_t)cus;
     std::vector<DiffWorld> ws(n);
     std::vector<float2> p0, q0, v0;
     std::vector<uint32_t> inc_count;
@@ -356,16 +363,38 @@ int Rollout::ensure_buffers(uint32_t n_steps) {
         HIP_TRY(dalloc(&d_ck_v_, (size_t)n_ck_buf * nb_));
         n_ck_alloc_ = n_ck_buf;
     }
-    const uint32_t seg_sub = (n_steps < ck_every_ ? n_steps : ck_every_) * substeps_;
-    if (seg_sub > tape_sub_alloc_) {
-        dfree(d_tape_s_), dfree(d_tape_nbr_), dfree(d_tape_v_), dfree(d_tape_pj_);
-        HIP_TRY(dalloc(&d_tape_s_, (size_t)seg_sub * nb_));
-        HIP_TRY(dalloc(&d_tape_nbr_, (size_t)seg_sub * nb_ * kDiffTapeNbr));
-        if (damped_) HIP_TRY(dalloc(&d_tape_v_, (size_t)seg_sub * nb_));
-        if (nj_ > 0 && j_iters_ > 0) HIP_TRY(dalloc(&d_tape_pj_, (size_t)seg_sub * nb_));
-        tape_sub_alloc_ = seg_sub;
-    }
+    return ensure_tape(segment_substeps(n_steps));
+}
+
+// Memory for `subs` substeps of tape.
+int Rollout::ensure_tape(uint32_t subs) {
+    if (subs <= tape_sub_alloc_) return BG_OK;
+    tape_sub_alloc_ = 0;
+    dfree(d_tape_s_), dfree(d_tape_nbr_), dfree(d_tape_v_), dfree(d_tape_pj_);
+    HIP_TRY(dalloc(&d_tape_s_, (size_t)subs * nb_));
+    HIP_TRY(dalloc(&d_tape_nbr_, (size_t)subs * nb_ * kDiffTapeNbr));
+    if (damped_) HIP_TRY(dalloc(&d_tape_v_, (size_t)subs * nb_));
+    if (nj_ > 0 && j_iters_ > 0) HIP_TRY(dalloc(&d_tape_pj_, (size_t)subs * nb_));
+    tape_sub_alloc_ = subs;
     return BG_OK;
+}
+
+// How many segments one recompute launch records: a segment takes one workgroup a world, so
+// with fewer worlds than CUs several fill the chip, as far as kTapeBytes of tape go (one
+// segment always does: a forward allocated it).
+uint32_t Rollout::recompute_segments() {
+    const uint32_t n_seg = (n_steps_ + ck_every_ - 1) / ck_every_;
+    const uint32_t seg_sub = segment_substeps(n_steps_);
+    const uint64_t per_sub = (uint64_t)nb_ * (sizeof(float2) * (1u + (d_tape_v_ ? 1u : 0u) + (d_tape_pj_ ? 1u : 0u)) +
+                                              sizeof(uint16_t) * kDiffTapeNbr);
+    uint64_t segs = std::min<uint64_t>(n_seg, cus_ / n_worlds_);
+    if (per_sub > 0) segs = std::min<uint64_t>(segs, kTapeBytes / (per_sub * seg_sub));
+    segs = std::max<uint64_t>(segs, 1);
+    if (segs > 1 && ensure_tape((uint32_t)segs * seg_sub) != BG_OK) {
+        (void)hipGetLastError();  // no room: one at a time
+        segs = 1;
+    }
+    return (uint32_t)segs;
 }
 
 DiffArgs Rollout::args() const {
@@ -439,6 +468,8 @@ int Rollout::forward(double delta, uint32_t n_steps, float* loss_per_world) {
 
 int Rollout::backward(const float* dl_dfinal, float* grad_vreq, float* grad_k) {
     if (!have_forward_) return fail(BG_ERR_INVALID_ARGUMENT, "backward needs a forward with the current parameters");
+    const uint32_t tape_segs = recompute_segments();
+    if (int st = ensure_tape(segment_substeps(n_steps_))) return st;
     DiffArgs a = args();
     if (dl_dfinal) {
         std::vector<float2> dl(nb_);
@@ -448,10 +479,12 @@ int Rollout::backward(const float* dl_dfinal, float* grad_vreq, float* grad_k) {
     }
     HIP_TRY(hipMemsetAsync(d_gk_, 0, sizeof(float) * (ns_ ? ns_ : 1), stream_));
     const uint32_t n_seg = (n_steps_ + ck_every_ - 1) / ck_every_;
-    for (uint32_t seg = n_seg; seg-- > 0;) {
-        const uint32_t first = seg * ck_every_;
-        const uint32_t steps = (n_steps_ - first) < ck_every_ ? (n_steps_ - first) : ck_every_;
-        HIP_TRY(launch_diff_backward_segment(a, seg, first, steps, seg == n_seg - 1, stream_));
+    for (uint32_t end = n_seg; end > 0;) {  // the last segments first
+        const uint32_t n = std::min(end, tape_segs), first = end - n;
+        HIP_TRY(launch_diff_recompute(a, first, n, ck_every_, n_steps_, stream_));
+        for (uint32_t seg = end; seg-- > first;)
+            HIP_TRY(launch_diff_reverse(a, seg, seg - first, ck_every_, n_steps_, stream_));
+        end = first;
     }
     std::vector<float2> gv(nb_);
     std::vector<float> gk(ns_);

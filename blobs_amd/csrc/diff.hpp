@@ -70,7 +70,7 @@ struct DiffArgs {
     float2* ck_v;
     float2* final_p;
     float* loss;  // per world: |centroid(final position) - target|^2
-    // tape of one segment, [substep in segment][nb_total]
+    // tape of the recorded segments, [substep][nb_total]
     float2* tape_s;
     uint16_t* tape_nbr;  // [..][nb_total][kDiffTapeNbr]
     float2* tape_v;      // calculated_velocity at the substep start (damped springs), else null
@@ -88,8 +88,12 @@ struct DiffArgs {
 };
 
 hipError_t launch_diff_forward(const DiffArgs& a, uint32_t n_steps, uint32_t ck_every, hipStream_t s);
-hipError_t launch_diff_backward_segment(const DiffArgs& a, uint32_t seg, uint32_t seg_first_step,
-                                        uint32_t seg_steps, bool last_segment, hipStream_t s);
+// Records the tapes of segments [first_seg, first_seg + n_seg), one after another.
+hipError_t launch_diff_recompute(const DiffArgs& a, uint32_t first_seg, uint32_t n_seg, uint32_t ck_every,
+                                 uint32_t n_steps, hipStream_t s);
+// Adjoint of segment `seg`, the tape_seg-th of the recorded ones.
+hipError_t launch_diff_reverse(const DiffArgs& a, uint32_t seg, uint32_t tape_seg, uint32_t ck_every, uint32_t n_steps,
+                               hipStream_t s);
 
 class World;
 
@@ -118,11 +122,14 @@ public:
 private:
     void release();
     int ensure_buffers(uint32_t n_steps);
+    int ensure_tape(uint32_t subs);
+    uint32_t recompute_segments();
+    uint32_t segment_substeps(uint32_t n_steps) const { return (n_steps < ck_every_ ? n_steps : ck_every_) * substeps_; }
     DiffArgs args() const;
 
     hipStream_t stream_ = nullptr;
     uint32_t n_worlds_ = 0, nb_ = 0, ns_ = 0, substeps_ = 8, ck_every_ = 20, n_steps_ = 0;
-    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, nj_ = 0, j_iters_ = 0;
+    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, cus_ = 1, nj_ = 0, j_iters_ = 0;
     float gx_ = 0.0f, gy_ = 0.0f, h_ = 0.0f;
     bool collisions_ = true, damped_ = false, have_forward_ = false;
     std::vector<uint8_t> nonfinite_;  // per world, after the last backward: a gradient entry is inf or NaN

@@ -1,15 +1,27 @@
 // diff_kernels.hip -- forward and adjoint of rollouts of single-sphere worlds
 // with springs, one 1024-thread workgroup per world for a whole segment of
-// steps (two bodies per thread; snapshot, velocities, the cell grid and the
-// adjoint vectors live in LDS).
+// steps (two bodies per thread; positions, velocities, the cell grid, the
+// spring forces, the joint records and the adjoint vectors live in LDS).
 //
 // Forward substep (physics.rs:401-421, same f32 operation order as the
 // general path): gravity and springs per body in ascending spring index
 // (springs.rs:25-47), contacts against the substep's snapshot summed in
 // ascending partner index (physics.rs:241-317), Verlet (physics.rs:323-358),
-// collider transform = position (zero offsets).  The grid is rebuilt in LDS
-// every substep: bounding box, cell counts with LDS atomics, a block scan,
-// and a scatter of body indices.
+// collider transform = position (zero offsets).  The bodies are filed by cell
+// in LDS every substep (lds_grid.hpp): counts with LDS atomics, a block scan,
+// and a scatter of (x, y, radius, index) records.
+//
+// A world has one workgroup, so a launch takes what its slowest world takes
+// and a substep is bound by VALU issue and by its chain of phases.  Hence
+// five barriers a substep; springs evaluated once each by a thread of their
+// own (at most kDiffLdsSprings; a body then sums its springs' terms from LDS
+// in ascending index), joints swept on records staged in LDS, and the next
+// tape slot loaded while the reverse works on the current one.  Recompute and
+// reverse are kernels of their own: in one, their state spilled 55 VGPRs.
+// Measured (forward + backward, against bounding box, grid and springs worked
+// out serially or per body each substep): 256 worlds of 2,048 bodies and 1,024
+// springs over 50 steps 33.1 -> 17.5 ms; 96 worlds of 700, 60 steps forward
+// 7.25 -> 3.62 ms; 12 worlds of 301 with 40 joints, 6 steps 3.78 -> 2.31 ms.
 //
 // Adjoint substep, exact derivative of that map with the substep's pair set
 // held fixed (pairs with dist < 1e-6 take the push-out branch and are held
@@ -26,225 +38,239 @@
 // anchor axis; dcorr/dd = I - (D/|d|)(I - n n^T), and the reverse sweep
 // walks the joints in the opposite order on the axes of the forward sweep.
 #include "diff.hpp"
-#include "step_common.hpp"
+
+#include <algorithm>
+
+#include "lds_grid.hpp"
 
 namespace bg {
 
 namespace {
 
 constexpr int kWaves = kDiffThreads / BG_WAVE;
+constexpr uint32_t kScanItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThreads;
+// Springs of a world whose terms are kept in LDS (32 KB of it); a world with more evaluates
+// them per body.
+constexpr uint32_t kDiffLdsSprings = 2048;
+constexpr uint32_t kDiffLdsJoints = 256;   // joints of a world whose records are staged in LDS
+constexpr uint32_t kDiffLdsAxes = 1024;    // solves of a world whose axes the reverse keeps in LDS
+constexpr uint32_t kCntStride = kDiffCells + 2;
+constexpr uint32_t kInc = 4;               // springs of a body kept as packed registers
 
-struct DiffGrid {
-    float ox, oy, inv_cell;
-    int32_t nx, ny;
-    uint32_t ncells;
+struct JointRec {
+    float4 anchor;   // a (x, y), b (z, w)
+    float4 mass;     // 1/m_a + 1/m_b, ratio, 1 - ratio, unused
+    float dist;
+    uint32_t ab;     // local a | local b << 16
+    uint32_t statics;  // bit 0: a is static, bit 1: b is
 };
 
 struct Ctx {
-    float4* snap;      // x, y, radius, mass
+    float2* xy;        // positions (the snapshot)
     float2* vel;       // calculated_velocity
-    uint32_t* cnt;     // cell counts, then cell starts
-    uint16_t* sorted;  // body index in cell order
-    uint32_t* red;     // [4][kWaves]
+    float* mass;
+    float4* rec;       // bodies in cell order; the reverse's snapshot (x, y, radius, mass) by index
+    float* gmod;       // gravity_mod; forward only
+    uint32_t* cnt;     // two tables of kCntStride: cell counts, then cell starts; the other one is cleared meanwhile
+    float4* force;     // per spring: (Fx / m_a, Fy / m_a, -Fx / m_b, -Fy / m_b); forward only
+    uint32_t* red;     // [kFitWords][kWaves]
     double* dred;      // [2][kWaves]
-    DiffGrid* grid;
-    float2* lam_pp;  // adjoint only
+    LdsGrid* grid;
+    JointRec* joints;  // the world's joints, if at most kDiffLdsJoints
+    float2* axes;      // the reverse's axes, if at most kDiffLdsAxes
+    float2* lam_pp;    // adjoint only (the memory of `force`)
     float2* lam_am;
 };
 
+// A thread's two bodies.  The phases loop over them at run time and pick the state by
+// selects: unrolled, two bodies' contact passes in flight spill 50 to 140 VGPRs.
 struct Own {
-    float2 p[kDiffPer], q[kDiffPer], v[kDiffPer];
-    float m[kDiffPer], r[kDiffPer], gm[kDiffPer];
-    uint32_t fl[kDiffPer], key[kDiffPer], rank[kDiffPer];
-    uint32_t li[kDiffPer], gi[kDiffPer];
-    bool live[kDiffPer];
+    float2 p[2], q[2];
+    float r[2];
+    uint32_t fl[2];             // body flags | springs of the body << 8 (at most kIncMany: more are counted anew)
+    uint32_t inc0[2], inc1[2];  // first kInc springs, two a word: local spring << 1 | (1: the body is its b)
+    // the spring this thread evaluates first
+    uint32_t s_ab;
+    float s_rest, s_k, s_c;
 };
+constexpr uint32_t kIncMany = 0xFFFFFFu;
+static_assert(kDiffPer == 2, "two bodies a thread");
+template <class T>
+__device__ __forceinline__ T pick(const T (&v)[2], uint32_t j) {
+    return j ? v[1] : v[0];
+}
+__device__ __forceinline__ float2 pick(const float2 (&v)[2], uint32_t j) {
+    return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
+}
+__device__ __forceinline__ void put(float2 (&v)[2], uint32_t j, float2 x) {
+    v[0].x = j ? v[0].x : x.x;
+    v[0].y = j ? v[0].y : x.y;
+    v[1].x = j ? x.x : v[1].x;
+    v[1].y = j ? x.y : v[1].y;
+}
+__device__ __forceinline__ uint32_t per_thread(const DiffWorld& W) { return W.nb > kDiffThreads ? 2u : 1u; }
 
-__device__ __forceinline__ void load_own(Own& o, const DiffArgs& a, const DiffWorld& W, const float2* p,
+// The thread's index, opaque to the compiler: the phases of a substep recompute what they
+// derive from it, where hoisted out of the substep loop those addresses spill.
+__device__ __forceinline__ uint32_t thread_index() {
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+__device__ __forceinline__ bool lds_springs(const DiffWorld& W) { return W.ns <= kDiffLdsSprings; }
+
+__device__ __forceinline__ JointRec joint_load(const DiffArgs& a, const DiffWorld& W, uint32_t q) {
+    JointRec r;
+    r.anchor = a.j_anchor[q];
+    r.mass = a.j_mass[q];
+    r.dist = a.j_dist[q];
+    r.ab = a.j_ab[q];
+    r.statics = ((a.flags[W.b0 + (r.ab & 0xFFFFu)] & BF_STATIC) ? 1u : 0u) |
+                ((a.flags[W.b0 + (r.ab >> 16)] & BF_STATIC) ? 2u : 0u);
+    return r;
+}
+
+__device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, const float2* p,
                                          const float2* q, const float2* v) {
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        o.li[j] = threadIdx.x + j * kDiffThreads;
-        o.live[j] = o.li[j] < W.nb;
-        o.gi[j] = W.b0 + (o.live[j] ? o.li[j] : 0u);
-        const uint32_t g = o.gi[j];
-        o.p[j] = o.live[j] ? p[g] : make_float2(0.0f, 0.0f);
-        o.q[j] = o.live[j] ? q[g] : make_float2(0.0f, 0.0f);
-        o.v[j] = o.live[j] ? v[g] : make_float2(0.0f, 0.0f);
-        o.m[j] = a.mass[g];
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t li = threadIdx.x + j * kDiffThreads;
+        const bool live = li < W.nb;
+        const uint32_t g = W.b0 + (live ? li : 0u);
+        o.p[j] = live ? p[g] : make_float2(0.0f, 0.0f);
+        o.q[j] = live ? q[g] : make_float2(0.0f, 0.0f);
         o.r[j] = a.radius[g];
-        o.gm[j] = a.gmod[g];
-        o.fl[j] = a.flags[g];
-        o.key[j] = 0;
-        o.rank[j] = 0;
+        o.fl[j] = a.flags[g] & 0xFFu;
+        o.inc0[j] = o.inc1[j] = 0;
+        if (!live) continue;
+        c.xy[li] = o.p[j];
+        c.vel[li] = v[g];
+        c.mass[li] = a.mass[g];
+        if (c.gmod) c.gmod[li] = a.gmod[g];
+        const uint32_t e0 = a.inc_start[g], n_inc = a.inc_start[g + 1] - e0;
+        o.fl[j] |= min(n_inc, kIncMany) << 8;
+        if (lds_springs(W)) {
+#pragma unroll
+            for (uint32_t t = 0; t < kInc; ++t)
+                if (t < n_inc) {
+                    const uint32_t s = a.inc_list[e0 + t];
+                    const uint32_t e = ((s - W.s0) << 1) | ((uint32_t)a.sp_a[s] == g ? 0u : 1u);
+                    (t < 2 ? o.inc0[j] : o.inc1[j]) |= e << (16u * (t & 1u));
+                }
+        }
     }
+    o.s_ab = 0;
+    o.s_rest = o.s_k = o.s_c = 0.0f;
+    if (threadIdx.x < W.ns) {
+        const uint32_t s = W.s0 + threadIdx.x;
+        o.s_ab = ((uint32_t)a.sp_a[s] - W.b0) | (((uint32_t)a.sp_b[s] - W.b0) << 16);
+        o.s_rest = a.sp_rest[s];
+        o.s_k = a.sp_k[s];
+        o.s_c = a.sp_c[s];
+    }
+    for (uint32_t i = threadIdx.x; i <= kDiffCells; i += kDiffThreads) c.cnt[i] = 0u;
+    const bool jointed = a.j_iters > 0 && W.njc > 0;
+    const uint32_t q0 = jointed ? a.jc_start[W.jc0] : 0u;
+    const uint32_t nj = jointed ? a.jc_start[W.jc0 + W.njc] - q0 : 0u;
+    if (nj <= kDiffLdsJoints)
+        for (uint32_t k = threadIdx.x; k < nj; k += kDiffThreads) c.joints[k] = joint_load(a, W, q0 + k);
 }
 
-__device__ __forceinline__ void publish(Ctx& c, const Own& o) {
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j)
-        if (o.live[j]) {
-            c.snap[o.li[j]] = make_float4(o.p[j].x, o.p[j].y, o.r[j], o.m[j]);
-            c.vel[o.li[j]] = o.v[j];
-        }
-}
-
-// Exclusive scan of cnt[0, n) by the block (n <= 5 * kDiffThreads).
-__device__ void block_scan_cnt(Ctx& c, uint32_t n) {
-    constexpr uint32_t kItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThreads;
-    const uint32_t base = threadIdx.x * kItems;
-    uint32_t v[kItems];
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kItems; ++k) {
-        v[k] = (base + k < n) ? c.cnt[base + k] : 0u;
-        sum += v[k];
-    }
-    const uint32_t incl = wave_incl_scan_u32(sum);
-    const int lane = threadIdx.x & (BG_WAVE - 1), wid = threadIdx.x / BG_WAVE;
-    if (lane == BG_WAVE - 1) c.red[wid] = incl;
-    __syncthreads();
-    uint32_t off = 0;
-    for (int w = 0; w < wid; ++w) off += c.red[w];
-    uint32_t run = off + incl - sum;
-#pragma unroll
-    for (uint32_t k = 0; k < kItems; ++k) {
-        if (base + k < n) c.cnt[base + k] = run;
-        run += v[k];
-    }
-    __syncthreads();
-}
-
-// Cell grid of the current snapshot in LDS (counting sort of body indices).
-__device__ void build_grid(Ctx& c, Own& o, const DiffWorld& W) {
-    const int lane = threadIdx.x & (BG_WAVE - 1), wid = threadIdx.x / BG_WAVE;
-    uint32_t b0 = 0xFFFFFFFFu, b1 = 0xFFFFFFFFu, b2 = 0u, b3 = 0u;
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        if (!o.live[j]) continue;
-        const float4 s = c.snap[o.li[j]];
-        if (!finitef(s.x) || !finitef(s.y)) continue;
-        b0 = min(b0, f2ord(s.x));
-        b1 = min(b1, f2ord(s.y));
-        b2 = max(b2, f2ord(s.x));
-        b3 = max(b3, f2ord(s.y));
-    }
-    b0 = wave_min_u32(b0);
-    b1 = wave_min_u32(b1);
-    b2 = wave_max_u32(b2);
-    b3 = wave_max_u32(b3);
-    if (lane == 0) {
-        c.red[wid] = b0;
-        c.red[kWaves + wid] = b1;
-        c.red[2 * kWaves + wid] = b2;
-        c.red[3 * kWaves + wid] = b3;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kWaves; ++w) {
-            b0 = min(b0, c.red[w]);
-            b1 = min(b1, c.red[kWaves + w]);
-            b2 = max(b2, c.red[2 * kWaves + w]);
-            b3 = max(b3, c.red[3 * kWaves + w]);
-        }
-        b0 = min(b0, c.red[0]);
-        b1 = min(b1, c.red[kWaves]);
-        b2 = max(b2, c.red[2 * kWaves]);
-        b3 = max(b3, c.red[3 * kWaves]);
-        float minx = 0.0f, miny = 0.0f, maxx = 0.0f, maxy = 0.0f;
-        if (b0 <= b2 && b1 <= b3) {
-            minx = ord2f(b0);
-            miny = ord2f(b1);
-            maxx = ord2f(b2);
-            maxy = ord2f(b3);
-        }
-        float cell = 2.0f * W.rmax;
-        if (!(cell > 0.0f) || !finitef(cell)) cell = 1.0f;
-        const float ex = maxx - minx, ey = maxy - miny;
-        int32_t nx = 1, ny = 1;
-        for (;;) {
-            const float fx = floorf(ex / cell) + 1.0f, fy = floorf(ey / cell) + 1.0f;
-            if (fx <= 65536.0f && fy <= 65536.0f && (uint64_t)fx * (uint64_t)fy <= (uint64_t)kDiffCells) {
-                nx = (int32_t)fx;
-                ny = (int32_t)fy;
-                break;
-            }
-            cell = cell * 2.0f;
-        }
-        c.grid->ox = minx;
-        c.grid->oy = miny;
-        c.grid->inv_cell = 1.0f / cell;
-        c.grid->nx = nx;
-        c.grid->ny = ny;
-        c.grid->ncells = (uint32_t)nx * (uint32_t)ny;
-    }
-    __syncthreads();
-    const DiffGrid g = *c.grid;
-    for (uint32_t i = threadIdx.x; i <= g.ncells; i += kDiffThreads) c.cnt[i] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        if (!o.live[j]) continue;
-        const float4 s = c.snap[o.li[j]];
-        const int32_t cx = cell_coord(s.x, g.ox, g.inv_cell, g.nx);
-        const int32_t cy = cell_coord(s.y, g.oy, g.inv_cell, g.ny);
-        o.key[j] = (uint32_t)cy * (uint32_t)g.nx + (uint32_t)cx;
-        o.rank[j] = atomicAdd(&c.cnt[o.key[j]], 1u);
-    }
-    __syncthreads();
-    block_scan_cnt(c, g.ncells + 1);
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j)
-        if (o.live[j]) c.sorted[c.cnt[o.key[j]] + o.rank[j]] = (uint16_t)o.li[j];
-    __syncthreads();
-}
-
-// Bodies of the grid rows overlapping the square of half-width Q around (qx, qy).
+// f(incidence) over body j's springs in ascending index; incidence as in Own::inc0.
 template <class F>
-__device__ __forceinline__ void grid_query(const Ctx& c, float qx, float qy, float Q, F&& visit) {
-    const DiffGrid g = *c.grid;
-    const float R = Q + (1e-5f * (fabsf(qx) + fabsf(qy) + Q) + 1e-6f);
-    int32_t cx0 = 0, cx1 = g.nx - 1, cy0 = 0, cy1 = g.ny - 1;
-    if (R < 1e30f && finitef(qx) && finitef(qy)) {
-        cx0 = cell_coord(qx - R, g.ox, g.inv_cell, g.nx);
-        cx1 = cell_coord(qx + R, g.ox, g.inv_cell, g.nx);
-        cy0 = cell_coord(qy - R, g.oy, g.inv_cell, g.ny);
-        cy1 = cell_coord(qy + R, g.oy, g.inv_cell, g.ny);
-    }
-    for (int32_t cy = cy0; cy <= cy1; ++cy) {
-        const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
-        const uint32_t t0 = c.cnt[row + (uint32_t)cx0], t1 = c.cnt[row + (uint32_t)cx1 + 1u];
-        for (uint32_t t = t0; t < t1; ++t) visit((uint32_t)c.sorted[t]);
+__device__ __forceinline__ void for_springs(const Own& o, uint32_t j, const DiffArgs& a, const DiffWorld& W, F&& f) {
+    const uint32_t n = pick(o.fl, j) >> 8, w0 = pick(o.inc0, j), w1 = pick(o.inc1, j);
+    if (n > 0) f(w0 & 0xFFFFu);
+    if (n > 1) f(w0 >> 16);
+    if (n > 2) f(w1 & 0xFFFFu);
+    if (n > 3) f(w1 >> 16);
+    static_assert(kInc == 4, "the four above");
+    if (n > kInc) {
+        const uint32_t g = W.b0 + threadIdx.x + j * kDiffThreads, e0 = a.inc_start[g], e1 = a.inc_start[g + 1];
+        for (uint32_t t = kInc; t < e1 - e0; ++t) {
+            const uint32_t s = a.inc_list[e0 + t];
+            f(((s - W.s0) << 1) | ((uint32_t)a.sp_a[s] == g ? 0u : 1u));
+        }
     }
 }
 
-// Joint weights (physics.rs:450-460): a static -> b moves by ims corr; b
-// static -> a does; otherwise a by ratio corr and b by (1 - ratio) corr.
-__device__ __forceinline__ void joint_weights(const DiffArgs& a, const DiffWorld& W, uint32_t q, uint32_t la,
-                                              uint32_t lb, bool& sa, bool& sb, float4& jm) {
-    sa = (a.flags[W.b0 + la] & BF_STATIC) != 0;
-    sb = (a.flags[W.b0 + lb] & BF_STATIC) != 0;
-    jm = a.j_mass[q];
+// f(local spring, local a, local b, rest, k, c) over the springs this thread evaluates.
+template <class F>
+__device__ __forceinline__ void own_springs(const Own& o, const DiffArgs& a, const DiffWorld& W, F&& f) {
+    uint32_t ab = o.s_ab;
+    float rest = o.s_rest, k = o.s_k, cc = o.s_c;
+    for (uint32_t t = threadIdx.x; t < W.ns;) {
+        f(t, ab & 0xFFFFu, ab >> 16, rest, k, cc);
+        t += kDiffThreads;
+        if (t < W.ns) {
+            const uint32_t s = W.s0 + t;
+            ab = ((uint32_t)a.sp_a[s] - W.b0) | (((uint32_t)a.sp_b[s] - W.b0) << 16);
+            rest = a.sp_rest[s];
+            k = a.sp_k[s];
+            cc = a.sp_c[s];
+        }
+    }
+}
+
+// Force of one spring on its body a (springs.rs:25-47); -F acts on b.
+__device__ __forceinline__ float2 spring_force(float2 pa, float2 pb, float2 va, float2 vb, float rest, float k, float c) {
+    const float dx = pb.x - pa.x, dy = pb.y - pa.y;
+    const float dist = vlen(dx, dy);
+    const float ux = dx / dist, uy = dy / dist;
+    const float rvx = va.x - vb.x, rvy = va.y - vb.y;
+    const float dot = rvx * ux + rvy * uy;
+    const float cd = c * dot;
+    const float dfx = cd * ux, dfy = cd * uy;
+    const float mag = k * (dist - rest);
+    return make_float2(ux * (mag - dfx), uy * (mag - dfy));
+}
+
+// One joint: its record from LDS, or from global memory in a world with more than
+// kDiffLdsJoints of them.  (A template: where the two meet in one load it becomes a flat one.)
+template <bool STAGED>
+__device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArgs& a, const DiffWorld& W, uint32_t q, uint32_t q0) {
+    if constexpr (STAGED)
+        return c.joints[q - q0];
+    else
+        return joint_load(a, W, q);
+}
+
+struct JointRange {
+    uint32_t q0, nj;   // the world's joints
+    bool staged;  // records and axes in LDS
+};
+__device__ __forceinline__ JointRange joint_range(const DiffArgs& a, const DiffWorld& W) {
+    JointRange j;
+    j.q0 = a.jc_start[W.jc0];
+    j.nj = a.jc_start[W.jc0 + W.njc] - j.q0;
+    j.staged = j.nj <= kDiffLdsJoints && (uint64_t)j.nj * a.j_iters <= kDiffLdsAxes;
+    return j;
 }
 
 // Position sweep of one joint component (physics.rs:426-460) on the LDS
-// positions P, joint_iterations times in arena order; with `axis`, every
-// solve's anchor axis goes to axis[it * n_joints + q].
-__device__ void joint_sweep(float2* P, uint32_t comp, const DiffArgs& a, const DiffWorld& W, float2* axis) {
-    const uint32_t q0 = a.jc_start[comp], q1 = a.jc_start[comp + 1];
+// positions P, joint_iterations times in arena order.  With REC every solve's
+// anchor axis is kept: in LDS at axes[it * nj + q - q0], or in j_axis.
+template <bool REC, bool STAGED>
+__device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, uint32_t comp, const DiffArgs& a, const DiffWorld& W,
+                                            const JointRange& jr) {
+    const uint32_t c0 = a.jc_start[comp], c1 = a.jc_start[comp + 1];
     uint32_t flags = 0;
     for (uint32_t it = 0; it < a.j_iters; ++it)
-        for (uint32_t q = q0; q < q1; ++q) {
-            const uint32_t ab = a.j_ab[q], la = ab & 0xFFFFu, lb = ab >> 16;
-            bool sa, sb;
-            float4 jm;
-            joint_weights(a, W, q, la, lb, sa, sb, jm);
-            const float4 an = a.j_anchor[q];
+        for (uint32_t q = c0; q < c1; ++q) {
+            const JointRec r = joint_rec<STAGED>(c, a, W, q, jr.q0);
+            const uint32_t la = r.ab & 0xFFFFu, lb = r.ab >> 16;
             float2 pa = P[la], pb = P[lb];
             float dx, dy;
-            const bool moved = joint_positions(pa, pb, make_float2(an.x, an.y), make_float2(an.z, an.w), a.j_dist[q],
-                                               jm, sa, sb, dx, dy, flags);
-            if (axis) axis[(size_t)it * a.n_joints + q] = make_float2(dx, dy);
+            const bool moved =
+                joint_positions(pa, pb, make_float2(r.anchor.x, r.anchor.y), make_float2(r.anchor.z, r.anchor.w),
+                                r.dist, r.mass, (r.statics & 1u) != 0u, (r.statics & 2u) != 0u, dx, dy, flags);
+            if (REC) {
+                if constexpr (STAGED)
+                    c.axes[it * jr.nj + (q - jr.q0)] = make_float2(dx, dy);
+                else
+                    a.j_axis[(size_t)it * a.n_joints + q] = make_float2(dx, dy);
+            }
             if (!moved) continue;
             P[la] = pa;
             P[lb] = pb;
@@ -253,312 +279,379 @@ __device__ void joint_sweep(float2* P, uint32_t comp, const DiffArgs& a, const D
 
 // Adjoint of joint_sweep on the LDS position adjoints L, from the axes the
 // forward sweep recorded: last solve first.
-__device__ void joint_sweep_reverse(float2* L, uint32_t comp, const DiffArgs& a, const DiffWorld& W,
-                                    const float2* axis) {
-    const uint32_t q0 = a.jc_start[comp], q1 = a.jc_start[comp + 1];
+template <bool STAGED>
+__device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, uint32_t comp, const DiffArgs& a,
+                                                    const DiffWorld& W, const JointRange& jr) {
+    const uint32_t c0 = a.jc_start[comp], c1 = a.jc_start[comp + 1];
     for (uint32_t it = a.j_iters; it-- > 0;)
-        for (uint32_t q = q1; q-- > q0;) {
-            const float2 d = axis[(size_t)it * a.n_joints + q];
+        for (uint32_t q = c1; q-- > c0;) {
+            float2 d;
+            if constexpr (STAGED)
+                d = c.axes[it * jr.nj + (q - jr.q0)];
+            else
+                d = a.j_axis[(size_t)it * a.n_joints + q];
             const float dist = vlen(d.x, d.y);
             if (dist < 1e-6f) continue;  // the reference skips the joint
-            const uint32_t ab = a.j_ab[q], la = ab & 0xFFFFu, lb = ab >> 16;
-            bool sa, sb;
-            float4 jm;
-            joint_weights(a, W, q, la, lb, sa, sb, jm);
-            const float wa = sa ? 0.0f : (sb ? jm.x : jm.y);
-            const float wb = sa ? jm.x : (sb ? 0.0f : jm.z);
+            const JointRec r = joint_rec<STAGED>(c, a, W, q, jr.q0);
+            const uint32_t la = r.ab & 0xFFFFu, lb = r.ab >> 16;
+            const bool sa = (r.statics & 1u) != 0u, sb = (r.statics & 2u) != 0u;
+            // weights (physics.rs:450-460): a static -> b moves by ims corr; b static -> a does;
+            // otherwise a by ratio corr and b by (1 - ratio) corr
+            const float wa = sa ? 0.0f : (sb ? r.mass.x : r.mass.y);
+            const float wb = sa ? r.mass.x : (sb ? 0.0f : r.mass.z);
             const float2 la2 = L[la], lb2 = L[lb];
             const float lcx = wa * la2.x - wb * lb2.x, lcy = wa * la2.y - wb * lb2.y;
             const float nx = d.x / dist, ny = d.y / dist;
             const float nm = nx * lcx + ny * lcy;
-            const float f = a.j_dist[q] / dist;
+            const float f = r.dist / dist;
             const float ldx = lcx - f * (lcx - nx * nm), ldy = lcy - f * (lcy - ny * nm);
             L[la] = make_float2(la2.x - ldx, la2.y - ldy);
             L[lb] = make_float2(lb2.x + ldx, lb2.y + ldy);
         }
 }
 
-// One forward substep of the world; with `rec`, records the snapshot,
-// contact partners, velocities (damped springs) and joint-stage positions
-// (joints) at tape slot `k`.
-__device__ void substep_forward(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub, bool rec,
-                                uint32_t k) {
+// update_objects of body j (physics.rs:326-358) from its position after the contact and joint
+// stages; the snapshot is the new position.
+__device__ __forceinline__ void verlet(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub, uint32_t j,
+                                       float2 pn, float2 acc) {
+    const uint32_t tid = thread_index();
     const float h = a.h;
-    float2* tape_s = rec ? a.tape_s : nullptr;
-    uint16_t* tape_nbr = rec ? a.tape_nbr : nullptr;
-    float2* tape_v = rec ? a.tape_v : nullptr;
-    if (a.collisions) build_grid(c, o, W);
-    float2 pnew[kDiffPer], acc[kDiffPer];
+    const uint32_t li = tid + j * kDiffThreads, fl = pick(o.fl, j);
+    BodyState st;
+    st.p = pn;
+    st.po = pick(o.q, j);
+    st.rot = 0.0f;
+    st.omega = 0.0f;
+    if (fl & BF_STATIC) {
+        st.po = pn;
+        st.vel = make_float2(0.0f, 0.0f);
+    } else {
+        const bool vr = gsub == 0 && (fl & BF_HAS_VREQ);
+        const float2 vq = vr ? a.vreq[W.b0 + li] : make_float2(0.0f, 0.0f);
+        const float ratio = ((int32_t)li == W.first_dyn && gsub == 0) ? h / W.old_dt0 : h / h;
+        verlet_dynamic(st, acc, 0.0f, vr, vq, h, ratio);
+    }
+    put(o.p, j, st.p);
+    put(o.q, j, st.po);
+    c.xy[li] = st.p;
+    c.vel[li] = st.vel;
+}
+
+// One forward substep of the world (`n` counts this launch's substeps); with
+// REC, records the snapshot, contact partners, velocities (damped springs) and
+// joint-stage positions (joints) at tape slot `slot`.
+template <bool REC>
+__device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub,
+                                                uint32_t n, uint32_t slot) {
+    const uint32_t tid = thread_index();
+    const bool springs_lds = lds_springs(W);
+    const bool joints = a.j_iters > 0 && W.njc > 0;
+    const uint32_t per = per_thread(W);
+    if (a.collisions && n % kFitEvery == 0) {
+        LdsFit f;
+        f.init();
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        pnew[j] = o.p[j];
-        acc[j] = make_float2(0.0f, 0.0f);
-        if (!o.live[j]) continue;
-        const uint32_t li = o.li[j], gi = o.gi[j];
-        const float4 own = c.snap[li];
-        if (tape_s) tape_s[(size_t)k * a.nb_total + gi] = make_float2(own.x, own.y);
-        if (tape_v) tape_v[(size_t)k * a.nb_total + gi] = c.vel[li];
-        // gravity + springs (physics.rs:369-375, springs.rs:25-47), ascending spring index
-        if (!(o.fl[j] & BF_STATIC)) {
+        for (uint32_t j = 0; j < 2; ++j)
+            if (tid + j * kDiffThreads < W.nb) f.point(o.p[j].x, o.p[j].y);
+        lds_fit<kDiffThreads>(f, 2.0f * W.rmax, kDiffCells, c.red, c.grid);
+    }
+    const LdsGrid g = lds_grid_uniform(*c.grid);
+    uint32_t* cnt = c.cnt + (n & 1u) * kCntStride;
+    uint32_t key[2] = {0u, 0u}, rank[2] = {0u, 0u};
+    if (a.collisions) {
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j)
+            if (tid + j * kDiffThreads < W.nb) {
+                key[j] = lds_cell(g, o.p[j].x, o.p[j].y);
+                rank[j] = atomicAdd(&cnt[key[j]], 1u);
+            }
+    }
+    if (springs_lds) {
+        own_springs(o, a, W, [&](uint32_t t, uint32_t ia, uint32_t ib, float rest, float k, float cc) {
+            const float2 f = spring_force(c.xy[ia], c.xy[ib], c.vel[ia], c.vel[ib], rest, k, cc);
+            const float ma = c.mass[ia], mb = c.mass[ib];
+            c.force[t] = make_float4(f.x / ma, f.y / ma, (-f.x) / mb, (-f.y) / mb);
+        });
+    } else {
+        // too many springs for LDS: each body sums its own into its entry of `force`
+        for (uint32_t j = 0; j < per; ++j) {
+            const uint32_t li = tid + j * kDiffThreads, gi = W.b0 + li;
+            if (li >= W.nb) continue;
             float2 ac = gsub == 0 ? a.acc0[gi] : make_float2(0.0f, 0.0f);
-            ac.x = ac.x + a.gx * o.gm[j];
-            ac.y = ac.y + a.gy * o.gm[j];
-            const float m = o.m[j];
+            ac.x = ac.x + a.gx * c.gmod[li];
+            ac.y = ac.y + a.gy * c.gmod[li];
+            const float m = c.mass[li];
             for (uint32_t e = a.inc_start[gi]; e < a.inc_start[gi + 1]; ++e) {
                 const uint32_t s = a.inc_list[e];
                 const uint32_t ia = (uint32_t)a.sp_a[s] - W.b0, ib = (uint32_t)a.sp_b[s] - W.b0;
-                const float4 pa = c.snap[ia], pb = c.snap[ib];
-                const float2 va = c.vel[ia], vb = c.vel[ib];
-                const float dx = pb.x - pa.x, dy = pb.y - pa.y;
-                const float dist = vlen(dx, dy);
-                const float ux = dx / dist, uy = dy / dist;
-                const float rvx = va.x - vb.x, rvy = va.y - vb.y;
-                const float dot = rvx * ux + rvy * uy;
-                const float cd = a.sp_c[s] * dot;
-                const float dfx = cd * ux, dfy = cd * uy;
-                const float mag = a.sp_k[s] * (dist - a.sp_rest[s]);
-                const float fx = ux * (mag - dfx), fy = uy * (mag - dfy);
-                if (li == ia) {
-                    ac.x = ac.x + fx / m;
-                    ac.y = ac.y + fy / m;
-                } else {
-                    ac.x = ac.x + (-fx) / m;
-                    ac.y = ac.y + (-fy) / m;
-                }
+                const float2 f =
+                    spring_force(c.xy[ia], c.xy[ib], c.vel[ia], c.vel[ib], a.sp_rest[s], a.sp_k[s], a.sp_c[s]);
+                ac.x = ac.x + (li == ia ? f.x : -f.x) / m;
+                ac.y = ac.y + (li == ia ? f.y : -f.y) / m;
             }
-            acc[j] = ac;
-        }
-        // contacts against the snapshot (physics.rs:241-317), ascending partner index
-        uint32_t nrec = 0;
-        uint16_t rec[kDiffTapeNbr - 1];
-#pragma unroll
-        for (uint32_t t = 0; t + 1 < kDiffTapeNbr; ++t) rec[t] = 0xFFFFu;
-        if (a.collisions && finitef(own.x) && finitef(own.y)) {
-            const float ra = own.z, ma = own.w;
-            auto enumerate = [&](auto&& sink) {
-                grid_query(c, own.x, own.y, ra + W.rmax, [&](uint32_t lj) {
-                    if (lj == li) return;
-                    const float4 sb = c.snap[lj];
-                    const bool isA = li > lj;
-                    const float ax = isA ? own.x - sb.x : sb.x - own.x;
-                    const float ay = isA ? own.y - sb.y : sb.y - own.y;
-                    const float rs = ra + sb.z;
-                    const float dot = ax * ax + ay * ay;
-                    if (dot > (rs * rs) * 1.00000095367431640625f) return;
-                    const float dist = sqrtf(dot);
-                    if (!(dist < rs)) return;
-                    sink(lj, sb.w, isA, ax, ay, dist, rs);
-                });
-            };
-            auto correction = [&](auto&& put, uint32_t lj, float mpart, bool isA, float ax, float ay, float dist,
-                                  float rs) {
-                float px = 0.0f, py = 0.0f;
-                const bool pushed = dist < 1e-6f;
-                if (pushed) {
-                    ax = ax + 0.02f;
-                    dist = vlen(ax, ay);
-                    px = isA ? 0.01f : -0.01f;
-                    py = isA ? 0.0f : -0.0f;
-                }
-                const float mA = isA ? ma : mpart, mB = isA ? mpart : ma;
-                const float ratio = 1.0f - mA / (mA + mB);
-                const float nx = ax / dist, ny = ay / dist;
-                const float delta = rs - dist;
-                float cx, cy;
-                if (isA) {
-                    const float kk = ratio * delta;
-                    cx = kk * nx;
-                    cy = kk * ny;
-                } else {
-                    const float kk = (1.0f - ratio) * delta;
-                    cx = -(kk * nx);
-                    cy = -(kk * ny);
-                }
-                if (pushed) {
-                    cx = px + cx;
-                    cy = py + cy;
-                }
-                put(lj, cx, cy);
-            };
-            ContactList<8, uint32_t> L;
-            L.init();
-            enumerate([&](uint32_t lj, float mpart, bool isA, float ax, float ay, float dist, float rs) {
-                correction([&](uint32_t kk, float x, float y) { L.add(kk, x, y); }, lj, mpart, isA, ax, ay, dist,
-                           rs);
-            });
-            nrec = L.n;
-#pragma unroll
-            for (uint32_t t = 0; t + 1 < kDiffTapeNbr; ++t)
-                if (t < L.n) rec[t] = (uint16_t)L.key[t];
-            if (L.n > 0) {
-                float2 p = pnew[j];
-                uint32_t last = L.apply(p);
-                uint32_t done = L.n < 8 ? L.n : 8;
-                while (done < L.n) {  // more than 8 contacts: next partner by selection, same order
-                    uint32_t best = kNil;
-                    float bx = 0.0f, by = 0.0f;
-                    enumerate([&](uint32_t lj, float mpart, bool isA, float ax, float ay, float dist, float rs) {
-                        correction(
-                            [&](uint32_t kk, float x, float y) {
-                                if (kk > last && kk < best) {
-                                    best = kk;
-                                    bx = x;
-                                    by = y;
-                                }
-                            },
-                            lj, mpart, isA, ax, ay, dist, rs);
-                    });
-                    if (best == kNil) break;
-                    p.x = p.x + bx;
-                    p.y = p.y + by;
-                    last = best;
-                    ++done;
-                }
-                pnew[j] = p;
-            }
-        }
-        if (tape_nbr) {
-            uint16_t* r = tape_nbr + ((size_t)k * a.nb_total + gi) * kDiffTapeNbr;
-            r[0] = (uint16_t)(nrec < 0xFFFFu ? nrec : 0xFFFFu);
-#pragma unroll
-            for (uint32_t t = 0; t + 1 < kDiffTapeNbr; ++t) r[t + 1] = rec[t];
+            c.force[li] = make_float4(ac.x, ac.y, 0.0f, 0.0f);
         }
     }
-    // fixed joints, positions (physics.rs:424-460): the LDS velocity array is free until
-    // publish, so it holds the positions while the component lanes sweep
-    if (a.j_iters > 0 && W.njc > 0) {
-        __syncthreads();  // every spring has read the velocities
-#pragma unroll
-        for (uint32_t j = 0; j < kDiffPer; ++j)
-            if (o.live[j]) {
-                c.vel[o.li[j]] = pnew[j];
-                if (rec) a.tape_pj[(size_t)k * a.nb_total + o.gi[j]] = pnew[j];
-            }
-        __syncthreads();
-        for (uint32_t comp = W.jc0 + threadIdx.x; comp < W.jc0 + W.njc; comp += kDiffThreads)
-            joint_sweep(c.vel, comp, a, W, nullptr);
-        __syncthreads();
-#pragma unroll
-        for (uint32_t j = 0; j < kDiffPer; ++j)
-            if (o.live[j]) pnew[j] = c.vel[o.li[j]];
-    }
-    // update_objects (physics.rs:326-358); the snapshot is the new position
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        if (!o.live[j]) continue;
-        if (o.fl[j] & BF_STATIC) {
-            o.p[j] = pnew[j];
-            o.q[j] = pnew[j];
-            o.v[j] = make_float2(0.0f, 0.0f);
-            continue;
-        }
-        BodyState st;
-        st.p = pnew[j];
-        st.po = o.q[j];
-        st.rot = 0.0f;
-        st.omega = 0.0f;
-        const bool vr = gsub == 0 && (o.fl[j] & BF_HAS_VREQ);
-        const float2 vq = vr ? a.vreq[o.gi[j]] : make_float2(0.0f, 0.0f);
-        const float ratio = ((int32_t)o.li[j] == W.first_dyn && gsub == 0) ? h / W.old_dt0 : h / h;
-        verlet_dynamic(st, acc[j], 0.0f, vr, vq, h, ratio);
-        o.p[j] = st.p;
-        o.q[j] = st.po;
-        o.v[j] = st.vel;
-    }
-    __syncthreads();  // everyone is done reading the snapshot
-    publish(c, o);
     __syncthreads();
+    if (a.collisions) {
+        lds_scan<kDiffThreads, kScanItems>(cnt, g.ncells + 1u, c.red);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) {
+            const uint32_t li = tid + j * kDiffThreads;
+            if (li < W.nb) c.rec[cnt[key[j]] + rank[j]] = make_float4(o.p[j].x, o.p[j].y, o.r[j], __uint_as_float(li));
+        }
+        // the other table is this substep's to clear: its last readers passed the barriers above
+        uint32_t* other = c.cnt + ((n & 1u) ^ 1u) * kCntStride;
+        for (uint32_t i = tid; i <= kDiffCells; i += kDiffThreads) other[i] = 0u;
+        __syncthreads();
+    }
+    // From here to the end of the substep a thread touches the positions and velocities of its
+    // own bodies only (springs are done, contacts read the records), so it may rewrite them.
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        const uint32_t li = tid + j * kDiffThreads, gi = W.b0 + li;
+        if (li >= W.nb) continue;
+        const float2 xy = pick(o.p, j);
+        const size_t tape = (size_t)slot * a.nb_total + gi;
+        if (REC) {
+            a.tape_s[tape] = xy;
+            if (a.tape_v) a.tape_v[tape] = c.vel[li];
+        }
+        // gravity + springs (physics.rs:369-375, springs.rs:25-47), ascending spring index
+        float2 ac = make_float2(0.0f, 0.0f);
+        if (springs_lds) {
+            if (!(pick(o.fl, j) & BF_STATIC)) {
+                if (gsub == 0) ac = a.acc0[gi];
+                ac.x = ac.x + a.gx * c.gmod[li];
+                ac.y = ac.y + a.gy * c.gmod[li];
+                for_springs(o, j, a, W, [&](uint32_t e) {
+                    const float2 f = reinterpret_cast<const float2*>(c.force)[e];
+                    ac.x = ac.x + f.x;
+                    ac.y = ac.y + f.y;
+                });
+            }
+        } else {
+            ac = make_float2(c.force[li].x, c.force[li].y);
+        }
+        // contacts against the snapshot (physics.rs:241-317), ascending partner index; the
+        // tape takes the first kDiffTapeNbr - 1 partners, so that its list holds as many
+        constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
+        ContactList<kList, uint32_t> L;
+        L.init();
+        float2 pn = xy;
+        if (a.collisions && finitef(xy.x) && finitef(xy.y))
+            lds_contacts(g, cnt, c.rec, xy, pick(o.r, j), c.mass[li], li, W.rmax, pn, L,
+                         [&](uint32_t lj) { return c.mass[lj]; }, [](uint32_t) { return false; },
+                         [](uint32_t) { return false; }, [](uint32_t, bool, bool, bool) {});
+        if (REC) {
+            uint32_t w[kDiffTapeNbr / 2];
+            auto half = [&](uint32_t t) -> uint32_t {
+                return t == 0 ? (L.n < 0xFFFFu ? L.n : 0xFFFFu) : (t - 1 < L.n ? (L.key[t - 1] & 0xFFFFu) : 0xFFFFu);
+            };
+#pragma unroll
+            for (uint32_t t = 0; t < kDiffTapeNbr / 2; ++t) w[t] = half(2 * t) | (half(2 * t + 1) << 16);
+            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        if (joints) {
+            c.vel[li] = pn;
+            c.xy[li] = ac;
+            if (REC) a.tape_pj[tape] = pn;
+        } else {
+            verlet(c, o, a, W, gsub, j, pn, ac);
+        }
+    }
+    __syncthreads();
+    // fixed joints, positions (physics.rs:424-460), on the velocities' memory
+    if (joints) {
+        const JointRange jr = joint_range(a, W);
+        for (uint32_t comp = W.jc0 + tid; comp < W.jc0 + W.njc; comp += kDiffThreads)
+            if (jr.staged)
+                joint_sweep<false, true>(c, c.vel, comp, a, W, jr);
+            else
+                joint_sweep<false, false>(c, c.vel, comp, a, W, jr);
+        __syncthreads();
+        for (uint32_t j = 0; j < per; ++j) {
+            const uint32_t li = tid + j * kDiffThreads;
+            if (li < W.nb) verlet(c, o, a, W, gsub, j, c.vel[li], c.xy[li]);
+        }
+        __syncthreads();
+    }
 }
 
-// Adjoint of substep `gsub` (tape slot k).  In: lp, lq, lv = d loss / d
-// (position, position_old, calculated_velocity) after the substep.  Out: the
-// same before it; gv += d loss / d velocity_request at the substep that
-// consumes it.
-__device__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub,
-                                uint32_t k, float2* lp, float2* lq, float2* lv, float2* gv) {
+// One tape slot of a thread's bodies (the contact partners are loaded by the substep itself,
+// which needs them late).
+struct Tape {
+    float2 s[2], v[2], pj[2];
+};
+
+__device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const DiffWorld& W, uint32_t k, bool joints) {
+    const uint32_t tid = thread_index();
+#pragma unroll
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        if (li >= W.nb) continue;
+        const size_t i = (size_t)k * a.nb_total + W.b0 + li;
+        t.s[j] = a.tape_s[i];
+        if (a.tape_v) t.v[j] = a.tape_v[i];
+        if (joints) t.pj[j] = a.tape_pj[i];
+    }
+}
+
+// Terms of one spring's adjoint: d loss / d (p_b - p_a) (kx, ky), d loss /
+// d (v_a - v_b) (rvx, rvy) and d loss / d stiffness.
+struct SpringAdj {
+    float kx, ky, rvx, rvy, gk;
+};
+__device__ __forceinline__ SpringAdj spring_adjoint(const Ctx& c, uint32_t ia, uint32_t ib, float rest, float kk, float cc) {
+    SpringAdj r;
+    const float4 pa = c.rec[ia], pb = c.rec[ib];
+    const float dx = pb.x - pa.x, dy = pb.y - pa.y;
+    const float L = sqrtf(dx * dx + dy * dy);
+    const float ux = dx / L, uy = dy / L;
+    const float2 la = c.lam_am[ia], lb = c.lam_am[ib];
+    const float lfx = la.x - lb.x, lfy = la.y - lb.y;
+    const float uf = ux * lfx + uy * lfy;
+    const float t = kk * (1.0f - rest / L);
+    r.kx = t * (lfx - ux * uf) + kk * ux * uf;
+    r.ky = t * (lfy - uy * uf) + kk * uy * uf;
+    r.rvx = r.rvy = 0.0f;
+    if (cc != 0.0f) {
+        const float2 va = c.vel[ia], vb = c.vel[ib];
+        const float vx = va.x - vb.x, vy = va.y - vb.y;
+        const float dot = vx * ux + vy * uy;
+        const float wl = ux * ux * lfx + uy * uy * lfy;
+        // d loss / d u of -c dot (u_x^2, u_y^2), then through du/dd = (I - u u^T)/L
+        const float gux = -cc * (vx * wl + 2.0f * dot * ux * lfx);
+        const float guy = -cc * (vy * wl + 2.0f * dot * uy * lfy);
+        const float gu = ux * gux + uy * guy;
+        r.kx += (gux - ux * gu) / L;
+        r.ky += (guy - uy * gu) / L;
+        r.rvx = -cc * wl * ux;
+        r.rvy = -cc * wl * uy;
+    }
+    r.gk = (L - rest) * uf;
+    return r;
+}
+
+// Adjoint of substep `gsub`, tape slot k, whose positions are in `t`.  In: lp,
+// lq, lv = d loss / d (position, position_old, calculated_velocity) after the
+// substep.  Out: the same before it; gv += d loss / d velocity_request at the
+// substep that consumes it; gk: the stiffness gradient of the thread's first
+// spring.  With `more`, `t` leaves with slot k - 1 on its way.
+__device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const DiffWorld& W,
+                                                uint32_t gsub, uint32_t k, bool more, Tape& t, float2 (&lp)[2],
+                                                float2 (&lq)[2], float2 (&lv)[2], float2 (&gv)[2], float& gk) {
+    const uint32_t tid = thread_index();
     const float h = a.h;
     const bool joints = a.j_iters > 0 && W.njc > 0;
-    float2 lpp[kDiffPer], lqin[kDiffPer];
+    const bool springs_lds = lds_springs(W);
+    const uint32_t per = per_thread(W);
+    // per spring (kx, ky) and, with damping, (rvx, rvy), and the joints' positions: the
+    // memory of the cell tables and of the forward's positions is free
+    float2* skx = reinterpret_cast<float2*>(c.cnt);
+    float2* jpos = reinterpret_cast<float2*>(c.cnt + kCntStride);
+    float2* srv = c.xy;
+    uint4 nbr[2];
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        lpp[j] = make_float2(0.0f, 0.0f);
-        lqin[j] = make_float2(0.0f, 0.0f);
-        if (!o.live[j]) continue;
-        const size_t t = (size_t)k * a.nb_total + o.gi[j];
-        const float2 s = a.tape_s[t];
-        c.snap[o.li[j]] = make_float4(s.x, s.y, o.r[j], o.m[j]);
-        if (joints) c.vel[o.li[j]] = a.tape_pj[t];  // positions entering the joint stage
-        else if (a.tape_v) c.vel[o.li[j]] = a.tape_v[t];
-        float2 lam_a = make_float2(0.0f, 0.0f);
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        nbr[j] = make_uint4(0u, 0u, 0u, 0u);
+        if (li >= W.nb) continue;
+        if (a.collisions)
+            nbr[j] = reinterpret_cast<const uint4*>(a.tape_nbr)[(size_t)k * a.nb_total + W.b0 + li];
+        const float m = c.mass[li];
+        c.rec[li] = make_float4(t.s[j].x, t.s[j].y, o.r[j], m);
+        if (a.tape_v) c.vel[li] = t.v[j];
+        if (joints) jpos[li] = t.pj[j];  // positions entering the joint stage
+        float2 lam_a = make_float2(0.0f, 0.0f), lpp, lqin = make_float2(0.0f, 0.0f);
         if (o.fl[j] & BF_STATIC) {  // p'' = p', q'' = p', v'' = 0
-            lpp[j] = make_float2(lp[j].x + lq[j].x, lp[j].y + lq[j].y);
+            lpp = make_float2(lp[j].x + lq[j].x, lp[j].y + lq[j].y);
         } else {
             // dx = (p' - q) r; p'' = p' + dx + a h^2, q'' = p', v'' = dx / h
-            const float ratio = ((int32_t)o.li[j] == W.first_dyn && gsub == 0) ? h / W.old_dt0 : h / h;
+            const float ratio = ((int32_t)li == W.first_dyn && gsub == 0) ? h / W.old_dt0 : h / h;
             const float ldx = lp[j].x + lv[j].x / h, ldy = lp[j].y + lv[j].y / h;
             if (gsub == 0 && (o.fl[j] & BF_HAS_VREQ)) {  // q = p' - vreq h: dx = vreq h r
-                lpp[j] = make_float2(lp[j].x + lq[j].x, lp[j].y + lq[j].y);
+                lpp = make_float2(lp[j].x + lq[j].x, lp[j].y + lq[j].y);
                 gv[j].x += h * ratio * ldx;
                 gv[j].y += h * ratio * ldy;
             } else {
-                lpp[j] = make_float2((lp[j].x + lq[j].x) + ratio * ldx, (lp[j].y + lq[j].y) + ratio * ldy);
-                lqin[j] = make_float2(-ratio * ldx, -ratio * ldy);
+                lpp = make_float2((lp[j].x + lq[j].x) + ratio * ldx, (lp[j].y + lq[j].y) + ratio * ldy);
+                lqin = make_float2(-ratio * ldx, -ratio * ldy);
             }
-            lam_a = make_float2(h * h * lp[j].x / o.m[j], h * h * lp[j].y / o.m[j]);
+            lam_a = make_float2(h * h * lp[j].x / m, h * h * lp[j].y / m);
         }
-        c.lam_pp[o.li[j]] = lpp[j];
-        c.lam_am[o.li[j]] = lam_a;
+        lq[j] = lqin;
+        c.lam_pp[li] = lpp;
+        c.lam_am[li] = lam_a;
     }
+    if (more) load_tape(t, a, W, k - 1, joints);
     __syncthreads();
     if (joints) {
         // replay each component's sweep from the recorded positions for its axes, then walk
         // it backwards on the position adjoints
-        for (uint32_t comp = W.jc0 + threadIdx.x; comp < W.jc0 + W.njc; comp += kDiffThreads) {
-            joint_sweep(c.vel, comp, a, W, a.j_axis);
-            joint_sweep_reverse(c.lam_pp, comp, a, W, a.j_axis);
+        const JointRange jr = joint_range(a, W);
+        for (uint32_t comp = W.jc0 + tid; comp < W.jc0 + W.njc; comp += kDiffThreads) {
+            if (jr.staged) {
+                joint_sweep<true, true>(c, jpos, comp, a, W, jr);
+                joint_sweep_reverse<true>(c, c.lam_pp, comp, a, W, jr);
+            } else {
+                joint_sweep<true, false>(c, jpos, comp, a, W, jr);
+                joint_sweep_reverse<false>(c, c.lam_pp, comp, a, W, jr);
+            }
         }
         __syncthreads();
-#pragma unroll
-        for (uint32_t j = 0; j < kDiffPer; ++j)
-            if (o.live[j]) {
-                lpp[j] = c.lam_pp[o.li[j]];
-                if (a.tape_v) c.vel[o.li[j]] = a.tape_v[(size_t)k * a.nb_total + o.gi[j]];
-            }
+    }
+    if (springs_lds && W.ns > 0) {
+        own_springs(o, a, W, [&](uint32_t s, uint32_t ia, uint32_t ib, float rest, float kk, float cc) {
+            const SpringAdj r = spring_adjoint(c, ia, ib, rest, kk, cc);
+            skx[s] = make_float2(r.kx, r.ky);
+            if (a.tape_v) srv[s] = make_float2(r.rvx, r.rvy);
+            if (s < kDiffThreads)
+                gk += r.gk;
+            else
+                a.grad_k[W.s0 + s] += r.gk;
+        });
         __syncthreads();
     }
-    float2 lvin[kDiffPer];
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        lvin[j] = make_float2(0.0f, 0.0f);
-        if (!o.live[j]) continue;
-        const uint32_t li = o.li[j], gi = o.gi[j];
-        const float4 si = c.snap[li];
-        float2 ls = make_float2(0.0f, 0.0f);
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        const uint32_t li = tid + j * kDiffThreads, gi = W.b0 + li;
+        if (li >= W.nb) continue;
+        const float4 si = c.rec[li];
+        const float2 lpp = c.lam_pp[li];
+        float2 ls = make_float2(0.0f, 0.0f), lvin = make_float2(0.0f, 0.0f);
         // contacts, pair set of the forward substep
         if (a.collisions && finitef(si.x) && finitef(si.y)) {
             auto pair = [&](uint32_t lj) {
-                const float4 sj = c.snap[lj];
+                const float4 sj = c.rec[lj];
                 const float ax = si.x - sj.x, ay = si.y - sj.y;
                 const float d = sqrtf(ax * ax + ay * ay);
                 if (!(d >= 1e-6f)) return;  // push-out branch: held constant
                 const float rs = si.z + sj.z;
                 const float wi = sj.w / (si.w + sj.w), wj = si.w / (si.w + sj.w);
                 const float2 lj2 = c.lam_pp[lj];
-                const float mux = wi * lpp[j].x - wj * lj2.x, muy = wi * lpp[j].y - wj * lj2.y;
+                const float mux = wi * lpp.x - wj * lj2.x, muy = wi * lpp.y - wj * lj2.y;
                 const float nx = ax / d, ny = ay / d;
                 const float nm = nx * mux + ny * muy;
                 const float f = rs / d;
                 ls.x += f * (mux - nx * nm) - mux;
                 ls.y += f * (muy - ny * nm) - muy;
             };
-            const uint16_t* r = a.tape_nbr + ((size_t)k * a.nb_total + gi) * kDiffTapeNbr;
-            const uint32_t n = r[0];
+            uint32_t w0 = j ? nbr[1].x : nbr[0].x, w1 = j ? nbr[1].y : nbr[0].y;
+            uint32_t w2 = j ? nbr[1].z : nbr[0].z, w3 = j ? nbr[1].w : nbr[0].w;
+            const uint32_t n = w0 & 0xFFFFu;
             if (n < kDiffTapeNbr) {
-                for (uint32_t t = 0; t < n; ++t) pair(r[1 + t]);
+                for (uint32_t i = 0; i < n; ++i) {  // shift the next partner down
+                    w0 = (w0 >> 16) | (w1 << 16);
+                    w1 = (w1 >> 16) | (w2 << 16);
+                    w2 = (w2 >> 16) | (w3 << 16);
+                    w3 >>= 16;
+                    pair(w0 & 0xFFFFu);
+                }
             } else {  // more partners than the tape holds: the same predicate over the world
                 for (uint32_t lj = 0; lj < W.nb; ++lj) {
                     if (lj == li) continue;
-                    const float4 sb = c.snap[lj];
+                    const float4 sb = c.rec[lj];
                     const bool isA = li > lj;
                     const float ax = isA ? si.x - sb.x : sb.x - si.x;
                     const float ay = isA ? si.y - sb.y : sb.y - si.y;
@@ -571,54 +664,37 @@ __device__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const D
             }
         }
         // springs
-        for (uint32_t e = a.inc_start[gi]; e < a.inc_start[gi + 1]; ++e) {
-            const uint32_t s = a.inc_list[e];
-            const uint32_t ia = (uint32_t)a.sp_a[s] - W.b0, ib = (uint32_t)a.sp_b[s] - W.b0;
-            const float4 pa = c.snap[ia], pb = c.snap[ib];
-            const float dx = pb.x - pa.x, dy = pb.y - pa.y;
-            const float L = sqrtf(dx * dx + dy * dy);
-            const float ux = dx / L, uy = dy / L;
-            const float2 la = c.lam_am[ia], lb = c.lam_am[ib];
-            const float lfx = la.x - lb.x, lfy = la.y - lb.y;
-            const float uf = ux * lfx + uy * lfy;
-            const float kk = a.sp_k[s], rest = a.sp_rest[s];
-            const float t = kk * (1.0f - rest / L);
-            float kx = t * (lfx - ux * uf) + kk * ux * uf;
-            float ky = t * (lfy - uy * uf) + kk * uy * uf;
-            float rvx = 0.0f, rvy = 0.0f;  // d loss / d (v_a - v_b)
-            const float cc = a.sp_c[s];
-            if (cc != 0.0f) {
-                const float2 va = c.vel[ia], vb = c.vel[ib];
-                const float vx = va.x - vb.x, vy = va.y - vb.y;
-                const float dot = vx * ux + vy * uy;
-                const float wl = ux * ux * lfx + uy * uy * lfy;
-                // d loss / d u of -c dot (u_x^2, u_y^2), then through du/dd = (I - u u^T)/L
-                const float gux = -cc * (vx * wl + 2.0f * dot * ux * lfx);
-                const float guy = -cc * (vy * wl + 2.0f * dot * uy * lfy);
-                const float gu = ux * gux + uy * guy;
-                kx += (gux - ux * gu) / L;
-                ky += (guy - uy * gu) / L;
-                rvx = -cc * wl * ux;
-                rvy = -cc * wl * uy;
-            }
-            if (li == ia) {
+        auto add = [&](bool is_a, float kx, float ky, float rvx, float rvy) {
+            if (is_a) {
                 ls.x -= kx;
                 ls.y -= ky;
-                lvin[j].x += rvx;
-                lvin[j].y += rvy;
-                a.grad_k[s] += (L - rest) * uf;
+                lvin.x += rvx;
+                lvin.y += rvy;
             } else {
                 ls.x += kx;
                 ls.y += ky;
-                lvin[j].x -= rvx;
-                lvin[j].y -= rvy;
+                lvin.x -= rvx;
+                lvin.y -= rvy;
+            }
+        };
+        if (springs_lds) {
+            for_springs(o, j, a, W, [&](uint32_t e) {
+                const float2 kxy = skx[e >> 1];
+                const float2 rv = a.tape_v ? srv[e >> 1] : make_float2(0.0f, 0.0f);
+                add((e & 1u) == 0u, kxy.x, kxy.y, rv.x, rv.y);
+            });
+        } else {
+            for (uint32_t e = a.inc_start[gi]; e < a.inc_start[gi + 1]; ++e) {
+                const uint32_t s = a.inc_list[e];
+                const uint32_t ia = (uint32_t)a.sp_a[s] - W.b0, ib = (uint32_t)a.sp_b[s] - W.b0;
+                const SpringAdj r = spring_adjoint(c, ia, ib, a.sp_rest[s], a.sp_k[s], a.sp_c[s]);
+                add(li == ia, r.kx, r.ky, r.rvx, r.rvy);
+                if (li == ia) a.grad_k[s] += r.gk;
             }
         }
-        lp[j] = make_float2(lpp[j].x + ls.x, lpp[j].y + ls.y);
-        lq[j] = lqin[j];
+        put(lp, j, make_float2(lpp.x + ls.x, lpp.y + ls.y));
+        put(lv, j, lvin);
     }
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) lv[j] = lvin[j];
     __syncthreads();  // snapshot and adjoint vectors are rewritten by the next substep
 }
 
@@ -626,8 +702,8 @@ __device__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const D
 __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     double sx = 0.0, sy = 0.0;
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j)
-        if (o.live[j]) {
+    for (uint32_t j = 0; j < 2; ++j)
+        if (threadIdx.x + j * kDiffThreads < W.nb) {
             sx += (double)o.p[j].x;
             sy += (double)o.p[j].y;
         }
@@ -651,49 +727,65 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     return make_double2(tx / n, ty / n);
 }
 
-#define BG_DIFF_SHARED                                 \
-    __shared__ float4 s_snap[kDiffMaxBodies];          \
-    __shared__ float2 s_vel[kDiffMaxBodies];           \
-    __shared__ uint32_t s_cnt[kDiffCells + 1];         \
-    __shared__ uint16_t s_sorted[kDiffMaxBodies];      \
-    __shared__ uint32_t s_red[4 * kWaves];             \
-    __shared__ double s_dred[2 * kWaves];              \
-    __shared__ DiffGrid s_grid;                        \
-    Ctx c;                                             \
-    c.snap = s_snap;                                   \
-    c.vel = s_vel;                                     \
-    c.cnt = s_cnt;                                     \
-    c.sorted = s_sorted;                               \
-    c.red = s_red;                                     \
-    c.dred = s_dred;                                   \
-    c.grid = &s_grid;                                  \
-    c.lam_pp = nullptr;                                \
-    c.lam_am = nullptr;
+// With the kernels' own arrays about 157 KB of the CU's 160 KB: one workgroup a CU either way (1,024 threads at 128
+// VGPRs fill its registers).
+#define BG_DIFF_SHARED                                               \
+    __shared__ float2 s_xy[kDiffMaxBodies];                          \
+    __shared__ float2 s_vel[kDiffMaxBodies];                         \
+    __shared__ float s_mass[kDiffMaxBodies];                         \
+    __shared__ float4 s_rec[kDiffMaxBodies];                         \
+    __shared__ uint64_t s_cnt[kCntStride];                           \
+    __shared__ float4 s_force[kDiffLdsSprings];                      \
+    __shared__ uint32_t s_red[kFitWords * kWaves];                   \
+    __shared__ double s_dred[2 * kWaves];                            \
+    __shared__ LdsGrid s_grid;                                       \
+    __shared__ JointRec s_joints[kDiffLdsJoints];                    \
+    static_assert(kDiffLdsSprings >= kDiffMaxBodies, "the adjoint vectors share the springs' memory"); \
+    static_assert(kDiffCells / 2 >= kDiffLdsSprings, "spring adjoints share a cell table's memory");   \
+    static_assert(kDiffMaxBodies >= kDiffLdsSprings, "and the positions'");                            \
+    Ctx c;                                                           \
+    c.xy = s_xy;                                                     \
+    c.vel = s_vel;                                                   \
+    c.mass = s_mass;                                                 \
+    c.rec = s_rec;                                                   \
+    c.cnt = reinterpret_cast<uint32_t*>(s_cnt);                      \
+    c.gmod = nullptr;                                                \
+    c.axes = nullptr;                                                \
+    c.force = s_force;                                               \
+    c.red = s_red;                                                   \
+    c.dred = s_dred;                                                 \
+    c.grid = &s_grid;                                                \
+    c.joints = s_joints;                                             \
+    c.lam_pp = reinterpret_cast<float2*>(s_force);                   \
+    c.lam_am = c.lam_pp + kDiffMaxBodies;
 
 __global__ __launch_bounds__(kDiffThreads) void k_diff_forward(DiffArgs a, uint32_t n_steps, uint32_t ck_every) {
     BG_DIFF_SHARED
+    __shared__ float s_gmod[kDiffMaxBodies];
+    c.gmod = s_gmod;
     const DiffWorld W = a.worlds[blockIdx.x];
     Own o;
-    load_own(o, a, W, a.ck_p, a.ck_q, a.ck_v);
-    publish(c, o);
+    load_own(c, o, a, W, a.ck_p, a.ck_q, a.ck_v);
     __syncthreads();
     for (uint32_t step = 0; step < n_steps; ++step) {
         if (step > 0 && step % ck_every == 0) {
-            const size_t base = (size_t)(step / ck_every) * a.nb_total;
+            const size_t base = (size_t)(step / ck_every) * a.nb_total + W.b0;
 #pragma unroll
-            for (uint32_t j = 0; j < kDiffPer; ++j)
-                if (o.live[j]) {
-                    a.ck_p[base + o.gi[j]] = o.p[j];
-                    a.ck_q[base + o.gi[j]] = o.q[j];
-                    a.ck_v[base + o.gi[j]] = o.v[j];
+            for (uint32_t j = 0; j < 2; ++j)
+                if (threadIdx.x + j * kDiffThreads < W.nb) {
+                    a.ck_p[base + threadIdx.x + j * kDiffThreads] = o.p[j];
+                    a.ck_q[base + threadIdx.x + j * kDiffThreads] = o.q[j];
+                    a.ck_v[base + threadIdx.x + j * kDiffThreads] = c.vel[threadIdx.x + j * kDiffThreads];
                 }
         }
-        for (uint32_t sub = 0; sub < a.substeps; ++sub)
-            substep_forward(c, o, a, W, step * a.substeps + sub, false, 0);
+        for (uint32_t sub = 0; sub < a.substeps; ++sub) {
+            const uint32_t n = step * a.substeps + sub;
+            substep_forward<false>(c, o, a, W, n, n, 0u);
+        }
     }
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j)
-        if (o.live[j]) a.final_p[o.gi[j]] = o.p[j];
+    for (uint32_t j = 0; j < 2; ++j)
+        if (threadIdx.x + j * kDiffThreads < W.nb) a.final_p[W.b0 + threadIdx.x + j * kDiffThreads] = o.p[j];
     const double2 cen = block_centroid(c, o, W);
     if (threadIdx.x == 0) {
         const double dx = cen.x - (double)W.tx, dy = cen.y - (double)W.ty;
@@ -701,53 +793,68 @@ __global__ __launch_bounds__(kDiffThreads) void k_diff_forward(DiffArgs a, uint3
     }
 }
 
-__global__ __launch_bounds__(kDiffThreads) void k_diff_backward(DiffArgs a, uint32_t seg, uint32_t first_step,
-                                                                uint32_t seg_steps, uint32_t last) {
+// Recomputes segments first_seg + blockIdx.y from their checkpoints, recording their tapes
+// one after another (seg_sub substeps each).
+__global__ __launch_bounds__(kDiffThreads) void k_diff_recompute(DiffArgs a, uint32_t first_seg, uint32_t ck_every,
+                                                                 uint32_t n_steps) {
     BG_DIFF_SHARED
-    __shared__ float2 s_lam_pp[kDiffMaxBodies];
-    __shared__ float2 s_lam_am[kDiffMaxBodies];
-    c.lam_pp = s_lam_pp;
-    c.lam_am = s_lam_am;
+    __shared__ float s_gmod[kDiffMaxBodies];
+    c.gmod = s_gmod;
+    const DiffWorld W = a.worlds[blockIdx.x];
+    const uint32_t seg = first_seg + blockIdx.y, first_step = seg * ck_every;
+    const uint32_t nsub = min(n_steps - first_step, ck_every) * a.substeps;
+    const uint32_t tape0 = blockIdx.y * ck_every * a.substeps;
+    const size_t ck = (size_t)seg * a.nb_total;
+    Own o;
+    load_own(c, o, a, W, a.ck_p + ck, a.ck_q + ck, a.ck_v + ck);
+    __syncthreads();
+    for (uint32_t k = 0; k < nsub; ++k)
+        substep_forward<true>(c, o, a, W, first_step * a.substeps + k, k, tape0 + k);
+}
+
+// Adjoint of one segment, its tape at slots tape0 ...
+__global__ __launch_bounds__(kDiffThreads) void k_diff_reverse(DiffArgs a, uint32_t seg, uint32_t tape0,
+                                                               uint32_t first_sub, uint32_t nsub, uint32_t last) {
+    BG_DIFF_SHARED
+    __shared__ float2 s_axes[kDiffLdsAxes];
+    c.axes = s_axes;
     const DiffWorld W = a.worlds[blockIdx.x];
     Own o;
-    const size_t ck = (size_t)seg * a.nb_total;
-    load_own(o, a, W, a.ck_p + ck, a.ck_q + ck, a.ck_v + ck);
-    publish(c, o);
+    // (only the last segment reads positions: the final ones, for the centroid)
+    load_own(c, o, a, W, a.final_p, a.final_p, a.final_p);
     __syncthreads();
-    // recompute the segment from its checkpoint, recording the tape
-    const uint32_t nsub = seg_steps * a.substeps;
-    for (uint32_t k = 0; k < nsub; ++k)
-        substep_forward(c, o, a, W, first_step * a.substeps + k, true, k);
-    float2 lp[kDiffPer], lq[kDiffPer], lv[kDiffPer], gv[kDiffPer];
-#pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j)  // the loss does not read the final velocities
-        lv[j] = (o.live[j] && !last) ? a.lam_v[o.gi[j]] : make_float2(0.0f, 0.0f);
-    if (last && !a.dl_dfinal) {  // d |centroid - target|^2 / d p_i = 2 (centroid - target) / n
+    float2 lp[2], lq[2], lv[2], gv[2];
+    const bool centroid = last && !a.dl_dfinal;
+    float2 g0 = make_float2(0.0f, 0.0f);
+    if (centroid) {  // d |centroid - target|^2 / d p_i = 2 (centroid - target) / n
         const double2 cen = block_centroid(c, o, W);
-        const float gx = (float)(2.0 * (cen.x - (double)W.tx) / (double)(W.nb > 0 ? W.nb : 1));
-        const float gy = (float)(2.0 * (cen.y - (double)W.ty) / (double)(W.nb > 0 ? W.nb : 1));
-#pragma unroll
-        for (uint32_t j = 0; j < kDiffPer; ++j) {
-            lp[j] = make_float2(gx, gy);
-            lq[j] = make_float2(0.0f, 0.0f);
-        }
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < kDiffPer; ++j) {
-            lp[j] = o.live[j] ? (last ? a.dl_dfinal[o.gi[j]] : a.lam_p[o.gi[j]]) : make_float2(0.0f, 0.0f);
-            lq[j] = (o.live[j] && !last) ? a.lam_q[o.gi[j]] : make_float2(0.0f, 0.0f);
-        }
+        g0.x = (float)(2.0 * (cen.x - (double)W.tx) / (double)(W.nb > 0 ? W.nb : 1));
+        g0.y = (float)(2.0 * (cen.y - (double)W.ty) / (double)(W.nb > 0 ? W.nb : 1));
     }
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) gv[j] = make_float2(0.0f, 0.0f);
-    for (uint32_t k = nsub; k-- > 0;) substep_reverse(c, o, a, W, first_step * a.substeps + k, k, lp, lq, lv, gv);
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t li = threadIdx.x + j * kDiffThreads, gi = W.b0 + li;
+        const bool live = li < W.nb;
+        lp[j] = centroid ? g0 : (live ? (last ? a.dl_dfinal[gi] : a.lam_p[gi]) : make_float2(0.0f, 0.0f));
+        lq[j] = (live && !last) ? a.lam_q[gi] : make_float2(0.0f, 0.0f);
+        lv[j] = (live && !last) ? a.lam_v[gi] : make_float2(0.0f, 0.0f);  // the loss does not read the final velocities
+        gv[j] = make_float2(0.0f, 0.0f);
+    }
+    const bool own_gk = lds_springs(W) && threadIdx.x < W.ns;
+    float gk = own_gk ? a.grad_k[W.s0 + threadIdx.x] : 0.0f;
+    Tape t;
+    if (nsub > 0) load_tape(t, a, W, tape0 + nsub - 1, a.j_iters > 0 && W.njc > 0);
+    for (uint32_t k = nsub; k-- > 0;)
+        substep_reverse(c, o, a, W, first_sub + k, tape0 + k, k > 0, t, lp, lq, lv, gv, gk);
+    if (own_gk) a.grad_k[W.s0 + threadIdx.x] = gk;
 #pragma unroll
-    for (uint32_t j = 0; j < kDiffPer; ++j) {
-        if (!o.live[j]) continue;
-        a.lam_p[o.gi[j]] = lp[j];
-        a.lam_q[o.gi[j]] = lq[j];
-        a.lam_v[o.gi[j]] = lv[j];
-        if (seg == 0) a.grad_vreq[o.gi[j]] = gv[j];
+    for (uint32_t j = 0; j < 2; ++j) {
+        const uint32_t li = threadIdx.x + j * kDiffThreads, gi = W.b0 + li;
+        if (li >= W.nb) continue;
+        a.lam_p[gi] = lp[j];
+        a.lam_q[gi] = lq[j];
+        a.lam_v[gi] = lv[j];
+        if (seg == 0) a.grad_vreq[gi] = gv[j];
     }
 }
 
@@ -759,10 +866,19 @@ hipError_t launch_diff_forward(const DiffArgs& a, uint32_t n_steps, uint32_t ck_
     return hipGetLastError();
 }
 
-hipError_t launch_diff_backward_segment(const DiffArgs& a, uint32_t seg, uint32_t seg_first_step,
-                                        uint32_t seg_steps, bool last_segment, hipStream_t s) {
+hipError_t launch_diff_recompute(const DiffArgs& a, uint32_t first_seg, uint32_t n_seg, uint32_t ck_every,
+                                 uint32_t n_steps, hipStream_t s) {
     if (a.n_worlds == 0) return hipSuccess;
-    k_diff_backward<<<a.n_worlds, kDiffThreads, 0, s>>>(a, seg, seg_first_step, seg_steps, last_segment ? 1u : 0u);
+    k_diff_recompute<<<dim3(a.n_worlds, n_seg), kDiffThreads, 0, s>>>(a, first_seg, ck_every, n_steps);
+    return hipGetLastError();
+}
+
+hipError_t launch_diff_reverse(const DiffArgs& a, uint32_t seg, uint32_t tape_seg, uint32_t ck_every, uint32_t n_steps,
+                               hipStream_t s) {
+    if (a.n_worlds == 0) return hipSuccess;
+    const uint32_t first = seg * ck_every, steps = std::min(n_steps - first, ck_every);
+    k_diff_reverse<<<a.n_worlds, kDiffThreads, 0, s>>>(a, seg, tape_seg * ck_every * a.substeps, first * a.substeps,
+                                                       steps * a.substeps, first + steps == n_steps ? 1u : 0u);
     return hipGetLastError();
 }
 
