@@ -187,11 +187,9 @@ __device__ __forceinline__ int32_t clampi(int32_t v, int32_t lo, int32_t hi) { r
 
 // Monotone cell coordinate: clamp(floor((x - o) * inv), 0, n-1).  Monotone
 // non-decreasing in x, so range queries over clamped cells stay supersets.
+// (Without a branch: a conversion truncates, which is floor from 0 up; a NaN becomes 0.)
 __device__ __forceinline__ int32_t cell_coord(float x, float o, float inv, int32_t n) {
-    float f = floorf((x - o) * inv);
-    if (!(f >= 0.0f)) return 0;  // also NaN
-    if (f >= (float)(n - 1)) return n - 1;
-    return (int32_t)f;
+    return (int32_t)fminf(fmaxf((x - o) * inv, 0.0f), (float)(n - 1));
 }
 
 }  // namespace bg

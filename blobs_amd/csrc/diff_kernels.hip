@@ -12,31 +12,17 @@
 // and a scatter of (x, y, radius, index) records.
 //
 // A world has one workgroup, so a launch takes what its slowest world takes
-// and a substep is bound by VALU issue and by its chain of phases.  Hence
-// five barriers a substep; springs evaluated once each by a thread of their
+// and a substep is bound by VALU issue and by its chain of phases (a barrier
+// between them).  Hence contacts worked out from a queue by all threads; springs evaluated once each by a thread of their
 // own (at most kDiffLdsSprings; a body then sums its springs' terms from LDS
 // in ascending index), joints swept on records staged in LDS, and the next
 // tape slot loaded while the reverse works on the current one.  Recompute and
 // reverse are kernels of their own: in one, their state spilled 55 VGPRs.
-// Measured (forward + backward, against bounding box, grid and springs worked
-// out serially or per body each substep): 256 worlds of 2,048 bodies and 1,024
-// springs over 50 steps 33.1 -> 17.5 ms; 96 worlds of 700, 60 steps forward
-// 7.25 -> 3.62 ms; 12 worlds of 301 with 40 joints, 6 steps 3.78 -> 2.31 ms.
-//
-// Adjoint substep, exact derivative of that map with the substep's pair set
-// held fixed (pairs with dist < 1e-6 take the push-out branch and are held
-// constant).  With w_i = m_j / (m_i + m_j) and a = s_i - s_j, the
-// correction on i is w_i f(a), f(a) = (r_i + r_j - |a|) a / |a|, whose
-// Jacobian is J = (rs/|a|)(I - n n^T) - I; the spring force
-// F = u k (L - rest) - c (rv . u) (u_x^2, u_y^2) (springs.rs:38-43, the
-// damping vector multiplies the direction componentwise), rv = v_a - v_b,
-// has dF/dd = k[(1 - rest/L)(I - u u^T) + u u^T] + (damping through u,
-// du/dd = (I - u u^T)/L), dF/drv = -c (u_x^2, u_y^2) u^T and
-// dF/dk = u (L - rest).  The velocity v = displacement / h of the previous
-// Verlet is part of the adjoint state with damping.  A fixed joint moves
-// p_a += w_a corr and p_b -= w_b corr, corr = (|d| - D) d/|d| with d the
-// anchor axis; dcorr/dd = I - (D/|d|)(I - n n^T), and the reverse sweep
-// walks the joints in the opposite order on the axes of the forward sweep.
+// Measured (forward + backward, against bounding box, grid, springs and contacts
+// worked out serially or per body each substep): 256 worlds of 2,048 bodies and
+// 1,024 springs over 50 steps 33.2 -> 15.4 ms (17.5 before the queue of pairs);
+// 96 worlds of 700, 60 steps forward 7.24 -> 3.24 ms (3.62); 12 worlds of 301
+// with 40 joints, 6 steps 3.80 -> 2.24 ms (2.31).
 #include "diff.hpp"
 
 #include <algorithm>
@@ -54,7 +40,9 @@ constexpr uint32_t kScanItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThrea
 constexpr uint32_t kDiffLdsSprings = 2048;
 constexpr uint32_t kDiffLdsJoints = 256;   // joints of a world whose records are staged in LDS
 constexpr uint32_t kDiffLdsAxes = 1024;    // solves of a world whose axes the reverse keeps in LDS
-constexpr uint32_t kCntStride = kDiffCells + 2;
+constexpr uint32_t kCntStride = kDiffCells + 4;  // (a multiple of 16 bytes)
+constexpr uint32_t kPairs = 1360;          // queued contact pairs of a substep: 12 bytes each of a cell table
+static_assert(12 * kPairs <= 4 * kDiffCells, "the queue fits the idle cell table");
 constexpr uint32_t kInc = 4;               // springs of a body kept as packed registers
 
 struct JointRec {
@@ -74,6 +62,7 @@ struct Ctx {
     uint32_t* cnt;     // two tables of kCntStride: cell counts, then cell starts; the other one is cleared meanwhile
     float4* force;     // per spring: (Fx / m_a, Fy / m_a, -Fx / m_b, -Fy / m_b); forward only
     uint32_t* red;     // [kFitWords][kWaves]
+    uint32_t* pairs;   // queued pairs of this substep
     double* dred;      // [2][kWaves]
     LdsGrid* grid;
     JointRec* joints;  // the world's joints, if at most kDiffLdsJoints
@@ -366,6 +355,7 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
                 rank[j] = atomicAdd(&cnt[key[j]], 1u);
             }
     }
+    if (tid == 0) *c.pairs = 0;
     if (springs_lds) {
         own_springs(o, a, W, [&](uint32_t t, uint32_t ia, uint32_t ib, float rest, float k, float cc) {
             const float2 f = spring_force(c.xy[ia], c.xy[ib], c.vel[ia], c.vel[ib], rest, k, cc);
@@ -398,11 +388,35 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) {
             const uint32_t li = tid + j * kDiffThreads;
-            if (li < W.nb) c.rec[cnt[key[j]] + rank[j]] = make_float4(o.p[j].x, o.p[j].y, o.r[j], __uint_as_float(li));
+            if (li >= W.nb) continue;
+            rank[j] += cnt[key[j]];  // the body's record
+            c.rec[rank[j]] = make_float4(o.p[j].x, o.p[j].y, o.r[j], __uint_as_float(li));
         }
-        // the other table is this substep's to clear: its last readers passed the barriers above
-        uint32_t* other = c.cnt + ((n & 1u) ^ 1u) * kCntStride;
-        for (uint32_t i = tid; i <= kDiffCells; i += kDiffThreads) other[i] = 0u;
+        __syncthreads();
+    }
+    // contacts against the snapshot (physics.rs:241-317); the queue is in the idle cell table
+    uint32_t* other = c.cnt + ((n & 1u) ^ 1u) * kCntStride;
+    float2* res = reinterpret_cast<float2*>(other);
+    uint32_t* entries = other + 2 * kPairs;
+    LdsPairs pr0 = {0u, 0u, false}, pr1 = {0u, 0u, false};
+    auto pair = [&](const float4 own, const float4 oth) {
+        const uint32_t li = __float_as_uint(own.w), lj = __float_as_uint(oth.w);
+        return lds_correction(own, oth, c.mass[li], c.mass[lj], li > lj, false);
+    };
+    if (a.collisions) {
+#pragma unroll 1
+        for (uint32_t j = 0; j < per; ++j) {
+            const float2 xy = pick(o.p, j);
+            const bool active = tid + j * kDiffThreads < W.nb && finitef(xy.x) && finitef(xy.y);
+            const LdsPairs pr = lds_mark<kPairs>(g, cnt, c.rec, active, xy, pick(o.r, j), j ? rank[1] : rank[0], W.rmax,
+                                                 entries, c.pairs);
+            if (j)
+                pr1 = pr;
+            else
+                pr0 = pr;
+        }
+        __syncthreads();
+        lds_correct<kPairs, kDiffThreads>(tid, *c.pairs, c.rec, entries, res, pair);
         __syncthreads();
     }
     // From here to the end of the substep a thread touches the positions and velocities of its
@@ -433,24 +447,39 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         } else {
             ac = make_float2(c.force[li].x, c.force[li].y);
         }
-        // contacts against the snapshot (physics.rs:241-317), ascending partner index; the
-        // tape takes the first kDiffTapeNbr - 1 partners, so that its list holds as many
-        constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
-        ContactList<kList, uint32_t> L;
-        L.init();
+        // contacts, ascending partner index; the tape takes the first kDiffTapeNbr - 1 partners
         float2 pn = xy;
-        if (a.collisions && finitef(xy.x) && finitef(xy.y))
-            lds_contacts(g, cnt, c.rec, xy, pick(o.r, j), c.mass[li], li, W.rmax, pn, L,
-                         [&](uint32_t lj) { return c.mass[lj]; }, [](uint32_t) { return false; },
-                         [](uint32_t) { return false; }, [](uint32_t, bool, bool, bool) {});
-        if (REC) {
-            uint32_t w[kDiffTapeNbr / 2];
-            auto half = [&](uint32_t t) -> uint32_t {
-                return t == 0 ? (L.n < 0xFFFFu ? L.n : 0xFFFFu) : (t - 1 < L.n ? (L.key[t - 1] & 0xFFFFu) : 0xFFFFu);
-            };
+        uint32_t w0 = 0xFFFF0000u, w1 = 0xFFFFFFFFu, w2 = 0xFFFFFFFFu, w3 = 0xFFFFFFFFu, found = 0;
+        auto record = [&](uint32_t t, uint32_t lj) {  // partner number t
+            if (!REC) return;
+            const uint32_t keep = t & 1u ? 0xFFFF0000u : 0xFFFFu, put_ = t & 1u ? lj : lj << 16;
+            if (t < 1) w0 = (w0 & keep) | put_;
+            else if (t < 3) w1 = (w1 & keep) | put_;
+            else if (t < 5) w2 = (w2 & keep) | put_;
+            else if (t < 7) w3 = (w3 & keep) | put_;
+        };
+        static_assert(kDiffTapeNbr == 8, "four words: the count and seven partners");
+        const LdsPairs pr = {j ? pr1.first : pr0.first, j ? pr1.n : pr0.n, j ? pr1.direct : pr0.direct};
+        if (pr.direct) {
+            constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
+            ContactList<kList, uint32_t> L;
+            const float4 own = make_float4(xy.x, xy.y, pick(o.r, j), __uint_as_float(li));
+            found = lds_contacts_direct(g, cnt, c.rec, xy, own.z, li, W.rmax, pn, L,
+                                        [&](const float4 oth) { return pair(own, oth); },
+                                        [](uint32_t, const LdsContact&) {});
 #pragma unroll
-            for (uint32_t t = 0; t < kDiffTapeNbr / 2; ++t) w[t] = half(2 * t) | (half(2 * t + 1) << 16);
-            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w[0], w[1], w[2], w[3]);
+            for (uint32_t t = 0; REC && t + 1 < kDiffTapeNbr; ++t)
+                if (t < L.n) record(t, L.key[t]);
+        } else {
+            found = lds_sum(pr, entries, res, [&](uint32_t t, uint32_t lj, float2 k) {
+                pn.x = pn.x + k.x;
+                pn.y = pn.y + k.y;
+                record(t, lj);
+            });
+        }
+        if (REC) {
+            w0 |= found < 0xFFFFu ? found : 0xFFFFu;
+            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w0, w1, w2, w3);
         }
         if (joints) {
             c.vel[li] = pn;
@@ -461,6 +490,9 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         }
     }
     __syncthreads();
+    // clear the queue's table for the next substep's counts: every sum has read it
+    if (a.collisions)
+        for (uint32_t i = tid; i <= kDiffCells; i += kDiffThreads) other[i] = 0u;
     // fixed joints, positions (physics.rs:424-460), on the velocities' memory
     if (joints) {
         const JointRange jr = joint_range(a, W);
@@ -474,8 +506,8 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
             const uint32_t li = tid + j * kDiffThreads;
             if (li < W.nb) verlet(c, o, a, W, gsub, j, c.vel[li], c.xy[li]);
         }
-        __syncthreads();
     }
+    __syncthreads();
 }
 
 // One tape slot of a thread's bodies (the contact partners are loaded by the substep itself,
@@ -733,10 +765,11 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     __shared__ float2 s_xy[kDiffMaxBodies];                          \
     __shared__ float2 s_vel[kDiffMaxBodies];                         \
     __shared__ float s_mass[kDiffMaxBodies];                         \
-    __shared__ float4 s_rec[kDiffMaxBodies];                         \
+    __shared__ float4 s_rec[kDiffMaxBodies + kLdsRecPad];            \
     __shared__ uint64_t s_cnt[kCntStride];                           \
     __shared__ float4 s_force[kDiffLdsSprings];                      \
     __shared__ uint32_t s_red[kFitWords * kWaves];                   \
+    __shared__ uint32_t s_pairs;                                     \
     __shared__ double s_dred[2 * kWaves];                            \
     __shared__ LdsGrid s_grid;                                       \
     __shared__ JointRec s_joints[kDiffLdsJoints];                    \
@@ -753,6 +786,7 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     c.axes = nullptr;                                                \
     c.force = s_force;                                               \
     c.red = s_red;                                                   \
+    c.pairs = &s_pairs;                                              \
     c.dred = s_dred;                                                 \
     c.grid = &s_grid;                                                \
     c.joints = s_joints;                                             \

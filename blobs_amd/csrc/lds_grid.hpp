@@ -7,10 +7,8 @@
 // barriers, not memory.  So the grid is fitted once every kFitEvery substeps
 // (bodies outside it clamp into border cells; any grid gives the same pairs),
 // the scans and reductions are DPP chains in registers (a ds_bpermute per
-// step costs the LDS latency six times over), and a body first marks its
-// candidates within reach in a bit mask with about 20 instructions each and
-// takes the exact test and the correction (three divides and a root, about
-// 130 instructions) for marked ones only.
+// step costs the LDS latency six times over), and contacts are worked out by
+// all threads from a queue of the pairs within reach.
 #pragma once
 
 #include "step_common.hpp"
@@ -207,10 +205,20 @@ __device__ __forceinline__ uint32_t lds_cell(const LdsGrid& g, float x, float y)
            (uint32_t)cell_coord(x, g.ox, g.inv_cell, g.nx);
 }
 
-// ---- one body's contacts ----------------------------------------------------
+// ---- contacts ----------------------------------------------------------------
+//
+// Three phases with a barrier between them.  Mark: each body walks the records
+// of its cells, about 20 instructions a candidate, and puts those within reach
+// into a queue.  Correct: a thread takes one queued pair, whoever's it is, and
+// works out its correction (a root and three divides, about 200 instructions):
+// with one contact among ten bodies a wave that corrected its own would run
+// that code once or twice for each of its bodies, almost all lanes idle.  Sum:
+// each body adds its corrections in ascending partner index.
 
-constexpr int kLdsRows = 3;          // grid rows of a flat candidate list (a query of cells of 2 r_max rarely spans 4)
-constexpr uint32_t kLdsFlat = 64;    // candidates of a flat list (one 64-bit mask)
+constexpr int kLdsRows = 3;        // grid rows of a flat candidate list (a query of cells of 2 r_max rarely spans 4)
+constexpr uint32_t kLdsFlat = 64;  // candidates of a flat list (one 64-bit mask)
+constexpr uint32_t kLdsRecPad = 4;
+constexpr uint32_t kNoPair = 0xFFFFFFFFu;
 
 // Cells of the square of half-width Q around (x, y); the whole grid when it is not finite.
 struct LdsRect {
@@ -228,174 +236,222 @@ __device__ __forceinline__ LdsRect lds_rect(const LdsGrid& g, float x, float y, 
     return c;
 }
 
-// The records of those cells, as one flat list where they are few enough.
-struct LdsQuery {
-    uint32_t end[kLdsRows - 1];  // flat end of each row but the last
-    uint32_t base[kLdsRows];     // record of flat index i in row r: base[r] + i (modulo 2^32)
-    uint32_t n;
-    bool flat;
-    __device__ __forceinline__ uint32_t slot(uint32_t i) const {
-        uint32_t b = base[0];
-#pragma unroll
-        for (int r = 1; r < kLdsRows; ++r) b = i >= end[r - 1] ? base[r] : b;
-        return b + i;
-    }
+// A body's pairs in the queue: `n` entries from `first`, or its contacts are left to
+// lds_contacts_direct (too many candidates, or no room).
+struct LdsPairs {
+    uint32_t first, n;
+    bool direct;
 };
 
-__device__ __forceinline__ LdsQuery lds_query(const LdsGrid& g, const uint32_t* start, float x, float y, float Q) {
-    const LdsRect c = lds_rect(g, x, y, Q);
-    LdsQuery q;
-    q.n = 0;
-#pragma unroll
-    for (int r = 0; r < kLdsRows; ++r) {
-        const int32_t cy = c.cy0 + r;
-        uint32_t lo = 0, hi = 0;
-        if (cy <= c.cy1) {
-            const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
-            lo = start[row + (uint32_t)c.cx0];
-            hi = start[row + (uint32_t)c.cx1 + 1u];
-        }
-        q.base[r] = lo - q.n;
-        q.n += hi - lo;
-        if (r + 1 < kLdsRows) q.end[r] = q.n;
+// Mark phase of one body a lane (`active`: the lane has one, with a finite snapshot xy),
+// called by whole waves.  rec[] = (x, y, radius, bits(local index)) in cell order, with
+// kLdsRecPad records of room behind them, `own` the body's own record.  *count was zero before the phase; entries from CAP on are not written.
+template <uint32_t CAP>
+__device__ __forceinline__ LdsPairs lds_mark(const LdsGrid& g, const uint32_t* start, const float4* rec, bool active,
+                                             float2 xy, float r, uint32_t own, float rmax, uint32_t* entries,
+                                             uint32_t* count) {
+    // The records of the cells as one flat list: index i is record base + i, plus step1 from
+    // end0 on (the second row), plus step2 from end1 on (all modulo 2^32).  (Sums, because a
+    // select between two variables here is compiled to a load through a selected address.)
+    uint32_t end0 = 0, end1 = 0, base = 0, step1 = 0, step2 = 0, n = 0;
+    bool flat = false;
+    if (active) {
+        const LdsRect c = lds_rect(g, xy.x, xy.y, r + rmax);
+        const uint32_t nx = (uint32_t)g.nx;
+        const uint32_t row0 = __umul24((uint32_t)c.cy0, nx), last = __umul24((uint32_t)c.cy1, nx);
+        const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
+        const uint32_t* s0 = start + c.cx0;
+        const uint32_t* s1 = start + c.cx1 + 1;
+        const uint32_t lo0 = s0[row0], hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
+        const int32_t rows = c.cy1 - c.cy0 + 1;
+        base = lo0;
+        end0 = hi0 - lo0;
+        step1 = lo1 - hi0;
+        end1 = end0 + (rows > 1 ? hi1 - lo1 : 0u);
+        step2 = (lo2 - end1) - (lo1 - end0);
+        n = end1 + (rows > 2 ? hi2 - lo2 : 0u);
+        flat = rows <= kLdsRows && n <= kLdsFlat;
+        if (!flat) n = 0;
     }
-    q.flat = c.cy1 - c.cy0 < kLdsRows && q.n <= kLdsFlat;
-    return q;
-}
-
-// Contacts of body `li` (snapshot xy, radius r, mass m) with the records
-// rec[] = (x, y, radius, bits(local index)) of the grid, summed into `p` in
-// ascending partner index.  A is the body of the higher index (local order is
-// arena order).  `mass(lj)` is a partner's mass, `skip(lj)` drops a candidate
-// (interaction groups), `sensor(lj)` keeps a contact out of the sums, and
-// `hit(lj, isA, pushed, nan)` is called once for each contact.  Returns their
-// number; L ends with the K smallest partners' corrections.
-template <int K, class Mass, class Skip, class Sensor, class Hit>
-__device__ __forceinline__ uint32_t lds_contacts(const LdsGrid& g, const uint32_t* start, const float4* rec, float2 xy,
-                                                 float r, float m, uint32_t li, float rmax, float2& p,
-                                                 ContactList<K, uint32_t>& L, Mass&& mass, Skip&& skip,
-                                                 Sensor&& sensor, Hit&& hit) {
-    const LdsQuery q = lds_query(g, start, xy.x, xy.y, r + rmax);
+    static_assert(kLdsRows == 3, "the rows above");
+    auto slot = [&](uint32_t i) {
+        return (i >= end0 ? step1 : 0u) + (i >= end1 ? step2 : 0u) + (base + i);
+    };
     uint32_t near_lo = 0, near_hi = 0;
-    auto mark = [&](uint32_t f) -> uint32_t {  // four candidates
+    // four candidates; past the last one it reads up to three records further (rec has room
+    // for that), whose bits are dropped below
+    auto mark = [&](uint32_t f) -> uint32_t {
         float4 sb[4];
+        uint32_t t[4];
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) sb[u] = rec[q.slot(min(f + u, q.n - 1u))];
+        for (uint32_t u = 0; u < 4; ++u) {
+            t[u] = slot(f + u);
+            sb[u] = rec[t[u]];
+        }
         uint32_t bits = 0;
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
             const float dx = xy.x - sb[u].x, dy = xy.y - sb[u].y;
             const float rs = r + sb[u].z;
-            const bool cand = f + u < q.n && __float_as_uint(sb[u].w) != li &&
-                              !(dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f);
-            bits |= cand ? 1u << u : 0u;
+            const bool far = dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f;
+            bits |= ((t[u] == own) | far) ? 0u : 1u << u;
         }
         return bits;
     };
-    if (q.flat) {
-        for (uint32_t f = 0; f < min(q.n, 32u); f += 4) near_lo |= mark(f) << f;
-        for (uint32_t f = 32; f < q.n; f += 4) near_hi |= mark(f) << (f - 32u);
+    for (uint32_t f = 0; f < min(n, 32u); f += 4) near_lo |= mark(f) << f;
+    for (uint32_t f = 32; f < n; f += 4) near_hi |= mark(f) << (f - 32u);
+    if (n < 32u) near_lo &= (1u << n) - 1u;
+    if (n < 64u) near_hi &= n > 32u ? (1u << (n - 32u)) - 1u : 0u;
+    LdsPairs pr;
+    pr.n = (uint32_t)(__popc(near_lo) + __popc(near_hi));
+    pr.direct = active && !flat;
+    const uint32_t incl = wave_prefix(pr.n, 0u, AddU32());
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, BG_WAVE - 1);
+    uint32_t at = 0;
+    if (total > 0) {
+        if ((threadIdx.x & (BG_WAVE - 1)) == 0) at = atomicAdd(count, total);
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
     }
-    // the reference predicate (physics.rs:264-269) and, for a contact, its correction
-    auto test = [&](const float4 sb, auto&& sink) {
-        const uint32_t lj = __float_as_uint(sb.w);
-        if (lj == li || skip(lj)) return;
-        const bool isA = li > lj;
-        const float dx = xy.x - sb.x, dy = xy.y - sb.y;
-        const float rs = r + sb.z;
-        const float dot = dx * dx + dy * dy;
-        if (dot > (rs * rs) * 1.00000095367431640625f) return;
-        const float dist = sqrtf(dot);
-        if (!(dist < rs)) return;
-        sink(lj, isA, isA ? dx : -dx, isA ? dy : -dy, dist, rs);
-    };
+    pr.first = at + incl - pr.n;
+    const bool fits = pr.first + pr.n <= CAP;
+    uint64_t m = ((uint64_t)near_hi << 32) | near_lo;
+    for (uint32_t e = pr.first; m != 0; ++e) {
+        const uint32_t i = (uint32_t)__builtin_ctzll(m);
+        m &= m - 1;
+        if (e < CAP) entries[e] = fits ? (own << 16) | slot(i) : kNoPair;
+    }
+    if (!fits) {
+        pr.direct = true;
+        pr.n = 0;
+    }
+    return pr;
+}
+
+// One pair: its contact (physics.rs:264-300) from the side of the body `own`.
+// A is the body of the higher index (local order is arena order).
+struct LdsContact {
+    float2 c;     // correction of the body's position
+    bool hit;     // a contact
+    bool pushed;  // took the push-out branch, folded into the correction by the pair rule
+    bool nan;     // its normal is not a number
+};
+__device__ __forceinline__ LdsContact lds_correction(const float4 own, const float4 other, float m_own, float m_other,
+                                                     bool is_a, bool sensor) {
+    LdsContact r = {make_float2(0.0f, 0.0f), false, false, false};
+    const float dx = own.x - other.x, dy = own.y - other.y;
+    const float rs = own.z + other.z;
+    const float dot = dx * dx + dy * dy;
+    if (dot > (rs * rs) * 1.00000095367431640625f) return r;
+    float dist = sqrtf(dot);
+    if (!(dist < rs)) return r;
+    r.hit = true;
+    float ax = is_a ? dx : -dx;
+    const float ay = is_a ? dy : -dy;
+    float px = 0.0f, py = 0.0f;
+    r.pushed = dist < 1e-6f;
+    if (r.pushed) {
+        ax = ax + 0.02f;
+        dist = vlen(ax, ay);
+        px = is_a ? 0.01f : -0.01f;
+        py = is_a ? 0.0f : -0.0f;
+    }
+    if (sensor) {
+        r.c = make_float2(px, py);
+        return r;
+    }
+    const float mA = is_a ? m_own : m_other, mB = is_a ? m_other : m_own;
+    const float ratio = 1.0f - mA / (mA + mB);
+    const float nx = ax / dist, ny = ay / dist;
+    r.nan = nx != nx || ny != ny;
+    const float delta = rs - dist;
+    const float kk = is_a ? ratio * delta : (1.0f - ratio) * delta;
+    r.c.x = is_a ? kk * nx : -(kk * nx);
+    r.c.y = is_a ? kk * ny : -(kk * ny);
+    if (r.pushed) {
+        r.c.x = px + r.c.x;
+        r.c.y = py + r.c.y;
+    }
+    return r;
+}
+
+// Correct phase: `pair(own record, other record)` gives the LdsContact of a queued pair; its
+// correction goes to res[e] and the partner's index (or kNoPair) to entries[e].
+template <uint32_t CAP, uint32_t NT, class Pair>
+__device__ __forceinline__ void lds_correct(uint32_t tid, uint32_t count, const float4* rec, uint32_t* entries,
+                                            float2* res, Pair&& pair) {
+    for (uint32_t e = tid; e < min(count, CAP); e += NT) {
+        const uint32_t w = entries[e];
+        if (w == kNoPair) continue;
+        const float4 other = rec[w & 0xFFFFu];
+        const LdsContact k = pair(rec[w >> 16], other);
+        entries[e] = k.hit ? __float_as_uint(other.w) : kNoPair;
+        res[e] = k.c;
+    }
+}
+
+// Sum phase: f(k, partner, correction) over the body's contacts in ascending partner index.
+template <class F>
+__device__ __forceinline__ uint32_t lds_sum(const LdsPairs& pr, const uint32_t* entries, const float2* res, F&& f) {
+    uint32_t k = 0;
+    for (uint32_t next = 0; k < pr.n; ++k) {
+        uint32_t best = kNoPair, at = 0;
+        for (uint32_t e = pr.first; e < pr.first + pr.n; ++e) {
+            const uint32_t key = entries[e];
+            if (key >= next && key < best) {
+                best = key;
+                at = e;
+            }
+        }
+        if (best == kNoPair) break;
+        f(k, best, res[at]);
+        next = best + 1u;
+    }
+    return k;
+}
+
+// The contacts of a body that did not go through the queue, summed into `p` in ascending
+// partner index: `pair(other record)` gives the LdsContact of a candidate, `once` is called
+// with each contact's.  L ends with the K smallest partners' corrections; returns the contacts.
+template <int K, class Pair, class Once>
+__device__ __forceinline__ uint32_t lds_contacts_direct(const LdsGrid& g, const uint32_t* start, const float4* rec,
+                                                        float2 xy, float r, uint32_t li, float rmax, float2& p,
+                                                        ContactList<K, uint32_t>& L, Pair&& pair, Once&& once) {
+    const LdsRect c = lds_rect(g, xy.x, xy.y, r + rmax);
     auto enumerate = [&](auto&& sink) {
-        if (q.flat) {
-            uint64_t mm = ((uint64_t)near_hi << 32) | near_lo;
-            while (mm != 0) {
-                const uint32_t i = (uint32_t)__builtin_ctzll(mm);
-                mm &= mm - 1;
-                test(rec[q.slot(i)], sink);
-            }
-        } else {
-            const LdsRect c = lds_rect(g, xy.x, xy.y, r + rmax);
-            for (int32_t cy = c.cy0; cy <= c.cy1; ++cy) {
-                const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
-                const uint32_t t1 = start[row + (uint32_t)c.cx1 + 1u];
-                for (uint32_t t = start[row + (uint32_t)c.cx0]; t < t1; ++t) test(rec[t], sink);
+        for (int32_t cy = c.cy0; cy <= c.cy1; ++cy) {
+            const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
+            const uint32_t t1 = start[row + (uint32_t)c.cx1 + 1u];
+            for (uint32_t t = start[row + (uint32_t)c.cx0]; t < t1; ++t) {
+                const float4 other = rec[t];
+                const uint32_t lj = __float_as_uint(other.w);
+                if (lj == li) continue;
+                const LdsContact k = pair(other);
+                if (k.hit) sink(lj, k);
             }
         }
-    };
-    // correction on this body from one pair (physics.rs:270-300); a push-out is folded into
-    // the same entry by the pair rule
-    auto correction = [&](auto&& put, auto&& once, uint32_t lj, bool isA, float ax, float ay, float dist, float rs) {
-        float px = 0.0f, py = 0.0f;
-        const bool pushed = dist < 1e-6f;
-        if (pushed) {
-            ax = ax + 0.02f;
-            dist = vlen(ax, ay);
-            px = isA ? 0.01f : -0.01f;
-            py = isA ? 0.0f : -0.0f;
-        }
-        if (sensor(lj)) {
-            once(pushed, false);
-            if (pushed) put(lj, px, py);
-            return;
-        }
-        const float mpart = mass(lj);
-        const float mA = isA ? m : mpart, mB = isA ? mpart : m;
-        const float ratio = 1.0f - mA / (mA + mB);
-        const float nx = ax / dist, ny = ay / dist;
-        once(pushed, nx != nx || ny != ny);
-        const float delta = rs - dist;
-        float cx, cy;
-        if (isA) {
-            const float kk = ratio * delta;
-            cx = kk * nx;
-            cy = kk * ny;
-        } else {
-            const float kk = (1.0f - ratio) * delta;
-            cx = -(kk * nx);
-            cy = -(kk * ny);
-        }
-        if (pushed) {
-            cx = px + cx;
-            cy = py + cy;
-        }
-        put(lj, cx, cy);
     };
     L.init();
-    uint32_t found = 0;
-    enumerate([&](uint32_t lj, bool isA, float ax, float ay, float dist, float rs) {
-        ++found;
-        correction([&](uint32_t kk, float x, float y) { L.add(kk, x, y); },
-                   [&](bool pushed, bool nan) { hit(lj, isA, pushed, nan); }, lj, isA, ax, ay, dist, rs);
+    enumerate([&](uint32_t lj, const LdsContact& k) {
+        once(lj, k);
+        L.add(lj, k.c.x, k.c.y);
     });
-    if (L.n > 0) {
-        uint32_t last = L.apply(p);
-        uint32_t done = L.n < (uint32_t)K ? L.n : (uint32_t)K;
-        while (done < L.n) {  // more than K: next partner by selection, same order
-            uint32_t best = 0xFFFFFFFFu;
-            float bx = 0.0f, by = 0.0f;
-            enumerate([&](uint32_t lj, bool isA, float ax, float ay, float dist, float rs) {
-                correction(
-                    [&](uint32_t kk, float x, float y) {
-                        if (kk > last && kk < best) {
-                            best = kk;
-                            bx = x;
-                            by = y;
-                        }
-                    },
-                    [](bool, bool) {}, lj, isA, ax, ay, dist, rs);
-            });
-            if (best == 0xFFFFFFFFu) break;
-            p.x = p.x + bx;
-            p.y = p.y + by;
-            last = best;
-            ++done;
-        }
+    if (L.n == 0) return 0;
+    uint32_t last = L.apply(p);
+    for (uint32_t done = L.n < (uint32_t)K ? L.n : (uint32_t)K; done < L.n; ++done) {  // more than K: one at a time
+        uint32_t best = kNoPair;
+        float2 b = make_float2(0.0f, 0.0f);
+        enumerate([&](uint32_t lj, const LdsContact& k) {
+            if (lj > last && lj < best) {
+                best = lj;
+                b = k.c;
+            }
+        });
+        if (best == kNoPair) break;
+        p.x = p.x + b.x;
+        p.y = p.y + b.y;
+        last = best;
     }
-    return found;
+    return L.n;
 }
 
 }  // namespace bg
