@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "joint_schedule.hpp"
 #include "world.hpp"
 
 namespace bg {
@@ -146,7 +147,8 @@ void Rollout::release() {
     dfree(d_ck_p_), dfree(d_ck_q_), dfree(d_ck_v_), dfree(d_final_), dfree(d_loss_);
     dfree(d_tape_s_), dfree(d_tape_nbr_), dfree(d_lam_p_), dfree(d_lam_q_), dfree(d_dl_), dfree(d_gv_),
         dfree(d_gk_);
-    dfree(d_tape_v_), dfree(d_tape_pj_), dfree(d_j_axis_), dfree(d_lam_v_), dfree(d_jc_start_), dfree(d_j_ab_),
+    dfree(d_tape_v_), dfree(d_tape_axis_), dfree(d_lam_v_), dfree(d_jg_level_), dfree(d_jl_start_),
+        dfree(d_j_entry_), dfree(d_j_ab_),
         dfree(d_j_anchor_), dfree(d_j_mass_), dfree(d_j_dist_);
     if (stream_) (void)hipStreamDestroy(stream_);
     stream_ = nullptr;
@@ -167,7 +169,8 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
     std::vector<DiffWorld> ws(n);
     std::vector<float2> p0, q0, v0;
     std::vector<uint32_t> inc_count;
-    std::vector<uint32_t> jc_start(1, 0), j_ab;
+    JointSchedule sched;
+    std::vector<uint32_t> j_ab;
     std::vector<float4> j_anchor, j_mass;
     std::vector<float> j_dist;
     damped_ = false;
@@ -210,11 +213,12 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
         radius_.insert(radius_.end(), h.radius.begin(), h.radius.end());
         gmod_.insert(gmod_.end(), h.gmod.begin(), h.gmod.end());
         flags_.insert(flags_.end(), h.flags.begin(), h.flags.end());
-        // joints: connected components of the world's joint graph (union-find over bodies), each
-        // component's joints contiguous and in arena order; components touch disjoint bodies, so
-        // sweeping them concurrently is the reference's sequential sweep
-        d.jc0 = (uint32_t)jc_start.size() - 1;
-        d.njc = 0;
+        // joints, component by component, and the schedule of their solves: components share no
+        // body, so up to a wave's lanes of them make a group
+        d.jq0 = (uint32_t)j_ab.size();
+        d.jg0 = sched.groups();
+        d.jl0 = (uint32_t)sched.level_start.size() - 1;
+        d.je0 = (uint32_t)sched.entry.size();
         if (!h.ja.empty()) {
             std::vector<int32_t> uf(d.nb);
             for (uint32_t i = 0; i < d.nb; ++i) uf[i] = (int32_t)i;
@@ -236,21 +240,32 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
                 }
                 comps[comp_of_root[r]].push_back((uint32_t)q);
             }
-            for (const auto& cq : comps) {
-                for (uint32_t q : cq) {
+            std::vector<std::pair<uint32_t, uint32_t>> joints;
+            std::vector<uint32_t> ids, last(d.nb, 0);
+            for (size_t cc = 0; cc < comps.size(); ++cc) {
+                for (uint32_t q : comps[cc]) {
                     const float ma = h.mass[h.ja[q]], mb = h.mass[h.jb[q]];
                     const float inv_a = 1.0f / ma, inv_b = 1.0f / mb;  // physics.rs:450-455
                     const float ims = inv_a + inv_b;
                     const float ratio = inv_a / ims;
+                    joints.push_back({(uint32_t)h.ja[q], (uint32_t)h.jb[q]});
+                    ids.push_back((uint32_t)j_ab.size() - d.jq0);
                     j_ab.push_back((uint32_t)h.ja[q] | ((uint32_t)h.jb[q] << 16));
                     j_anchor.push_back(make_float4(h.jan_a[q].x, h.jan_a[q].y, h.jan_b[q].x, h.jan_b[q].y));
                     j_dist.push_back(h.jdist[q]);
                     j_mass.push_back(make_float4(ims, ratio, 1.0f - ratio, 1.0f));
                 }
-                jc_start.push_back((uint32_t)j_ab.size());
+                if (cc + 1 == comps.size() || (cc + 1) % BG_WAVE == 0) {
+                    sched.add_group(joints, ids, j_iters_, last, BG_WAVE);
+                    joints.clear();
+                    ids.clear();
+                }
             }
-            d.njc = (uint32_t)comps.size();
         }
+        d.njq = (uint32_t)j_ab.size() - d.jq0;
+        d.njg = sched.groups() - d.jg0;
+        d.njl = (uint32_t)sched.level_start.size() - 1 - d.jl0;
+        d.nje = (uint32_t)sched.entry.size() - d.je0;
         for (size_t s = 0; s < h.k.size(); ++s) {
             sa_.push_back((int32_t)d.b0 + h.sa[s]);
             sb_.push_back((int32_t)d.b0 + h.sb[s]);
@@ -263,6 +278,7 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
     nb_ = (uint32_t)mass_.size();
     ns_ = (uint32_t)k_.size();
     nj_ = (uint32_t)j_ab.size();
+    n_solves_ = (uint32_t)sched.entry.size();
     n_worlds_ = n;
     body0_.resize(n + 1);
     for (uint32_t w = 0; w < n; ++w) body0_[w] = ws[w].b0;
@@ -307,13 +323,16 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
     HIP_TRY(dalloc(&d_gv_, nb_));
     HIP_TRY(dalloc(&d_gk_, ns_));
     HIP_TRY(dalloc(&d_lam_v_, nb_));
-    HIP_TRY(dalloc(&d_jc_start_, jc_start.size()));
+    HIP_TRY(dalloc(&d_jg_level_, sched.group_level.size()));
+    HIP_TRY(dalloc(&d_jl_start_, sched.level_start.size()));
+    HIP_TRY(dalloc(&d_j_entry_, sched.entry.size()));
     HIP_TRY(dalloc(&d_j_ab_, nj_));
     HIP_TRY(dalloc(&d_j_anchor_, nj_));
     HIP_TRY(dalloc(&d_j_mass_, nj_));
     HIP_TRY(dalloc(&d_j_dist_, nj_));
-    HIP_TRY(dalloc(&d_j_axis_, (size_t)nj_ * (j_iters_ ? j_iters_ : 1)));
-    HIP_TRY(up(d_jc_start_, jc_start, s));
+    HIP_TRY(up(d_jg_level_, sched.group_level, s));
+    HIP_TRY(up(d_jl_start_, sched.level_start, s));
+    HIP_TRY(up(d_j_entry_, sched.entry, s));
     HIP_TRY(up(d_j_ab_, j_ab, s));
     HIP_TRY(up(d_j_anchor_, j_anchor, s));
     HIP_TRY(up(d_j_mass_, j_mass, s));
@@ -370,11 +389,11 @@ int Rollout::ensure_buffers(uint32_t n_steps) {
 int Rollout::ensure_tape(uint32_t subs) {
     if (subs <= tape_sub_alloc_) return BG_OK;
     tape_sub_alloc_ = 0;
-    dfree(d_tape_s_), dfree(d_tape_nbr_), dfree(d_tape_v_), dfree(d_tape_pj_);
+    dfree(d_tape_s_), dfree(d_tape_nbr_), dfree(d_tape_v_), dfree(d_tape_axis_);
     HIP_TRY(dalloc(&d_tape_s_, (size_t)subs * nb_));
     HIP_TRY(dalloc(&d_tape_nbr_, (size_t)subs * nb_ * kDiffTapeNbr));
     if (damped_) HIP_TRY(dalloc(&d_tape_v_, (size_t)subs * nb_));
-    if (nj_ > 0 && j_iters_ > 0) HIP_TRY(dalloc(&d_tape_pj_, (size_t)subs * nb_));
+    if (n_solves_ > 0) HIP_TRY(dalloc(&d_tape_axis_, (size_t)subs * n_solves_));
     tape_sub_alloc_ = subs;
     return BG_OK;
 }
@@ -385,8 +404,8 @@ int Rollout::ensure_tape(uint32_t subs) {
 uint32_t Rollout::recompute_segments() {
     const uint32_t n_seg = (n_steps_ + ck_every_ - 1) / ck_every_;
     const uint32_t seg_sub = segment_substeps(n_steps_);
-    const uint64_t per_sub = (uint64_t)nb_ * (sizeof(float2) * (1u + (d_tape_v_ ? 1u : 0u) + (d_tape_pj_ ? 1u : 0u)) +
-                                              sizeof(uint16_t) * kDiffTapeNbr);
+    const uint64_t per_sub = (uint64_t)nb_ * (sizeof(float2) * (1u + (d_tape_v_ ? 1u : 0u)) + sizeof(uint16_t) * kDiffTapeNbr) +
+                             (uint64_t)n_solves_ * sizeof(float2);
     uint64_t segs = std::min<uint64_t>(n_seg, cus_ / n_worlds_);
     if (per_sub > 0) segs = std::min<uint64_t>(segs, kTapeBytes / (per_sub * seg_sub));
     segs = std::max<uint64_t>(segs, 1);
@@ -416,13 +435,14 @@ DiffArgs Rollout::args() const {
     a.sp_c = d_c_;
     a.inc_start = d_inc_start_;
     a.inc_list = d_inc_list_;
-    a.jc_start = d_jc_start_;
+    a.jg_level = d_jg_level_;
+    a.jl_start = d_jl_start_;
+    a.j_entry = d_j_entry_;
     a.j_ab = d_j_ab_;
     a.j_anchor = d_j_anchor_;
     a.j_dist = d_j_dist_;
     a.j_mass = d_j_mass_;
-    a.n_joints = nj_;
-    a.j_iters = nj_ > 0 ? j_iters_ : 0u;
+    a.n_solves = n_solves_;
     a.ck_p = d_ck_p_;
     a.ck_q = d_ck_q_;
     a.ck_v = d_ck_v_;
@@ -431,8 +451,7 @@ DiffArgs Rollout::args() const {
     a.tape_s = d_tape_s_;
     a.tape_nbr = d_tape_nbr_;
     a.tape_v = d_tape_v_;
-    a.tape_pj = d_tape_pj_;
-    a.j_axis = d_j_axis_;
+    a.tape_axis = d_tape_axis_;
     a.lam_p = d_lam_p_;
     a.lam_q = d_lam_q_;
     a.lam_v = d_lam_v_;

@@ -36,7 +36,10 @@ struct DiffWorld {
     int32_t first_dyn;  // local index of the first non-static body, -1 if none
     float rmax;         // largest radius of the world
     float tx, ty;       // target point of the centroid loss
-    uint32_t jc0, njc;  // joint components [jc0, jc0 + njc) (their joints are contiguous)
+    uint32_t jq0, njq;  // joints [jq0, jq0 + njq)
+    uint32_t jg0, njg;  // groups of joints [jg0, jg0 + njg) (see JointSchedule)
+    uint32_t jl0, njl;  // their levels
+    uint32_t je0, nje;  // their solves
 };
 
 struct DiffArgs {
@@ -57,13 +60,16 @@ struct DiffArgs {
     const float* sp_c;
     const uint32_t* inc_start;  // per body: its springs in ascending index
     const uint32_t* inc_list;
-    // fixed joints, grouped by connected component (arena order inside one)
-    const uint32_t* jc_start;  // per component: first joint, n_components + 1 entries
+    // fixed joints: the schedule of their solves (entries are joints of their world), then
+    // per joint
+    const uint32_t* jg_level;
+    const uint32_t* jl_start;
+    const uint32_t* j_entry;
     const uint32_t* j_ab;      // local body a | local body b << 16
     const float4* j_anchor;    // anchor a (x, y), anchor b (z, w)
     const float* j_dist;
     const float4* j_mass;  // 1/m_a + 1/m_b, ratio, 1 - ratio, unused
-    uint32_t n_joints, j_iters;
+    uint32_t n_solves;         // of all worlds, per substep
     // checkpoints [n_ck][nb_total] of position, position_old, calculated_velocity
     float2* ck_p;
     float2* ck_q;
@@ -74,8 +80,7 @@ struct DiffArgs {
     float2* tape_s;
     uint16_t* tape_nbr;  // [..][nb_total][kDiffTapeNbr]
     float2* tape_v;      // calculated_velocity at the substep start (damped springs), else null
-    float2* tape_pj;     // positions entering the joint stage (joints), else null
-    float2* j_axis;      // [j_iters][n_joints]: anchor axes of the reverse pass's joint sweep
+    float2* tape_axis;   // [..][n_solves]: each solve's anchor axis (joints), else null
     // adjoint
     float2* lam_p;  // d loss / d position at a segment boundary
     float2* lam_q;  // d loss / d position_old
@@ -129,7 +134,7 @@ private:
 
     hipStream_t stream_ = nullptr;
     uint32_t n_worlds_ = 0, nb_ = 0, ns_ = 0, substeps_ = 8, ck_every_ = 20, n_steps_ = 0;
-    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, cus_ = 1, nj_ = 0, j_iters_ = 0;
+    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, cus_ = 1, nj_ = 0, n_solves_ = 0, j_iters_ = 0;
     float gx_ = 0.0f, gy_ = 0.0f, h_ = 0.0f;
     bool collisions_ = true, damped_ = false, have_forward_ = false;
     std::vector<uint8_t> nonfinite_;  // per world, after the last backward: a gradient entry is inf or NaN
@@ -148,8 +153,8 @@ private:
            *d_final_ = nullptr, *d_tape_s_ = nullptr, *d_lam_p_ = nullptr, *d_lam_q_ = nullptr, *d_dl_ = nullptr,
            *d_gv_ = nullptr;
     uint16_t* d_tape_nbr_ = nullptr;
-    float2 *d_tape_v_ = nullptr, *d_tape_pj_ = nullptr, *d_j_axis_ = nullptr, *d_lam_v_ = nullptr;
-    uint32_t *d_jc_start_ = nullptr, *d_j_ab_ = nullptr;
+    float2 *d_tape_v_ = nullptr, *d_tape_axis_ = nullptr, *d_lam_v_ = nullptr;
+    uint32_t *d_jg_level_ = nullptr, *d_jl_start_ = nullptr, *d_j_entry_ = nullptr, *d_j_ab_ = nullptr;
     float4 *d_j_anchor_ = nullptr, *d_j_mass_ = nullptr;
     float* d_j_dist_ = nullptr;
 };

@@ -38,19 +38,24 @@ constexpr uint32_t kScanItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThrea
 // Springs of a world whose terms are kept in LDS (32 KB of it); a world with more evaluates
 // them per body.
 constexpr uint32_t kDiffLdsSprings = 2048;
-constexpr uint32_t kDiffLdsJoints = 256;   // joints of a world whose records are staged in LDS
-constexpr uint32_t kDiffLdsAxes = 1024;    // solves of a world whose axes the reverse keeps in LDS
+// A world whose joint records and schedule are staged in LDS has at most so many joints,
+// solves a substep and levels of them.
+constexpr uint32_t kDiffLdsJoints = 256, kDiffLdsSolves = 1024, kDiffLdsLevels = 512;
 constexpr uint32_t kCntStride = kDiffCells + 4;  // (a multiple of 16 bytes)
 constexpr uint32_t kPairs = 1360;          // queued contact pairs of a substep: 12 bytes each of a cell table
+static_assert(kDiffLdsSolves <= kDiffThreads, "a thread stages one axis");
 static_assert(12 * kPairs <= 4 * kDiffCells, "the queue fits the idle cell table");
 constexpr uint32_t kInc = 4;               // springs of a body kept as packed registers
 
 struct JointRec {
-    float4 anchor;   // a (x, y), b (z, w)
-    float4 mass;     // 1/m_a + 1/m_b, ratio, 1 - ratio, unused
-    float dist;
-    uint32_t ab;     // local a | local b << 16
-    uint32_t statics;  // bit 0: a is static, bit 1: b is
+    float4 anchor;  // a (x, y), b (z, w)
+    float4 mass;    // 1/m_a + 1/m_b, ratio, 1 - ratio, distance
+    uint32_t ab;    // local a | a is static << 15 | local b << 16 | b is static << 31
+};
+struct JointStage {
+    float4 anchor[kDiffLdsJoints], mass[kDiffLdsJoints];
+    uint32_t ab[kDiffLdsJoints];
+    uint16_t entry[kDiffLdsSolves], level[kDiffLdsLevels + 1];
 };
 
 struct Ctx {
@@ -65,8 +70,8 @@ struct Ctx {
     uint32_t* pairs;   // queued pairs of this substep
     double* dred;      // [2][kWaves]
     LdsGrid* grid;
-    JointRec* joints;  // the world's joints, if at most kDiffLdsJoints
-    float2* axes;      // the reverse's axes, if at most kDiffLdsAxes
+    JointStage* joints;  // of a staged world
+    float2* axes;        // its solves' axes; reverse only
     float2* lam_pp;    // adjoint only (the memory of `force`)
     float2* lam_am;
 };
@@ -109,15 +114,74 @@ __device__ __forceinline__ uint32_t thread_index() {
 
 __device__ __forceinline__ bool lds_springs(const DiffWorld& W) { return W.ns <= kDiffLdsSprings; }
 
-__device__ __forceinline__ JointRec joint_load(const DiffArgs& a, const DiffWorld& W, uint32_t q) {
+__device__ __forceinline__ bool joints_staged(const DiffWorld& W) {
+    return W.njq <= kDiffLdsJoints && W.nje <= kDiffLdsSolves && W.njl <= kDiffLdsLevels;
+}
+
+// Joint q of the world: from LDS in a staged world, else from global memory.  (Templates:
+// where the two meet in one load it becomes a flat one.)
+template <bool STAGED>
+__device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArgs& a, const DiffWorld& W, uint32_t q) {
     JointRec r;
-    r.anchor = a.j_anchor[q];
-    r.mass = a.j_mass[q];
-    r.dist = a.j_dist[q];
-    r.ab = a.j_ab[q];
-    r.statics = ((a.flags[W.b0 + (r.ab & 0xFFFFu)] & BF_STATIC) ? 1u : 0u) |
-                ((a.flags[W.b0 + (r.ab >> 16)] & BF_STATIC) ? 2u : 0u);
+    if constexpr (STAGED) {
+        r.anchor = c.joints->anchor[q];
+        r.mass = c.joints->mass[q];
+        r.ab = c.joints->ab[q];
+    } else {
+        r.anchor = a.j_anchor[W.jq0 + q];
+        r.mass = a.j_mass[W.jq0 + q];
+        r.mass.w = a.j_dist[W.jq0 + q];
+        r.ab = a.j_ab[W.jq0 + q];
+        if (a.flags[W.b0 + (r.ab & 0x7FFFu)] & BF_STATIC) r.ab |= 1u << 15;
+        if (a.flags[W.b0 + ((r.ab >> 16) & 0x7FFFu)] & BF_STATIC) r.ab |= 1u << 31;
+    }
     return r;
+}
+static_assert(kDiffMaxBodies <= 0x7FFF, "15-bit body indices in JointRec::ab");
+
+// Runs the world's joint solves level by level, a wave a group: solve(e, record) for solve e
+// of the world.  REVERSE: from the last level to the first.  The next level's records load
+// while the current one works.
+template <bool STAGED, bool REVERSE, class Solve>
+__device__ __forceinline__ void joint_levels(const Ctx& c, const DiffArgs& a, const DiffWorld& W, Solve&& solve) {
+    const uint32_t lane = threadIdx.x & (BG_WAVE - 1);
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / BG_WAVE));
+    for (uint32_t grp = W.jg0 + wave; grp < W.jg0 + W.njg; grp += kWaves) {
+        const uint32_t l0 = a.jg_level[grp] - W.jl0, n = a.jg_level[grp + 1] - W.jl0 - l0;
+        uint32_t e, q;
+        JointRec r;
+        bool have;
+        auto load = [&](uint32_t k) {
+            const uint32_t l = l0 + (REVERSE ? n - 1u - k : k);
+            uint32_t end;
+            if constexpr (STAGED) {
+                e = c.joints->level[l] + lane;
+                end = c.joints->level[l + 1];
+            } else {
+                e = a.jl_start[W.jl0 + l] - W.je0 + lane;
+                end = a.jl_start[W.jl0 + l + 1] - W.je0;
+            }
+            have = e < end;
+            if (!have) return;
+            if constexpr (STAGED)
+                q = c.joints->entry[e];
+            else
+                q = a.j_entry[W.je0 + e];
+            r = joint_rec<STAGED>(c, a, W, q);
+        };
+        if (n > 0) load(0);
+        for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t e_now = e;
+            const JointRec r_now = r;
+            const bool have_now = have;
+            if (k + 1 < n) load(k + 1);
+            if (have_now) solve(e_now, r_now);
+            // the next level's lanes read what this one's wrote: one wave's LDS accesses keep
+            // their order, the compiler has to as well
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
 }
 
 __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, const float2* p,
@@ -159,11 +223,18 @@ __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, cons
         o.s_c = a.sp_c[s];
     }
     for (uint32_t i = threadIdx.x; i <= kDiffCells; i += kDiffThreads) c.cnt[i] = 0u;
-    const bool jointed = a.j_iters > 0 && W.njc > 0;
-    const uint32_t q0 = jointed ? a.jc_start[W.jc0] : 0u;
-    const uint32_t nj = jointed ? a.jc_start[W.jc0 + W.njc] - q0 : 0u;
-    if (nj <= kDiffLdsJoints)
-        for (uint32_t k = threadIdx.x; k < nj; k += kDiffThreads) c.joints[k] = joint_load(a, W, q0 + k);
+    if (W.njg > 0 && joints_staged(W)) {
+        for (uint32_t k = threadIdx.x; k < W.njq; k += kDiffThreads) {
+            const JointRec r = joint_rec<false>(c, a, W, k);
+            c.joints->anchor[k] = r.anchor;
+            c.joints->mass[k] = r.mass;
+            c.joints->ab[k] = r.ab;
+        }
+        for (uint32_t k = threadIdx.x; k < W.nje; k += kDiffThreads)
+            c.joints->entry[k] = (uint16_t)a.j_entry[W.je0 + k];
+        for (uint32_t k = threadIdx.x; k <= W.njl; k += kDiffThreads)
+            c.joints->level[k] = (uint16_t)(a.jl_start[W.jl0 + k] - W.je0);
+    }
 }
 
 // f(incidence) over body j's springs in ascending index; incidence as in Own::inc0.
@@ -215,88 +286,54 @@ __device__ __forceinline__ float2 spring_force(float2 pa, float2 pb, float2 va, 
     return make_float2(ux * (mag - dfx), uy * (mag - dfy));
 }
 
-// One joint: its record from LDS, or from global memory in a world with more than
-// kDiffLdsJoints of them.  (A template: where the two meet in one load it becomes a flat one.)
-template <bool STAGED>
-__device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArgs& a, const DiffWorld& W, uint32_t q, uint32_t q0) {
-    if constexpr (STAGED)
-        return c.joints[q - q0];
-    else
-        return joint_load(a, W, q);
-}
-
-struct JointRange {
-    uint32_t q0, nj;   // the world's joints
-    bool staged;  // records and axes in LDS
-};
-__device__ __forceinline__ JointRange joint_range(const DiffArgs& a, const DiffWorld& W) {
-    JointRange j;
-    j.q0 = a.jc_start[W.jc0];
-    j.nj = a.jc_start[W.jc0 + W.njc] - j.q0;
-    j.staged = j.nj <= kDiffLdsJoints && (uint64_t)j.nj * a.j_iters <= kDiffLdsAxes;
-    return j;
-}
-
-// Position sweep of one joint component (physics.rs:426-460) on the LDS
-// positions P, joint_iterations times in arena order.  With REC every solve's
-// anchor axis is kept: in LDS at axes[it * nj + q - q0], or in j_axis.
+// Position sweep of the world's joints (physics.rs:426-460) on the LDS positions P; with REC
+// every solve's anchor axis is recorded.
 template <bool REC, bool STAGED>
-__device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, uint32_t comp, const DiffArgs& a, const DiffWorld& W,
-                                            const JointRange& jr) {
-    const uint32_t c0 = a.jc_start[comp], c1 = a.jc_start[comp + 1];
+__device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, const DiffArgs& a, const DiffWorld& W, uint32_t slot) {
     uint32_t flags = 0;
-    for (uint32_t it = 0; it < a.j_iters; ++it)
-        for (uint32_t q = c0; q < c1; ++q) {
-            const JointRec r = joint_rec<STAGED>(c, a, W, q, jr.q0);
-            const uint32_t la = r.ab & 0xFFFFu, lb = r.ab >> 16;
-            float2 pa = P[la], pb = P[lb];
-            float dx, dy;
-            const bool moved =
-                joint_positions(pa, pb, make_float2(r.anchor.x, r.anchor.y), make_float2(r.anchor.z, r.anchor.w),
-                                r.dist, r.mass, (r.statics & 1u) != 0u, (r.statics & 2u) != 0u, dx, dy, flags);
-            if (REC) {
-                if constexpr (STAGED)
-                    c.axes[it * jr.nj + (q - jr.q0)] = make_float2(dx, dy);
-                else
-                    a.j_axis[(size_t)it * a.n_joints + q] = make_float2(dx, dy);
-            }
-            if (!moved) continue;
-            P[la] = pa;
-            P[lb] = pb;
-        }
+    joint_levels<STAGED, false>(c, a, W, [&](uint32_t e, const JointRec& r) {
+        const uint32_t la = r.ab & 0x7FFFu, lb = (r.ab >> 16) & 0x7FFFu;
+        float2 pa = P[la], pb = P[lb];
+        float dx, dy;
+        const bool moved =
+            joint_positions(pa, pb, make_float2(r.anchor.x, r.anchor.y), make_float2(r.anchor.z, r.anchor.w), r.mass.w,
+                            make_float4(r.mass.x, r.mass.y, r.mass.z, 1.0f), (r.ab & (1u << 15)) != 0u,
+                            (r.ab & (1u << 31)) != 0u, dx, dy, flags);
+        if (REC) a.tape_axis[(size_t)slot * a.n_solves + W.je0 + e] = make_float2(dx, dy);
+        if (!moved) return;
+        P[la] = pa;
+        P[lb] = pb;
+    });
 }
 
 // Adjoint of joint_sweep on the LDS position adjoints L, from the axes the
 // forward sweep recorded: last solve first.
 template <bool STAGED>
-__device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, uint32_t comp, const DiffArgs& a,
-                                                    const DiffWorld& W, const JointRange& jr) {
-    const uint32_t c0 = a.jc_start[comp], c1 = a.jc_start[comp + 1];
-    for (uint32_t it = a.j_iters; it-- > 0;)
-        for (uint32_t q = c1; q-- > c0;) {
-            float2 d;
-            if constexpr (STAGED)
-                d = c.axes[it * jr.nj + (q - jr.q0)];
-            else
-                d = a.j_axis[(size_t)it * a.n_joints + q];
-            const float dist = vlen(d.x, d.y);
-            if (dist < 1e-6f) continue;  // the reference skips the joint
-            const JointRec r = joint_rec<STAGED>(c, a, W, q, jr.q0);
-            const uint32_t la = r.ab & 0xFFFFu, lb = r.ab >> 16;
-            const bool sa = (r.statics & 1u) != 0u, sb = (r.statics & 2u) != 0u;
-            // weights (physics.rs:450-460): a static -> b moves by ims corr; b static -> a does;
-            // otherwise a by ratio corr and b by (1 - ratio) corr
-            const float wa = sa ? 0.0f : (sb ? r.mass.x : r.mass.y);
-            const float wb = sa ? r.mass.x : (sb ? 0.0f : r.mass.z);
-            const float2 la2 = L[la], lb2 = L[lb];
-            const float lcx = wa * la2.x - wb * lb2.x, lcy = wa * la2.y - wb * lb2.y;
-            const float nx = d.x / dist, ny = d.y / dist;
-            const float nm = nx * lcx + ny * lcy;
-            const float f = r.dist / dist;
-            const float ldx = lcx - f * (lcx - nx * nm), ldy = lcy - f * (lcy - ny * nm);
-            L[la] = make_float2(la2.x - ldx, la2.y - ldy);
-            L[lb] = make_float2(lb2.x + ldx, lb2.y + ldy);
-        }
+__device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, const DiffArgs& a, const DiffWorld& W,
+                                                    uint32_t slot) {
+    joint_levels<STAGED, true>(c, a, W, [&](uint32_t e, const JointRec& r) {
+        float2 d;
+        if constexpr (STAGED)
+            d = c.axes[e];
+        else
+            d = a.tape_axis[(size_t)slot * a.n_solves + W.je0 + e];
+        const float dist = vlen(d.x, d.y);
+        if (dist < 1e-6f) return;  // the reference skips the joint
+        const uint32_t la = r.ab & 0x7FFFu, lb = (r.ab >> 16) & 0x7FFFu;
+        const bool sa = (r.ab & (1u << 15)) != 0u, sb = (r.ab & (1u << 31)) != 0u;
+        // weights (physics.rs:450-460): a static -> b moves by ims corr; b static -> a does;
+        // otherwise a by ratio corr and b by (1 - ratio) corr
+        const float wa = sa ? 0.0f : (sb ? r.mass.x : r.mass.y);
+        const float wb = sa ? r.mass.x : (sb ? 0.0f : r.mass.z);
+        const float2 la2 = L[la], lb2 = L[lb];
+        const float lcx = wa * la2.x - wb * lb2.x, lcy = wa * la2.y - wb * lb2.y;
+        const float nx = d.x / dist, ny = d.y / dist;
+        const float nm = nx * lcx + ny * lcy;
+        const float f = r.mass.w / dist;
+        const float ldx = lcx - f * (lcx - nx * nm), ldy = lcy - f * (lcy - ny * nm);
+        L[la] = make_float2(la2.x - ldx, la2.y - ldy);
+        L[lb] = make_float2(lb2.x + ldx, lb2.y + ldy);
+    });
 }
 
 // update_objects of body j (physics.rs:326-358) from its position after the contact and joint
@@ -334,7 +371,7 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
                                                 uint32_t n, uint32_t slot) {
     const uint32_t tid = thread_index();
     const bool springs_lds = lds_springs(W);
-    const bool joints = a.j_iters > 0 && W.njc > 0;
+    const bool joints = W.njg > 0;
     const uint32_t per = per_thread(W);
     if (a.collisions && n % kFitEvery == 0) {
         LdsFit f;
@@ -484,7 +521,6 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         if (joints) {
             c.vel[li] = pn;
             c.xy[li] = ac;
-            if (REC) a.tape_pj[tape] = pn;
         } else {
             verlet(c, o, a, W, gsub, j, pn, ac);
         }
@@ -495,12 +531,10 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         for (uint32_t i = tid; i <= kDiffCells; i += kDiffThreads) other[i] = 0u;
     // fixed joints, positions (physics.rs:424-460), on the velocities' memory
     if (joints) {
-        const JointRange jr = joint_range(a, W);
-        for (uint32_t comp = W.jc0 + tid; comp < W.jc0 + W.njc; comp += kDiffThreads)
-            if (jr.staged)
-                joint_sweep<false, true>(c, c.vel, comp, a, W, jr);
-            else
-                joint_sweep<false, false>(c, c.vel, comp, a, W, jr);
+        if (joints_staged(W))
+            joint_sweep<REC, true>(c, c.vel, a, W, slot);
+        else
+            joint_sweep<REC, false>(c, c.vel, a, W, slot);
         __syncthreads();
         for (uint32_t j = 0; j < per; ++j) {
             const uint32_t li = tid + j * kDiffThreads;
@@ -513,10 +547,11 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
 // One tape slot of a thread's bodies (the contact partners are loaded by the substep itself,
 // which needs them late).
 struct Tape {
-    float2 s[2], v[2], pj[2];
+    float2 s[2], v[2];
+    float2 axis;  // of one of a staged world's solves
 };
 
-__device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const DiffWorld& W, uint32_t k, bool joints) {
+__device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const DiffWorld& W, uint32_t k) {
     const uint32_t tid = thread_index();
 #pragma unroll
     for (uint32_t j = 0; j < 2; ++j) {
@@ -525,8 +560,8 @@ __device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const Diff
         const size_t i = (size_t)k * a.nb_total + W.b0 + li;
         t.s[j] = a.tape_s[i];
         if (a.tape_v) t.v[j] = a.tape_v[i];
-        if (joints) t.pj[j] = a.tape_pj[i];
     }
+    if (joints_staged(W) && tid < W.nje) t.axis = a.tape_axis[(size_t)k * a.n_solves + W.je0 + tid];
 }
 
 // Terms of one spring's adjoint: d loss / d (p_b - p_a) (kx, ky), d loss /
@@ -575,13 +610,12 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
                                                 float2 (&lq)[2], float2 (&lv)[2], float2 (&gv)[2], float& gk) {
     const uint32_t tid = thread_index();
     const float h = a.h;
-    const bool joints = a.j_iters > 0 && W.njc > 0;
+    const bool joints = W.njg > 0;
     const bool springs_lds = lds_springs(W);
     const uint32_t per = per_thread(W);
-    // per spring (kx, ky) and, with damping, (rvx, rvy), and the joints' positions: the
-    // memory of the cell tables and of the forward's positions is free
+    // per spring (kx, ky) and, with damping, (rvx, rvy): the memory of a cell table and of the
+    // forward's positions is free
     float2* skx = reinterpret_cast<float2*>(c.cnt);
-    float2* jpos = reinterpret_cast<float2*>(c.cnt + kCntStride);
     float2* srv = c.xy;
     uint4 nbr[2];
 #pragma unroll
@@ -594,7 +628,6 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
         const float m = c.mass[li];
         c.rec[li] = make_float4(t.s[j].x, t.s[j].y, o.r[j], m);
         if (a.tape_v) c.vel[li] = t.v[j];
-        if (joints) jpos[li] = t.pj[j];  // positions entering the joint stage
         float2 lam_a = make_float2(0.0f, 0.0f), lpp, lqin = make_float2(0.0f, 0.0f);
         if (o.fl[j] & BF_STATIC) {  // p'' = p', q'' = p', v'' = 0
             lpp = make_float2(lp[j].x + lq[j].x, lp[j].y + lq[j].y);
@@ -616,21 +649,14 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
         c.lam_pp[li] = lpp;
         c.lam_am[li] = lam_a;
     }
-    if (more) load_tape(t, a, W, k - 1, joints);
+    if (joints && joints_staged(W) && tid < W.nje) c.axes[tid] = t.axis;
+    if (more) load_tape(t, a, W, k - 1);
     __syncthreads();
     if (joints) {
-        // replay each component's sweep from the recorded positions for its axes, then walk
-        // it backwards on the position adjoints
-        const JointRange jr = joint_range(a, W);
-        for (uint32_t comp = W.jc0 + tid; comp < W.jc0 + W.njc; comp += kDiffThreads) {
-            if (jr.staged) {
-                joint_sweep<true, true>(c, jpos, comp, a, W, jr);
-                joint_sweep_reverse<true>(c, c.lam_pp, comp, a, W, jr);
-            } else {
-                joint_sweep<true, false>(c, jpos, comp, a, W, jr);
-                joint_sweep_reverse<false>(c, c.lam_pp, comp, a, W, jr);
-            }
-        }
+        if (joints_staged(W))
+            joint_sweep_reverse<true>(c, c.lam_pp, a, W, k);
+        else
+            joint_sweep_reverse<false>(c, c.lam_pp, a, W, k);
         __syncthreads();
     }
     if (springs_lds && W.ns > 0) {
@@ -772,7 +798,7 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     __shared__ uint32_t s_pairs;                                     \
     __shared__ double s_dred[2 * kWaves];                            \
     __shared__ LdsGrid s_grid;                                       \
-    __shared__ JointRec s_joints[kDiffLdsJoints];                    \
+    __shared__ JointStage s_joints;                                  \
     static_assert(kDiffLdsSprings >= kDiffMaxBodies, "the adjoint vectors share the springs' memory"); \
     static_assert(kDiffCells / 2 >= kDiffLdsSprings, "spring adjoints share a cell table's memory");   \
     static_assert(kDiffMaxBodies >= kDiffLdsSprings, "and the positions'");                            \
@@ -789,7 +815,7 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     c.pairs = &s_pairs;                                              \
     c.dred = s_dred;                                                 \
     c.grid = &s_grid;                                                \
-    c.joints = s_joints;                                             \
+    c.joints = &s_joints;                                            \
     c.lam_pp = reinterpret_cast<float2*>(s_force);                   \
     c.lam_am = c.lam_pp + kDiffMaxBodies;
 
@@ -850,7 +876,7 @@ __global__ __launch_bounds__(kDiffThreads) void k_diff_recompute(DiffArgs a, uin
 __global__ __launch_bounds__(kDiffThreads) void k_diff_reverse(DiffArgs a, uint32_t seg, uint32_t tape0,
                                                                uint32_t first_sub, uint32_t nsub, uint32_t last) {
     BG_DIFF_SHARED
-    __shared__ float2 s_axes[kDiffLdsAxes];
+    __shared__ float2 s_axes[kDiffLdsSolves];
     c.axes = s_axes;
     const DiffWorld W = a.worlds[blockIdx.x];
     Own o;
@@ -877,7 +903,7 @@ __global__ __launch_bounds__(kDiffThreads) void k_diff_reverse(DiffArgs a, uint3
     const bool own_gk = lds_springs(W) && threadIdx.x < W.ns;
     float gk = own_gk ? a.grad_k[W.s0 + threadIdx.x] : 0.0f;
     Tape t;
-    if (nsub > 0) load_tape(t, a, W, tape0 + nsub - 1, a.j_iters > 0 && W.njc > 0);
+    if (nsub > 0) load_tape(t, a, W, tape0 + nsub - 1);
     for (uint32_t k = nsub; k-- > 0;)
         substep_reverse(c, o, a, W, first_sub + k, tape0 + k, k > 0, t, lp, lq, lv, gv, gk);
     if (own_gk) a.grad_k[W.s0 + threadIdx.x] = gk;
