@@ -197,7 +197,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         st = launch_steps(delta, chunk_steps * n_chunks);
         if (st) return st;
         advance_time(delta, chunk_steps * n_chunks);
-        host_stale_ = true;
+        host_behind();
         return check_and_process();
     }
     // the first chunk after an upload runs eagerly (user inputs are consumed once)
@@ -270,7 +270,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
     hipError_t e = hipStreamSynchronize(d.stream);
     release();
     if (e != hipSuccess && result == BG_OK) result = fail(BG_ERR_HIP, hipGetErrorString(e));
-    host_stale_ = true;
+    host_behind();
     if (result != BG_OK) return result;
     return check_and_process();
 }
@@ -339,7 +339,7 @@ int World::autotune(double delta, uint32_t steps_per_trial, float* cell_scale, f
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    host_stale_ = true;
+    host_behind();
     if (st) return st;
     if (!have) return fail(BG_ERR_HIP, "autotune: event timing failed");
     st = set_broadphase(best.cs, best.sk, best.iv);
@@ -365,7 +365,7 @@ int World::autotune(double delta, uint32_t steps_per_trial, float* cell_scale, f
         }
         (void)hipEventDestroy(p0);
         (void)hipEventDestroy(p1);
-        host_stale_ = true;
+        host_behind();
         if (st) return st;
         if (e != hipSuccess) return fail(BG_ERR_HIP, std::string("autotune: ") + hipGetErrorString(e));
         if (persist_ms > best_ms) {

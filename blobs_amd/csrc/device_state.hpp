@@ -236,6 +236,9 @@ struct DeviceWorld {
     // (default priority; forked from and joined to `stream` by events)
     hipStream_t p_stream = nullptr;
     hipEvent_t p_fork = nullptr, p_join = nullptr;
+    // state gathered for the host (sphere path; see World::export_state)
+    char *export_buf = nullptr;
+    size_t export_size = 0;
     // collision events (optional): buffer of event_cap records, count in accum
     DevEvent *events = nullptr;
     uint32_t event_cap = 0;
@@ -326,6 +329,14 @@ hipError_t launch_sphere_substep(DeviceWorld& d, const SubstepArgs& a, bool grou
 // Launcher (ordered_contacts.hip): the ordered replay after k_contacts (exits at once
 // when no pair of the substep's snapshot coincides).
 hipError_t launch_contacts_ordered(DeviceWorld& d, const SubstepArgs& a, bool groups, bool sensors);
+// Launchers (export_kernels.hip): state for the host in dense order.  Any output may be null;
+// the outputs are device memory or pinned host memory.
+struct ExportOut {
+    float2 *pos, *pos_old, *vel;
+    float *rot, *omega, *old_dt;
+    float2 *col_pos;
+};
+hipError_t launch_export(const DeviceWorld& d, bool sphere, uint32_t id_mask, const ExportOut& out);
 // fills n copies of v (graph-safe replacement of hipMemsetAsync)
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 

@@ -31,6 +31,11 @@ float col_inertia(const bg_collider& c) {
 // Steps a single-sphere world stays on the general path after a push-out.
 constexpr uint32_t kPushOutHold = 4;
 
+// Exports: state up to kExportDirect bytes is stored to pinned memory by the kernel;
+// more comes through pinned staging of two halves of at most kStageHalf bytes.
+constexpr size_t kExportDirect = 256 << 10;
+constexpr size_t kStageHalf = 4 << 20;
+
 template <class T>
 hipError_t dmalloc(T** p, size_t n) {
     *p = nullptr;
@@ -88,6 +93,9 @@ World::~World() {
     if (d_.stream) (void)hipStreamSynchronize(d_.stream);
     if (check_event_) (void)hipEventDestroy(check_event_);
     if (host_acc_) (void)hipHostFree(host_acc_);
+    if (stage_) (void)hipHostFree(stage_);
+    for (hipEvent_t e : stage_event_)
+        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : event_pool_) (void)hipEventDestroy(e);
     for (auto& v : pending_)
         for (auto& pr : v) {
@@ -386,7 +394,7 @@ int World::reset() {
 }
 
 int World::get_params(bg_params* p) {
-    if (host_stale_) {
+    if (host_stale_ && !old_dt_known_) {
         // old_dt lives on the device between steps
         if (d_.accum) {
             StepAccum acc;
@@ -449,6 +457,10 @@ int World::get_col(bg_handle h, bg_collider* out) {
 }
 
 int World::get_bodies(float* pos, float* pos_old, float* vel, float* rot, float* omega, bg_handle* handles) {
+    if (host_stale_ && d_.allocated) {
+        if (handles) std::copy(body_handle_of_dense_.begin(), body_handle_of_dense_.end(), handles);
+        return export_state(pos, pos_old, vel, rot, omega, nullptr);
+    }
     if (sync_host()) return BG_ERR_HIP;
     uint32_t k = 0;
     for (uint32_t s = 0; s < bodies_.capacity_slots(); ++s) {
@@ -475,6 +487,10 @@ int World::get_bodies(float* pos, float* pos_old, float* vel, float* rot, float*
 }
 
 int World::get_collider_positions(float* abs, uint32_t* count) {
+    if (host_stale_ && d_.allocated) {
+        if (count) *count = d_.nc;
+        return abs ? export_state(nullptr, nullptr, nullptr, nullptr, nullptr, abs) : BG_OK;
+    }
     if (sync_host()) return BG_ERR_HIP;
     uint32_t k = 0;
     for (uint32_t s = 0; s < colliders_.capacity_slots(); ++s) {
@@ -486,6 +502,105 @@ int World::get_collider_positions(float* abs, uint32_t* count) {
         ++k;
     }
     if (count) *count = k;
+    return BG_OK;
+}
+
+int World::ensure_staging(size_t bytes) {
+    const size_t half = std::min<size_t>(kStageHalf, (bytes + 4095) & ~(size_t)4095);
+    for (hipEvent_t& e : stage_event_)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (half <= stage_half_) return BG_OK;
+    if (stage_) (void)hipHostFree(stage_);
+    stage_ = nullptr;
+    stage_half_ = 0;
+    HIP_TRY(hipHostMalloc((void**)&stage_, 2 * half, hipHostMallocDefault));
+    stage_half_ = half;
+    return BG_OK;
+}
+
+// Device arrays to pageable host memory, a piece through one half of the staging while the
+// previous piece is copied out of the other.
+int World::copy_to_host(const CopyOut* c, uint32_t n) {
+    size_t most = 0;
+    for (uint32_t i = 0; i < n; ++i) most = std::max(most, c[i].bytes);
+    if (most == 0) return BG_OK;
+    if (int st = ensure_staging(most)) return st;
+    struct Piece {
+        char* dst = nullptr;
+        size_t bytes = 0;
+    } prev;
+    uint32_t k = 0;
+    auto finish = [&](const Piece& p, uint32_t half) -> int {
+        HIP_TRY(hipEventSynchronize(stage_event_[half]));
+        memcpy(p.dst, stage_ + half * stage_half_, p.bytes);
+        return BG_OK;
+    };
+    for (uint32_t i = 0; i < n; ++i)
+        for (size_t at = 0; at < c[i].bytes; at += stage_half_, ++k) {
+            Piece p;
+            p.dst = (char*)c[i].dst + at;
+            p.bytes = std::min(stage_half_, c[i].bytes - at);
+            HIP_TRY(hipMemcpyAsync(stage_ + (k & 1u) * stage_half_, (const char*)c[i].src + at, p.bytes,
+                                   hipMemcpyDeviceToHost, d_.stream));
+            HIP_TRY(hipEventRecord(stage_event_[k & 1u], d_.stream));
+            if (prev.dst)
+                if (int st = finish(prev, (k & 1u) ^ 1u)) return st;
+            prev = p;
+        }
+    return finish(prev, (k & 1u) ^ 1u);
+}
+
+// The state the caller asked for (null: not wanted), in dense order, from the device.  A small
+// world's kernel stores straight into pinned memory; a large one's gathers into device memory
+// (the general path's arrays are in dense order already), which then comes over in pieces.
+int World::export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos) {
+    DeviceWorld& d = d_;
+    const bool sphere = path_ == StepPath::Sphere;
+    const uint32_t id_mask = snap_flags_ ? kSnapIdMask : ~kSnapOutlier;
+    const uint32_t n_old = sphere ? d.n_worlds : 1u;
+    std::vector<float> old_dt(n_old);
+    enum { kPos, kPosOld, kVel, kRot, kOmega, kOldDt, kCol, kParts };
+    void* dst[kParts] = {pos, pos_old, vel, rot, omega, old_dt.data(), col_pos};
+    const size_t size[kParts] = {8ull * d.nb, 8ull * d.nb, 8ull * d.nb, 4ull * d.nb, 4ull * d.nb, 4ull * n_old, 8ull * d.nc};
+    size_t at[kParts], total = 0;
+    for (int i = 0; i < kParts; ++i) {
+        at[i] = total;
+        if (dst[i]) total += (size[i] + 15) & ~(size_t)15;
+    }
+    auto outputs = [&](char* base) {
+        auto f2 = [&](int i) { return dst[i] ? (float2*)(base + at[i]) : nullptr; };
+        auto f1 = [&](int i) { return dst[i] ? (float*)(base + at[i]) : nullptr; };
+        return ExportOut{f2(kPos), f2(kPosOld), f2(kVel), f1(kRot), f1(kOmega), f1(kOldDt), f2(kCol)};
+    };
+    if (total <= kExportDirect) {
+        if (int st = ensure_staging(total)) return st;
+        HIP_TRY(launch_export(d, sphere, id_mask, outputs(stage_)));
+        HIP_TRY(hipStreamSynchronize(d.stream));
+        for (int i = 0; i < kParts; ++i)
+            if (dst[i]) memcpy(dst[i], stage_ + at[i], size[i]);
+    } else {
+        const void* src[kParts] = {d.b.pos, d.b.pos_old, d.b.vel, d.b.rot, d.b.omega, &d.accum->old_dt, d.c.abs};
+        if (sphere) {
+            if (total > d.export_size) {
+                dfree(d.export_buf);
+                d.export_size = 0;
+                HIP_TRY(dmalloc(&d.export_buf, total));
+                d.export_size = total;
+            }
+            HIP_TRY(launch_export(d, sphere, id_mask, outputs(d.export_buf)));
+            for (int i = 0; i < kParts; ++i) src[i] = d.export_buf + at[i];
+        }
+        CopyOut c[kParts];
+        uint32_t n = 0;
+        for (int i = 0; i < kParts; ++i)
+            if (dst[i]) c[n++] = {dst[i], src[i], size[i]};
+        if (int st = copy_to_host(c, n)) return st;
+    }
+    if (sphere && !batch_start_.empty())
+        batch_old_dt_ = old_dt;
+    else
+        params_.old_dt = old_dt[0];
+    old_dt_known_ = true;
     return BG_OK;
 }
 
@@ -709,6 +824,7 @@ void World::free_arrays() {
     dfree(d.jc_start), dfree(d.jc_list), dfree(d.jb_start), dfree(d.jb_list), dfree(d.j_local), dfree(d.jq_anchor), dfree(d.jq_mass), dfree(d.jq_len), dfree(d.con_pos),
         dfree(d.con_r);
     dfree(d.keys), dfree(d.vals), dfree(d.keys_tmp), dfree(d.vals_tmp), dfree(d.cell_start), dfree(d.crec);
+    dfree(d.export_buf);
     dfree(d.grid), dfree(d.accum), dfree(d.block_contacts), dfree(d.events), dfree(d.vel_next);
     dfree(d.ord_rows), dfree(d.ord_n), dfree(d.ord_mark), dfree(d.pos_pre), dfree(d.mv_key), dfree(d.mv_abs);
     dfree(d.mv_list), dfree(d.ord_heap), dfree(d.ord_log), dfree(d.aff_list), dfree(d.aff_mark), dfree(d.ord_cand);
@@ -785,6 +901,7 @@ int World::upload() {
     // dense maps
     const uint32_t nb = bodies_.len(), nc = colliders_.len();
     body_slot_of_dense_.clear();
+    body_handle_of_dense_.clear();
     col_slot_of_dense_.clear();
     body_dense_of_slot_.assign(bodies_.capacity_slots(), -1);
     col_dense_of_slot_.assign(colliders_.capacity_slots(), -1);
@@ -792,6 +909,7 @@ int World::upload() {
         if (bodies_.occupied(s)) {
             body_dense_of_slot_[s] = (int32_t)body_slot_of_dense_.size();
             body_slot_of_dense_.push_back(s);
+            body_handle_of_dense_.push_back(bodies_.handle_at(s));
         }
     for (uint32_t s = 0; s < colliders_.capacity_slots(); ++s)
         if (colliders_.occupied(s)) {
@@ -1840,7 +1958,7 @@ int World::step(double delta, uint32_t n) {
     st = launch_steps(delta, n);
     if (st) return st;
     advance_time(delta, n);
-    host_stale_ = true;
+    host_behind();
     if (deferred_checks_) {
         // wait for the previous record before its pinned buffer is reused
         st = finish_deferred_check(true);

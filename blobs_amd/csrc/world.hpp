@@ -127,6 +127,20 @@ private:
     int upload();
     int download();
     int sync_host() { return host_stale_ ? download() : BG_OK; }
+    // the device has run ahead of the host mirror
+    void host_behind() {
+        host_stale_ = true;
+        old_dt_known_ = false;
+    }
+    // device arrays for the caller, without touching the host mirror
+    struct CopyOut {
+        void* dst;
+        const void* src;
+        size_t bytes;
+    };
+    int ensure_staging(size_t bytes);
+    int copy_to_host(const CopyOut* c, uint32_t n);
+    int export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos);
     void mark_dirty() { dev_dirty_ = true; }
     int rebuild();
     int run_substep(float h, bool fresh, bool last);
@@ -167,6 +181,13 @@ private:
     StepPath path_ = StepPath::None;
     bool dev_dirty_ = true;
     bool host_stale_ = false;
+    bool old_dt_known_ = false;  // host_stale_, but an export brought the worlds' old_dt
+    // pinned staging of exports: two halves of stage_half_ bytes (allocated by the first
+    // export, at most 2 x kStageHalf), an event each
+    char* stage_ = nullptr;
+    size_t stage_half_ = 0;
+    hipEvent_t stage_event_[2] = {nullptr, nullptr};
+    std::vector<bg_handle> body_handle_of_dense_;
     bool stepped_since_upload_ = false;
     bool fresh_ = true;
     bool need_rebuild_ = true;

@@ -585,12 +585,12 @@ class Physics:
     def bodies(self) -> dict:
         """Body state in arena order as numpy arrays."""
         n = self.rbd_count()
-        pos = np.zeros((n, 2), np.float32)
-        pos_old = np.zeros((n, 2), np.float32)
-        vel = np.zeros((n, 2), np.float32)
-        rot = np.zeros(n, np.float32)
-        om = np.zeros(n, np.float32)
-        hs = np.zeros(n, np.uint64)
+        pos = np.empty((n, 2), np.float32)
+        pos_old = np.empty((n, 2), np.float32)
+        vel = np.empty((n, 2), np.float32)
+        rot = np.empty(n, np.float32)
+        om = np.empty(n, np.float32)
+        hs = np.empty(n, np.uint64)
         self._chk(self._lib.bg_get_bodies(self._w, L.fptr(pos), L.fptr(pos_old), L.fptr(vel), L.fptr(rot),
                                           L.fptr(om), L.hptr(hs)))
         return {"position": pos, "position_old": pos_old, "velocity": vel, "rotation": rot,
@@ -599,7 +599,7 @@ class Physics:
     def collider_positions(self) -> np.ndarray:
         n = C.c_uint32()
         self._chk(self._lib.bg_get_collider_positions(self._w, None, C.byref(n)))
-        out = np.zeros((n.value, 2), np.float32)
+        out = np.empty((n.value, 2), np.float32)
         self._chk(self._lib.bg_get_collider_positions(self._w, L.fptr(out), C.byref(n)))
         return out
 
