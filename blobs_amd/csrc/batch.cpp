@@ -183,10 +183,10 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         s.p[6] = p_src_.pp;  // the persistent launch reads its worlds from here
         s.p[7] = p_src_.snap;
         s.u[0] = bbox_parity_;
-        s.u[1] = steps_since_rebuild_;
+        s.u[1] = 0;
         s.u[2] = (need_rebuild_ ? 1u : 0u) | (d.gather_pending ? 2u : 0u) | (fresh_ ? 4u : 0u);
         s.u[3] = sub_since_rebuild_;
-        s.u[4] = rebuild_interval_;
+        s.u[4] = interval_substeps();
         return s;
     };
     const bool prof = profiling_;
@@ -198,7 +198,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         if (st) return st;
         advance_time(delta, chunk_steps * n_chunks);
         host_behind();
-        return check_and_process();
+        return check_and_process(chunk_steps * n_chunks);
     }
     // the first chunk after an upload runs eagerly (user inputs are consumed once)
     if (fresh_) {
@@ -272,7 +272,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
     if (e != hipSuccess && result == BG_OK) result = fail(BG_ERR_HIP, hipGetErrorString(e));
     host_behind();
     if (result != BG_OK) return result;
-    return check_and_process();
+    return check_and_process(chunk_steps * n_chunks);
 }
 
 int World::set_persistent(bool enable) {
@@ -376,7 +376,7 @@ int World::autotune(double delta, uint32_t steps_per_trial, float* cell_scale, f
     if (cell_scale) *cell_scale = best.cs;
     if (skin) *skin = best.sk;
     if (interval) *interval = best.iv;
-    return check_and_process();
+    return check_and_process(0);
 }
 
 }  // namespace bg

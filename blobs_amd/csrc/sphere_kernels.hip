@@ -828,6 +828,7 @@ __global__ __launch_bounds__(BG_WAVE) void k_world_grids(uint32_t n_worlds, uint
     const uint32_t lane = threadIdx.x;
     if (w == 0 && lane == 0) {
         accum->dmax = 0u;
+        accum->last_outliers = accum->n_outliers;
         accum->n_outliers = 0u;
     }
     if (w >= n_worlds) return;

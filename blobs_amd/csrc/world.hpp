@@ -151,11 +151,11 @@ private:
     void advance_time(double delta, uint32_t n);
     bool sphere_eligible() const;
     void dense_slots(std::vector<uint32_t>& bodies, std::vector<uint32_t>& cols) const;
-    int check_errors(uint32_t* flags_out = nullptr);
+    int check_errors(uint32_t* flags_out, uint32_t n_steps);
     int process_flags(uint32_t flags);
-    int check_and_process() {
+    int check_and_process(uint32_t n_steps) {
         uint32_t f = 0;
-        int st = check_errors(&f);
+        int st = check_errors(&f, n_steps);
         return st ? st : process_flags(f);
     }
     int finish_deferred_check(bool wait);
@@ -194,7 +194,6 @@ private:
     // general path: the rebuild's key pass waits for the substep's first launch
     bool keys_pending_ = false;
     KeysArgs keys_{};
-    uint32_t steps_since_rebuild_ = 0;
     uint32_t bbox_parity_ = 0;
     // broadphase settings until bg_set_broadphase: measured defaults (the small plain scene
     // steps 2.6x faster than with a skin of half a cell; large worlds gain from rebuilding
@@ -203,7 +202,11 @@ private:
     float skin_scale_ = 0.25f;  // outlier skin as a fraction of the cell size
     float skin_ = 0.0f;
     uint32_t sub_since_rebuild_ = 0;
-    uint32_t rebuild_interval_ = 0;  // 0: every step below 65,536 bodies, every third step from there
+    uint32_t rebuild_interval_ = 0;  // in steps; 0: adapted to the outliers (adapt_interval)
+    uint32_t interval_level_ = kLevelUnset, interval_calm_ = 0, interval_backoff_ = 0;
+    static constexpr uint32_t kLevelUnset = 0xFFu, kLevels = 5;
+    uint32_t interval_substeps();
+    void adapt_interval(const StepAccum& acc, uint32_t n_steps);
     // world properties fixed at upload
     float rmax_ = 0.0f;
     float mass_per_r_ = 0.0f;  // sphere path: every body's mass is exactly this times its radius (0: not so)
@@ -220,6 +223,7 @@ private:
     // deferred checks: the step record's flags arrive in pinned host memory
     bool deferred_checks_ = false, check_pending_ = false;
     StepAccum* host_acc_ = nullptr;
+    uint32_t check_steps_ = 0;  // steps the pending check covers
     hipEvent_t check_event_ = nullptr;
     uint64_t pairwise_push_out_steps_ = 0;  // fused-path steps that resolved push-outs pair by pair
     // dense <-> slot maps of the last upload
