@@ -191,9 +191,10 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
     };
     const bool prof = profiling_;
     uint32_t done = 0;
-    if (event_cap_ > 0) {
-        // events are stamped with the substep index the host passes: a replayed graph would
-        // repeat the stamps, so a world that records events runs its chunks eagerly
+    if (event_cap_ > 0 || small_active()) {
+        // Events are stamped with the substep index the host passes: a replayed graph would
+        // repeat the stamps, so a world that records events runs its chunks eagerly.  So do
+        // small worlds, whose chunks are a launch or two.
         st = launch_steps(delta, chunk_steps * n_chunks);
         if (st) return st;
         advance_time(delta, chunk_steps * n_chunks);

@@ -110,6 +110,13 @@ constexpr uint32_t kPersistClassThreads[kPersistClasses] = {1024};
 constexpr uint32_t kLdsBodies = kPersistPer * 1024;
 constexpr uint32_t kPersistMinBodies = 1025;
 
+// Worlds of at most kSmallBodies single centred spheres: every substep of a launch by one
+// workgroup a world (small_kernels.hip).
+constexpr uint32_t kSmallClasses = 4;
+constexpr uint32_t kSmallClassThreads[kSmallClasses] = {1024, 1024, 512, 256};
+constexpr uint32_t kSmallClassBodies[kSmallClasses] = {2048, 1024, 512, 256};
+constexpr uint32_t kSmallBodies = kSmallClassBodies[0];
+
 struct DeviceWorld {
     uint32_t nb = 0, nc = 0, ns = 0, nj = 0, nk = 0;
     uint32_t cells_cap = 0;
@@ -232,6 +239,9 @@ struct DeviceWorld {
     uint32_t p_class_start[kPersistClasses + 1] = {};
     uint32_t p_groups[kPersistClasses] = {};
     uint32_t p_grid_worlds = 0;  // worlds left to the grid path
+    // small worlds (small_kernels.hip): slot ranges [n_worlds + 1], then the worlds by class [n_worlds]
+    uint32_t *small_worlds = nullptr;
+    uint32_t small_class_start[kSmallClasses + 1] = {};
     // the persistent launch runs on its own stream beside the grid path's substeps
     // (default priority; forked from and joined to `stream` by events)
     hipStream_t p_stream = nullptr;
@@ -273,6 +283,27 @@ struct PersistArgs {
 };
 
 hipError_t launch_batch_persistent(const PersistArgs& k, hipStream_t s);
+
+struct SmallArgs {
+    SphereArrays s;          // read and written in place
+    const uint32_t* wstart;  // [n_worlds + 1] slot range of each world
+    const uint32_t* order;   // worlds by class
+    uint32_t class_start[kSmallClasses + 1];
+    float* wold_dt;
+    StepAccum* accum;
+    unsigned long long* block_contacts;
+    const float2* con_pos;
+    const float* con_r;
+    uint32_t nk;
+    DevEvent* events;  // null: no event recording
+    uint32_t event_cap;
+    float2* vel_scratch;  // with events: the velocities between substeps, where LDS has no room for them
+    float h, ratio_rest, gx, gy;
+    uint32_t nsub, fresh, collisions;
+    uint32_t sub_global;  // substeps since the world was created, before this launch
+    uint32_t snap_flags;  // snapshot words carry the body flags
+};
+hipError_t launch_small_step(const SmallArgs& k, hipStream_t s);
 
 // Scalars of one substep launch.
 struct SubstepArgs {

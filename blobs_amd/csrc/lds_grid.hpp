@@ -88,14 +88,15 @@ struct LdsGrid {
     float ox, oy, inv_cell;
     int32_t nx, ny;
     uint32_t ncells;
+    float ex, ey;  // mean of the extra vectors
 };
 
-// Sums of one thread's points for the fit.
+// Sums of one thread's points for the fit, and of an extra vector of some of them.
 struct LdsFit {
-    float n, sx, sy, sxx, syy;
+    float n, sx, sy, sxx, syy, ne, ex, ey;
     uint32_t b0, b1, b2, b3;  // f2ord bounding box
     __device__ __forceinline__ void init() {
-        n = sx = sy = sxx = syy = 0.0f;
+        n = sx = sy = sxx = syy = ne = ex = ey = 0.0f;
         b0 = b1 = 0xFFFFFFFFu;
         b2 = b3 = 0u;
     }
@@ -111,8 +112,14 @@ struct LdsFit {
         b2 = max(b2, f2ord(x));
         b3 = max(b3, f2ord(y));
     }
+    __device__ __forceinline__ void extra(float x, float y) {
+        if (!finitef(x) || !finitef(y)) return;
+        ne += 1.0f;
+        ex += x;
+        ey += y;
+    }
 };
-constexpr uint32_t kFitWords = 9;
+constexpr uint32_t kFitWords = 12;
 
 // Fits `grid` to the workgroup's points: cells of side `cell` over their
 // bounding box, clipped to the centroid +- 3 sigma so that a few bodies thrown
@@ -125,14 +132,15 @@ __device__ __forceinline__ void lds_fit(const LdsFit& f, float cell, uint32_t ce
     const uint32_t lane = threadIdx.x & (BG_WAVE - 1), wid = threadIdx.x / BG_WAVE;
     auto fold = [](uint32_t (&v)[kFitWords]) {
 #pragma unroll
-        for (int q = 0; q < 5; ++q) v[q] = wave_prefix(v[q], 0u, AddF32());
-        v[5] = wave_prefix(v[5], 0xFFFFFFFFu, MinU32());
-        v[6] = wave_prefix(v[6], 0xFFFFFFFFu, MinU32());
-        v[7] = wave_prefix(v[7], 0u, MaxU32());
-        v[8] = wave_prefix(v[8], 0u, MaxU32());
+        for (int q = 0; q < 8; ++q) v[q] = wave_prefix(v[q], 0u, AddF32());
+        v[8] = wave_prefix(v[8], 0xFFFFFFFFu, MinU32());
+        v[9] = wave_prefix(v[9], 0xFFFFFFFFu, MinU32());
+        v[10] = wave_prefix(v[10], 0u, MaxU32());
+        v[11] = wave_prefix(v[11], 0u, MaxU32());
     };
     uint32_t v[kFitWords] = {__float_as_uint(f.n),   __float_as_uint(f.sx), __float_as_uint(f.sy),
-                             __float_as_uint(f.sxx), __float_as_uint(f.syy), f.b0, f.b1, f.b2, f.b3};
+                             __float_as_uint(f.sxx), __float_as_uint(f.syy), __float_as_uint(f.ne),
+                             __float_as_uint(f.ex),  __float_as_uint(f.ey),  f.b0, f.b1, f.b2, f.b3};
     fold(v);
     if (lane == BG_WAVE - 1) {
 #pragma unroll
@@ -141,17 +149,17 @@ __device__ __forceinline__ void lds_fit(const LdsFit& f, float cell, uint32_t ce
     __syncthreads();
     if (wid == 0) {
 #pragma unroll
-        for (uint32_t q = 0; q < kFitWords; ++q) v[q] = lane < kNW ? red[q * kNW + lane] : (q < 5 || q > 6 ? 0u : 0xFFFFFFFFu);
+        for (uint32_t q = 0; q < kFitWords; ++q) v[q] = lane < kNW ? red[q * kNW + lane] : (q < 8 || q > 9 ? 0u : 0xFFFFFFFFu);
         fold(v);
         if (lane == BG_WAVE - 1) {
             const float n = __uint_as_float(v[0]);
             float minx = 0.0f, miny = 0.0f, maxx = 0.0f, maxy = 0.0f;
             if (!(cell > 0.0f) || !finitef(cell)) cell = 1.0f;
             if (n > 0.0f) {
-                minx = ord2f(v[5]);
-                miny = ord2f(v[6]);
-                maxx = ord2f(v[7]);
-                maxy = ord2f(v[8]);
+                minx = ord2f(v[8]);
+                miny = ord2f(v[9]);
+                maxx = ord2f(v[10]);
+                maxy = ord2f(v[11]);
                 const float mx = __uint_as_float(v[1]) / n, my = __uint_as_float(v[2]) / n;
                 const float dx = 3.0f * sqrtf(fmaxf(__uint_as_float(v[3]) / n - mx * mx, 0.0f)) + cell;
                 const float dy = 3.0f * sqrtf(fmaxf(__uint_as_float(v[4]) / n - my * my, 0.0f)) + cell;
@@ -182,6 +190,9 @@ __device__ __forceinline__ void lds_fit(const LdsFit& f, float cell, uint32_t ce
             grid->nx = nx;
             grid->ny = ny;
             grid->ncells = (uint32_t)nx * (uint32_t)ny;
+            const float ne = __uint_as_float(v[5]);
+            grid->ex = ne > 0.0f ? __uint_as_float(v[6]) / ne : 0.0f;
+            grid->ey = ne > 0.0f ? __uint_as_float(v[7]) / ne : 0.0f;
         }
     }
     __syncthreads();
@@ -197,6 +208,8 @@ __device__ __forceinline__ LdsGrid lds_grid_uniform(const LdsGrid& g) {
     u.nx = __builtin_amdgcn_readfirstlane(g.nx);
     u.ny = __builtin_amdgcn_readfirstlane(g.ny);
     u.ncells = (uint32_t)__builtin_amdgcn_readfirstlane((int)g.ncells);
+    u.ex = f(g.ex);
+    u.ey = f(g.ey);
     return u;
 }
 
@@ -243,68 +256,15 @@ struct LdsPairs {
     bool direct;
 };
 
-// Mark phase of one body a lane (`active`: the lane has one, with a finite snapshot xy),
-// called by whole waves.  rec[] = (x, y, radius, bits(local index)) in cell order, with
-// kLdsRecPad records of room behind them, `own` the body's own record.  *count was zero before the phase; entries from CAP on are not written.
-template <uint32_t CAP>
-__device__ __forceinline__ LdsPairs lds_mark(const LdsGrid& g, const uint32_t* start, const float4* rec, bool active,
-                                             float2 xy, float r, uint32_t own, float rmax, uint32_t* entries,
-                                             uint32_t* count) {
-    // The records of the cells as one flat list: index i is record base + i, plus step1 from
-    // end0 on (the second row), plus step2 from end1 on (all modulo 2^32).  (Sums, because a
-    // select between two variables here is compiled to a load through a selected address.)
-    uint32_t end0 = 0, end1 = 0, base = 0, step1 = 0, step2 = 0, n = 0;
-    bool flat = false;
-    if (active) {
-        const LdsRect c = lds_rect(g, xy.x, xy.y, r + rmax);
-        const uint32_t nx = (uint32_t)g.nx;
-        const uint32_t row0 = __umul24((uint32_t)c.cy0, nx), last = __umul24((uint32_t)c.cy1, nx);
-        const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
-        const uint32_t* s0 = start + c.cx0;
-        const uint32_t* s1 = start + c.cx1 + 1;
-        const uint32_t lo0 = s0[row0], hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
-        const int32_t rows = c.cy1 - c.cy0 + 1;
-        base = lo0;
-        end0 = hi0 - lo0;
-        step1 = lo1 - hi0;
-        end1 = end0 + (rows > 1 ? hi1 - lo1 : 0u);
-        step2 = (lo2 - end1) - (lo1 - end0);
-        n = end1 + (rows > 2 ? hi2 - lo2 : 0u);
-        flat = rows <= kLdsRows && n <= kLdsFlat;
-        if (!flat) n = 0;
-    }
-    static_assert(kLdsRows == 3, "the rows above");
-    auto slot = [&](uint32_t i) {
-        return (i >= end0 ? step1 : 0u) + (i >= end1 ? step2 : 0u) + (base + i);
-    };
-    uint32_t near_lo = 0, near_hi = 0;
-    // four candidates; past the last one it reads up to three records further (rec has room
-    // for that), whose bits are dropped below
-    auto mark = [&](uint32_t f) -> uint32_t {
-        float4 sb[4];
-        uint32_t t[4];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            t[u] = slot(f + u);
-            sb[u] = rec[t[u]];
-        }
-        uint32_t bits = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const float dx = xy.x - sb[u].x, dy = xy.y - sb[u].y;
-            const float rs = r + sb[u].z;
-            const bool far = dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f;
-            bits |= ((t[u] == own) | far) ? 0u : 1u << u;
-        }
-        return bits;
-    };
-    for (uint32_t f = 0; f < min(n, 32u); f += 4) near_lo |= mark(f) << f;
-    for (uint32_t f = 32; f < n; f += 4) near_hi |= mark(f) << (f - 32u);
-    if (n < 32u) near_lo &= (1u << n) - 1u;
-    if (n < 64u) near_hi &= n > 32u ? (1u << (n - 32u)) - 1u : 0u;
+// Queue a body's marked candidates (bit i: other(i)), a body a lane, by whole waves.  *count
+// was zero before the phase; entries from CAP on are not written, and a body that has some
+// there is left to the caller.
+template <uint32_t CAP, class Other>
+__device__ __forceinline__ LdsPairs lds_queue(uint64_t marked, uint32_t own, uint32_t* entries, uint32_t* count,
+                                              Other&& other) {
     LdsPairs pr;
-    pr.n = (uint32_t)(__popc(near_lo) + __popc(near_hi));
-    pr.direct = active && !flat;
+    pr.n = (uint32_t)__popcll(marked);
+    pr.direct = false;
     const uint32_t incl = wave_prefix(pr.n, 0u, AddU32());
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, BG_WAVE - 1);
     uint32_t at = 0;
@@ -314,16 +274,93 @@ __device__ __forceinline__ LdsPairs lds_mark(const LdsGrid& g, const uint32_t* s
     }
     pr.first = at + incl - pr.n;
     const bool fits = pr.first + pr.n <= CAP;
-    uint64_t m = ((uint64_t)near_hi << 32) | near_lo;
-    for (uint32_t e = pr.first; m != 0; ++e) {
-        const uint32_t i = (uint32_t)__builtin_ctzll(m);
-        m &= m - 1;
-        if (e < CAP) entries[e] = fits ? (own << 16) | slot(i) : kNoPair;
+    for (uint32_t e = pr.first; marked != 0; ++e) {
+        const uint32_t i = (uint32_t)__builtin_ctzll(marked);
+        marked &= marked - 1;
+        if (e < CAP) entries[e] = fits ? (own << 16) | other(i) : kNoPair;
     }
     if (!fits) {
         pr.direct = true;
         pr.n = 0;
     }
+    return pr;
+}
+
+// The records of up to kLdsRows rows of cells as one flat list: entry i is record base + i, plus
+// step1 from end0 on (the second row), plus step2 from end1 on (all modulo 2^32).  (Sums,
+// because a select between two variables here is compiled to a load through a selected address.)
+struct LdsRows {
+    uint32_t base, end0, step1, end1, step2, n;
+    bool flat;  // the rows and records fit (else n is 0)
+    __device__ __forceinline__ uint32_t slot(uint32_t i) const {
+        return (i >= end0 ? step1 : 0u) + (i >= end1 ? step2 : 0u) + (base + i);
+    }
+};
+__device__ __forceinline__ LdsRows lds_rows(const LdsGrid& g, const uint32_t* start, bool active, float2 xy, float Q) {
+    LdsRows l = {0, 0, 0, 0, 0, 0, false};
+    if (active) {
+        const LdsRect c = lds_rect(g, xy.x, xy.y, Q);
+        const uint32_t nx = (uint32_t)g.nx;
+        const uint32_t row0 = __umul24((uint32_t)c.cy0, nx), last = __umul24((uint32_t)c.cy1, nx);
+        const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
+        const uint32_t* s0 = start + c.cx0;
+        const uint32_t* s1 = start + c.cx1 + 1;
+        const uint32_t lo0 = s0[row0], hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
+        const int32_t rows = c.cy1 - c.cy0 + 1;
+        l.base = lo0;
+        l.end0 = hi0 - lo0;
+        l.step1 = lo1 - hi0;
+        l.end1 = l.end0 + (rows > 1 ? hi1 - lo1 : 0u);
+        l.step2 = (lo2 - l.end1) - (lo1 - l.end0);
+        l.n = l.end1 + (rows > 2 ? hi2 - lo2 : 0u);
+        l.flat = rows <= kLdsRows && l.n <= kLdsFlat;
+        if (!l.flat) l.n = 0;
+    }
+    static_assert(kLdsRows == 3, "the rows above");
+    return l;
+}
+
+// The entries of a flat list that near(slot, record) accepts, one bit each.  (Past the last one it
+// reads up to three records further -- rec has kLdsRecPad records of room -- and drops their bits.)
+template <class Near>
+__device__ __forceinline__ uint64_t lds_near(const LdsRows& l, const float4* rec, Near&& near) {
+    uint32_t near_lo = 0, near_hi = 0;
+    auto four = [&](uint32_t f) -> uint32_t {
+        float4 sb[4];
+        uint32_t t[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            t[u] = l.slot(f + u);
+            sb[u] = rec[t[u]];
+        }
+        uint32_t bits = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) bits |= near(t[u], sb[u]) ? 1u << u : 0u;
+        return bits;
+    };
+    for (uint32_t f = 0; f < min(l.n, 32u); f += 4) near_lo |= four(f) << f;
+    for (uint32_t f = 32; f < l.n; f += 4) near_hi |= four(f) << (f - 32u);
+    if (l.n < 32u) near_lo &= (1u << l.n) - 1u;
+    if (l.n < 64u) near_hi &= l.n > 32u ? (1u << (l.n - 32u)) - 1u : 0u;
+    return ((uint64_t)near_hi << 32) | near_lo;
+}
+
+// Mark phase of one body a lane (`active`: the lane has one, with a finite snapshot xy),
+// called by whole waves.  rec[] = (x, y, radius, bits(local index)) in cell order, with
+// kLdsRecPad records of room behind them, `own` the body's own record.
+template <uint32_t CAP>
+__device__ __forceinline__ LdsPairs lds_mark(const LdsGrid& g, const uint32_t* start, const float4* rec, bool active,
+                                             float2 xy, float r, uint32_t own, float rmax, uint32_t* entries,
+                                             uint32_t* count) {
+    const LdsRows l = lds_rows(g, start, active, xy, r + rmax);
+    const uint64_t marked = lds_near(l, rec, [&](uint32_t t, const float4& b) {
+        const float dx = xy.x - b.x, dy = xy.y - b.y;
+        const float rs = r + b.z;
+        const bool far = dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f;
+        return !((t == own) | far);
+    });
+    LdsPairs pr = lds_queue<CAP>(marked, own, entries, count, [&](uint32_t i) { return l.slot(i); });
+    pr.direct |= active && !l.flat;
     return pr;
 }
 

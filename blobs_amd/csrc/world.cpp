@@ -814,6 +814,7 @@ void World::free_arrays() {
     dfree(d.cell_count), dfree(d.perm);
     dfree(d.wid), dfree(d.cell_base), dfree(d.tile_seg), dfree(d.grids), dfree(d.wbbox), dfree(d.wold_dt), dfree(d.wstat), dfree(d.wvel);
     dfree(d.p_order), dfree(d.p_wstart), dfree(d.p_counter), dfree(d.p_skip);
+    dfree(d.small_worlds);
     for (uint32_t c = 0; c < kPersistClasses; ++c) d.p_groups[c] = 0;
     d.p_grid_worlds = 0;
     dfree(d.snap_next), dfree(d.x0), dfree(d.bc_start), dfree(d.bc_list), dfree(d.nbr), dfree(d.nbr_len);
@@ -1548,6 +1549,43 @@ int World::upload() {
             persist_ = true;
         }
     }
+    // Small worlds, all of at most kSmallBodies.  With a workgroup a CU for each they all take the
+    // largest's size, in one launch; otherwise each its own size's, so that more of them share a CU.
+    // Small path against the grid path at one rebuild a step, us a step, best of three runs:
+    // 364 bodies 47 / 131 (and 55 / 139 as a settled pile), 1,288 62 / 131 (102 / 197), 2,000 free
+    // 85 / 117; batches 128 worlds of 64-512 31 / 106, 1,024 of 512-1,024 163 / 296, 512 of
+    // 1,024-2,048 127 / 286, 4,096 of 64-256 123 / 311: never slower over the sizes it takes.
+    small_ = false;
+    std::vector<uint32_t> small_worlds;  // slot ranges [W + 1], then the worlds by class [W]
+    if (sphere && !persist_ && zero_off_ && !groups_ && !sensors_) {
+        small_worlds = batch_start_.empty() ? std::vector<uint32_t>{0u, nb} : batch_start_;
+        const uint32_t W = (uint32_t)small_worlds.size() - 1;
+        const std::vector<uint32_t>& wstart = small_worlds;
+        uint32_t largest = 0;
+        for (uint32_t w = 0; w < W; ++w) largest = std::max(largest, wstart[w + 1] - wstart[w]);
+        if (largest <= kSmallBodies) {
+            int cus = 0;
+            if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d.device) != hipSuccess || cus < 1)
+                cus = 1;
+            auto class_of = [](uint32_t n) {
+                uint32_t c = kSmallClasses - 1;
+                while (n > kSmallClassBodies[c]) --c;
+                return c;
+            };
+            std::vector<uint32_t> cls(W);
+            for (uint32_t w = 0; w < W; ++w)
+                cls[w] = class_of(W <= (uint32_t)cus ? largest : wstart[w + 1] - wstart[w]);
+            for (uint32_t c = 0; c < kSmallClasses; ++c) {
+                d.small_class_start[c] = (uint32_t)small_worlds.size() - (W + 1);
+                for (uint32_t w = 0; w < W; ++w)
+                    if (cls[w] == c) small_worlds.push_back(w);
+            }
+            d.small_class_start[kSmallClasses] = W;
+            HIP_TRY(dmalloc(&d.small_worlds, small_worlds.size()));
+            HIP_TRY(h2d(d.small_worlds, small_worlds, s));
+            small_ = true;
+        }
+    }
     HIP_TRY(sort_temp_reserve(d.sort, std::max<uint32_t>(nc, cell_rows + 1)));
     HIP_TRY(hipMemsetAsync(d.cell_start, 0, sizeof(uint32_t) * ((size_t)cell_rows + 1), d.stream));
     d.allocated = true;
@@ -1786,6 +1824,7 @@ int World::run_substep(float h, bool fresh, bool last) {
 // Panics and routing from the step record's error flags (physics.rs:293,
 // 447-448, 471-474).
 int World::process_flags(uint32_t flags) {
+    if (flags & INFO_LISTS_FULL) small_hold_ = kSmallHold;
     const uint32_t panic_bits = flags & (ERR_NAN_NORMAL | ERR_JOINT_MASS | ERR_JOINT_ROT | ERR_ORDERED_CAP);
     route_after_step(flags);
     if (panic_bits & ERR_NAN_NORMAL) return fail(BG_ERR_PANIC, "assertion failed: !n.is_nan() (physics.rs:293)");
@@ -1885,7 +1924,54 @@ int World::launch_persistent(double delta, uint32_t n, bool fresh, hipStream_t s
     return BG_OK;
 }
 
+// Small worlds (small_kernels.hip).  A setting made with bg_set_broadphase, and stage timing,
+// are the grid path's; so is a world with more partners about a body than a list holds, for a while.
+bool World::small_active() const {
+    return small_ && path_ == StepPath::Sphere && rebuild_interval_ == 0 && !profiling_ && small_hold_ == 0 &&
+           !d_.gather_pending;
+}
+
+int World::launch_small(double delta, uint32_t n) {
+    DeviceWorld& d = d_;
+    const float df = (float)delta;                 // physics.rs:80
+    const float h = df / (float)params_.substeps;  // physics.rs:399
+    SmallArgs k{};
+    k.s = d.s;
+    k.wstart = d.small_worlds;
+    k.order = d.small_worlds + d.n_worlds + 1;
+    for (uint32_t c = 0; c <= kSmallClasses; ++c) k.class_start[c] = d.small_class_start[c];
+    k.wold_dt = d.wold_dt;
+    k.accum = d.accum;
+    k.block_contacts = d.block_contacts;
+    k.con_pos = d.con_pos;
+    k.con_r = d.con_r;
+    k.nk = d.nk;
+    k.events = d.events;
+    k.event_cap = d.event_cap;
+    k.vel_scratch = d.vel_next;
+    k.h = h;
+    k.ratio_rest = h / h;
+    k.gx = params_.gravity[0];
+    k.gy = params_.gravity[1];
+    k.collisions = params_.collisions_enabled ? 1u : 0u;
+    k.snap_flags = snap_flags_ ? 1u : 0u;
+    for (uint64_t left = (uint64_t)n * params_.substeps; left > 0;) {
+        k.nsub = (uint32_t)std::min<uint64_t>(left, kSmallSubsteps);
+        k.fresh = fresh_ ? 1u : 0u;
+        k.sub_global = substep_seq_;
+        HIP_TRY(launch_small_step(k, d.stream));
+        substep_seq_ += k.nsub;
+        left -= k.nsub;
+        fresh_ = false;
+        stepped_since_upload_ = true;
+    }
+    need_rebuild_ = true;  // the grid, should the grid path go on from here
+    return BG_OK;
+}
+
 int World::launch_steps(double delta, uint32_t n) {
+    if (small_active()) return launch_small(delta, n);
+    small_hold_ -= std::min(small_hold_, n);
     if (persist_ && path_ == StepPath::Sphere && n > 0) {
         DeviceWorld& d = d_;
         const bool fresh = fresh_;
@@ -1960,7 +2046,7 @@ uint32_t World::interval_substeps() {
 // and 100 us a rebuild), and after a calm while up again, the longer the more often that went
 // wrong.  Results never depend on it.
 void World::adapt_interval(const StepAccum& acc, uint32_t n_steps) {
-    if (rebuild_interval_ || path_ != StepPath::Sphere || !params_.collisions_enabled || n_steps == 0) return;
+    if (rebuild_interval_ || small_active() || path_ != StepPath::Sphere || !params_.collisions_enabled || n_steps == 0) return;
     (void)interval_substeps();
     static constexpr uint32_t kOutlierShare[kLevels] = {512, 200, 64, 32, 32};  // one body in so many
     // (A second rebuild within a step is another 40 us of launches however small the world, the

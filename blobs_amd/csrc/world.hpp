@@ -245,6 +245,13 @@ private:
     // constraints or events, worlds of at most kPersistMaxBodies bodies).  Off by default:
     // over long runs of spreading worlds the grid path alone is faster
     bool persist_enabled_ = false, persist_ = false;
+    // small worlds (small_kernels.hip): the uploaded worlds all fit, and the steps left on the
+    // grid path since a list overflowed
+    bool small_ = false;
+    uint32_t small_hold_ = 0;
+    static constexpr uint32_t kSmallHold = 256, kSmallSubsteps = 512;  // substeps of a launch
+    bool small_active() const;
+    int launch_small(double delta, uint32_t n);
     SphereArrays p_src_{};  // where the last persistent launch (or the upload) left its worlds' records
     std::vector<float> batch_old_dt_;
     std::vector<double> batch_time_;

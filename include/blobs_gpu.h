@@ -304,7 +304,9 @@ int bg_debug_data(bg_world *w, bg_affine2 *bodies, bg_affine2 *colliders, float 
  * depend on any of them; only speed does.  Until it is called: cell scale
  * 1.25 (1.5 for a batch), skin 0.25, and a rebuild interval that follows the
  * outliers (from a quarter of a step to three steps, starting at one step
- * below 65,536 bodies and at three from there). */
+ * below 65,536 bodies and at three from there); worlds of at most 2,048
+ * centred single spheres without groups or sensors (each of a batch) then step
+ * without that grid, one workgroup a world. */
 int bg_set_broadphase(bg_world *w, float cell_scale, float skin, uint32_t rebuild_interval);
 /* Which device path the last step ran: 0 none, 1 general, 2 fused spheres. */
 int bg_step_path(bg_world *w, uint32_t *out);
