@@ -216,9 +216,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         atomicMin(&s_rmin, least);
     }
     __syncthreads();
-    const float rmax = ord2f(s_rmax);
+    const float rmax = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(ord2f(s_rmax))));
     const bool alike = s_rmax == s_rmin;  // one radius: the mark phase needs no partner's
-    float span = kSkinSubsteps, rest = kSkinRest * 2.0f * rmax, age = 0.0f;
+    float span = kSkinSubsteps, rest = kSkinRest * 2.0f * rmax;
+    uint32_t age = 0;  // substeps since the build
     float2 drift = make_float2(0.0f, 0.0f);
     bool build = true;
     uint32_t count = 0, pushes = 0, flags = 0;
@@ -257,6 +258,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     };
 
     for (uint32_t sub = 0; sub < k.nsub; ++sub) {
+        uint32_t t = threadIdx.x;
+        asm volatile("" : "+v"(t));  // (or what is derived from it is kept from phase to phase, and spills)
         const bool fresh = k.fresh && sub == 0;
         const uint32_t par = sub & 1u;
         LdsPairs pr[PER];
@@ -288,7 +291,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             lds_fit<NT>(fit, 2.004f * (rmax + rest), Scratch::kCells, sc.b.red, &s_grid);
             const LdsGrid gr = lds_grid_uniform(s_grid);
             drift = make_float2(gr.ex, gr.ey);
-            age = 0.0f;
+            age = 0;
             for (uint32_t i = t; i <= gr.ncells; i += NT) sc.b.start[i] = 0u;
             __syncthreads();
             const float margin = 1e-4f * (2.0f * rmax + 2.0f * rest) + 1e-5f;
@@ -493,7 +496,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
         // sum, update_objects (physics.rs:326-358), collider transform, constraints
         bool left = false;
-        age += 1.0f;
+        ++age;
 #pragma unroll 1
         for (uint32_t j = 0; j < per; ++j) {
             if (t + j * NT >= nb) continue;
@@ -546,10 +549,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             if (sub + 1 == k.nsub) k.s.vel[g] = st.vel;
             const float2 x0 = pick(o.x0, j);
             const float skin = pick(o.skin, j);
-            const float dx = (x.x - x0.x) - age * drift.x, dy = (x.y - x0.y) - age * drift.y;
+            const float dx = (x.x - x0.x) - (float)age * drift.x, dy = (x.y - x0.y) - (float)age * drift.y;
             left |= finitef(x.x) && finitef(x.y) && !(dx * dx + dy * dy <= skin * skin);
         }
-        left |= !(age * (fabsf(drift.x) + fabsf(drift.y)) <= kMaxDrift);
+        left |= !((float)age * (fabsf(drift.x) + fabsf(drift.y)) <= kMaxDrift);
         if (__any(left) && lane == 0) s_left[par] = 1u;
         if (t == 0) s_left[par ^ 1u] = s_count[par ^ 1u] = s_direct[par ^ 1u] = 0u;
         __syncthreads();
