@@ -68,12 +68,16 @@ __device__ __forceinline__ float atan2_f32(float y, float x) { return (float)ata
 
 // Affine2(rot, p) * offset, translation part: Mat2*Vec2 = c0*x + c1*y with
 // columns (cos, sin), (-sin, cos), then + p (physics.rs:363).
-__device__ __forceinline__ float2 body_xform(float rot, float2 p, float2 off) {
-    float s, c;
-    rot_sincos(rot, &s, &c);
+__device__ __forceinline__ float2 body_xform(float s, float c, float2 p, float2 off) {
     float rx = c * off.x + (-s) * off.y;
     float ry = s * off.x + c * off.y;
     return make_float2(rx + p.x, ry + p.y);
+}
+
+__device__ __forceinline__ float2 body_xform(float rot, float2 p, float2 off) {
+    float s, c;
+    rot_sincos(rot, &s, &c);
+    return body_xform(s, c, p, off);
 }
 
 // Out-of-line copy for rarely taken paths, so its f64 sincos does not

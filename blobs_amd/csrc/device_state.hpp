@@ -59,7 +59,13 @@ constexpr uint32_t kNil = 0xFFFFFFFFu;
 constexpr uint32_t kNbrCap = 32;      // partner-list entries per body (sphere path)
 constexpr uint8_t kNbrNone = 0xFF;    // no list: the body walks the grid
 
-constexpr uint32_t kJointBodies = 16, kJointJoints = 16;
+// Joints of a group and where its part of each table starts (k_joints).
+struct JointGroup {
+    uint32_t q0, q1;  // joints
+    uint32_t b0, b1;  // body list
+    uint32_t l0, l1;  // levels
+};
+constexpr uint32_t kGroupJoints = 64;  // joints of a group (a larger component is a group by itself)
 
 // Ordered contact pass (general path).  A push-out (physics.rs:272-286)
 // rewrites the two colliders' snapshots from their bodies' live positions,
@@ -170,32 +176,25 @@ struct DeviceWorld {
     int32_t *sp_a = nullptr, *sp_b = nullptr;
     float *sp_rest = nullptr, *sp_k = nullptr, *sp_c = nullptr;
     uint32_t *bs_start = nullptr, *bs_list = nullptr;
-    // joints, grouped into independent components (disjoint body sets)
-    int32_t *j_a = nullptr, *j_b = nullptr;
-    float2 *j_anchor_a = nullptr, *j_anchor_b = nullptr;
-    float *j_dist = nullptr, *j_target = nullptr;
-    // per joint: 1/m_a + 1/m_b, (1/m_a)/ims, 1 - that, and 1 if both masses are positive
-    // (physics.rs:447-460; the same f32 operations, evaluated at upload)
-    float4 *j_mass = nullptr;
-    // deferred joint rotations: per solve (component-major, then iteration, then joint),
-    // the axis record (dx, dy, target angle, 1; 0 for a skipped solve); per body, its joints
-    // in arena order (entry = position in jc_list << 1 | 1 if the body is the joint's b) and
-    // component
-    uint32_t j_iters = 0;  // joint_iterations the records are sized for
-    float4 *jrec = nullptr;
-    uint32_t *bj_start = nullptr, *bj_list = nullptr;
-    int32_t *bj_comp = nullptr;
-    uint32_t *jc_start = nullptr, *jc_list = nullptr;
+    // joints, in component order (components of the joint graph, arena order inside each):
+    // anchors (a.x, a.y, b.x, b.y); mass terms 1/m_a + 1/m_b, (1/m_a)/ims, 1 - that, and 1 if both
+    // masses are positive (physics.rs:447-460; the same f32 operations, evaluated at upload);
+    // and (distance, target angle)
     uint32_t n_jcomp = 0;
-    // components of at most kJointBodies bodies and kJointJoints joints iterate in LDS:
-    // their bodies (jb_start/jb_list, empty for a larger component) and, per entry of
-    // jc_list, the joint's two bodies as local indices (a | b << 8)
-    uint32_t *jb_start = nullptr, *j_local = nullptr;
-    int32_t *jb_list = nullptr;
-    // per entry of jc_list: the joint's anchors (a.x, a.y, b.x, b.y), mass terms and
-    // (distance, target angle), so that a block stages its components' joints coalesced
     float4 *jq_anchor = nullptr, *jq_mass = nullptr;
     float2 *jq_len = nullptr;
+    uint2 *jq_ab = nullptr;  // body a | static << 31, body b | static << 31: indices of the group's body list
+    // groups of components, each swept by one workgroup level by level (joint_schedule.hpp),
+    // for j_iters iterations; per solve (level order) its joint and where its rotation goes
+    uint32_t j_iters = 0, n_jgroups = 0;
+    JointGroup *jg = nullptr;
+    uint32_t *jl_start = nullptr;
+    uint2 *j_entry = nullptr;
+    int32_t *jg_body = nullptr;
+    // per solve, at iteration * joints + joint: the rotation step (corr * h, 1; second 0 for a
+    // skipped solve); per body, its joints in arena order (entry = joint << 1 | 1 if the body is the joint's b)
+    float2 *jrot = nullptr;
+    uint32_t *bj_start = nullptr, *bj_list = nullptr;
     // constraints
     float2 *con_pos = nullptr;
     float *con_r = nullptr;
@@ -328,7 +327,7 @@ struct SubstepArgs {
     uint32_t write_vel;   // sphere path: store calculated_velocity (last substep of a step, or
                           // every substep when collision events read it)
     uint32_t joint_rot;   // general path: k_integrate applies the joint stage's rotation corrections
-    uint32_t joint_iters;
+    uint32_t joint_iters, joint_count;
 };
 
 // A general-path rebuild's key pass (step_kernels.hip): the grid from the
@@ -351,8 +350,8 @@ struct KeysArgs {
 // Launchers (step_kernels.hip: general path + broadphase build).  A substep
 // that rebuilds passes its key pass (launched with the substep's forces).
 hipError_t launch_rebuild_sort_and_cells(DeviceWorld& d);
-hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, uint32_t joint_iterations, bool groups,
-                                  bool sensors, const KeysArgs* rebuild);
+hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, bool groups, bool sensors,
+                                  const KeysArgs* rebuild);
 // Launchers (sphere_kernels.hip).
 hipError_t launch_sphere_rebuild(DeviceWorld& d, float cell, uint32_t parity);
 hipError_t launch_sphere_substep(DeviceWorld& d, const SubstepArgs& a, bool groups, bool sensors, bool zero_off,

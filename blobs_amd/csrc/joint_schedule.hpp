@@ -23,6 +23,7 @@ struct JointSchedule {
     std::vector<uint32_t> group_level{0};  // levels of group g: [group_level[g], group_level[g + 1])
     std::vector<uint32_t> level_start{0};  // solves of level l: entry[level_start[l] .. level_start[l + 1])
     std::vector<uint32_t> entry;           // a solve's joint
+    std::vector<uint32_t> iteration;       // and its iteration
 
     uint32_t groups() const { return (uint32_t)group_level.size() - 1; }
 
@@ -30,7 +31,7 @@ struct JointSchedule {
     // n_bodies), numbered `ids`, swept `iterations` times.  `last` is scratch, all zero.
     void add_group(const std::vector<std::pair<uint32_t, uint32_t>>& joints, const std::vector<uint32_t>& ids,
                    uint32_t iterations, std::vector<uint32_t>& last, uint32_t width) {
-        std::vector<std::vector<uint32_t>> levels;
+        std::vector<std::vector<std::pair<uint32_t, uint32_t>>> levels;
         for (uint32_t it = 0; it < iterations; ++it)
             for (size_t k = 0; k < joints.size(); ++k) {
                 uint32_t& la = last[joints[k].first];
@@ -38,12 +39,15 @@ struct JointSchedule {
                 uint32_t l = std::max(la, lb);
                 while (l < levels.size() && levels[l].size() >= width) ++l;
                 if (l >= levels.size()) levels.resize(l + 1);
-                levels[l].push_back(ids[k]);
+                levels[l].push_back({ids[k], it});
                 la = lb = l + 1;
             }
         for (const auto& j : joints) last[j.first] = last[j.second] = 0;
         for (const auto& l : levels) {
-            entry.insert(entry.end(), l.begin(), l.end());
+            for (const auto& e : l) {
+                entry.push_back(e.first);
+                iteration.push_back(e.second);
+            }
             level_start.push_back((uint32_t)entry.size());
         }
         group_level.push_back((uint32_t)level_start.size() - 1);

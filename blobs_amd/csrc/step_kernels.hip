@@ -646,12 +646,6 @@ __global__ __launch_bounds__(kContactThreads) void k_contact_merge(DeviceWorld d
     d.b.pos[b] = p;
 }
 
-// One fixed joint (physics.rs:424-477) on body positions pa, pb and rotations
-// ra, rb (read before any write of this joint).  Returns false for coincident
-// anchors, which the reference skips; the caller then writes nothing.
-// The joint's mass terms (physics.rs:447-460) depend on the two bodies'
-// calculated_mass only, which no stage of a step changes: they come in
-// precomputed (DeviceWorld::j_mass, same f32 operations) and stay off the chain.
 // Rotation correction of one joint from its axis (physics.rs:462-469): the
 // reference adds corr * dt to rotation a and subtracts it from rotation b.
 // Positions never read rotations inside the joint stage (anchors are not
@@ -663,141 +657,130 @@ __device__ __forceinline__ float joint_rotation_corr(float dx, float dy, float j
     return diff * 0.5f;
 }
 
-__device__ __forceinline__ void joint_rotate(float& ra, float& rb, float corr, float h, uint32_t& flags) {
-    ra = ra + corr * h;
-    rb = rb - corr * h;
-    if (!finitef(ra) || !finitef(rb)) flags |= ERR_JOINT_ROT;
-}
+// Fixed joints (physics.rs:424-477): a workgroup a group of components
+// (components touch disjoint bodies).  Its first wave sweeps the positions
+// level by level, a lane a solve (joint_schedule.hpp: the sequential sweep's
+// very positions), on LDS copies of the bodies and joint records; the joint's
+// mass terms depend on calculated_mass only, so they come in precomputed and
+// stay off the chain.  Then all the threads work out the solves' rotation
+// steps from the axes, an atan2 pair each, and k_integrate adds them per body
+// in the order of the sweep: iterations, then joints in arena order.
+//
+// Bound by the chain: a level is two LDS reads, a root, two divides and two
+// writes, and a lane a component took one such step for each of the largest's
+// solves (52, against 24 levels), with two f64 atan2 a solve left to its two
+// bodies' threads in a row.  16,384 joints: this kernel and k_integrate took
+// 27.6 + 24.6 us a substep that way; a pass of 64 substeps fell from 14.1 to 9.9 ms.
+constexpr uint32_t kJointThreads = 256;
+constexpr uint32_t kStageJoints = 256, kStageBodies = 384, kStageSolves = 1024, kStageLevels = 512;
 
-// One fixed joint, positions then rotations.
-__device__ __forceinline__ bool joint_solve(float2& pa, float2& pb, float& ra, float& rb, float2 an_a, float2 an_b,
-                                            float jdist, float jtarget, float4 jm, bool sa, bool sb, float h,
-                                            uint32_t& flags) {
-    float dx, dy;
-    if (!joint_positions(pa, pb, an_a, an_b, jdist, jm, sa, sb, dx, dy, flags)) return false;
-    joint_rotate(ra, rb, joint_rotation_corr(dx, dy, jtarget), h, flags);
-    return true;
-}
+struct JointRec {
+    float4 anchor, mass;
+    float dist;
+    uint32_t a, b;  // body list index | static << 31
+};
 
-// Fixed joints (physics.rs:424-477), positions: Gauss-Seidel in arena order
-// inside each connected component of the joint graph (components touch
-// disjoint bodies, so they run in parallel, one lane each).  A block of 64
-// components first stages, with coalesced loads, the constant records of all
-// their joints (stored in component order at upload) and the positions of
-// the bodies of its components of at most kJointBodies bodies and
-// kJointJoints joints; each such component then iterates on those LDS copies
-// (the sweep is a chain of dependent reads and writes, so each step costs an
-// LDS round trip instead of a cache round trip), and the block writes its
-// bodies back.  A larger component, or every component of a block whose
-// joints or bodies exceed the block's LDS, iterates in global memory.
-// Writes keep the reference's order (a's position, b's, a's rotation, b's),
-// which decides a joint of a body to itself.  With `defer`,
-// every solve's axis goes to jrec[iterations * jc_start[c] + it * nq + q] --
-// record (dx, dy, target angle, 1), or 0 when the anchors coincide and the
-// reference skips the joint -- and the rotations are applied later:
-// k_integrate evaluates each of its body's solves' atan2 pairs and adds the
-// corrections in sequence order.  Without it
-// (joint_iterations changed since the upload) the rotations are applied here.
-constexpr uint32_t kBlockJoints = 512;  // joints of a block's components staged in LDS
-constexpr uint32_t kBlockBodies = 640;  // bodies of its small components staged in LDS
-
-__global__ __launch_bounds__(64) void k_joints(DeviceWorld d, SubstepArgs a, uint32_t iterations, bool defer) {
-    __shared__ float4 s_anchor[kBlockJoints];  // anchor a, anchor b
-    __shared__ float4 s_jm[kBlockJoints];      // mass terms
-    __shared__ float2 s_len[kBlockJoints];     // distance, target angle
-    __shared__ uint32_t s_loc[kBlockJoints];   // local a | local b << 8
-    __shared__ float2 s_pos[kBlockBodies];
-    __shared__ float s_rot[kBlockBodies];
-    __shared__ int32_t s_gid[kBlockBodies];    // body index
-    __shared__ uint8_t s_stat[kBlockBodies];   // 1: static body
-    const uint32_t lane = threadIdx.x;
-    const uint32_t c0 = blockIdx.x * 64u, c1 = min(c0 + 64u, d.n_jcomp);
-    const uint32_t comp = c0 + lane;
-    const uint32_t q0 = d.jc_start[c0], q1 = d.jc_start[c1];
-    const uint32_t b0 = d.jb_start[c0], b1 = d.jb_start[c1];
-    const bool staged = q1 - q0 <= kBlockJoints && b1 - b0 <= kBlockBodies;  // the same for the block
+__global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h) {
+    __shared__ float4 s_anchor[kStageJoints], s_mass[kStageJoints];
+    __shared__ float2 s_len[kStageJoints];
+    __shared__ uint2 s_ab[kStageJoints];
+    __shared__ float2 s_pos[kStageBodies];
+    __shared__ int32_t s_gid[kStageBodies];
+    __shared__ uint32_t s_level[kStageLevels + 1];
+    __shared__ uint2 s_entry[kStageSolves];
+    __shared__ float2 s_axis[kStageSolves];
+    const JointGroup g = d.jg[blockIdx.x];
+    const uint32_t tid = threadIdx.x, nq = g.q1 - g.q0, nbod = g.b1 - g.b0, nl = g.l1 - g.l0;
+    const uint32_t e0 = d.jl_start[g.l0], n = d.jl_start[g.l1] - e0;
+    const bool staged = nq <= kStageJoints && nbod <= kStageBodies && nl <= kStageLevels && n <= kStageSolves;
+    if (staged) {
+        for (uint32_t i = tid; i < nbod; i += kJointThreads) {
+            const int32_t b = d.jg_body[g.b0 + i];
+            s_gid[i] = b;
+            s_pos[i] = d.b.pos[b];
+        }
+        for (uint32_t i = tid; i < nq; i += kJointThreads) {
+            s_anchor[i] = d.jq_anchor[g.q0 + i];
+            s_mass[i] = d.jq_mass[g.q0 + i];
+            s_len[i] = d.jq_len[g.q0 + i];
+            s_ab[i] = d.jq_ab[g.q0 + i];
+        }
+        for (uint32_t i = tid; i <= nl; i += kJointThreads) s_level[i] = d.jl_start[g.l0 + i] - e0;
+        for (uint32_t i = tid; i < n; i += kJointThreads) s_entry[i] = d.j_entry[e0 + i];
+    }
+    __syncthreads();
     uint32_t flags = 0;
-    if (staged) {
-        for (uint32_t i = lane; i < q1 - q0; i += 64u) {
-            s_anchor[i] = d.jq_anchor[q0 + i];
-            s_jm[i] = d.jq_mass[q0 + i];
-            s_len[i] = d.jq_len[q0 + i];
-            s_loc[i] = d.j_local[q0 + i];
+    // one solve: axis to `axis`, positions through get and put; body a's write comes first
+    auto solve = [&](const JointRec& r, auto&& get, auto&& put) {
+        const uint32_t ia = r.a & 0x7FFFFFFFu, ib = r.b & 0x7FFFFFFFu;
+        float2 pa = get(ia), pb = get(ib), axis;
+        if (joint_positions(pa, pb, make_float2(r.anchor.x, r.anchor.y), make_float2(r.anchor.z, r.anchor.w), r.dist,
+                            r.mass, (r.a >> 31) != 0u, (r.b >> 31) != 0u, axis.x, axis.y, flags)) {
+            put(ia, pa);
+            put(ib, pb);
         }
-        for (uint32_t i = lane; i < b1 - b0; i += 64u) {
-            const int32_t g = d.jb_list[b0 + i];
-            s_gid[i] = g;
-            s_pos[i] = d.b.pos[g];
-            if (!defer) s_rot[i] = d.b.rot[g];
-            s_stat[i] = (d.b.bflags[g] & BF_STATIC) ? 1u : 0u;
-        }
-        __syncthreads();
-    }
-    if (comp < c1) {
-        const uint32_t k0 = d.jc_start[comp], k1 = d.jc_start[comp + 1];
-        const uint32_t lb = d.jb_start[comp] - b0, nbl = d.jb_start[comp + 1] - d.jb_start[comp];
-        const uint32_t nq = k1 - k0;
-        float4* rec = defer ? d.jrec + (size_t)iterations * k0 : nullptr;
-        if (staged && nbl > 0) {
-            const uint32_t lq = k0 - q0;
-            for (uint32_t it = 0; it < iterations; ++it) {
-                for (uint32_t q = 0; q < nq; ++q) {
-                    const uint32_t loc = s_loc[lq + q];
-                    const uint32_t la = lb + (loc & 0xFFu), lbb = lb + ((loc >> 8) & 0xFFu);
-                    const float4 an = s_anchor[lq + q];
-                    const float2 len = s_len[lq + q];
-                    float2 pa = s_pos[la], pb = s_pos[lbb];
-                    float dx, dy;
-                    const bool moved = joint_positions(pa, pb, make_float2(an.x, an.y), make_float2(an.z, an.w),
-                                                       len.x, s_jm[lq + q], s_stat[la] != 0u, s_stat[lbb] != 0u,
-                                                       dx, dy, flags);
-                    if (defer) rec[it * nq + q] = moved ? make_float4(dx, dy, len.y, 1.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (!moved) continue;
-                    s_pos[la] = pa;
-                    s_pos[lbb] = pb;
-                    if (!defer) {
-                        float ra = s_rot[la], rb = s_rot[lbb];
-                        joint_rotate(ra, rb, joint_rotation_corr(dx, dy, len.y), a.h, flags);
-                        s_rot[la] = ra;
-                        s_rot[lbb] = rb;
-                    }
-                }
+        return axis;
+    };
+    if (tid < BG_WAVE) {
+        if (staged) {
+            // the next level's record loads while the current one works
+            uint32_t e = 0, e_next = 0;
+            bool have = false, have_next = false;
+            JointRec r, r_next;
+            auto load = [&](uint32_t l) {
+                e_next = s_level[l] + tid;
+                have_next = e_next < s_level[l + 1];
+                if (!have_next) return;
+                const uint32_t q = s_entry[e_next].x;
+                r_next.anchor = s_anchor[q];
+                r_next.mass = s_mass[q];
+                r_next.dist = s_len[q].x;
+                const uint2 ab = s_ab[q];
+                r_next.a = ab.x;
+                r_next.b = ab.y;
+            };
+            if (nl > 0) load(0);
+            for (uint32_t l = 0; l < nl; ++l) {
+                e = e_next;
+                have = have_next;
+                r = r_next;
+                if (l + 1 < nl) load(l + 1);
+                if (have)
+                    s_axis[e] = solve(r, [&](uint32_t i) { return s_pos[i]; },
+                                      [&](uint32_t i, float2 p) { s_pos[i] = p; });
+                // the next level's lanes read what this one's wrote: one wave's LDS accesses keep
+                // their order, the compiler has to as well
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
-        } else if (!staged || nbl == 0) {
-            for (uint32_t it = 0; it < iterations; ++it) {
-                for (uint32_t kk = k0; kk < k1; ++kk) {
-                    const uint32_t j = d.jc_list[kk];
-                    const int32_t ia = d.j_a[j], ib = d.j_b[j];
-                    float2 pa = d.b.pos[ia], pb = d.b.pos[ib];
-                    float dx, dy;
-                    const bool moved =
-                        joint_positions(pa, pb, d.j_anchor_a[j], d.j_anchor_b[j], d.j_dist[j], d.j_mass[j],
-                                        d.b.bflags[ia] & BF_STATIC, d.b.bflags[ib] & BF_STATIC, dx, dy, flags);
-                    if (defer)
-                        rec[it * nq + (kk - k0)] =
-                            moved ? make_float4(dx, dy, d.j_target[j], 1.0f) : make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (!moved) continue;
-                    d.b.pos[ia] = pa;
-                    d.b.pos[ib] = pb;
-                    if (!defer) {
-                        float ra = d.b.rot[ia], rb = d.b.rot[ib];
-                        joint_rotate(ra, rb, joint_rotation_corr(dx, dy, d.j_target[j]), a.h, flags);
-                        d.b.rot[ia] = ra;
-                        d.b.rot[ib] = rb;
-                    }
+        } else {
+            for (uint32_t l = 0; l < nl; ++l) {
+                const uint32_t end = d.jl_start[g.l0 + l + 1];
+                for (uint32_t e = d.jl_start[g.l0 + l] + tid; e < end; e += BG_WAVE) {
+                    const uint2 en = d.j_entry[e];
+                    const uint2 ab = d.jq_ab[g.q0 + en.x];
+                    const JointRec r = {d.jq_anchor[g.q0 + en.x], d.jq_mass[g.q0 + en.x], d.jq_len[g.q0 + en.x].x,
+                                        ab.x, ab.y};
+                    d.jrot[en.y] = solve(r, [&](uint32_t i) { return d.b.pos[d.jg_body[g.b0 + i]]; },
+                                         [&](uint32_t i, float2 p) { d.b.pos[d.jg_body[g.b0 + i]] = p; });
                 }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // memory: wait for the writes
+                __builtin_amdgcn_wave_barrier();
             }
-        }
-    }
-    if (staged) {
-        __syncthreads();
-        for (uint32_t i = lane; i < b1 - b0; i += 64u) {
-            const int32_t g = s_gid[i];
-            d.b.pos[g] = s_pos[i];
-            if (!defer) d.b.rot[g] = s_rot[i];
         }
     }
     if (flags) atomicOr(&d.accum->error_flags, flags);
+    __syncthreads();
+    if (staged)
+        for (uint32_t i = tid; i < nbod; i += kJointThreads) d.b.pos[s_gid[i]] = s_pos[i];
+    for (uint32_t e = tid; e < n; e += kJointThreads) {
+        const uint2 en = staged ? s_entry[e] : d.j_entry[e0 + e];
+        const float2 axis = staged ? s_axis[e] : d.jrot[en.y];
+        const float target = staged ? s_len[en.x].y : d.jq_len[g.q0 + en.x].y;
+        float2 step = make_float2(0.0f, 0.0f);  // coincident anchors: the reference skips the solve
+        if (!(vlen(axis.x, axis.y) < 1e-6f)) step = make_float2(joint_rotation_corr(axis.x, axis.y, target) * h, 1.0f);
+        d.jrot[en.y] = step;
+    }
 }
 
 // Verlet + collider transforms + constraints (physics.rs:323-395).
@@ -813,23 +796,29 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
         s.omega = d.b.omega[b];
         const float rot_in = s.rot;
         if (a.joint_rot) {
-            // this body's joint rotation corrections (physics.rs:468-469), in the order the
-            // joint stage made them: iterations, then the component's joints in arena order
-            const int32_t c = d.bj_comp[b];
-            if (c >= 0) {
-                const uint32_t k0 = d.jc_start[c], nq = d.jc_start[c + 1] - k0;
-                const uint32_t e0 = d.bj_start[b], e1 = d.bj_start[b + 1];
-                const float4* rec = d.jrec + (size_t)a.joint_iters * k0;
-                for (uint32_t it = 0; it < a.joint_iters; ++it)
-                    for (uint32_t e = e0; e < e1; ++e) {
-                        const uint32_t ent = d.bj_list[e];
-                        const float4 x = rec[it * nq + ((ent >> 1) - k0)];
-                        if (x.w == 0.0f) continue;  // the reference skipped that solve
-                        // both bodies of the solve evaluate its atan2 pair (the same f32 result)
-                        const float dlt = joint_rotation_corr(x.x, x.y, x.z) * a.h;
-                        s.rot = (ent & 1u) ? s.rot - dlt : s.rot + dlt;
-                        if (!finitef(s.rot)) la.flags |= ERR_JOINT_ROT;
+            // this body's joint rotation steps (physics.rs:468-469), in the order of the sweep:
+            // iterations, then joints in arena order; a few load at a time
+            const uint32_t e0 = d.bj_start[b], n = d.bj_start[b + 1] - e0;
+            const uint32_t total = n * a.joint_iters;
+            uint32_t i = 0, it = 0;  // position m is entry i of iteration it
+            for (uint32_t m = 0; m < total; m += 4) {
+                uint32_t ent[4];
+                float2 step[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    ent[u] = d.bj_list[e0 + i];
+                    step[u] = d.jrot[(size_t)it * a.joint_count + (ent[u] >> 1)];
+                    if (m + u + 1 < total && ++i == n) {
+                        i = 0;
+                        ++it;
                     }
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) {
+                    if (m + u >= total || step[u].y == 0.0f) continue;
+                    s.rot = (ent[u] & 1u) ? s.rot - step[u].x : s.rot + step[u].x;
+                    if (!finitef(s.rot)) la.flags |= ERR_JOINT_ROT;
+                }
             }
         }
         if (fl & BF_STATIC) {  // :327-332
@@ -869,6 +858,8 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
         // round so that their loads overlap (an index past the end repeats the last collider:
         // the same store, and the bounding box and displacement maximum are idempotent)
         const uint32_t c0 = d.bc_start[b], c1 = d.bc_start[b + 1];
+        float sn = 0.0f, cs = 1.0f;
+        if (c1 > c0) rot_sincos(s.rot, &sn, &cs);
         for (uint32_t k0 = c0; k0 < c1; k0 += 4) {
             uint32_t c[4];
             float2 off[4], x0[4];
@@ -881,7 +872,7 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
             }
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) {
-                const float2 x = body_xform(s.rot, s.p, off[u]);
+                const float2 x = body_xform(sn, cs, s.p, off[u]);
                 d.c.abs[c[u]] = x;
                 la.point(x.x, x.y, x0[u].x, x0[u].y, a.drift_x, a.drift_y);
             }
@@ -912,8 +903,8 @@ hipError_t launch_rebuild_sort_and_cells(DeviceWorld& d) {
     return hipGetLastError();
 }
 
-hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, uint32_t joint_iterations, bool groups,
-                                  bool sensors, const KeysArgs* rebuild) {
+hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, bool groups, bool sensors,
+                                  const KeysArgs* rebuild) {
     if (d.nb == 0) return hipSuccess;
     const uint32_t blocks = div_up(d.nb, kThreads);
     // the rebuild's keys and the substep's forces in one launch, then the rest of the rebuild
@@ -958,13 +949,11 @@ hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, uint32_t
     }
     SubstepArgs ai = a;
     ai.joint_rot = 0u;
-    if (d.n_jcomp > 0 && joint_iterations > 0) {
-        const bool defer = d.jrec && joint_iterations == d.j_iters;
-        k_joints<<<div_up(d.n_jcomp, 64), 64, 0, d.stream>>>(d, a, joint_iterations, defer);
-        if (defer) {
-            ai.joint_rot = 1u;
-            ai.joint_iters = joint_iterations;
-        }
+    if (d.n_jgroups > 0 && d.j_iters > 0) {
+        k_joints<<<d.n_jgroups, kJointThreads, 0, d.stream>>>(d, a.h);
+        ai.joint_rot = 1u;
+        ai.joint_iters = d.j_iters;
+        ai.joint_count = d.nj;
     }
     k_integrate<<<blocks, kThreads, 0, d.stream>>>(d, ai);
     return hipGetLastError();

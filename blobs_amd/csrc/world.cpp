@@ -1,4 +1,5 @@
 // world.cpp -- host side of the `Physics` drop-in (see world.hpp).
+#include "joint_schedule.hpp"
 #include "world.hpp"
 
 #include <hip/hip_runtime.h>
@@ -820,9 +821,9 @@ void World::free_arrays() {
     dfree(d.snap_next), dfree(d.x0), dfree(d.bc_start), dfree(d.bc_list), dfree(d.nbr), dfree(d.nbr_len);
     dfree(d.sp_a), dfree(d.sp_b), dfree(d.sp_rest), dfree(d.sp_k), dfree(d.sp_c), dfree(d.bs_start),
         dfree(d.bs_list);
-    dfree(d.j_a), dfree(d.j_b), dfree(d.j_anchor_a), dfree(d.j_anchor_b), dfree(d.j_dist), dfree(d.j_target);
-    dfree(d.j_mass), dfree(d.jrec), dfree(d.bj_start), dfree(d.bj_list), dfree(d.bj_comp);
-    dfree(d.jc_start), dfree(d.jc_list), dfree(d.jb_start), dfree(d.jb_list), dfree(d.j_local), dfree(d.jq_anchor), dfree(d.jq_mass), dfree(d.jq_len), dfree(d.con_pos),
+    dfree(d.jq_anchor), dfree(d.jq_mass), dfree(d.jq_len), dfree(d.jq_ab);
+    dfree(d.jg), dfree(d.jl_start), dfree(d.j_entry), dfree(d.jg_body), dfree(d.jrot), dfree(d.bj_start), dfree(d.bj_list);
+    dfree(d.con_pos),
         dfree(d.con_r);
     dfree(d.keys), dfree(d.vals), dfree(d.keys_tmp), dfree(d.vals_tmp), dfree(d.cell_start), dfree(d.crec);
     dfree(d.export_buf);
@@ -1065,8 +1066,7 @@ int World::upload() {
         const float ratio = inv_a / ims;
         j_mass[k] = make_float4(ims, ratio, 1.0f - ratio, (ma > 0.0f && mb > 0.0f) ? 1.0f : 0.0f);
     }
-    std::vector<uint32_t> jc_start, jc_list, jb_start, j_local;
-    std::vector<int32_t> jb_list;
+    std::vector<uint32_t> jc_start, jc_list;
     uint32_t n_jcomp = 0;
     if (nj > 0 && !structure_error_) {
         std::vector<int32_t> uf(nb);
@@ -1099,43 +1099,25 @@ int World::upload() {
         jc_list.resize(nj);
         std::vector<uint32_t> fillp(jc_start.begin(), jc_start.end() - 1);
         for (uint32_t k = 0; k < nj; ++k) jc_list[fillp[jcomp[k]]++] = k;
-        // local body indices of the components small enough to iterate in LDS
-        jb_start.assign(n_jcomp + 1, 0);
-        j_local.assign(nj, 0);
-        std::vector<int32_t> local_of(nb, -1), bodies;
-        for (uint32_t c = 0; c < n_jcomp; ++c) {
-            bodies.clear();
-            for (uint32_t kk = jc_start[c]; kk < jc_start[c + 1]; ++kk) {
-                const uint32_t j = jc_list[kk];
-                for (int32_t bi : {j_a[j], j_b[j]})
-                    if (local_of[bi] < 0) {
-                        local_of[bi] = (int32_t)bodies.size();
-                        bodies.push_back(bi);
-                    }
-                j_local[kk] = (uint32_t)(local_of[j_a[j]] & 0xFF) | ((uint32_t)(local_of[j_b[j]] & 0xFF) << 8);
-            }
-            const bool fits = jc_start[c + 1] - jc_start[c] <= kJointJoints && bodies.size() <= kJointBodies;
-            for (int32_t bi : bodies) {
-                local_of[bi] = -1;
-                if (fits) jb_list.push_back(bi);
-            }
-            jb_start[c + 1] = (uint32_t)jb_list.size();
-        }
     }
-    // the joints' constant records in component order (entry kk of jc_list), for the joint
-    // stage's coalesced staging
+    // the joints' constant records in component order (entry kk of jc_list)
     std::vector<float4> jq_anchor(jc_list.size()), jq_mass(jc_list.size());
     std::vector<float2> jq_len(jc_list.size());
+    joint_bodies_.assign(jc_list.size(), {0, 0});
     for (size_t kk = 0; kk < jc_list.size(); ++kk) {
         const uint32_t j = jc_list[kk];
         jq_anchor[kk] = make_float4(j_an_a[j].x, j_an_a[j].y, j_an_b[j].x, j_an_b[j].y);
         jq_mass[kk] = j_mass[j];
         jq_len[kk] = make_float2(j_dist[j], j_target[j]);
+        joint_bodies_[kk] = {j_a[j], j_b[j]};
     }
-    // per body: its joints in arena order and its component (deferred joint rotations)
-    std::vector<uint32_t> bj_start(nb + 1, 0), bj_list;
-    std::vector<int32_t> bj_comp(nb, -1);
+    joint_static_.clear();
+    if (n_jcomp > 0)
+        for (uint32_t i = 0; i < nb; ++i) joint_static_.push_back((bflags[i] & BF_STATIC) ? 1 : 0);
+    // per body: its joints in arena order (deferred joint rotations)
+    std::vector<uint32_t> bj_start, bj_list;
     if (n_jcomp > 0) {
+        bj_start.assign(nb + 1, 0);
         for (uint32_t k = 0; k < nj; ++k) {
             bj_start[j_a[k] + 1]++;
             bj_start[j_b[k] + 1]++;
@@ -1143,14 +1125,13 @@ int World::upload() {
         for (uint32_t i = 0; i < nb; ++i) bj_start[i + 1] += bj_start[i];
         bj_list.resize(bj_start[nb]);
         std::vector<uint32_t> fillb(bj_start.begin(), bj_start.end() - 1);
-        for (uint32_t c = 0; c < n_jcomp; ++c)
-            for (uint32_t kk = jc_start[c]; kk < jc_start[c + 1]; ++kk) {
-                const uint32_t j = jc_list[kk];
-                bj_list[fillb[j_a[j]]++] = kk << 1;
-                bj_list[fillb[j_b[j]]++] = (kk << 1) | 1u;
-                bj_comp[j_a[j]] = bj_comp[j_b[j]] = (int32_t)c;
-            }
+        for (uint32_t kk = 0; kk < nj; ++kk) {  // (inside a component in arena order)
+            const uint32_t j = jc_list[kk];
+            bj_list[fillb[j_a[j]]++] = kk << 1;
+            bj_list[fillb[j_b[j]]++] = (kk << 1) | 1u;
+        }
     }
+    joint_comp_start_ = jc_start;
 
     // constraints
     const uint32_t nk = (uint32_t)constraints_.size();
@@ -1418,25 +1399,9 @@ int World::upload() {
     HIP_TRY(dmalloc(&d.sp_c, ns));
     HIP_TRY(dmalloc(&d.bs_start, nb + 1));
     HIP_TRY(dmalloc(&d.bs_list, bs_list.size()));
-    HIP_TRY(dmalloc(&d.j_a, nj));
-    HIP_TRY(dmalloc(&d.j_b, nj));
-    HIP_TRY(dmalloc(&d.j_anchor_a, nj));
-    HIP_TRY(dmalloc(&d.j_anchor_b, nj));
-    HIP_TRY(dmalloc(&d.j_dist, nj));
-    HIP_TRY(dmalloc(&d.j_target, nj));
-    HIP_TRY(dmalloc(&d.j_mass, nj));
-    if (n_jcomp > 0 && params_.joint_iterations > 0) {
-        d.j_iters = params_.joint_iterations;
-        HIP_TRY(dmalloc(&d.jrec, (size_t)d.j_iters * nj));
-        HIP_TRY(dmalloc(&d.bj_start, nb + 1));
-        HIP_TRY(dmalloc(&d.bj_list, bj_list.size()));
-        HIP_TRY(dmalloc(&d.bj_comp, nb));
-    }
-    HIP_TRY(dmalloc(&d.jc_start, n_jcomp + 1));
-    HIP_TRY(dmalloc(&d.jc_list, nj));
-    HIP_TRY(dmalloc(&d.jb_start, n_jcomp + 1));
-    HIP_TRY(dmalloc(&d.jb_list, jb_list.size()));
-    HIP_TRY(dmalloc(&d.j_local, nj));
+    d.j_iters = d.n_jgroups = 0;  // the schedule of the sweep: ensure_joint_schedule
+    HIP_TRY(dmalloc(&d.bj_start, bj_start.size()));
+    HIP_TRY(dmalloc(&d.bj_list, bj_list.size()));
     HIP_TRY(dmalloc(&d.jq_anchor, jq_anchor.size()));
     HIP_TRY(dmalloc(&d.jq_mass, jq_mass.size()));
     HIP_TRY(dmalloc(&d.jq_len, jq_len.size()));
@@ -1599,23 +1564,8 @@ int World::upload() {
     HIP_TRY(h2d(d.sp_c, sp_c, s));
     HIP_TRY(h2d(d.bs_start, bs_start, s));
     HIP_TRY(h2d(d.bs_list, bs_list, s));
-    HIP_TRY(h2d(d.j_a, j_a, s));
-    HIP_TRY(h2d(d.j_b, j_b, s));
-    HIP_TRY(h2d(d.j_anchor_a, j_an_a, s));
-    HIP_TRY(h2d(d.j_anchor_b, j_an_b, s));
-    HIP_TRY(h2d(d.j_dist, j_dist, s));
-    HIP_TRY(h2d(d.j_target, j_target, s));
-    HIP_TRY(h2d(d.j_mass, j_mass, s));
-    if (d.jrec) {
-        HIP_TRY(h2d(d.bj_start, bj_start, s));
-        HIP_TRY(h2d(d.bj_list, bj_list, s));
-        HIP_TRY(h2d(d.bj_comp, bj_comp, s));
-    }
-    HIP_TRY(h2d(d.jc_start, jc_start, s));
-    HIP_TRY(h2d(d.jc_list, jc_list, s));
-    HIP_TRY(h2d(d.jb_start, jb_start, s));
-    HIP_TRY(h2d(d.jb_list, jb_list, s));
-    HIP_TRY(h2d(d.j_local, j_local, s));
+    HIP_TRY(h2d(d.bj_start, bj_start, s));
+    HIP_TRY(h2d(d.bj_list, bj_list, s));
     HIP_TRY(h2d(d.jq_anchor, jq_anchor, s));
     HIP_TRY(h2d(d.jq_mass, jq_mass, s));
     HIP_TRY(h2d(d.jq_len, jq_len, s));
@@ -1817,7 +1767,7 @@ int World::run_substep(float h, bool fresh, bool last) {
     if (int st = stage_begin(BG_STAGE_SUBSTEP)) return st;
     const KeysArgs* keys = keys_pending_ ? &keys_ : nullptr;
     keys_pending_ = false;
-    HIP_TRY(launch_general_substep(d, a, params_.joint_iterations, groups_, sensors_, keys));
+    HIP_TRY(launch_general_substep(d, a, groups_, sensors_, keys));
     return stage_end(BG_STAGE_SUBSTEP);
 }
 
@@ -1890,6 +1840,77 @@ int World::prepare_step() {
         if (st) return st;
     }
     if (structure_error_) return fail(BG_ERR_PANIC, structure_msg_);
+    return ensure_joint_schedule();
+}
+
+// The sweep of the joint stage for the present joint_iterations (k_joints): groups of whole
+// components, and each group's solves by levels.
+int World::ensure_joint_schedule() {
+    DeviceWorld& d = d_;
+    const uint32_t iters = params_.joint_iterations;
+    if (path_ != StepPath::General || d.n_jcomp == 0 || d.j_iters == iters) return BG_OK;
+    dfree(d.jg), dfree(d.jl_start), dfree(d.j_entry), dfree(d.jg_body), dfree(d.jrot), dfree(d.jq_ab);
+    d.j_iters = d.n_jgroups = 0;
+    if (iters == 0) return BG_OK;
+    const uint32_t nj = (uint32_t)joint_bodies_.size();
+    if ((uint64_t)nj * iters > 0xFFFFFFFFull) return fail(BG_ERR_CAPACITY, "joint solves of a substep exceed 2^32");
+    JointSchedule sched;
+    std::vector<JointGroup> groups;
+    std::vector<int32_t> bodies, local(d.nb, -1);
+    std::vector<uint2> ab(nj);
+    std::vector<std::pair<uint32_t, uint32_t>> joints;
+    std::vector<uint32_t> ids, last;
+    for (uint32_t c = 0; c < d.n_jcomp;) {
+        JointGroup g;
+        g.q0 = joint_comp_start_[c];
+        g.b0 = (uint32_t)bodies.size();
+        g.l0 = (uint32_t)sched.level_start.size() - 1;
+        do
+            ++c;
+        while (c < d.n_jcomp && joint_comp_start_[c + 1] - g.q0 <= kGroupJoints);
+        g.q1 = joint_comp_start_[c];
+        joints.clear();
+        ids.clear();
+        for (uint32_t q = g.q0; q < g.q1; ++q) {
+            uint32_t l[2];
+            for (int e = 0; e < 2; ++e) {
+                const int32_t b = e ? joint_bodies_[q].second : joint_bodies_[q].first;
+                if (local[b] < 0) {
+                    local[b] = (int32_t)(bodies.size() - g.b0);
+                    bodies.push_back(b);
+                }
+                l[e] = (uint32_t)local[b];
+            }
+            ab[q].x = l[0] | (uint32_t)joint_static_[joint_bodies_[q].first] << 31;
+            ab[q].y = l[1] | (uint32_t)joint_static_[joint_bodies_[q].second] << 31;
+            joints.push_back({l[0], l[1]});
+            ids.push_back(q - g.q0);
+        }
+        g.b1 = (uint32_t)bodies.size();
+        last.assign(g.b1 - g.b0, 0);
+        sched.add_group(joints, ids, iters, last, BG_WAVE);
+        g.l1 = (uint32_t)sched.level_start.size() - 1;
+        groups.push_back(g);
+    }
+    std::vector<uint2> entry(sched.entry.size());
+    for (const JointGroup& g : groups)
+        for (uint32_t e = sched.level_start[g.l0]; e < sched.level_start[g.l1]; ++e)
+            entry[e] = make_uint2(sched.entry[e], sched.iteration[e] * nj + g.q0 + sched.entry[e]);
+    hipStream_t s = d.stream;
+    HIP_TRY(dmalloc(&d.jg, groups.size()));
+    HIP_TRY(dmalloc(&d.jl_start, sched.level_start.size()));
+    HIP_TRY(dmalloc(&d.j_entry, entry.size()));
+    HIP_TRY(dmalloc(&d.jg_body, bodies.size()));
+    HIP_TRY(dmalloc(&d.jq_ab, ab.size()));
+    HIP_TRY(dmalloc(&d.jrot, (size_t)iters * nj));
+    HIP_TRY(h2d(d.jg, groups, s));
+    HIP_TRY(h2d(d.jl_start, sched.level_start, s));
+    HIP_TRY(h2d(d.j_entry, entry, s));
+    HIP_TRY(h2d(d.jg_body, bodies, s));
+    HIP_TRY(h2d(d.jq_ab, ab, s));
+    HIP_TRY(hipStreamSynchronize(s));  // host vectors die at return
+    d.n_jgroups = (uint32_t)groups.size();
+    d.j_iters = iters;
     return BG_OK;
 }
 

@@ -145,6 +145,7 @@ private:
     int rebuild();
     int run_substep(float h, bool fresh, bool last);
     int prepare_step();
+    int ensure_joint_schedule();
     int launch_steps(double delta, uint32_t n);
     int launch_grid_steps(double delta, uint32_t n);
     int launch_persistent(double delta, uint32_t n, bool fresh, hipStream_t stream);
@@ -229,6 +230,11 @@ private:
     // dense <-> slot maps of the last upload
     std::vector<uint32_t> body_slot_of_dense_, col_slot_of_dense_;
     std::vector<int32_t> body_dense_of_slot_, col_dense_of_slot_;
+    // joints of the last upload in component order: their bodies (dense), the components'
+    // ranges, and per body whether it is static
+    std::vector<std::pair<int32_t, int32_t>> joint_bodies_;
+    std::vector<uint32_t> joint_comp_start_;
+    std::vector<uint8_t> joint_static_;
     // broadphase drift of the current rebuild period
     double drift_x_ = 0, drift_y_ = 0, vdrift_x_ = 0, vdrift_y_ = 0, h_prev_ = 0;
     uint64_t contact_base_ = 0;
