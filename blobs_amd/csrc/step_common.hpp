@@ -73,6 +73,11 @@ struct ContactList {
     }
 };
 
+// Q padded for the rounding of cell coordinates.
+__device__ __forceinline__ float stencil_reach(float2 q, float Q) {
+    return Q + (1e-5f * (fabsf(q.x) + fabsf(q.y) + Q) + 1e-6f);
+}
+
 // Visit every slot in the cells overlapping the square of half-width Q
 // around (qx, qy), in slot order, four at a time: visit(t, r, nv) gets slots
 // t .. t+nv-1 (nv in 1..4) with their records r[0..nv-1] (loaded together,
@@ -82,7 +87,7 @@ struct ContactList {
 template <class F>
 __device__ __forceinline__ void scan_stencil(const GridParams& g, const uint32_t* __restrict__ cell_start, uint32_t n,
                                              const float4* __restrict__ rec, float qx, float qy, float Q, F&& visit) {
-    float R = Q + (1e-5f * (fabsf(qx) + fabsf(qy) + Q) + 1e-6f);
+    const float R = stencil_reach(make_float2(qx, qy), Q);
     int32_t cx0, cx1, cy0, cy1;
     if (R < 1e30f && finitef(qx) && finitef(qy)) {
         cx0 = cell_coord(qx - R, g.ox, g.inv_cell, g.nx);
