@@ -131,7 +131,7 @@ struct DeviceWorld {
     // general path
     BodyArrays b{};
     ColliderArrays c{};
-    float2 *x0 = nullptr;  // collider snapshot at the last rebuild (sphere path: per slot)
+    float2 *x0 = nullptr;  // sphere path: snapshot at the last rebuild, per slot
     uint32_t *bc_start = nullptr, *bc_list = nullptr;  // body -> colliders
     // sphere path
     SphereArrays s{}, s_alt{};
@@ -173,9 +173,10 @@ struct DeviceWorld {
     uint32_t total_cells = 0;       // cell_base[n_worlds]
     uint32_t *tile_seg = nullptr;   // batch: per scan tile of the cell table, the world holding its first cell
     // springs
-    int32_t *sp_a = nullptr, *sp_b = nullptr;
-    float *sp_rest = nullptr, *sp_k = nullptr, *sp_c = nullptr;
-    uint32_t *bs_start = nullptr, *bs_list = nullptr;
+    // per body, a record for each of its springs in arena order: (other body | body is the
+    // spring's b << 31, rest length, stiffness, damping)
+    uint32_t *bs_start = nullptr;
+    float4 *bs_rec = nullptr;
     // joints, in component order (components of the joint graph, arena order inside each):
     // anchors (a.x, a.y, b.x, b.y); mass terms 1/m_a + 1/m_b, (1/m_a)/ims, 1 - that, and 1 if both
     // masses are positive (physics.rs:447-460; the same f32 operations, evaluated at upload);
@@ -344,7 +345,6 @@ struct KeysArgs {
     uint32_t* keys;
     uint32_t* rank;
     uint32_t* cnt;
-    float2* x0;
 };
 
 // Launchers (step_kernels.hip: general path + broadphase build).  A substep

@@ -827,7 +827,6 @@ __global__ __launch_bounds__(BG_WAVE) void k_world_grids(uint32_t n_worlds, uint
     const uint32_t w = blockIdx.x;
     const uint32_t lane = threadIdx.x;
     if (w == 0 && lane == 0) {
-        accum->dmax = 0u;
         accum->last_outliers = accum->n_outliers;
         accum->n_outliers = 0u;
     }

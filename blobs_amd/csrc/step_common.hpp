@@ -114,39 +114,6 @@ __device__ __forceinline__ void scan_stencil(const GridParams& g, const uint32_t
     }
 }
 
-__device__ __forceinline__ float read_dmax(const StepAccum* acc) {
-    float d = __uint_as_float(__hip_atomic_load(&acc->dmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    return d;
-}
-
-// Block-level reduction of the per-thread step records, one atomic each.
-struct LocalAccum {
-    float dmax;
-    float minx, miny, maxx, maxy;
-    uint32_t contacts;
-    uint32_t flags;
-    uint32_t push_outs;
-    __device__ __forceinline__ void init() {
-        dmax = 0.0f;
-        minx = miny = FLT_MAX;
-        maxx = maxy = -FLT_MAX;
-        contacts = 0;
-        flags = 0;
-        push_outs = 0;
-    }
-    __device__ __forceinline__ void point(float x, float y, float x0, float y0, float dx, float dy) {
-        if (finitef(x) && finitef(y)) {
-            minx = fminf(minx, x);
-            maxx = fmaxf(maxx, x);
-            miny = fminf(miny, y);
-            maxy = fmaxf(maxy, y);
-            float ex = (x - x0) - dx, ey = (y - y0) - dy;
-            float d = sqrtf(ex * ex + ey * ey);
-            if (finitef(d)) dmax = fmaxf(dmax, d);
-        }
-    }
-};
-
 // Only blocks that extend the running extremum issue an atomic (a relaxed
 // read first): thousands of blocks hitting one word serialize otherwise.
 __device__ __forceinline__ void atomic_max_if_greater(uint32_t* p, uint32_t v) {
@@ -154,58 +121,6 @@ __device__ __forceinline__ void atomic_max_if_greater(uint32_t* p, uint32_t v) {
 }
 __device__ __forceinline__ void atomic_min_if_less(uint32_t* p, uint32_t v) {
     if (v < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, v);
-}
-
-// Contacts go to a per-block slot (summed on the host when queried), never
-// to one shared counter.  Blocks of 64 to kThreads threads.
-static __device__ void flush_accum(const LocalAccum& l, StepAccum* g, unsigned long long* block_contacts, uint32_t parity,
-                            bool with_points) {
-    __shared__ uint32_t s_red[8][kThreads / BG_WAVE];
-    __shared__ unsigned long long s_cnt[kThreads / BG_WAVE];
-    const int lane = threadIdx.x & (BG_WAVE - 1), wid = threadIdx.x / BG_WAVE;
-    uint32_t v[8];
-    v[0] = with_points ? __float_as_uint(l.dmax) : 0u;
-    v[1] = f2ord(l.minx);
-    v[2] = f2ord(l.miny);
-    v[3] = f2ord(l.maxx);
-    v[4] = f2ord(l.maxy);
-    v[5] = l.flags;
-    v[6] = l.push_outs;
-    v[0] = wave_max_u32(v[0]);
-    v[1] = wave_min_u32(v[1]);
-    v[2] = wave_min_u32(v[2]);
-    v[3] = wave_max_u32(v[3]);
-    v[4] = wave_max_u32(v[4]);
-    for (int o = 32; o > 0; o >>= 1) v[5] |= __shfl_xor(v[5], o, BG_WAVE);
-    v[6] = wave_sum_u32(v[6]);
-    uint64_t c = wave_sum_u64((uint64_t)l.contacts);
-    if (lane == 0) {
-        for (int k = 0; k < 7; ++k) s_red[k][wid] = v[k];
-        s_cnt[wid] = c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x / BG_WAVE); ++w) {
-            s_red[0][0] = s_red[0][w] > s_red[0][0] ? s_red[0][w] : s_red[0][0];
-            s_red[1][0] = s_red[1][w] < s_red[1][0] ? s_red[1][w] : s_red[1][0];
-            s_red[2][0] = s_red[2][w] < s_red[2][0] ? s_red[2][w] : s_red[2][0];
-            s_red[3][0] = s_red[3][w] > s_red[3][0] ? s_red[3][w] : s_red[3][0];
-            s_red[4][0] = s_red[4][w] > s_red[4][0] ? s_red[4][w] : s_red[4][0];
-            s_red[5][0] |= s_red[5][w];
-            s_red[6][0] += s_red[6][w];
-            s_cnt[0] += s_cnt[w];
-        }
-        if (with_points) {
-            atomic_max_if_greater(&g->dmax, s_red[0][0]);
-            atomic_min_if_less(&g->bbox[parity][0], s_red[1][0]);
-            atomic_min_if_less(&g->bbox[parity][1], s_red[2][0]);
-            atomic_max_if_greater(&g->bbox[parity][2], s_red[3][0]);
-            atomic_max_if_greater(&g->bbox[parity][3], s_red[4][0]);
-        }
-        if (s_red[5][0]) atomicOr(&g->error_flags, s_red[5][0]);
-        if (s_red[6][0]) atomicAdd(&g->push_outs, s_red[6][0]);
-        if (s_cnt[0]) block_contacts[blockIdx.x] += s_cnt[0];
-    }
 }
 
 // ---- Verlet update of one body, physics.rs:326-358 -----------------------

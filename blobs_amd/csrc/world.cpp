@@ -126,7 +126,7 @@ int World::debug_accum(uint32_t* out4) {
     HIP_TRY(hipMemcpyAsync(&acc, d_.accum, sizeof(acc), hipMemcpyDeviceToHost, d_.stream));
     HIP_TRY(hipStreamSynchronize(d_.stream));
     out4[0] = acc.n_outliers;
-    out4[1] = acc.dmax;
+    out4[1] = 0;
     out4[2] = acc.push_outs;
     out4[3] = acc.error_flags;
     return BG_OK;
@@ -819,8 +819,7 @@ void World::free_arrays() {
     for (uint32_t c = 0; c < kPersistClasses; ++c) d.p_groups[c] = 0;
     d.p_grid_worlds = 0;
     dfree(d.snap_next), dfree(d.x0), dfree(d.bc_start), dfree(d.bc_list), dfree(d.nbr), dfree(d.nbr_len);
-    dfree(d.sp_a), dfree(d.sp_b), dfree(d.sp_rest), dfree(d.sp_k), dfree(d.sp_c), dfree(d.bs_start),
-        dfree(d.bs_list);
+    dfree(d.bs_start), dfree(d.bs_rec);
     dfree(d.jq_anchor), dfree(d.jq_mass), dfree(d.jq_len), dfree(d.jq_ab);
     dfree(d.jg), dfree(d.jl_start), dfree(d.j_entry), dfree(d.jg_body), dfree(d.jrot), dfree(d.bj_start), dfree(d.bj_list);
     dfree(d.con_pos),
@@ -1006,7 +1005,8 @@ int World::upload() {
     const uint32_t ns = springs_.len();
     std::vector<int32_t> sp_a, sp_b;
     std::vector<float> sp_rest, sp_k, sp_c;
-    std::vector<uint32_t> bs_count(nb + 1, 0), bs_start(nb + 1, 0), bs_list;
+    std::vector<uint32_t> bs_count(nb + 1, 0), bs_start(nb + 1, 0);
+    std::vector<float4> bs_rec;
     for (uint32_t s = 0; s < springs_.capacity_slots(); ++s) {
         if (!springs_.occupied(s)) continue;
         const bg_spring& sp = springs_.at_slot(s);
@@ -1028,12 +1028,16 @@ int World::upload() {
             bs_count[sp_b[s]]++;
         }
         for (uint32_t i = 0; i < nb; ++i) bs_start[i + 1] = bs_start[i] + bs_count[i];
-        bs_list.resize(bs_start[nb]);
+        bs_rec.resize(bs_start[nb]);
         std::vector<uint32_t> fillp(bs_start.begin(), bs_start.end() - 1);
-        for (uint32_t s = 0; s < ns; ++s) {
-            bs_list[fillp[sp_a[s]]++] = s;
-            bs_list[fillp[sp_b[s]]++] = s;
-        }
+        for (uint32_t s = 0; s < ns; ++s)
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t k = fillp[e ? sp_b[s] : sp_a[s]]++;
+                const uint32_t other = (uint32_t)(e ? sp_a[s] : sp_b[s]) | (e ? 0x80000000u : 0u);
+                float w;
+                memcpy(&w, &other, 4);
+                bs_rec[k] = make_float4(w, sp_rest[s], sp_k[s], sp_c[s]);
+            }
     }
 
     // joints (arena order), grouped into components of the body graph
@@ -1389,16 +1393,11 @@ int World::upload() {
         HIP_TRY(h2d(d.c.groups, cgrp, s));
         HIP_TRY(h2d(d.c.cflags, cfl, s));
     }
-    HIP_TRY(dmalloc(&d.x0, nc));
+    if (sphere) HIP_TRY(dmalloc(&d.x0, nb));
     HIP_TRY(dmalloc(&d.bc_start, nb + 1));
     HIP_TRY(dmalloc(&d.bc_list, bc_list.size()));
-    HIP_TRY(dmalloc(&d.sp_a, ns));
-    HIP_TRY(dmalloc(&d.sp_b, ns));
-    HIP_TRY(dmalloc(&d.sp_rest, ns));
-    HIP_TRY(dmalloc(&d.sp_k, ns));
-    HIP_TRY(dmalloc(&d.sp_c, ns));
     HIP_TRY(dmalloc(&d.bs_start, nb + 1));
-    HIP_TRY(dmalloc(&d.bs_list, bs_list.size()));
+    HIP_TRY(dmalloc(&d.bs_rec, bs_rec.size()));
     d.j_iters = d.n_jgroups = 0;  // the schedule of the sweep: ensure_joint_schedule
     HIP_TRY(dmalloc(&d.bj_start, bj_start.size()));
     HIP_TRY(dmalloc(&d.bj_list, bj_list.size()));
@@ -1557,13 +1556,8 @@ int World::upload() {
 
     HIP_TRY(h2d(d.bc_start, bc_start, s));
     HIP_TRY(h2d(d.bc_list, bc_list, s));
-    HIP_TRY(h2d(d.sp_a, sp_a, s));
-    HIP_TRY(h2d(d.sp_b, sp_b, s));
-    HIP_TRY(h2d(d.sp_rest, sp_rest, s));
-    HIP_TRY(h2d(d.sp_k, sp_k, s));
-    HIP_TRY(h2d(d.sp_c, sp_c, s));
     HIP_TRY(h2d(d.bs_start, bs_start, s));
-    HIP_TRY(h2d(d.bs_list, bs_list, s));
+    HIP_TRY(h2d(d.bs_rec, bs_rec, s));
     HIP_TRY(h2d(d.bj_start, bj_start, s));
     HIP_TRY(h2d(d.bj_list, bj_list, s));
     HIP_TRY(h2d(d.jq_anchor, jq_anchor, s));
@@ -1698,7 +1692,7 @@ int World::rebuild() {
     } else {
         // launched by the substep, beside its forces
         keys_ = KeysArgs{d.c.abs, d.nc, d.accum, bbox_parity_, cell, d.cells_cap, d.grid, d.keys, d.vals_tmp,
-                         d.cell_count, d.x0};
+                         d.cell_count};
         keys_pending_ = true;
     }
     if (int st = stage_end(BG_STAGE_REBUILD)) return st;
