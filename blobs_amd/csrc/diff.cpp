@@ -279,6 +279,14 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
     ns_ = (uint32_t)k_.size();
     nj_ = (uint32_t)j_ab.size();
     n_solves_ = (uint32_t)sched.entry.size();
+    // One workgroup size for all: a thread for each body of the largest world (two each past 1,024),
+    // and for each solve of a world whose joints are staged in LDS.
+    threads_ = 256;
+    for (const DiffWorld& w : ws) {
+        uint32_t need = w.nb;
+        if (w.nje <= kDiffThreads) need = std::max(need, w.nje);
+        while (threads_ < need && threads_ < kDiffMaxBodies) threads_ *= 2;
+    }
     n_worlds_ = n;
     body0_.resize(n + 1);
     for (uint32_t w = 0; w < n; ++w) body0_[w] = ws[w].b0;
@@ -422,6 +430,7 @@ DiffArgs Rollout::args() const {
     a.worlds = d_worlds_;
     a.n_worlds = n_worlds_;
     a.nb_total = nb_;
+    a.threads = threads_;
     a.mass = d_mass_;
     a.radius = d_radius_;
     a.gmod = d_gmod_;

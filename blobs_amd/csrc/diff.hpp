@@ -26,7 +26,6 @@ namespace bg {
 constexpr uint32_t kDiffThreads = 1024;
 constexpr uint32_t kDiffPer = 2;                                // bodies per thread
 constexpr uint32_t kDiffMaxBodies = kDiffThreads * kDiffPer;    // per world
-constexpr uint32_t kDiffCells = 4096;                           // LDS grid cells per world
 constexpr uint32_t kDiffTapeNbr = 8;                            // u16 per tape record: count + 7 partners
 
 struct DiffWorld {
@@ -45,6 +44,7 @@ struct DiffWorld {
 struct DiffArgs {
     const DiffWorld* worlds;
     uint32_t n_worlds, nb_total;
+    uint32_t threads;  // of a workgroup, a body each: 256, 512, 1,024, or more for kDiffThreads with two bodies each
     // bodies, global index
     const float* mass;
     const float* radius;
@@ -134,7 +134,7 @@ private:
 
     hipStream_t stream_ = nullptr;
     uint32_t n_worlds_ = 0, nb_ = 0, ns_ = 0, substeps_ = 8, ck_every_ = 20, n_steps_ = 0;
-    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, cus_ = 1, nj_ = 0, n_solves_ = 0, j_iters_ = 0;
+    uint32_t n_ck_alloc_ = 0, tape_sub_alloc_ = 0, cus_ = 1, nj_ = 0, n_solves_ = 0, j_iters_ = 0, threads_ = 0;
     float gx_ = 0.0f, gy_ = 0.0f, h_ = 0.0f;
     bool collisions_ = true, damped_ = false, have_forward_ = false;
     std::vector<uint8_t> nonfinite_;  // per world, after the last backward: a gradient entry is inf or NaN

@@ -1,28 +1,39 @@
 // diff_kernels.hip -- forward and adjoint of rollouts of single-sphere worlds
-// with springs, one 1024-thread workgroup per world for a whole segment of
-// steps (two bodies per thread; positions, velocities, the cell grid, the
-// spring forces, the joint records and the adjoint vectors live in LDS).
+// with springs, one workgroup per world for a whole segment of steps: a body a
+// thread and as few threads as hold the largest world (256, 512, 1,024; two
+// bodies a thread past that).  Positions, velocities, partner lists, the spring
+// forces, the joint records and the adjoint vectors live in LDS.
 //
 // Forward substep (physics.rs:401-421, same f32 operation order as the
 // general path): gravity and springs per body in ascending spring index
 // (springs.rs:25-47), contacts against the substep's snapshot summed in
 // ascending partner index (physics.rs:241-317), Verlet (physics.rs:323-358),
-// collider transform = position (zero offsets).  The bodies are filed by cell
-// in LDS every substep (lds_grid.hpp): counts with LDS atomics, a block scan,
-// and a scatter of (x, y, radius, index) records.
+// collider transform = position (zero offsets).
 //
 // A world has one workgroup, so a launch takes what its slowest world takes
 // and a substep is bound by VALU issue and by its chain of phases (a barrier
-// between them).  Hence contacts worked out from a queue by all threads; springs evaluated once each by a thread of their
-// own (at most kDiffLdsSprings; a body then sums its springs' terms from LDS
-// in ascending index), joints swept on records staged in LDS, and the next
-// tape slot loaded while the reverse works on the current one.  Recompute and
-// reverse are kernels of their own: in one, their state spilled 55 VGPRs.
+// between them).  Hence contacts worked out from a queue by all threads;
+// springs evaluated once each by a thread of their own (at most
+// kDiffLdsSprings; a body then sums its springs' terms from LDS in ascending
+// index); joints swept level by level on records staged in LDS
+// (joint_schedule.hpp); and the next tape slot loaded while the reverse works
+// on the current one.  Recompute and reverse are kernels of their own: in one,
+// their state spilled 55 VGPRs.
+//
+// Partner lists.  Most bodies of such worlds move a thousandth of a diameter a
+// substep and a few a twentieth, so a list of the bodies within two skins of
+// reach serves for tens of substeps.  A body is in reach of another only if
+// the two paths since the build, the world's mean motion taken out, add up to
+// the rest, so a body whose path exceeds the skin leaves the lists and is tested
+// by everyone (its own pairs come from those tests), until the tests cost as
+// much as a build.  A world too dense for lists is filed by cell every substep.
+//
 // Measured (forward + backward, against bounding box, grid, springs and contacts
-// worked out serially or per body each substep): 256 worlds of 2,048 bodies and
-// 1,024 springs over 50 steps 33.2 -> 15.4 ms (17.5 before the queue of pairs);
-// 96 worlds of 700, 60 steps forward 7.24 -> 3.24 ms (3.62); 12 worlds of 301
-// with 40 joints, 6 steps 3.80 -> 2.24 ms (2.31).
+// worked out serially or per body each substep; in brackets with a grid and
+// 1,024 threads for every world in every substep): 256 worlds of 2,048 bodies and
+// 1,024 springs over 50 steps 33.2 -> 14.8 ms (15.4); 96 worlds of 700, 60 steps
+// forward 7.24 -> 2.66 ms (3.13); 12 worlds of 301 with 40 joints, 6 steps 3.80 ->
+// 1.51 ms (1.61); 512 worlds of 300, 20 steps 1.11 ms (1.98).
 #include "diff.hpp"
 
 #include <algorithm>
@@ -33,19 +44,30 @@ namespace bg {
 
 namespace {
 
-constexpr int kWaves = kDiffThreads / BG_WAVE;
-constexpr uint32_t kScanItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThreads;
+// A world's workgroup: NT threads, PER bodies a thread.
+template <uint32_t NT, uint32_t PER>
+struct Rollout {
+static constexpr uint32_t kDiffThreads = NT, kDiffMaxBodies = NT * PER;
+static constexpr uint32_t kDiffCells = PER == 1 ? 2 * NT : 3 * NT;
+static constexpr uint32_t kPairs = PER == 1 ? NT + NT / 4 : 1200;  // queued contact pairs of a substep
+static constexpr int kWaves = NT / BG_WAVE;
+static constexpr uint32_t kScanItems = (kDiffCells + 1 + kDiffThreads - 1) / kDiffThreads;
 // Springs of a world whose terms are kept in LDS (32 KB of it); a world with more evaluates
 // them per body.
-constexpr uint32_t kDiffLdsSprings = 2048;
+static constexpr uint32_t kDiffLdsSprings = 2048;
 // A world whose joint records and schedule are staged in LDS has at most so many joints,
 // solves a substep and levels of them.
-constexpr uint32_t kDiffLdsJoints = 256, kDiffLdsSolves = 1024, kDiffLdsLevels = 512;
-constexpr uint32_t kCntStride = kDiffCells + 4;  // (a multiple of 16 bytes)
-constexpr uint32_t kPairs = 1360;          // queued contact pairs of a substep: 12 bytes each of a cell table
+static constexpr uint32_t kDiffLdsJoints = 256, kDiffLdsSolves = NT, kDiffLdsLevels = 512;
+// Partner lists: entries of a body, bodies outside the lists and queued pairs of each, builds with
+// the skin halved while too many lists overflow, and the substeps a world that overflows them all
+// goes without.  The skin in diameters of the largest body: with 0.1 the four cases above take
+// 15.6, 3.03, 1.50 and 1.17 ms, with 0.3 16.3, 2.79, 1.54 and 1.11.
+static constexpr uint32_t kListCap = 8, kOutMax = 16, kOutPairs = 8, kListTries = 3, kGridHold = 64;
+static constexpr float kSkin = 0.2f;
+static constexpr uint32_t kTested = 24;           // a build costs about what so many tests of a body outside the lists do
+static constexpr uint32_t kOut = 15;              // Own::nl of a body outside the lists
 static_assert(kDiffLdsSolves <= kDiffThreads, "a thread stages one axis");
-static_assert(12 * kPairs <= 4 * kDiffCells, "the queue fits the idle cell table");
-constexpr uint32_t kInc = 4;               // springs of a body kept as packed registers
+static constexpr uint32_t kInc = 4;               // springs of a body kept as packed registers
 
 struct JointRec {
     float4 anchor;  // a (x, y), b (z, w)
@@ -58,16 +80,38 @@ struct JointStage {
     uint16_t entry[kDiffLdsSolves], level[kDiffLdsLevels + 1];
 };
 
+// Bodies outside the lists, by substep parity where a phase clears what another reads.
+struct Outliers {
+    uint32_t n;           // (may exceed kOutMax: then the lists are built anew)
+    uint32_t pairs[2];    // queued pairs
+    uint16_t id[kOutMax];
+    uint32_t count[2][kOutMax];  // pairs of an outlier, in the queue's entries from kPairs + u * kOutPairs
+};
+// The lists' state, the same in every thread.
+struct Walk {
+    float skin;
+    float2 drift;  // the world's common motion a substep
+    uint32_t grid; // substeps left without lists
+    uint32_t tested;  // bodies outside the lists, summed over the substeps since the build
+    bool build;
+};
+
 struct Ctx {
     float2* xy;        // positions (the snapshot)
     float2* vel;       // calculated_velocity
     float* mass;
-    float4* rec;       // bodies in cell order; the reverse's snapshot (x, y, radius, mass) by index
+    float* rad;        // radii
+    float4* rec;       // bodies in cell order (the memory of `force` or of `lists`); the reverse's
+                       // snapshot (x, y, radius, mass) by index
+    uint16_t (*lists)[kDiffMaxBodies][4];  // [kListCap / 4]: partners by body; forward only
+    float2* res;       // [kPairs] corrections of the queue; forward only
+    uint32_t* entries; // [kPairs] its pairs
+    Outliers* out;
     float* gmod;       // gravity_mod; forward only
-    uint32_t* cnt;     // two tables of kCntStride: cell counts, then cell starts; the other one is cleared meanwhile
+    uint32_t* cnt;     // [kDiffCells + 1] cell counts, then cell starts; forward only
+    float2 *spring_k, *spring_v;  // spring adjoints; reverse only
     float4* force;     // per spring: (Fx / m_a, Fy / m_a, -Fx / m_b, -Fy / m_b); forward only
     uint32_t* red;     // [kFitWords][kWaves]
-    uint32_t* pairs;   // queued pairs of this substep
     double* dred;      // [2][kWaves]
     LdsGrid* grid;
     JointStage* joints;  // of a staged world
@@ -79,49 +123,69 @@ struct Ctx {
 // A thread's two bodies.  The phases loop over them at run time and pick the state by
 // selects: unrolled, two bodies' contact passes in flight spill 50 to 140 VGPRs.
 struct Own {
-    float2 p[2], q[2];
-    float r[2];
-    uint32_t fl[2];             // body flags | springs of the body << 8 (at most kIncMany: more are counted anew)
-    uint32_t inc0[2], inc1[2];  // first kInc springs, two a word: local spring << 1 | (1: the body is its b)
+    float2 p[PER], q[PER];
+    float travel[PER];            // path since the lists were built, the common motion taken out
+    uint32_t nl;                // list lengths, four bits each (kOut: outside the lists)
+    uint32_t fl[PER];             // body flags | springs of the body << 8 (at most kIncMany: more are counted anew)
+    uint32_t inc0[PER], inc1[PER];  // first kInc springs, two a word: local spring << 1 | (1: the body is its b)
     // the spring this thread evaluates first
     uint32_t s_ab;
     float s_rest, s_k, s_c;
 };
-constexpr uint32_t kIncMany = 0xFFFFFFu;
-static_assert(kDiffPer == 2, "two bodies a thread");
+static constexpr uint32_t kIncMany = 0xFFFFFFu;
+static_assert(PER == 1 || PER == 2, "the picks");
 template <class T>
-__device__ __forceinline__ T pick(const T (&v)[2], uint32_t j) {
-    return j ? v[1] : v[0];
+static __device__ __forceinline__ T pick(const T (&v)[PER], uint32_t j) {
+    if constexpr (PER == 1)
+        return v[0];
+    else
+        return j ? v[1] : v[0];
 }
-__device__ __forceinline__ float2 pick(const float2 (&v)[2], uint32_t j) {
-    return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
+static __device__ __forceinline__ float2 pick(const float2 (&v)[PER], uint32_t j) {
+    if constexpr (PER == 1)
+        return v[0];
+    else
+        return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
 }
-__device__ __forceinline__ void put(float2 (&v)[2], uint32_t j, float2 x) {
-    v[0].x = j ? v[0].x : x.x;
-    v[0].y = j ? v[0].y : x.y;
-    v[1].x = j ? x.x : v[1].x;
-    v[1].y = j ? x.y : v[1].y;
+template <class T>
+static __device__ __forceinline__ void put(T (&v)[PER], uint32_t j, T x) {
+    if constexpr (PER == 1) {
+        v[0] = x;
+    } else {
+        v[0] = j ? v[0] : x;
+        v[1] = j ? x : v[1];
+    }
 }
-__device__ __forceinline__ uint32_t per_thread(const DiffWorld& W) { return W.nb > kDiffThreads ? 2u : 1u; }
+static __device__ __forceinline__ void put(float2 (&v)[PER], uint32_t j, float2 x) {
+    if constexpr (PER == 1) {
+        v[0] = x;
+    } else {
+        v[0].x = j ? v[0].x : x.x;
+        v[0].y = j ? v[0].y : x.y;
+        v[1].x = j ? x.x : v[1].x;
+        v[1].y = j ? x.y : v[1].y;
+    }
+}
+static __device__ __forceinline__ uint32_t per_thread(const DiffWorld& W) { return PER == 1 || W.nb <= NT ? 1u : 2u; }
 
 // The thread's index, opaque to the compiler: the phases of a substep recompute what they
 // derive from it, where hoisted out of the substep loop those addresses spill.
-__device__ __forceinline__ uint32_t thread_index() {
+static __device__ __forceinline__ uint32_t thread_index() {
     uint32_t t = threadIdx.x;
     asm volatile("" : "+v"(t));
     return t;
 }
 
-__device__ __forceinline__ bool lds_springs(const DiffWorld& W) { return W.ns <= kDiffLdsSprings; }
+static __device__ __forceinline__ bool lds_springs(const DiffWorld& W) { return W.ns <= kDiffLdsSprings; }
 
-__device__ __forceinline__ bool joints_staged(const DiffWorld& W) {
+static __device__ __forceinline__ bool joints_staged(const DiffWorld& W) {
     return W.njq <= kDiffLdsJoints && W.nje <= kDiffLdsSolves && W.njl <= kDiffLdsLevels;
 }
 
 // Joint q of the world: from LDS in a staged world, else from global memory.  (Templates:
 // where the two meet in one load it becomes a flat one.)
 template <bool STAGED>
-__device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArgs& a, const DiffWorld& W, uint32_t q) {
+static __device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArgs& a, const DiffWorld& W, uint32_t q) {
     JointRec r;
     if constexpr (STAGED) {
         r.anchor = c.joints->anchor[q];
@@ -143,7 +207,7 @@ static_assert(kDiffMaxBodies <= 0x7FFF, "15-bit body indices in JointRec::ab");
 // of the world.  REVERSE: from the last level to the first.  The next level's records load
 // while the current one works.
 template <bool STAGED, bool REVERSE, class Solve>
-__device__ __forceinline__ void joint_levels(const Ctx& c, const DiffArgs& a, const DiffWorld& W, Solve&& solve) {
+static __device__ __forceinline__ void joint_levels(const Ctx& c, const DiffArgs& a, const DiffWorld& W, Solve&& solve) {
     const uint32_t lane = threadIdx.x & (BG_WAVE - 1);
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / BG_WAVE));
     for (uint32_t grp = W.jg0 + wave; grp < W.jg0 + W.njg; grp += kWaves) {
@@ -184,22 +248,23 @@ __device__ __forceinline__ void joint_levels(const Ctx& c, const DiffArgs& a, co
     }
 }
 
-__device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, const float2* p,
+static __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, const float2* p,
                                          const float2* q, const float2* v) {
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
+    for (uint32_t j = 0; j < PER; ++j) {
         const uint32_t li = threadIdx.x + j * kDiffThreads;
         const bool live = li < W.nb;
         const uint32_t g = W.b0 + (live ? li : 0u);
         o.p[j] = live ? p[g] : make_float2(0.0f, 0.0f);
         o.q[j] = live ? q[g] : make_float2(0.0f, 0.0f);
-        o.r[j] = a.radius[g];
+        o.travel[j] = 0.0f;
         o.fl[j] = a.flags[g] & 0xFFu;
         o.inc0[j] = o.inc1[j] = 0;
         if (!live) continue;
         c.xy[li] = o.p[j];
         c.vel[li] = v[g];
         c.mass[li] = a.mass[g];
+        c.rad[li] = a.radius[g];
         if (c.gmod) c.gmod[li] = a.gmod[g];
         const uint32_t e0 = a.inc_start[g], n_inc = a.inc_start[g + 1] - e0;
         o.fl[j] |= min(n_inc, kIncMany) << 8;
@@ -213,6 +278,7 @@ __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, cons
                 }
         }
     }
+    o.nl = 0;
     o.s_ab = 0;
     o.s_rest = o.s_k = o.s_c = 0.0f;
     if (threadIdx.x < W.ns) {
@@ -222,7 +288,6 @@ __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, cons
         o.s_k = a.sp_k[s];
         o.s_c = a.sp_c[s];
     }
-    for (uint32_t i = threadIdx.x; i <= kDiffCells; i += kDiffThreads) c.cnt[i] = 0u;
     if (W.njg > 0 && joints_staged(W)) {
         for (uint32_t k = threadIdx.x; k < W.njq; k += kDiffThreads) {
             const JointRec r = joint_rec<false>(c, a, W, k);
@@ -239,7 +304,7 @@ __device__ __forceinline__ void load_own(Ctx& c, Own& o, const DiffArgs& a, cons
 
 // f(incidence) over body j's springs in ascending index; incidence as in Own::inc0.
 template <class F>
-__device__ __forceinline__ void for_springs(const Own& o, uint32_t j, const DiffArgs& a, const DiffWorld& W, F&& f) {
+static __device__ __forceinline__ void for_springs(const Own& o, uint32_t j, const DiffArgs& a, const DiffWorld& W, F&& f) {
     const uint32_t n = pick(o.fl, j) >> 8, w0 = pick(o.inc0, j), w1 = pick(o.inc1, j);
     if (n > 0) f(w0 & 0xFFFFu);
     if (n > 1) f(w0 >> 16);
@@ -257,7 +322,7 @@ __device__ __forceinline__ void for_springs(const Own& o, uint32_t j, const Diff
 
 // f(local spring, local a, local b, rest, k, c) over the springs this thread evaluates.
 template <class F>
-__device__ __forceinline__ void own_springs(const Own& o, const DiffArgs& a, const DiffWorld& W, F&& f) {
+static __device__ __forceinline__ void own_springs(const Own& o, const DiffArgs& a, const DiffWorld& W, F&& f) {
     uint32_t ab = o.s_ab;
     float rest = o.s_rest, k = o.s_k, cc = o.s_c;
     for (uint32_t t = threadIdx.x; t < W.ns;) {
@@ -274,7 +339,7 @@ __device__ __forceinline__ void own_springs(const Own& o, const DiffArgs& a, con
 }
 
 // Force of one spring on its body a (springs.rs:25-47); -F acts on b.
-__device__ __forceinline__ float2 spring_force(float2 pa, float2 pb, float2 va, float2 vb, float rest, float k, float c) {
+static __device__ __forceinline__ float2 spring_force(float2 pa, float2 pb, float2 va, float2 vb, float rest, float k, float c) {
     const float dx = pb.x - pa.x, dy = pb.y - pa.y;
     const float dist = vlen(dx, dy);
     const float ux = dx / dist, uy = dy / dist;
@@ -289,7 +354,7 @@ __device__ __forceinline__ float2 spring_force(float2 pa, float2 pb, float2 va, 
 // Position sweep of the world's joints (physics.rs:426-460) on the LDS positions P; with REC
 // every solve's anchor axis is recorded.
 template <bool REC, bool STAGED>
-__device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, const DiffArgs& a, const DiffWorld& W, uint32_t slot) {
+static __device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, const DiffArgs& a, const DiffWorld& W, uint32_t slot) {
     uint32_t flags = 0;
     joint_levels<STAGED, false>(c, a, W, [&](uint32_t e, const JointRec& r) {
         const uint32_t la = r.ab & 0x7FFFu, lb = (r.ab >> 16) & 0x7FFFu;
@@ -309,7 +374,7 @@ __device__ __forceinline__ void joint_sweep(Ctx& c, float2* P, const DiffArgs& a
 // Adjoint of joint_sweep on the LDS position adjoints L, from the axes the
 // forward sweep recorded: last solve first.
 template <bool STAGED>
-__device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, const DiffArgs& a, const DiffWorld& W,
+static __device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, const DiffArgs& a, const DiffWorld& W,
                                                     uint32_t slot) {
     joint_levels<STAGED, true>(c, a, W, [&](uint32_t e, const JointRec& r) {
         float2 d;
@@ -338,8 +403,8 @@ __device__ __forceinline__ void joint_sweep_reverse(Ctx& c, float2* L, const Dif
 
 // update_objects of body j (physics.rs:326-358) from its position after the contact and joint
 // stages; the snapshot is the new position.
-__device__ __forceinline__ void verlet(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub, uint32_t j,
-                                       float2 pn, float2 acc) {
+static __device__ __forceinline__ void verlet(Ctx& c, Own& o, const Walk& w, const DiffArgs& a, const DiffWorld& W,
+                                       uint32_t gsub, uint32_t j, float2 pn, float2 acc) {
     const uint32_t tid = thread_index();
     const float h = a.h;
     const uint32_t li = tid + j * kDiffThreads, fl = pick(o.fl, j);
@@ -357,42 +422,198 @@ __device__ __forceinline__ void verlet(Ctx& c, Own& o, const DiffArgs& a, const 
         const float ratio = ((int32_t)li == W.first_dyn && gsub == 0) ? h / W.old_dt0 : h / h;
         verlet_dynamic(st, acc, 0.0f, vr, vq, h, ratio);
     }
+    const float2 before = pick(o.p, j);
     put(o.p, j, st.p);
     put(o.q, j, st.po);
     c.xy[li] = st.p;
     c.vel[li] = st.vel;
+    // (an upper bound will do: the root's last bits do not matter)
+    const float tx = (st.p.x - before.x) - w.drift.x, ty = (st.p.y - before.y) - w.drift.y;
+    const float travel = pick(o.travel, j) + 1.0001f * __builtin_amdgcn_sqrtf(tx * tx + ty * ty);
+    put(o.travel, j, travel);
+    if (finitef(st.p.x) && finitef(st.p.y) && !(travel <= w.skin) && ((o.nl >> (4u * j)) & 15u) != kOut) {
+        const uint32_t u = atomicAdd(&c.out->n, 1u);
+        if (u < kOutMax) {
+            c.out->id[u] = (uint16_t)li;
+            o.nl |= kOut << (4u * j);
+        }
+    }
+}
+
+// The bodies filed by cell (rec, c.cnt) and, unless w.grid, everyone's list of the bodies it could
+// touch until one of the two has travelled w.skin.
+static __device__ __forceinline__ void build_lists(Ctx& c, Own& o, Walk& w, const DiffArgs& a, const DiffWorld& W) {
+    const uint32_t tid = thread_index();
+    const uint32_t per = per_thread(W);
+    if (w.grid == 0 || w.grid % kFitEvery == 0) {
+        LdsFit f;
+        f.init();
+#pragma unroll
+        for (uint32_t j = 0; j < PER; ++j)
+            if (tid + j * kDiffThreads < W.nb) {
+                f.point(o.p[j].x, o.p[j].y);
+                if (!(o.fl[j] & BF_STATIC)) f.extra(o.p[j].x - o.q[j].x, o.p[j].y - o.q[j].y);
+            }
+        lds_fit<kDiffThreads>(f, 2.004f * (W.rmax + (w.grid ? 0.0f : w.skin)), kDiffCells, c.red, c.grid);
+    }
+    const LdsGrid g = lds_grid_uniform(*c.grid);
+    w.drift = make_float2(g.ex, g.ey);
+    w.tested = 0;
+    for (uint32_t i = tid; i <= g.ncells; i += kDiffThreads) c.cnt[i] = 0u;
+    if (tid == 0) c.out->n = 0;
+    __syncthreads();
+    uint32_t key[PER] = {}, at[PER] = {};
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j)
+        if (tid + j * kDiffThreads < W.nb) {
+            key[j] = lds_cell(g, o.p[j].x, o.p[j].y);
+            at[j] = atomicAdd(&c.cnt[key[j]], 1u);
+        }
+    __syncthreads();
+    lds_scan<kDiffThreads, kScanItems>(c.cnt, g.ncells + 1u, c.red);
+    c.rec = w.grid ? reinterpret_cast<float4*>(c.lists) : c.force;
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        if (li >= W.nb) continue;
+        at[j] += c.cnt[key[j]];
+        c.rec[at[j]] = make_float4(o.p[j].x, o.p[j].y, c.rad[li], __uint_as_float(li));
+        o.travel[j] = 0.0f;
+    }
+    __syncthreads();
+    if (w.grid) return;
+    for (uint32_t tries = 1;; ++tries) {
+        o.nl = 0;
+#pragma unroll 1
+        for (uint32_t j = 0; j < per; ++j) {
+            const uint32_t li = tid + j * kDiffThreads;
+            const float2 xy = pick(o.p, j);
+            if (li >= W.nb || !finitef(xy.x) || !finitef(xy.y)) continue;
+            const float r = c.rad[li];
+            const float reach = r + 2.0f * w.skin + (1e-4f * (r + W.rmax + 2.0f * w.skin) + 1e-5f);
+            const LdsRows l = lds_rows(g, c.cnt, true, xy, reach + W.rmax);
+            const uint64_t near = lds_near(l, c.rec, [&](uint32_t, const float4& b) {
+                const float dx = xy.x - b.x, dy = xy.y - b.y, rs = reach + b.z;
+                return !((__float_as_uint(b.w) == li) | (dx * dx + dy * dy > rs * rs));
+            });
+            const uint32_t n = (uint32_t)__popcll(near);
+            if (l.flat && n <= kListCap) {
+                uint32_t i = 0;
+                for (uint64_t m = near; m != 0; m &= m - 1, ++i)
+                    c.lists[i >> 2][li][i & 3u] =
+                        (uint16_t)__float_as_uint(c.rec[l.slot((uint32_t)__builtin_ctzll(m))].w);
+                for (; (i & 3u) != 0u; ++i) c.lists[i >> 2][li][i & 3u] = (uint16_t)li;  // (whole groups are read)
+                o.nl |= n << (4u * j);
+            } else {
+                const uint32_t u = atomicAdd(&c.out->n, 1u);
+                if (u < kOutMax) c.out->id[u] = (uint16_t)li;
+                o.nl |= kOut << (4u * j);
+            }
+        }
+        static_assert(kListCap < kOut && kListCap <= 8, "four bits; the mask below");
+        __syncthreads();
+        if (c.out->n <= kOutMax) break;
+        __syncthreads();
+        if (tries == kListTries) {  // the world is too dense for lists: file it every substep
+            w.grid = kGridHold;
+            w.skin = kSkin * 2.0f * W.rmax;
+            c.rec = reinterpret_cast<float4*>(c.lists);
+#pragma unroll
+            for (uint32_t j = 0; j < PER; ++j) {
+                const uint32_t li = tid + j * kDiffThreads;
+                if (li < W.nb) c.rec[at[j]] = make_float4(o.p[j].x, o.p[j].y, c.rad[li], __uint_as_float(li));
+            }
+            if (tid == 0) c.out->n = 0;
+            __syncthreads();
+            break;
+        }
+        w.skin *= 0.5f;
+        if (tid == 0) c.out->n = 0;
+        __syncthreads();
+    }
+}
+
+// Mark phase of the lists: the pairs within reach go into the queue.  Returns body 0's and body
+// 1's pairs, first | n << 16 (n kNoRoom: worked out by the body's thread).
+static constexpr uint32_t kNoRoom = 0xFFFFu;
+static __device__ __forceinline__ void mark_lists(Ctx& c, const Own& o, const DiffWorld& W, uint32_t par,
+                                           uint32_t (&pr)[PER]) {
+    const uint32_t tid = thread_index();
+    const uint32_t per = per_thread(W);
+    const uint32_t nout = (uint32_t)__builtin_amdgcn_readfirstlane((int)c.out->n);
+    uint32_t* count = &c.out->pairs[par];
+    auto within = [&](float2 p, float r, float2 b, float rb) {
+        const float dx = p.x - b.x, dy = p.y - b.y, rs = r + rb;
+        return !(dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f);
+    };
+    auto near = [&](float2 p, float r, uint32_t lj) { return within(p, r, c.xy[lj], c.rad[lj]); };
+    // the outliers, one a lane, read from there by every lane
+    const uint32_t lane = tid & (BG_WAVE - 1);
+    const uint32_t out_id = lane < nout ? c.out->id[lane] : 0u;
+    const float2 out_p = c.xy[out_id];
+    const float out_r = c.rad[out_id];
+    auto of_lane = [](float v, uint32_t u) {
+        return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (int)u));
+    };
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        uint32_t marked = 0;
+        const uint32_t nl = (o.nl >> (4u * j)) & 15u;
+        const float2 p = pick(o.p, j);
+        if (li < W.nb && finitef(p.x) && finitef(p.y)) {
+            const float r = c.rad[li];
+            const uint32_t n = nl != kOut ? nl : 0u;
+            uint2 l[kListCap / 4];
+#pragma unroll
+            for (uint32_t f = 0; f < kListCap / 4; ++f) {
+                l[f] = make_uint2(0u, 0u);
+                if (4 * f >= n) continue;
+                l[f] = *(const uint2*)c.lists[f][li];
+                marked |= ((near(p, r, l[f].x & 0xFFFFu) ? 1u : 0u) | (near(p, r, l[f].x >> 16) ? 2u : 0u) |
+                           (near(p, r, l[f].y & 0xFFFFu) ? 4u : 0u) | (near(p, r, l[f].y >> 16) ? 8u : 0u))
+                          << (4 * f);
+            }
+            marked &= (1u << n) - 1u;
+            // (a body outside the lists leaves its pairs with the others to them)
+            for (uint32_t u = 0; u < nout; ++u) {
+                const uint32_t lj = (uint32_t)__builtin_amdgcn_readlane((int)out_id, (int)u);
+                if (lj == li || !within(p, r, make_float2(of_lane(out_p.x, u), of_lane(out_p.y, u)), of_lane(out_r, u)))
+                    continue;
+                bool listed = false;  // (then its entry has been marked)
+#pragma unroll
+                for (uint32_t f = 0; f < kListCap / 4; ++f) {
+                    listed |= 4 * f < n && (l[f].x & 0xFFFFu) == lj;
+                    listed |= 4 * f + 1 < n && (l[f].x >> 16) == lj;
+                    listed |= 4 * f + 2 < n && (l[f].y & 0xFFFFu) == lj;
+                    listed |= 4 * f + 3 < n && (l[f].y >> 16) == lj;
+                }
+                if (!listed && nl != kOut) marked |= 1u << (kListCap + u);
+                // and the pair from the other's side
+                const uint32_t k = atomicAdd(&c.out->count[par][u], 1u);
+                if (k < kOutPairs) c.entries[kPairs + u * kOutPairs + k] = (lj << 16) | li;
+            }
+        }
+        const LdsPairs q = lds_queue<kPairs>(marked, li, c.entries, count, [&](uint32_t i) {
+            return i < kListCap ? (uint32_t)c.lists[i >> 2][li][i & 3u] : (uint32_t)c.out->id[i - kListCap];
+        });
+        put(pr, j, q.first | (q.direct ? kNoRoom : q.n) << 16);
+    }
+    static_assert(kListCap + kOutMax <= 32, "the mask");
 }
 
 // One forward substep of the world (`n` counts this launch's substeps); with
 // REC, records the snapshot, contact partners, velocities (damped springs) and
 // joint-stage positions (joints) at tape slot `slot`.
 template <bool REC>
-__device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& a, const DiffWorld& W, uint32_t gsub,
-                                                uint32_t n, uint32_t slot) {
+static __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, Walk& w, const DiffArgs& a, const DiffWorld& W,
+                                                uint32_t gsub, uint32_t n, uint32_t slot) {
     const uint32_t tid = thread_index();
     const bool springs_lds = lds_springs(W);
     const bool joints = W.njg > 0;
-    const uint32_t per = per_thread(W);
-    if (a.collisions && n % kFitEvery == 0) {
-        LdsFit f;
-        f.init();
-#pragma unroll
-        for (uint32_t j = 0; j < 2; ++j)
-            if (tid + j * kDiffThreads < W.nb) f.point(o.p[j].x, o.p[j].y);
-        lds_fit<kDiffThreads>(f, 2.0f * W.rmax, kDiffCells, c.red, c.grid);
-    }
-    const LdsGrid g = lds_grid_uniform(*c.grid);
-    uint32_t* cnt = c.cnt + (n & 1u) * kCntStride;
-    uint32_t key[2] = {0u, 0u}, rank[2] = {0u, 0u};
-    if (a.collisions) {
-#pragma unroll
-        for (uint32_t j = 0; j < 2; ++j)
-            if (tid + j * kDiffThreads < W.nb) {
-                key[j] = lds_cell(g, o.p[j].x, o.p[j].y);
-                rank[j] = atomicAdd(&cnt[key[j]], 1u);
-            }
-    }
-    if (tid == 0) *c.pairs = 0;
+    const uint32_t per = per_thread(W), par = n & 1u;
+    if (a.collisions && w.build) build_lists(c, o, w, a, W);
+    const bool lists = a.collisions && w.grid == 0;
     if (springs_lds) {
         own_springs(o, a, W, [&](uint32_t t, uint32_t ia, uint32_t ib, float rest, float k, float cc) {
             const float2 f = spring_force(c.xy[ia], c.xy[ib], c.vel[ia], c.vel[ib], rest, k, cc);
@@ -419,55 +640,130 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
             c.force[li] = make_float4(ac.x, ac.y, 0.0f, 0.0f);
         }
     }
-    __syncthreads();
-    if (a.collisions) {
-        lds_scan<kDiffThreads, kScanItems>(cnt, g.ncells + 1u, c.red);
-#pragma unroll
-        for (uint32_t j = 0; j < 2; ++j) {
-            const uint32_t li = tid + j * kDiffThreads;
-            if (li >= W.nb) continue;
-            rank[j] += cnt[key[j]];  // the body's record
-            c.rec[rank[j]] = make_float4(o.p[j].x, o.p[j].y, o.r[j], __uint_as_float(li));
-        }
-        __syncthreads();
-    }
-    // contacts against the snapshot (physics.rs:241-317); the queue is in the idle cell table
-    uint32_t* other = c.cnt + ((n & 1u) ^ 1u) * kCntStride;
-    float2* res = reinterpret_cast<float2*>(other);
-    uint32_t* entries = other + 2 * kPairs;
-    LdsPairs pr0 = {0u, 0u, false}, pr1 = {0u, 0u, false};
-    auto pair = [&](const float4 own, const float4 oth) {
-        const uint32_t li = __float_as_uint(own.w), lj = __float_as_uint(oth.w);
-        return lds_correction(own, oth, c.mass[li], c.mass[lj], li > lj, false);
+    // contacts against the snapshot (physics.rs:241-317)
+    uint32_t pr[PER] = {}, nout = 0;
+    bool crowd = false;
+    auto contact = [&](uint32_t li, uint32_t lj) {
+        const float2 p = c.xy[li], b = c.xy[lj];
+        return lds_correction(make_float4(p.x, p.y, c.rad[li], 0.0f), make_float4(b.x, b.y, c.rad[lj], 0.0f),
+                              c.mass[li], c.mass[lj], li > lj, false);
     };
-    if (a.collisions) {
-#pragma unroll 1
-        for (uint32_t j = 0; j < per; ++j) {
-            const float2 xy = pick(o.p, j);
-            const bool active = tid + j * kDiffThreads < W.nb && finitef(xy.x) && finitef(xy.y);
-            const LdsPairs pr = lds_mark<kPairs>(g, cnt, c.rec, active, xy, pick(o.r, j), j ? rank[1] : rank[0], W.rmax,
-                                                 entries, c.pairs);
-            if (j)
-                pr1 = pr;
-            else
-                pr0 = pr;
+    if (lists) {
+        mark_lists(c, o, W, par, pr);
+        __syncthreads();
+        // (read here: past the next barrier somebody may already be at the end of the substep)
+        nout = (uint32_t)__builtin_amdgcn_readfirstlane((int)c.out->n);
+        crowd = c.out->pairs[par] > kPairs;
+        crowd |= __any((tid & (BG_WAVE - 1)) < nout && c.out->count[par][tid & (kOutMax - 1)] > kOutPairs) != 0;
+        const uint32_t queued = min(c.out->pairs[par], kPairs);
+        const uint32_t total = queued + nout * kOutPairs;
+        for (uint32_t i = tid; i < total; i += kDiffThreads) {
+            uint32_t e = i;
+            if (i >= queued) {
+                const uint32_t u = (i - queued) / kOutPairs, k = (i - queued) % kOutPairs;
+                if (k >= c.out->count[par][u]) continue;
+                e = kPairs + i - queued;
+            }
+            const uint32_t pair = c.entries[e];
+            if (pair == kNoPair) continue;
+            const LdsContact k = contact(pair >> 16, pair & 0xFFFFu);
+            c.entries[e] = k.hit ? pair & 0xFFFFu : kNoPair;
+            c.res[e] = k.c;
         }
-        __syncthreads();
-        lds_correct<kPairs, kDiffThreads>(tid, *c.pairs, c.rec, entries, res, pair);
-        __syncthreads();
     }
+    __syncthreads();
+    // A body's corrections, ascending partner index; the tape takes the first kDiffTapeNbr - 1 partners.
+    float2 sums[PER] = {};
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        if (li >= W.nb) continue;
+        float2 pn = pick(o.p, j);
+        const size_t tape = (size_t)slot * a.nb_total + W.b0 + li;
+        if (REC) a.tape_s[tape] = pn;
+        uint32_t w0 = 0xFFFF0000u, w1 = 0xFFFFFFFFu, w2 = 0xFFFFFFFFu, w3 = 0xFFFFFFFFu, found = 0;
+        auto record = [&](uint32_t t, uint32_t lj) {  // partner number t
+            if (!REC) return;
+            const uint32_t keep = t & 1u ? 0xFFFF0000u : 0xFFFFu, put_ = t & 1u ? lj : lj << 16;
+            if (t < 1) w0 = (w0 & keep) | put_;
+            else if (t < 3) w1 = (w1 & keep) | put_;
+            else if (t < 5) w2 = (w2 & keep) | put_;
+            else if (t < 7) w3 = (w3 & keep) | put_;
+        };
+        static_assert(kDiffTapeNbr == 8, "four words: the count and seven partners");
+        if (lists) {
+            const uint32_t n = (o.nl >> (4u * j)) & 15u;
+            uint32_t first = pick(pr, j) & 0xFFFFu, count = pick(pr, j) >> 16;
+            if (n == kOut)
+                for (uint32_t u = 0; u < nout; ++u)
+                    if (c.out->id[u] == li) {
+                        first = kPairs + u * kOutPairs;
+                        count = c.out->count[par][u] <= kOutPairs ? c.out->count[par][u] : kNoRoom;
+                    }
+            if (count != kNoRoom) {
+                found = lds_sum({first, count, false}, c.entries, c.res, [&](uint32_t t, uint32_t lj, float2 k) {
+                    pn.x = pn.x + k.x;
+                    pn.y = pn.y + k.y;
+                    record(t, lj);
+                });
+            } else {
+                // no room in the queue: its partners one after the other
+                for (uint32_t lj = 0;; ++lj) {
+                    uint32_t best = kNoPair;
+                    if (n == kOut) {
+                        best = lj;
+                    } else {
+                        for (uint32_t i = 0; i < n; ++i) {
+                            const uint32_t x = c.lists[i >> 2][li][i & 3u];
+                            best = x >= lj ? min(best, x) : best;
+                        }
+                        for (uint32_t u = 0; u < nout; ++u) {
+                            const uint32_t x = c.out->id[u];
+                            best = x >= lj ? min(best, x) : best;
+                        }
+                    }
+                    if (best >= W.nb) break;
+                    lj = best;
+                    if (lj == li) continue;
+                    const LdsContact k = contact(li, lj);
+                    if (!k.hit) continue;
+                    pn.x = pn.x + k.c.x;
+                    pn.y = pn.y + k.c.y;
+                    record(found++, lj);
+                }
+            }
+        } else if (a.collisions && finitef(pn.x) && finitef(pn.y)) {
+            constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
+            ContactList<kList, uint32_t> L;
+            const float4 own = make_float4(pn.x, pn.y, c.rad[li], __uint_as_float(li));
+            found = lds_contacts_direct(lds_grid_uniform(*c.grid), c.cnt, c.rec, make_float2(pn.x, pn.y), own.z, li,
+                                        W.rmax, pn, L,
+                                        [&](const float4 oth) {
+                                            const uint32_t lj = __float_as_uint(oth.w);
+                                            return lds_correction(own, oth, c.mass[li], c.mass[lj], li > lj, false);
+                                        },
+                                        [](uint32_t, const LdsContact&) {});
+#pragma unroll
+            for (uint32_t t = 0; REC && t + 1 < kDiffTapeNbr; ++t)
+                if (t < L.n) record(t, L.key[t]);
+        }
+        if (REC && a.collisions) {
+            w0 |= found < 0xFFFFu ? found : 0xFFFFu;
+            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w0, w1, w2, w3);
+        }
+        put(sums, j, pn);
+    }
+    if (crowd) __syncthreads();  // bodies without room read others' snapshots
+    if (tid == 0) c.out->pairs[par ^ 1u] = 0;
+    if (tid < kOutMax) c.out->count[par ^ 1u][tid] = 0;
     // From here to the end of the substep a thread touches the positions and velocities of its
-    // own bodies only (springs are done, contacts read the records), so it may rewrite them.
+    // own bodies only, so it may rewrite them.
 #pragma unroll 1
     for (uint32_t j = 0; j < per; ++j) {
         const uint32_t li = tid + j * kDiffThreads, gi = W.b0 + li;
         if (li >= W.nb) continue;
-        const float2 xy = pick(o.p, j);
-        const size_t tape = (size_t)slot * a.nb_total + gi;
-        if (REC) {
-            a.tape_s[tape] = xy;
-            if (a.tape_v) a.tape_v[tape] = c.vel[li];
-        }
+        const float2 pn = pick(sums, j);
+        if (REC && a.tape_v) a.tape_v[(size_t)slot * a.nb_total + gi] = c.vel[li];
         // gravity + springs (physics.rs:369-375, springs.rs:25-47), ascending spring index
         float2 ac = make_float2(0.0f, 0.0f);
         if (springs_lds) {
@@ -484,51 +780,14 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         } else {
             ac = make_float2(c.force[li].x, c.force[li].y);
         }
-        // contacts, ascending partner index; the tape takes the first kDiffTapeNbr - 1 partners
-        float2 pn = xy;
-        uint32_t w0 = 0xFFFF0000u, w1 = 0xFFFFFFFFu, w2 = 0xFFFFFFFFu, w3 = 0xFFFFFFFFu, found = 0;
-        auto record = [&](uint32_t t, uint32_t lj) {  // partner number t
-            if (!REC) return;
-            const uint32_t keep = t & 1u ? 0xFFFF0000u : 0xFFFFu, put_ = t & 1u ? lj : lj << 16;
-            if (t < 1) w0 = (w0 & keep) | put_;
-            else if (t < 3) w1 = (w1 & keep) | put_;
-            else if (t < 5) w2 = (w2 & keep) | put_;
-            else if (t < 7) w3 = (w3 & keep) | put_;
-        };
-        static_assert(kDiffTapeNbr == 8, "four words: the count and seven partners");
-        const LdsPairs pr = {j ? pr1.first : pr0.first, j ? pr1.n : pr0.n, j ? pr1.direct : pr0.direct};
-        if (pr.direct) {
-            constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
-            ContactList<kList, uint32_t> L;
-            const float4 own = make_float4(xy.x, xy.y, pick(o.r, j), __uint_as_float(li));
-            found = lds_contacts_direct(g, cnt, c.rec, xy, own.z, li, W.rmax, pn, L,
-                                        [&](const float4 oth) { return pair(own, oth); },
-                                        [](uint32_t, const LdsContact&) {});
-#pragma unroll
-            for (uint32_t t = 0; REC && t + 1 < kDiffTapeNbr; ++t)
-                if (t < L.n) record(t, L.key[t]);
-        } else {
-            found = lds_sum(pr, entries, res, [&](uint32_t t, uint32_t lj, float2 k) {
-                pn.x = pn.x + k.x;
-                pn.y = pn.y + k.y;
-                record(t, lj);
-            });
-        }
-        if (REC) {
-            w0 |= found < 0xFFFFu ? found : 0xFFFFu;
-            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w0, w1, w2, w3);
-        }
         if (joints) {
             c.vel[li] = pn;
             c.xy[li] = ac;
         } else {
-            verlet(c, o, a, W, gsub, j, pn, ac);
+            verlet(c, o, w, a, W, gsub, j, pn, ac);
         }
     }
     __syncthreads();
-    // clear the queue's table for the next substep's counts: every sum has read it
-    if (a.collisions)
-        for (uint32_t i = tid; i <= kDiffCells; i += kDiffThreads) other[i] = 0u;
     // fixed joints, positions (physics.rs:424-460), on the velocities' memory
     if (joints) {
         if (joints_staged(W))
@@ -538,23 +797,27 @@ __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, const DiffArgs& 
         __syncthreads();
         for (uint32_t j = 0; j < per; ++j) {
             const uint32_t li = tid + j * kDiffThreads;
-            if (li < W.nb) verlet(c, o, a, W, gsub, j, c.vel[li], c.xy[li]);
+            if (li < W.nb) verlet(c, o, w, a, W, gsub, j, c.vel[li], c.xy[li]);
         }
+        __syncthreads();
     }
-    __syncthreads();
+    if (w.grid) --w.grid;
+    nout = (uint32_t)__builtin_amdgcn_readfirstlane((int)c.out->n);
+    w.tested += nout;
+    w.build = !lists || nout > kOutMax || w.tested > kTested;
 }
 
 // One tape slot of a thread's bodies (the contact partners are loaded by the substep itself,
 // which needs them late).
 struct Tape {
-    float2 s[2], v[2];
+    float2 s[PER], v[PER];
     float2 axis;  // of one of a staged world's solves
 };
 
-__device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const DiffWorld& W, uint32_t k) {
+static __device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const DiffWorld& W, uint32_t k) {
     const uint32_t tid = thread_index();
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
+    for (uint32_t j = 0; j < PER; ++j) {
         const uint32_t li = tid + j * kDiffThreads;
         if (li >= W.nb) continue;
         const size_t i = (size_t)k * a.nb_total + W.b0 + li;
@@ -569,7 +832,7 @@ __device__ __forceinline__ void load_tape(Tape& t, const DiffArgs& a, const Diff
 struct SpringAdj {
     float kx, ky, rvx, rvy, gk;
 };
-__device__ __forceinline__ SpringAdj spring_adjoint(const Ctx& c, uint32_t ia, uint32_t ib, float rest, float kk, float cc) {
+static __device__ __forceinline__ SpringAdj spring_adjoint(const Ctx& c, uint32_t ia, uint32_t ib, float rest, float kk, float cc) {
     SpringAdj r;
     const float4 pa = c.rec[ia], pb = c.rec[ib];
     const float dx = pb.x - pa.x, dy = pb.y - pa.y;
@@ -605,9 +868,9 @@ __device__ __forceinline__ SpringAdj spring_adjoint(const Ctx& c, uint32_t ia, u
 // substep.  Out: the same before it; gv += d loss / d velocity_request at the
 // substep that consumes it; gk: the stiffness gradient of the thread's first
 // spring.  With `more`, `t` leaves with slot k - 1 on its way.
-__device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const DiffWorld& W,
-                                                uint32_t gsub, uint32_t k, bool more, Tape& t, float2 (&lp)[2],
-                                                float2 (&lq)[2], float2 (&lv)[2], float2 (&gv)[2], float& gk) {
+static __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const DiffArgs& a, const DiffWorld& W,
+                                                uint32_t gsub, uint32_t k, bool more, Tape& t, float2 (&lp)[PER],
+                                                float2 (&lq)[PER], float2 (&lv)[PER], float2 (&gv)[PER], float& gk) {
     const uint32_t tid = thread_index();
     const float h = a.h;
     const bool joints = W.njg > 0;
@@ -615,18 +878,18 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
     const uint32_t per = per_thread(W);
     // per spring (kx, ky) and, with damping, (rvx, rvy): the memory of a cell table and of the
     // forward's positions is free
-    float2* skx = reinterpret_cast<float2*>(c.cnt);
-    float2* srv = c.xy;
-    uint4 nbr[2];
+    float2* skx = c.spring_k;
+    float2* srv = c.spring_v;
+    uint4 nbr[PER];
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
+    for (uint32_t j = 0; j < PER; ++j) {
         const uint32_t li = tid + j * kDiffThreads;
         nbr[j] = make_uint4(0u, 0u, 0u, 0u);
         if (li >= W.nb) continue;
         if (a.collisions)
             nbr[j] = reinterpret_cast<const uint4*>(a.tape_nbr)[(size_t)k * a.nb_total + W.b0 + li];
         const float m = c.mass[li];
-        c.rec[li] = make_float4(t.s[j].x, t.s[j].y, o.r[j], m);
+        c.rec[li] = make_float4(t.s[j].x, t.s[j].y, c.rad[li], m);
         if (a.tape_v) c.vel[li] = t.v[j];
         float2 lam_a = make_float2(0.0f, 0.0f), lpp, lqin = make_float2(0.0f, 0.0f);
         if (o.fl[j] & BF_STATIC) {  // p'' = p', q'' = p', v'' = 0
@@ -695,8 +958,10 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
                 ls.x += f * (mux - nx * nm) - mux;
                 ls.y += f * (muy - ny * nm) - muy;
             };
-            uint32_t w0 = j ? nbr[1].x : nbr[0].x, w1 = j ? nbr[1].y : nbr[0].y;
-            uint32_t w2 = j ? nbr[1].z : nbr[0].z, w3 = j ? nbr[1].w : nbr[0].w;
+            uint4 words = nbr[0];
+            if constexpr (PER == 2) words = make_uint4(j ? nbr[1].x : words.x, j ? nbr[1].y : words.y,
+                                                       j ? nbr[1].z : words.z, j ? nbr[1].w : words.w);
+            uint32_t w0 = words.x, w1 = words.y, w2 = words.z, w3 = words.w;
             const uint32_t n = w0 & 0xFFFFu;
             if (n < kDiffTapeNbr) {
                 for (uint32_t i = 0; i < n; ++i) {  // shift the next partner down
@@ -757,10 +1022,10 @@ __device__ __forceinline__ void substep_reverse(Ctx& c, const Own& o, const Diff
 }
 
 // Centroid of the world's positions (f64 sums) by the block.
-__device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
+static __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     double sx = 0.0, sy = 0.0;
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j)
+    for (uint32_t j = 0; j < PER; ++j)
         if (threadIdx.x + j * kDiffThreads < W.nb) {
             sx += (double)o.p[j].x;
             sy += (double)o.p[j].y;
@@ -784,69 +1049,92 @@ __device__ double2 block_centroid(Ctx& c, const Own& o, const DiffWorld& W) {
     const double n = W.nb > 0 ? (double)W.nb : 1.0;
     return make_double2(tx / n, ty / n);
 }
+// Before a launch's first substep.
+static __device__ __forceinline__ void start_walk(Ctx& c, Walk& w, const DiffWorld& W) {
+    w.skin = kSkin * 2.0f * W.rmax;
+    w.drift = make_float2(0.0f, 0.0f);
+    w.grid = 0;
+    w.tested = 0;
+    w.build = true;
+    if (threadIdx.x == 0) c.out->n = c.out->pairs[0] = c.out->pairs[1] = 0;
+    if (threadIdx.x < 2 * kOutMax) c.out->count[threadIdx.x / kOutMax][threadIdx.x % kOutMax] = 0;
+}
+};  // Rollout
 
-// With the kernels' own arrays about 157 KB of the CU's 160 KB: one workgroup a CU either way (1,024 threads at 128
-// VGPRs fill its registers).
+// With the kernels' own arrays nearly the CU's 160 KB: one workgroup a CU either way (1,024 threads
+// at 128 VGPRs fill its registers).
 #define BG_DIFF_SHARED                                               \
+    using X = Rollout<NT, PER>;                                      \
+    constexpr uint32_t kDiffMaxBodies = X::kDiffMaxBodies, kDiffLdsSprings = X::kDiffLdsSprings;       \
+    constexpr int kWaves = X::kWaves;                                \
     __shared__ float2 s_xy[kDiffMaxBodies];                          \
     __shared__ float2 s_vel[kDiffMaxBodies];                         \
-    __shared__ float s_mass[kDiffMaxBodies];                         \
-    __shared__ float4 s_rec[kDiffMaxBodies + kLdsRecPad];            \
-    __shared__ uint64_t s_cnt[kCntStride];                           \
-    __shared__ float4 s_force[kDiffLdsSprings];                      \
-    __shared__ uint32_t s_red[kFitWords * kWaves];                   \
-    __shared__ uint32_t s_pairs;                                     \
-    __shared__ double s_dred[2 * kWaves];                            \
-    __shared__ LdsGrid s_grid;                                       \
-    __shared__ JointStage s_joints;                                  \
-    static_assert(kDiffLdsSprings >= kDiffMaxBodies, "the adjoint vectors share the springs' memory"); \
-    static_assert(kDiffCells / 2 >= kDiffLdsSprings, "spring adjoints share a cell table's memory");   \
-    static_assert(kDiffMaxBodies >= kDiffLdsSprings, "and the positions'");                            \
-    Ctx c;                                                           \
+    __shared__ float s_mass[kDiffMaxBodies], s_rad[kDiffMaxBodies];  \
+    __shared__ float4 s_force[kDiffLdsSprings + kLdsRecPad];         \
+    __shared__ typename X::JointStage s_joints;                      \
+    static_assert(kDiffLdsSprings >= kDiffMaxBodies, "the adjoint vectors and the records share the springs' memory"); \
+    typename X::Ctx c{};                                                         \
     c.xy = s_xy;                                                     \
     c.vel = s_vel;                                                   \
     c.mass = s_mass;                                                 \
-    c.rec = s_rec;                                                   \
-    c.cnt = reinterpret_cast<uint32_t*>(s_cnt);                      \
-    c.gmod = nullptr;                                                \
-    c.axes = nullptr;                                                \
+    c.rad = s_rad;                                                   \
     c.force = s_force;                                               \
-    c.red = s_red;                                                   \
-    c.pairs = &s_pairs;                                              \
-    c.dred = s_dred;                                                 \
-    c.grid = &s_grid;                                                \
     c.joints = &s_joints;                                            \
     c.lam_pp = reinterpret_cast<float2*>(s_force);                   \
     c.lam_am = c.lam_pp + kDiffMaxBodies;
 
-__global__ __launch_bounds__(kDiffThreads) void k_diff_forward(DiffArgs a, uint32_t n_steps, uint32_t ck_every) {
-    BG_DIFF_SHARED
-    __shared__ float s_gmod[kDiffMaxBodies];
-    c.gmod = s_gmod;
+// The forward's.  The scans' and the centroid's scratch is the idle queue's.
+#define BG_DIFF_FORWARD                                              \
+    BG_DIFF_SHARED                                                   \
+    constexpr uint32_t kPairs = X::kPairs, kQueue = kPairs + X::kOutMax * X::kOutPairs;                   \
+    __shared__ float s_gmod[kDiffMaxBodies];                         \
+    __shared__ float4 s_lists[kDiffMaxBodies + kLdsRecPad];          \
+    __shared__ uint32_t s_cnt[X::kDiffCells + 1];                    \
+    __shared__ float2 s_res[kQueue];                                 \
+    __shared__ uint32_t s_entries[kQueue];                           \
+    __shared__ typename X::Outliers s_out;                                       \
+    __shared__ LdsGrid s_grid;                                       \
+    static_assert(sizeof(uint16_t[X::kListCap / 4][kDiffMaxBodies][4]) <= sizeof(s_lists), "lists, or records"); \
+    static_assert(kQueue >= kFitWords * kWaves && kQueue >= 2 * kWaves, "the scratch");                  \
+    c.gmod = s_gmod;                                                 \
+    c.lists = reinterpret_cast<uint16_t(*)[kDiffMaxBodies][4]>(s_lists); \
+    c.cnt = s_cnt;                                                   \
+    c.res = s_res;                                                   \
+    c.entries = s_entries;                                           \
+    c.out = &s_out;                                                  \
+    c.grid = &s_grid;                                                \
+    c.red = s_entries;                                               \
+    c.dred = reinterpret_cast<double*>(s_res);                       \
+    typename X::Walk w;
+
+template <uint32_t NT, uint32_t PER>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_diff_forward(DiffArgs a, uint32_t n_steps, uint32_t ck_every) {
+    BG_DIFF_FORWARD
     const DiffWorld W = a.worlds[blockIdx.x];
-    Own o;
-    load_own(c, o, a, W, a.ck_p, a.ck_q, a.ck_v);
+    typename X::Own o;
+    X::load_own(c, o, a, W, a.ck_p, a.ck_q, a.ck_v);
+    X::start_walk(c, w, W);
     __syncthreads();
     for (uint32_t step = 0; step < n_steps; ++step) {
         if (step > 0 && step % ck_every == 0) {
             const size_t base = (size_t)(step / ck_every) * a.nb_total + W.b0;
 #pragma unroll
-            for (uint32_t j = 0; j < 2; ++j)
-                if (threadIdx.x + j * kDiffThreads < W.nb) {
-                    a.ck_p[base + threadIdx.x + j * kDiffThreads] = o.p[j];
-                    a.ck_q[base + threadIdx.x + j * kDiffThreads] = o.q[j];
-                    a.ck_v[base + threadIdx.x + j * kDiffThreads] = c.vel[threadIdx.x + j * kDiffThreads];
+            for (uint32_t j = 0; j < PER; ++j)
+                if (threadIdx.x + j * NT < W.nb) {
+                    a.ck_p[base + threadIdx.x + j * NT] = o.p[j];
+                    a.ck_q[base + threadIdx.x + j * NT] = o.q[j];
+                    a.ck_v[base + threadIdx.x + j * NT] = c.vel[threadIdx.x + j * NT];
                 }
         }
         for (uint32_t sub = 0; sub < a.substeps; ++sub) {
             const uint32_t n = step * a.substeps + sub;
-            substep_forward<false>(c, o, a, W, n, n, 0u);
+            X::template substep_forward<false>(c, o, w, a, W, n, n, 0u);
         }
     }
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j)
-        if (threadIdx.x + j * kDiffThreads < W.nb) a.final_p[W.b0 + threadIdx.x + j * kDiffThreads] = o.p[j];
-    const double2 cen = block_centroid(c, o, W);
+    for (uint32_t j = 0; j < PER; ++j)
+        if (threadIdx.x + j * NT < W.nb) a.final_p[W.b0 + threadIdx.x + j * NT] = o.p[j];
+    const double2 cen = X::block_centroid(c, o, W);
     if (threadIdx.x == 0) {
         const double dx = cen.x - (double)W.tx, dy = cen.y - (double)W.ty;
         a.loss[blockIdx.x] = (float)(dx * dx + dy * dy);
@@ -855,61 +1143,70 @@ __global__ __launch_bounds__(kDiffThreads) void k_diff_forward(DiffArgs a, uint3
 
 // Recomputes segments first_seg + blockIdx.y from their checkpoints, recording their tapes
 // one after another (seg_sub substeps each).
-__global__ __launch_bounds__(kDiffThreads) void k_diff_recompute(DiffArgs a, uint32_t first_seg, uint32_t ck_every,
+template <uint32_t NT, uint32_t PER>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_diff_recompute(DiffArgs a, uint32_t first_seg, uint32_t ck_every,
                                                                  uint32_t n_steps) {
-    BG_DIFF_SHARED
-    __shared__ float s_gmod[kDiffMaxBodies];
-    c.gmod = s_gmod;
+    BG_DIFF_FORWARD
     const DiffWorld W = a.worlds[blockIdx.x];
     const uint32_t seg = first_seg + blockIdx.y, first_step = seg * ck_every;
     const uint32_t nsub = min(n_steps - first_step, ck_every) * a.substeps;
     const uint32_t tape0 = blockIdx.y * ck_every * a.substeps;
     const size_t ck = (size_t)seg * a.nb_total;
-    Own o;
-    load_own(c, o, a, W, a.ck_p + ck, a.ck_q + ck, a.ck_v + ck);
+    typename X::Own o;
+    X::load_own(c, o, a, W, a.ck_p + ck, a.ck_q + ck, a.ck_v + ck);
+    X::start_walk(c, w, W);
     __syncthreads();
     for (uint32_t k = 0; k < nsub; ++k)
-        substep_forward<true>(c, o, a, W, first_step * a.substeps + k, k, tape0 + k);
+        X::template substep_forward<true>(c, o, w, a, W, first_step * a.substeps + k, k, tape0 + k);
 }
 
 // Adjoint of one segment, its tape at slots tape0 ...
-__global__ __launch_bounds__(kDiffThreads) void k_diff_reverse(DiffArgs a, uint32_t seg, uint32_t tape0,
+template <uint32_t NT, uint32_t PER>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_diff_reverse(DiffArgs a, uint32_t seg, uint32_t tape0,
                                                                uint32_t first_sub, uint32_t nsub, uint32_t last) {
     BG_DIFF_SHARED
-    __shared__ float2 s_axes[kDiffLdsSolves];
+    __shared__ float4 s_rec[kDiffMaxBodies];
+    __shared__ float2 s_spring_k[kDiffLdsSprings], s_spring_v[PER == 1 ? kDiffLdsSprings : 1];
+    __shared__ float2 s_axes[X::kDiffLdsSolves];
+    __shared__ double s_dred[2 * kWaves];
+    c.rec = s_rec;
+    c.spring_k = s_spring_k;
+    c.spring_v = PER == 1 ? s_spring_v : s_xy;
+    static_assert(PER == 1 || kDiffMaxBodies >= kDiffLdsSprings, "spring adjoints in the positions' memory");
     c.axes = s_axes;
+    c.dred = s_dred;
     const DiffWorld W = a.worlds[blockIdx.x];
-    Own o;
+    typename X::Own o;
     // (only the last segment reads positions: the final ones, for the centroid)
-    load_own(c, o, a, W, a.final_p, a.final_p, a.final_p);
+    X::load_own(c, o, a, W, a.final_p, a.final_p, a.final_p);
     __syncthreads();
-    float2 lp[2], lq[2], lv[2], gv[2];
+    float2 lp[PER], lq[PER], lv[PER], gv[PER];
     const bool centroid = last && !a.dl_dfinal;
     float2 g0 = make_float2(0.0f, 0.0f);
     if (centroid) {  // d |centroid - target|^2 / d p_i = 2 (centroid - target) / n
-        const double2 cen = block_centroid(c, o, W);
+        const double2 cen = X::block_centroid(c, o, W);
         g0.x = (float)(2.0 * (cen.x - (double)W.tx) / (double)(W.nb > 0 ? W.nb : 1));
         g0.y = (float)(2.0 * (cen.y - (double)W.ty) / (double)(W.nb > 0 ? W.nb : 1));
     }
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
-        const uint32_t li = threadIdx.x + j * kDiffThreads, gi = W.b0 + li;
+    for (uint32_t j = 0; j < PER; ++j) {
+        const uint32_t li = threadIdx.x + j * NT, gi = W.b0 + li;
         const bool live = li < W.nb;
         lp[j] = centroid ? g0 : (live ? (last ? a.dl_dfinal[gi] : a.lam_p[gi]) : make_float2(0.0f, 0.0f));
         lq[j] = (live && !last) ? a.lam_q[gi] : make_float2(0.0f, 0.0f);
         lv[j] = (live && !last) ? a.lam_v[gi] : make_float2(0.0f, 0.0f);  // the loss does not read the final velocities
         gv[j] = make_float2(0.0f, 0.0f);
     }
-    const bool own_gk = lds_springs(W) && threadIdx.x < W.ns;
+    const bool own_gk = X::lds_springs(W) && threadIdx.x < W.ns;
     float gk = own_gk ? a.grad_k[W.s0 + threadIdx.x] : 0.0f;
-    Tape t;
-    if (nsub > 0) load_tape(t, a, W, tape0 + nsub - 1);
+    typename X::Tape t;
+    if (nsub > 0) X::load_tape(t, a, W, tape0 + nsub - 1);
     for (uint32_t k = nsub; k-- > 0;)
-        substep_reverse(c, o, a, W, first_sub + k, tape0 + k, k > 0, t, lp, lq, lv, gv, gk);
+        X::substep_reverse(c, o, a, W, first_sub + k, tape0 + k, k > 0, t, lp, lq, lv, gv, gk);
     if (own_gk) a.grad_k[W.s0 + threadIdx.x] = gk;
 #pragma unroll
-    for (uint32_t j = 0; j < 2; ++j) {
-        const uint32_t li = threadIdx.x + j * kDiffThreads, gi = W.b0 + li;
+    for (uint32_t j = 0; j < PER; ++j) {
+        const uint32_t li = threadIdx.x + j * NT, gi = W.b0 + li;
         if (li >= W.nb) continue;
         a.lam_p[gi] = lp[j];
         a.lam_q[gi] = lq[j];
@@ -920,16 +1217,26 @@ __global__ __launch_bounds__(kDiffThreads) void k_diff_reverse(DiffArgs a, uint3
 
 }  // namespace
 
+#define BG_DIFF_LAUNCH(KERNEL, GRID, ...)                                                                     \
+    do {                                                                                                      \
+        switch (a.threads) {                                                                                  \
+            case 256: KERNEL<256, 1><<<GRID, 256, 0, s>>>(__VA_ARGS__); break;                                \
+            case 512: KERNEL<512, 1><<<GRID, 512, 0, s>>>(__VA_ARGS__); break;                                \
+            case 1024: KERNEL<1024, 1><<<GRID, 1024, 0, s>>>(__VA_ARGS__); break;                             \
+            default: KERNEL<kDiffThreads, kDiffPer><<<GRID, kDiffThreads, 0, s>>>(__VA_ARGS__); break;        \
+        }                                                                                                     \
+    } while (0)
+
 hipError_t launch_diff_forward(const DiffArgs& a, uint32_t n_steps, uint32_t ck_every, hipStream_t s) {
     if (a.n_worlds == 0) return hipSuccess;
-    k_diff_forward<<<a.n_worlds, kDiffThreads, 0, s>>>(a, n_steps, ck_every);
+    BG_DIFF_LAUNCH(k_diff_forward, a.n_worlds, a, n_steps, ck_every);
     return hipGetLastError();
 }
 
 hipError_t launch_diff_recompute(const DiffArgs& a, uint32_t first_seg, uint32_t n_seg, uint32_t ck_every,
                                  uint32_t n_steps, hipStream_t s) {
     if (a.n_worlds == 0) return hipSuccess;
-    k_diff_recompute<<<dim3(a.n_worlds, n_seg), kDiffThreads, 0, s>>>(a, first_seg, ck_every, n_steps);
+    BG_DIFF_LAUNCH(k_diff_recompute, dim3(a.n_worlds, n_seg), a, first_seg, ck_every, n_steps);
     return hipGetLastError();
 }
 
@@ -937,8 +1244,8 @@ hipError_t launch_diff_reverse(const DiffArgs& a, uint32_t seg, uint32_t tape_se
                                hipStream_t s) {
     if (a.n_worlds == 0) return hipSuccess;
     const uint32_t first = seg * ck_every, steps = std::min(n_steps - first, ck_every);
-    k_diff_reverse<<<a.n_worlds, kDiffThreads, 0, s>>>(a, seg, tape_seg * ck_every * a.substeps, first * a.substeps,
-                                                       steps * a.substeps, first + steps == n_steps ? 1u : 0u);
+    BG_DIFF_LAUNCH(k_diff_reverse, a.n_worlds, a, seg, tape_seg * ck_every * a.substeps, first * a.substeps,
+                   steps * a.substeps, first + steps == n_steps ? 1u : 0u);
     return hipGetLastError();
 }
 

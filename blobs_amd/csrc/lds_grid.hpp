@@ -220,13 +220,12 @@ __device__ __forceinline__ uint32_t lds_cell(const LdsGrid& g, float x, float y)
 
 // ---- contacts ----------------------------------------------------------------
 //
-// Three phases with a barrier between them.  Mark: each body walks the records
-// of its cells, about 20 instructions a candidate, and puts those within reach
-// into a queue.  Correct: a thread takes one queued pair, whoever's it is, and
-// works out its correction (a root and three divides, about 200 instructions):
-// with one contact among ten bodies a wave that corrected its own would run
-// that code once or twice for each of its bodies, almost all lanes idle.  Sum:
-// each body adds its corrections in ascending partner index.
+// Three phases with a barrier between them.  Mark: each body puts its partners
+// within reach into a queue.  Correct: a thread takes one queued pair, whoever's
+// it is, and works out its correction (a root and three divides, about 200
+// instructions): with one contact among ten bodies a wave that corrected its own
+// would run that code once or twice for each of its bodies, almost all lanes idle.
+// Sum: each body adds its corrections in ascending partner index.
 
 constexpr int kLdsRows = 3;        // grid rows of a flat candidate list (a query of cells of 2 r_max rarely spans 4)
 constexpr uint32_t kLdsFlat = 64;  // candidates of a flat list (one 64-bit mask)
@@ -345,25 +344,6 @@ __device__ __forceinline__ uint64_t lds_near(const LdsRows& l, const float4* rec
     return ((uint64_t)near_hi << 32) | near_lo;
 }
 
-// Mark phase of one body a lane (`active`: the lane has one, with a finite snapshot xy),
-// called by whole waves.  rec[] = (x, y, radius, bits(local index)) in cell order, with
-// kLdsRecPad records of room behind them, `own` the body's own record.
-template <uint32_t CAP>
-__device__ __forceinline__ LdsPairs lds_mark(const LdsGrid& g, const uint32_t* start, const float4* rec, bool active,
-                                             float2 xy, float r, uint32_t own, float rmax, uint32_t* entries,
-                                             uint32_t* count) {
-    const LdsRows l = lds_rows(g, start, active, xy, r + rmax);
-    const uint64_t marked = lds_near(l, rec, [&](uint32_t t, const float4& b) {
-        const float dx = xy.x - b.x, dy = xy.y - b.y;
-        const float rs = r + b.z;
-        const bool far = dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f;
-        return !((t == own) | far);
-    });
-    LdsPairs pr = lds_queue<CAP>(marked, own, entries, count, [&](uint32_t i) { return l.slot(i); });
-    pr.direct |= active && !l.flat;
-    return pr;
-}
-
 // One pair: its contact (physics.rs:264-300) from the side of the body `own`.
 // A is the body of the higher index (local order is arena order).
 struct LdsContact {
@@ -409,21 +389,6 @@ __device__ __forceinline__ LdsContact lds_correction(const float4 own, const flo
         r.c.y = py + r.c.y;
     }
     return r;
-}
-
-// Correct phase: `pair(own record, other record)` gives the LdsContact of a queued pair; its
-// correction goes to res[e] and the partner's index (or kNoPair) to entries[e].
-template <uint32_t CAP, uint32_t NT, class Pair>
-__device__ __forceinline__ void lds_correct(uint32_t tid, uint32_t count, const float4* rec, uint32_t* entries,
-                                            float2* res, Pair&& pair) {
-    for (uint32_t e = tid; e < min(count, CAP); e += NT) {
-        const uint32_t w = entries[e];
-        if (w == kNoPair) continue;
-        const float4 other = rec[w & 0xFFFFu];
-        const LdsContact k = pair(rec[w >> 16], other);
-        entries[e] = k.hit ? __float_as_uint(other.w) : kNoPair;
-        res[e] = k.c;
-    }
 }
 
 // Sum phase: f(k, partner, correction) over the body's contacts in ascending partner index.
