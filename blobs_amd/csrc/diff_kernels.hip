@@ -31,9 +31,9 @@
 // Measured (forward + backward, against bounding box, grid, springs and contacts
 // worked out serially or per body each substep; in brackets with a grid and
 // 1,024 threads for every world in every substep): 256 worlds of 2,048 bodies and
-// 1,024 springs over 50 steps 33.2 -> 14.8 ms (15.4); 96 worlds of 700, 60 steps
-// forward 7.24 -> 2.66 ms (3.13); 12 worlds of 301 with 40 joints, 6 steps 3.80 ->
-// 1.51 ms (1.61); 512 worlds of 300, 20 steps 1.11 ms (1.98).
+// 1,024 springs over 50 steps 33.2 -> 14.5 ms (15.4); 96 worlds of 700, 60 steps
+// forward 7.24 -> 2.68 ms (3.13); 12 worlds of 301 with 40 joints, 6 steps 3.80 ->
+// 1.53 ms (1.61); 512 worlds of 300, 20 steps 1.10 ms (1.98).
 #include "diff.hpp"
 
 #include <algorithm>
@@ -61,7 +61,7 @@ static constexpr uint32_t kDiffLdsJoints = 256, kDiffLdsSolves = NT, kDiffLdsLev
 // Partner lists: entries of a body, bodies outside the lists and queued pairs of each, builds with
 // the skin halved while too many lists overflow, and the substeps a world that overflows them all
 // goes without.  The skin in diameters of the largest body: with 0.1 the four cases above take
-// 15.6, 3.03, 1.50 and 1.17 ms, with 0.3 16.3, 2.79, 1.54 and 1.11.
+// 15.6, 3.03, 1.50 and 1.17 ms, with 0.3 16.3, 2.79, 1.54 and 1.11, with 0.2 14.8, 2.66, 1.53 and 1.10.
 static constexpr uint32_t kListCap = 8, kOutMax = 16, kOutPairs = 8, kListTries = 3, kGridHold = 64;
 static constexpr float kSkin = 0.2f;
 static constexpr uint32_t kTested = 24;           // a build costs about what so many tests of a body outside the lists do
@@ -84,6 +84,7 @@ struct JointStage {
 struct Outliers {
     uint32_t n;           // (may exceed kOutMax: then the lists are built anew)
     uint32_t pairs[2];    // queued pairs
+    uint32_t round, more; // and of a round of queue_rounds; somebody has contacts left
     uint16_t id[kOutMax];
     uint32_t count[2][kOutMax];  // pairs of an outlier, in the queue's entries from kPairs + u * kOutPairs
 };
@@ -602,6 +603,135 @@ static __device__ __forceinline__ void mark_lists(Ctx& c, const Own& o, const Di
     static_assert(kListCap + kOutMax <= 32, "the mask");
 }
 
+// The contacts of the bodies still to do (bit j of `pending`), as many of them at a time as the
+// queue has room for: a world of thousands of pairs, or one without lists.  (A thread doing all of
+// its body's, candidate by candidate, leaves the wave to its busiest: 4 worlds of 2,048 bodies
+// thrown on eight times their area's worth, 10 steps: 28.6 ms, 88.0 that way.)
+template <class Contact, class Finish>
+static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const DiffWorld& W, bool lists, uint32_t nout,
+                                                    uint32_t pending, Contact&& contact, Finish&& finish) {
+    const uint32_t tid = thread_index();
+    const uint32_t per = per_thread(W);
+    // f(partner) for the candidates of body j within reach
+    auto partners = [&](uint32_t j, auto&& f) {
+        const uint32_t li = tid + j * kDiffThreads;
+        const float2 p = pick(o.p, j);
+        const float r = c.rad[li];
+        auto test = [&](uint32_t lj, float2 b, float rb) {
+            const float dx = p.x - b.x, dy = p.y - b.y, rs = r + rb;
+            if ((lj != li) & !(dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f)) f(lj);
+        };
+        const uint32_t n = (o.nl >> (4u * j)) & 15u;
+        if (!lists) {
+            const LdsGrid g = lds_grid_uniform(*c.grid);
+            const LdsRect q = lds_rect(g, p.x, p.y, r + W.rmax);
+            for (int32_t cy = q.cy0; cy <= q.cy1; ++cy) {
+                const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
+                const uint32_t t1 = c.cnt[row + (uint32_t)q.cx1 + 1u];
+                for (uint32_t t = c.cnt[row + (uint32_t)q.cx0]; t < t1; t += 4) {
+                    float4 b[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) b[u] = c.rec[t + u];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u)
+                        if (t + u < t1) test(__float_as_uint(b[u].w), make_float2(b[u].x, b[u].y), b[u].z);
+                }
+            }
+            static_assert(kLdsRecPad >= 3, "reads past the last record");
+        } else if (n == kOut) {
+            for (uint32_t lj = 0; lj < W.nb; ++lj) test(lj, c.xy[lj], c.rad[lj]);
+        } else {
+            for (uint32_t i = 0; i < n; ++i) {
+                const uint32_t lj = c.lists[i >> 2][li][i & 3u];
+                test(lj, c.xy[lj], c.rad[lj]);
+            }
+            for (uint32_t u = 0; u < nout; ++u) {
+                const uint32_t lj = c.out->id[u];
+                bool listed = false;
+                for (uint32_t i = 0; i < n; ++i) listed |= c.lists[i >> 2][li][i & 3u] == lj;
+                if (!listed) test(lj, c.xy[lj], c.rad[lj]);
+            }
+        }
+    };
+    uint32_t need[PER] = {};
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        uint32_t n = 0;
+        if ((pending >> j) & 1u) partners(j, [&](uint32_t) { ++n; });
+        put(need, j, n);
+        if (n > kPairs) {  // never fits
+            finish(j, 0u, kNoRoom, false);
+            pending &= ~(1u << j);
+        }
+    }
+    for (;;) {  // (the first body in line fits, so every round does some)
+        __syncthreads();
+        if (tid == 0) c.out->round = c.out->more = 0;
+        __syncthreads();
+        uint32_t at[PER] = {}, placed = 0;
+#pragma unroll 1
+        for (uint32_t j = 0; j < per; ++j) {
+            const bool todo = (pending >> j) & 1u;
+            const uint32_t n = todo ? pick(need, j) : 0u;
+            const uint32_t incl = wave_prefix(n, 0u, AddU32());
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, BG_WAVE - 1);
+            uint32_t first = 0;
+            if (total > 0 && (tid & (BG_WAVE - 1)) == 0) first = atomicAdd(&c.out->round, total);
+            first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + incl - n;
+            put(at, j, first);
+            if (!todo) continue;
+            if (first + n <= kPairs) {
+                placed |= 1u << j;
+                const uint32_t own = (tid + j * kDiffThreads) << 16;
+                uint32_t e = first;
+                const float2 range = make_float2(__uint_as_float(first), __uint_as_float(first + n));
+                partners(j, [&](uint32_t lj) {
+                    c.entries[e] = own | lj;
+                    c.res[e++] = range;
+                });
+            } else {
+                for (uint32_t e = first; e < kPairs; ++e) c.entries[e] = kNoPair;
+            }
+        }
+        __syncthreads();
+        // a pair's correction, and its place in its body's ascending order (dozens of partners would
+        // take a thread by itself long to sort)
+        uint32_t to[2], key[2];
+        float2 k[2];
+        static_assert(kPairs <= 2 * kDiffThreads, "the two");
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            const uint32_t e = tid + i * kDiffThreads;
+            to[i] = kNoPair;
+            if (e >= min(c.out->round, kPairs)) continue;
+            const uint32_t pair = c.entries[e];
+            if (pair == kNoPair) continue;
+            to[i] = __float_as_uint(c.res[e].x);
+            const uint32_t end = __float_as_uint(c.res[e].y);
+#pragma unroll 4
+            for (uint32_t f = __float_as_uint(c.res[e].x); f < end; ++f) to[i] += c.entries[f] < pair ? 1u : 0u;
+            const LdsContact ct = contact(pair >> 16, pair & 0xFFFFu);
+            key[i] = ct.hit ? pair & 0xFFFFu : kNoPair;
+            k[i] = ct.c;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i)
+            if (to[i] != kNoPair) {
+                c.entries[to[i]] = key[i];
+                c.res[to[i]] = k[i];
+            }
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t j = 0; j < per; ++j)
+            if ((placed >> j) & 1u) finish(j, pick(at, j), pick(need, j), true);
+        pending &= ~placed;
+        if (pending) c.out->more = 1;
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane((int)c.out->more) == 0) break;
+    }
+}
+
 // One forward substep of the world (`n` counts this launch's substeps); with
 // REC, records the snapshot, contact partners, velocities (damped springs) and
 // joint-stage positions (joints) at tape slot `slot`.
@@ -642,7 +772,7 @@ static __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, Walk& w, 
     }
     // contacts against the snapshot (physics.rs:241-317)
     uint32_t pr[PER] = {}, nout = 0;
-    bool crowd = false;
+    bool crowd = a.collisions && !lists;
     auto contact = [&](uint32_t li, uint32_t lj) {
         const float2 p = c.xy[li], b = c.xy[lj];
         return lds_correction(make_float4(p.x, p.y, c.rad[li], 0.0f), make_float4(b.x, b.y, c.rad[lj], 0.0f),
@@ -672,17 +802,16 @@ static __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, Walk& w, 
         }
     }
     __syncthreads();
-    // A body's corrections, ascending partner index; the tape takes the first kDiffTapeNbr - 1 partners.
+    // A body's corrections, ascending partner index, from `count` entries of the queue (kNoRoom: from
+    // all bodies, one after the other); the tape takes the first kDiffTapeNbr - 1 partners.
     float2 sums[PER] = {};
-#pragma unroll 1
-    for (uint32_t j = 0; j < per; ++j) {
+    auto finish = [&](uint32_t j, uint32_t first, uint32_t count, bool sorted) {
         const uint32_t li = tid + j * kDiffThreads;
-        if (li >= W.nb) continue;
         float2 pn = pick(o.p, j);
-        const size_t tape = (size_t)slot * a.nb_total + W.b0 + li;
-        if (REC) a.tape_s[tape] = pn;
         uint32_t w0 = 0xFFFF0000u, w1 = 0xFFFFFFFFu, w2 = 0xFFFFFFFFu, w3 = 0xFFFFFFFFu, found = 0;
-        auto record = [&](uint32_t t, uint32_t lj) {  // partner number t
+        auto add = [&](uint32_t t, uint32_t lj, float2 k) {  // partner number t
+            pn.x = pn.x + k.x;
+            pn.y = pn.y + k.y;
             if (!REC) return;
             const uint32_t keep = t & 1u ? 0xFFFF0000u : 0xFFFFu, put_ = t & 1u ? lj : lj << 16;
             if (t < 1) w0 = (w0 & keep) | put_;
@@ -691,69 +820,49 @@ static __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, Walk& w, 
             else if (t < 7) w3 = (w3 & keep) | put_;
         };
         static_assert(kDiffTapeNbr == 8, "four words: the count and seven partners");
+        if (sorted) {
+            for (uint32_t e = first; e < first + count; ++e)
+                if (c.entries[e] != kNoPair) add(found++, c.entries[e], c.res[e]);
+        } else if (count != kNoRoom) {
+            found = lds_sum({first, count, false}, c.entries, c.res, add);
+        } else {
+            for (uint32_t lj = 0; lj < W.nb; ++lj) {
+                const LdsContact k = contact(li, lj);
+                if (lj != li && k.hit) add(found++, lj, k.c);
+            }
+        }
+        if (REC && a.collisions) {
+            w0 |= found < 0xFFFFu ? found : 0xFFFFu;
+            reinterpret_cast<uint4*>(a.tape_nbr)[(size_t)slot * a.nb_total + W.b0 + li] = make_uint4(w0, w1, w2, w3);
+        }
+        put(sums, j, pn);
+    };
+    uint32_t pending = 0;  // bit j: body j's contacts are still to do
+#pragma unroll 1
+    for (uint32_t j = 0; j < per; ++j) {
+        const uint32_t li = tid + j * kDiffThreads;
+        if (li >= W.nb) continue;
+        const float2 xy = pick(o.p, j);
+        if (REC) a.tape_s[(size_t)slot * a.nb_total + W.b0 + li] = xy;
+        uint32_t first = 0, count = 0;
         if (lists) {
-            const uint32_t n = (o.nl >> (4u * j)) & 15u;
-            uint32_t first = pick(pr, j) & 0xFFFFu, count = pick(pr, j) >> 16;
-            if (n == kOut)
+            first = pick(pr, j) & 0xFFFFu;
+            count = pick(pr, j) >> 16;
+            if (((o.nl >> (4u * j)) & 15u) == kOut)
                 for (uint32_t u = 0; u < nout; ++u)
                     if (c.out->id[u] == li) {
                         first = kPairs + u * kOutPairs;
                         count = c.out->count[par][u] <= kOutPairs ? c.out->count[par][u] : kNoRoom;
                     }
-            if (count != kNoRoom) {
-                found = lds_sum({first, count, false}, c.entries, c.res, [&](uint32_t t, uint32_t lj, float2 k) {
-                    pn.x = pn.x + k.x;
-                    pn.y = pn.y + k.y;
-                    record(t, lj);
-                });
-            } else {
-                // no room in the queue: its partners one after the other
-                for (uint32_t lj = 0;; ++lj) {
-                    uint32_t best = kNoPair;
-                    if (n == kOut) {
-                        best = lj;
-                    } else {
-                        for (uint32_t i = 0; i < n; ++i) {
-                            const uint32_t x = c.lists[i >> 2][li][i & 3u];
-                            best = x >= lj ? min(best, x) : best;
-                        }
-                        for (uint32_t u = 0; u < nout; ++u) {
-                            const uint32_t x = c.out->id[u];
-                            best = x >= lj ? min(best, x) : best;
-                        }
-                    }
-                    if (best >= W.nb) break;
-                    lj = best;
-                    if (lj == li) continue;
-                    const LdsContact k = contact(li, lj);
-                    if (!k.hit) continue;
-                    pn.x = pn.x + k.c.x;
-                    pn.y = pn.y + k.c.y;
-                    record(found++, lj);
-                }
-            }
-        } else if (a.collisions && finitef(pn.x) && finitef(pn.y)) {
-            constexpr int kList = REC ? (int)kDiffTapeNbr : 4;
-            ContactList<kList, uint32_t> L;
-            const float4 own = make_float4(pn.x, pn.y, c.rad[li], __uint_as_float(li));
-            found = lds_contacts_direct(lds_grid_uniform(*c.grid), c.cnt, c.rec, make_float2(pn.x, pn.y), own.z, li,
-                                        W.rmax, pn, L,
-                                        [&](const float4 oth) {
-                                            const uint32_t lj = __float_as_uint(oth.w);
-                                            return lds_correction(own, oth, c.mass[li], c.mass[lj], li > lj, false);
-                                        },
-                                        [](uint32_t, const LdsContact&) {});
-#pragma unroll
-            for (uint32_t t = 0; REC && t + 1 < kDiffTapeNbr; ++t)
-                if (t < L.n) record(t, L.key[t]);
+        } else if (a.collisions && finitef(xy.x) && finitef(xy.y)) {
+            count = kNoRoom;
         }
-        if (REC && a.collisions) {
-            w0 |= found < 0xFFFFu ? found : 0xFFFFu;
-            reinterpret_cast<uint4*>(a.tape_nbr)[tape] = make_uint4(w0, w1, w2, w3);
-        }
-        put(sums, j, pn);
+        if (count == kNoRoom)
+            pending |= 1u << j;
+        else
+            finish(j, first, count, false);
     }
-    if (crowd) __syncthreads();  // bodies without room read others' snapshots
+    if (crowd) queue_rounds(c, o, W, lists, nout, pending, contact, finish);
     if (tid == 0) c.out->pairs[par ^ 1u] = 0;
     if (tid < kOutMax) c.out->count[par ^ 1u][tid] = 0;
     // From here to the end of the substep a thread touches the positions and velocities of its

@@ -411,49 +411,4 @@ __device__ __forceinline__ uint32_t lds_sum(const LdsPairs& pr, const uint32_t* 
     return k;
 }
 
-// The contacts of a body that did not go through the queue, summed into `p` in ascending
-// partner index: `pair(other record)` gives the LdsContact of a candidate, `once` is called
-// with each contact's.  L ends with the K smallest partners' corrections; returns the contacts.
-template <int K, class Pair, class Once>
-__device__ __forceinline__ uint32_t lds_contacts_direct(const LdsGrid& g, const uint32_t* start, const float4* rec,
-                                                        float2 xy, float r, uint32_t li, float rmax, float2& p,
-                                                        ContactList<K, uint32_t>& L, Pair&& pair, Once&& once) {
-    const LdsRect c = lds_rect(g, xy.x, xy.y, r + rmax);
-    auto enumerate = [&](auto&& sink) {
-        for (int32_t cy = c.cy0; cy <= c.cy1; ++cy) {
-            const uint32_t row = (uint32_t)cy * (uint32_t)g.nx;
-            const uint32_t t1 = start[row + (uint32_t)c.cx1 + 1u];
-            for (uint32_t t = start[row + (uint32_t)c.cx0]; t < t1; ++t) {
-                const float4 other = rec[t];
-                const uint32_t lj = __float_as_uint(other.w);
-                if (lj == li) continue;
-                const LdsContact k = pair(other);
-                if (k.hit) sink(lj, k);
-            }
-        }
-    };
-    L.init();
-    enumerate([&](uint32_t lj, const LdsContact& k) {
-        once(lj, k);
-        L.add(lj, k.c.x, k.c.y);
-    });
-    if (L.n == 0) return 0;
-    uint32_t last = L.apply(p);
-    for (uint32_t done = L.n < (uint32_t)K ? L.n : (uint32_t)K; done < L.n; ++done) {  // more than K: one at a time
-        uint32_t best = kNoPair;
-        float2 b = make_float2(0.0f, 0.0f);
-        enumerate([&](uint32_t lj, const LdsContact& k) {
-            if (lj > last && lj < best) {
-                best = lj;
-                b = k.c;
-            }
-        });
-        if (best == kNoPair) break;
-        p.x = p.x + b.x;
-        p.y = p.y + b.y;
-        last = best;
-    }
-    return L.n;
-}
-
 }  // namespace bg
