@@ -408,7 +408,7 @@ int bg_spatial_hash_query_host(float cell_size, const bg_spatial_point *points, 
 
 /* bg_spatial_hash_query without any allocation: the same arguments, results
  * and kernels, with the scratch in a device array the library holds on each
- * GPU until the process ends (36 MiB).  For callers that cannot allocate
+ * GPU until the process ends (52 MiB).  For callers that cannot allocate
  * device memory (code under stream capture, serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  Limits: at most
  * 1,048,576 points and 1,048,576 queries (BG_ERR_CAPACITY beyond, nothing
