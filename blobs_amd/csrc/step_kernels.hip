@@ -61,31 +61,41 @@ __device__ __forceinline__ void rebuild_key_at(uint32_t i, const KeysArgs& k) {
     }
 }
 
-// Colliders into cell order: slot = cell_start[key] + rank (cell_start is the
-// exclusive scan of the counts); the counts are cleared for the next rebuild.
-// Beside the collider index, each slot gets the record the contact pass tests
+// Collider i into cell order: slot = cell_start[key] + rank (cell_start is the exclusive scan of
+// the counts).  Beside the collider index, each slot gets the record the contact pass tests
 // (position, radius, parent body), so a candidate is one load from a cell run.
-__global__ __launch_bounds__(kThreads) void k_cell_scatter(const uint32_t* __restrict__ keys,
-                                                           const uint32_t* __restrict__ rank, uint32_t nc,
-                                                           const uint32_t* __restrict__ cell_start,
-                                                           uint32_t* __restrict__ vals, uint32_t* cnt,
-                                                           uint32_t n_cnt, const float2* __restrict__ abs,
-                                                           const float* __restrict__ radius,
-                                                           const int32_t* __restrict__ parent,
-                                                           float4* __restrict__ rec,
+struct CellScatter {
+    const uint32_t* keys;
+    const uint32_t* rank;
+    uint32_t nc;
+    const uint32_t* cell_start;
+    uint32_t* vals;
+    const float2* abs;
+    const float* radius;
+    const int32_t* parent;
+    float4* rec;
+};
+__device__ __forceinline__ void scatter_at(uint32_t i, const CellScatter& k) {
+    if (i >= k.nc) return;
+    const uint32_t slot = k.cell_start[k.keys[i]] + k.rank[i];
+    if (slot < k.nc) {  // consistent counts and scan never fail this
+        k.vals[slot] = i;
+        const float2 x = k.abs[i];
+        k.rec[slot] = make_float4(x.x, x.y, k.radius[i], __int_as_float(k.parent[i]));
+    }
+}
+CellScatter cell_scatter_of(const DeviceWorld& d) {
+    return {d.keys, d.vals_tmp, d.nc, d.cell_start, d.vals, d.c.abs, d.c.radius, d.c.parent, d.crec};
+}
+
+// The counts are cleared for the next rebuild.
+__global__ __launch_bounds__(kThreads) void k_cell_scatter(CellScatter k, uint32_t* cnt, uint32_t n_cnt,
                                                            const GridParams* __restrict__ grid) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // only the grid's cells were counted (and scanned): clear those
     const uint32_t n_used = grid->ncells + 1u < n_cnt ? grid->ncells + 1u : n_cnt;
     for (uint32_t c = i; c < n_used; c += gridDim.x * blockDim.x) cnt[c] = 0u;
-    if (i < nc) {
-        const uint32_t slot = cell_start[keys[i]] + rank[i];
-        if (slot < nc) {  // consistent counts and scan never fail this
-            vals[slot] = i;
-            const float2 x = abs[i];
-            rec[slot] = make_float4(x.x, x.y, radius[i], __int_as_float(parent[i]));
-        }
-    }
+    scatter_at(i, k);
 }
 
 // ============================================================ general path
@@ -384,20 +394,29 @@ constexpr int kDirectRegs = 4;      // corrections of a collider outside the que
 // its own in ascending partner: 36.4 us over the scene's first 112 steps, against 48.1 with a
 // thread doing all of its collider's contacts, sixteen sorted in registers (166
 // registers, three waves a SIMD); 6.2 against 14.2 at 1,115 colliders.
+struct ListsLds {
+    float4 own[BG_WAVE];     // (x, y, radius, body's mass)
+    uint2 id[BG_WAVE];       // collider, body
+    uint2 pair[kPairCap];    // own lane, partner's slot; then (partner, -) or (kNil, -)
+    float2 res[kPairCap];
+};
+// One wave's LDS accesses keep their order; the compiler has to as well.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 template <bool GROUPS, bool SENSORS>
-__global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d, SubstepArgs a) {
-    static_assert(kContactThreads == BG_WAVE, "a block is one wave");
-    __shared__ float4 s_own[kContactThreads];   // (x, y, radius, body's mass)
-    __shared__ uint2 s_id[kContactThreads];     // collider, body
-    __shared__ uint2 s_pair[kPairCap];          // own lane, partner's slot; then (partner, -) or (kNil, -)
-    __shared__ float2 s_res[kPairCap];
+__device__ __forceinline__ void contact_lists(const DeviceWorld& d, const SubstepArgs& a, ListsLds& lds, uint32_t slot,
+                                              uint32_t count_slot) {
     // threads walk the colliders in cell order (the order the key pass just sorted them
     // into): a wave's colliders are neighbours, so their candidate records overlap in cache
     // (an XCD takes a contiguous range of them), and each one's own record is the slot's
     // (x, y, radius, parent), loaded coalesced
-    const uint32_t lane = threadIdx.x;
-    const uint32_t slot = xcd_block(blockIdx.x, gridDim.x) * kContactThreads + lane;
-    if (slot == 0) d.cfb_n[0] = 0u;  // k_contact_merge fills the fallback list after this kernel
+    float4* s_own = lds.own;
+    uint2 *s_id = lds.id, *s_pair = lds.pair;
+    float2* s_res = lds.res;
+    const uint32_t lane = threadIdx.x & (BG_WAVE - 1);
+    if (slot == 0) d.cfb_n[0] = 0u;  // k_contact_merge fills the fallback list after this
     uint32_t count = 0, flags = 0;
     uint32_t c = 0, n = 0, first = 0, n_put = 0;
     bool direct = false;
@@ -550,9 +569,9 @@ __global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d
     if (fits)
         for (uint32_t e = first; marked != 0; ++e, marked &= marked - 1)
             s_pair[e] = make_uint2(lane, flat_slot((uint32_t)__builtin_ctzll(marked)));
-    __syncthreads();
+    wave_sync();
     // ---- correct: a pair a lane
-    for (uint32_t e = lane; e < queued; e += kContactThreads) {
+    for (uint32_t e = lane; e < queued; e += BG_WAVE) {
         const uint2 pr = s_pair[e];
         const float4 rb = d.crec[pr.y];
         const uint32_t j = d.vals[pr.y];
@@ -563,7 +582,7 @@ __global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d
             s_res[e] = make_float2(x, y);
         });
     }
-    __syncthreads();
+    wave_sync();
     // ---- each collider's own, in ascending partner: for this collider c the pair key (max, min) of
     // (c, j) orders as j does (every j < c before every j > c, each side by j)
     for (uint32_t next = 0; n_put < n; ++n_put) {
@@ -611,7 +630,16 @@ __global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d
     if (slot < d.nc) d.ccnt[c] = n_put;
     if (flags) atomicOr(&d.accum->error_flags, flags);
     const uint32_t sum = wave_sum_u32(count);
-    if (lane == 0 && sum) d.block_contacts[blockIdx.x] += sum;
+    if (lane == 0 && sum) d.block_contacts[count_slot] += sum;
+    wave_sync();  // (the wave's next pass writes the same memory)
+}
+
+template <bool GROUPS, bool SENSORS>
+__global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d, SubstepArgs a) {
+    static_assert(kContactThreads == BG_WAVE, "a block is one wave");
+    __shared__ ListsLds lds;
+    contact_lists<GROUPS, SENSORS>(d, a, lds, xcd_block(blockIdx.x, gridDim.x) * kContactThreads + threadIdx.x,
+                                   blockIdx.x);
 }
 
 // Second half: adds each body's corrections to its position in key order --
@@ -633,8 +661,8 @@ __device__ __forceinline__ uint64_t merge_key(float4 v) {
     return ((uint64_t)__float_as_uint(v.x) << 32) | __float_as_uint(v.y);
 }
 
-__global__ __launch_bounds__(kThreads) void k_contact_merge(DeviceWorld d) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+// (whole waves: thread t of the pass)
+__device__ __forceinline__ void contact_merge(const DeviceWorld& d, uint32_t t) {
     const uint32_t b = t / kMergeLanes, r = t % kMergeLanes;
     uint32_t k0 = 0, k1 = 0;
     float2 p = make_float2(0.0f, 0.0f);
@@ -712,6 +740,10 @@ __global__ __launch_bounds__(kThreads) void k_contact_merge(DeviceWorld d) {
     if (fallback) d.cfb_list[atomicAdd(d.cfb_n, 1u)] = b;
 }
 
+__global__ __launch_bounds__(kThreads) void k_contact_merge(DeviceWorld d) {
+    contact_merge(d, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
 // Rotation correction of one joint from its axis (physics.rs:462-469): the
 // reference adds corr * dt to rotation a and subtracts it from rotation b.
 // Positions never read rotations inside the joint stage (anchors are not
@@ -746,33 +778,44 @@ struct JointRec {
     uint32_t a, b;  // body list index | static << 31
 };
 
-__global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h) {
-    __shared__ float4 s_anchor[kStageJoints], s_mass[kStageJoints];
-    __shared__ float2 s_len[kStageJoints];
-    __shared__ uint2 s_ab[kStageJoints];
-    __shared__ float2 s_pos[kStageBodies];
-    __shared__ int32_t s_gid[kStageBodies];
-    __shared__ uint32_t s_level[kStageLevels + 1];
-    __shared__ uint2 s_entry[kStageSolves];
-    __shared__ float2 s_axis[kStageSolves];
-    const JointGroup g = d.jg[blockIdx.x];
+struct JointsLds {
+    float4 s_anchor[kStageJoints], s_mass[kStageJoints];
+    float2 s_len[kStageJoints];
+    uint2 s_ab[kStageJoints];
+    float2 s_pos[kStageBodies];
+    int32_t s_gid[kStageBodies];
+    uint32_t s_level[kStageLevels + 1];
+    uint2 s_entry[kStageSolves];
+    float2 s_axis[kStageSolves];
+};
+template <uint32_t NT>
+__device__ __forceinline__ void joint_group(const DeviceWorld& d, float h, uint32_t group, JointsLds& lds) {
+    auto &s_anchor = lds.s_anchor, &s_mass = lds.s_mass;
+    auto& s_len = lds.s_len;
+    auto& s_pos = lds.s_pos;
+    auto& s_axis = lds.s_axis;
+    auto& s_ab = lds.s_ab;
+    auto& s_entry = lds.s_entry;
+    auto& s_gid = lds.s_gid;
+    auto& s_level = lds.s_level;
+    const JointGroup g = d.jg[group];
     const uint32_t tid = threadIdx.x, nq = g.q1 - g.q0, nbod = g.b1 - g.b0, nl = g.l1 - g.l0;
     const uint32_t e0 = d.jl_start[g.l0], n = d.jl_start[g.l1] - e0;
     const bool staged = nq <= kStageJoints && nbod <= kStageBodies && nl <= kStageLevels && n <= kStageSolves;
     if (staged) {
-        for (uint32_t i = tid; i < nbod; i += kJointThreads) {
+        for (uint32_t i = tid; i < nbod; i += NT) {
             const int32_t b = d.jg_body[g.b0 + i];
             s_gid[i] = b;
             s_pos[i] = d.b.pos[b];
         }
-        for (uint32_t i = tid; i < nq; i += kJointThreads) {
+        for (uint32_t i = tid; i < nq; i += NT) {
             s_anchor[i] = d.jq_anchor[g.q0 + i];
             s_mass[i] = d.jq_mass[g.q0 + i];
             s_len[i] = d.jq_len[g.q0 + i];
             s_ab[i] = d.jq_ab[g.q0 + i];
         }
-        for (uint32_t i = tid; i <= nl; i += kJointThreads) s_level[i] = d.jl_start[g.l0 + i] - e0;
-        for (uint32_t i = tid; i < n; i += kJointThreads) s_entry[i] = d.j_entry[e0 + i];
+        for (uint32_t i = tid; i <= nl; i += NT) s_level[i] = d.jl_start[g.l0 + i] - e0;
+        for (uint32_t i = tid; i < n; i += NT) s_entry[i] = d.j_entry[e0 + i];
     }
     __syncthreads();
     uint32_t flags = 0;
@@ -838,8 +881,8 @@ __global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h
     if (flags) atomicOr(&d.accum->error_flags, flags);
     __syncthreads();
     if (staged)
-        for (uint32_t i = tid; i < nbod; i += kJointThreads) d.b.pos[s_gid[i]] = s_pos[i];
-    for (uint32_t e = tid; e < n; e += kJointThreads) {
+        for (uint32_t i = tid; i < nbod; i += NT) d.b.pos[s_gid[i]] = s_pos[i];
+    for (uint32_t e = tid; e < n; e += NT) {
         const uint2 en = staged ? s_entry[e] : d.j_entry[e0 + e];
         const float2 axis = staged ? s_axis[e] : d.jrot[en.y];
         const float target = staged ? s_len[en.x].y : d.jq_len[g.q0 + en.x].y;
@@ -847,6 +890,11 @@ __global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h
         if (!(vlen(axis.x, axis.y) < 1e-6f)) step = make_float2(joint_rotation_corr(axis.x, axis.y, target) * h, 1.0f);
         d.jrot[en.y] = step;
     }
+}
+
+__global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h) {
+    __shared__ JointsLds lds;
+    joint_group<kJointThreads>(d, h, blockIdx.x, lds);
 }
 
 // Verlet + collider transforms + constraints (physics.rs:323-395), and the
@@ -857,12 +905,13 @@ __global__ __launch_bounds__(kJointThreads) void k_joints(DeviceWorld d, float h
 // 294,249 colliders against 24.9 (6.0 against 10.4 at 250 bodies).
 constexpr uint32_t kBodyLanes = 4;
 
-__global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepArgs a) {
-    __shared__ uint32_t s_box[4][kThreads / BG_WAVE];
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+struct Box {
+    uint32_t b0 = 0xFFFFFFFFu, b1 = 0xFFFFFFFFu, b2 = 0u, b3 = 0u;  // f2ord bounding box
+};
+// (whole waves: thread t of the pass)
+__device__ __forceinline__ void integrate_at(const DeviceWorld& d, const SubstepArgs& a, uint32_t t, Box& box) {
     const uint32_t b = t / kBodyLanes, r = t % kBodyLanes;
     uint32_t flags = 0;
-    uint32_t b0 = 0xFFFFFFFFu, b1 = 0xFFFFFFFFu, b2 = 0u, b3 = 0u;  // f2ord bounding box
     if (b < d.nb) {
         const uint32_t fl = d.b.bflags[b];
         const uint32_t c0 = d.bc_start[b], c1 = d.bc_start[b + 1];
@@ -938,10 +987,10 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
                 const float2 x = body_xform(sn, cs, s.p, off);
                 d.c.abs[c] = x;
                 if (finitef(x.x) && finitef(x.y)) {
-                    b0 = min(b0, f2ord(x.x));
-                    b1 = min(b1, f2ord(x.y));
-                    b2 = max(b2, f2ord(x.x));
-                    b3 = max(b3, f2ord(x.y));
+                    box.b0 = min(box.b0, f2ord(x.x));
+                    box.b1 = min(box.b1, f2ord(x.y));
+                    box.b2 = max(box.b2, f2ord(x.x));
+                    box.b3 = max(box.b3, f2ord(x.y));
                 }
                 k += kBodyLanes;
                 if (k >= c1) break;
@@ -966,10 +1015,16 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
         }
     }
     static_assert(BG_WAVE % kBodyLanes == 0, "a body's lanes in one wave");
-    b0 = wave_prefix(b0, 0xFFFFFFFFu, MinU32());
-    b1 = wave_prefix(b1, 0xFFFFFFFFu, MinU32());
-    b2 = wave_prefix(b2, 0u, MaxU32());
-    b3 = wave_prefix(b3, 0u, MaxU32());
+    if (flags) atomicOr(&d.accum->error_flags, flags);
+}
+// The block's box into the substep's record.
+template <uint32_t NT>
+__device__ __forceinline__ void box_flush(const DeviceWorld& d, uint32_t parity, const Box& box,
+                                          uint32_t (&s_box)[4][NT / BG_WAVE]) {
+    const uint32_t b0 = wave_prefix(box.b0, 0xFFFFFFFFu, MinU32());
+    const uint32_t b1 = wave_prefix(box.b1, 0xFFFFFFFFu, MinU32());
+    const uint32_t b2 = wave_prefix(box.b2, 0u, MaxU32());
+    const uint32_t b3 = wave_prefix(box.b3, 0u, MaxU32());
     const uint32_t wv = threadIdx.x / BG_WAVE;
     if ((threadIdx.x & (BG_WAVE - 1)) == BG_WAVE - 1) {
         s_box[0][wv] = b0;
@@ -977,17 +1032,106 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
         s_box[2][wv] = b2;
         s_box[3][wv] = b3;
     }
-    if (flags) atomicOr(&d.accum->error_flags, flags);
     __syncthreads();
     if (threadIdx.x < 4) {
         const uint32_t* v = s_box[threadIdx.x];
-        uint32_t* to = &d.accum->bbox[a.parity][threadIdx.x];
-        static_assert(kThreads / BG_WAVE == 4, "the four below");
+        uint32_t* to = &d.accum->bbox[parity][threadIdx.x];
+        uint32_t m = v[0];
+#pragma unroll
+        for (uint32_t i = 1; i < NT / BG_WAVE; ++i) m = threadIdx.x < 2 ? min(m, v[i]) : max(m, v[i]);
         if (threadIdx.x < 2)
-            atomic_min_if_less(to, min(min(v[0], v[1]), min(v[2], v[3])));
+            atomic_min_if_less(to, m);
         else
-            atomic_max_if_greater(to, max(max(v[0], v[1]), max(v[2], v[3])));
+            atomic_max_if_greater(to, m);
     }
+}
+
+__global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepArgs a) {
+    __shared__ uint32_t s_box[4][kThreads / BG_WAVE];
+    Box box;
+    integrate_at(d, a, blockIdx.x * blockDim.x + threadIdx.x, box);
+    box_flush<kThreads>(d, a.parity, box, s_box);
+}
+
+// ---- small worlds ------------------------------------------------------------
+//
+// A world of at most kSmallColliders colliders and kSmallGeneral bodies takes its substep in four
+// launches instead of ten: one workgroup sorts and works out the contacts, one solves the
+// joints and integrates (the fallback and the ordered pass in between, which have nothing to do
+// in most substeps).  A pass of such a world is a launch's few microseconds whatever it does, and
+// a barrier a tenth of one; but one workgroup has one CU's latency to hide its loads in, so a
+// second round over the colliders costs what the launches did.  A step: 48 bodies 251 us against
+// 319 in ten launches, 120 285 against 359, 250 (1,115 colliders) 359 against 379, but 300
+// 460 against 395.
+constexpr uint32_t kSmallThreads = 1024;
+
+template <bool GROUPS, bool SENSORS>
+__global__ __launch_bounds__(kSmallThreads) void k_small_contacts(KeysArgs k, CellScatter sc, DeviceWorld d,
+                                                                  SubstepArgs a) {
+    __shared__ ListsLds lds[kSmallThreads / BG_WAVE];
+    __shared__ uint32_t red[kSmallThreads / BG_WAVE];
+    const uint32_t t = threadIdx.x;
+    for (uint32_t i = t; i < d.nc + (a.has_springs ? d.nb : 0u); i += kSmallThreads) {
+        if (i < d.nc)
+            rebuild_key_at(i, k);
+        else
+            forces_at(i - d.nc, d, a);
+    }
+    __syncthreads();
+    {  // exclusive scan of the cells' counts, which are cleared: up to four times four a thread
+        const uint32_t n = d.grid->ncells, n4 = (n + 3u) / 4u, per = (n4 + kSmallThreads - 1u) / kSmallThreads;
+        uint4* cnt = reinterpret_cast<uint4*>(k.cnt);
+        uint4* start = reinterpret_cast<uint4*>(d.cell_start);
+        uint4 v[4];
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; ++g) {
+            const uint32_t i = t * per + g;
+            v[g] = g < per && i < n4 ? cnt[i] : make_uint4(0u, 0u, 0u, 0u);
+        }
+#pragma unroll
+        for (uint32_t g = 0; g < 4; ++g) sum += v[g].x + v[g].y + v[g].z + v[g].w;
+        const uint32_t incl = wave_prefix(sum, 0u, AddU32()), lane = t & (BG_WAVE - 1);
+        if (lane == BG_WAVE - 1) red[t / BG_WAVE] = incl;
+        __syncthreads();
+        const uint32_t tot = wave_prefix(lane < kSmallThreads / BG_WAVE ? red[lane] : 0u, 0u, AddU32());
+        const int w = __builtin_amdgcn_readfirstlane((int)(t / BG_WAVE));
+        uint32_t run = (w > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)tot, w - 1) : 0u) + incl - sum;
+#pragma unroll
+        for (uint32_t g = 0; g < 4; ++g) {
+            const uint32_t i = t * per + g;
+            if (g >= per || i >= n4) continue;
+            const uint4 c = v[g];
+            start[i] = make_uint4(run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z);
+            run += c.x + c.y + c.z + c.w;
+            cnt[i] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        __syncthreads();
+        if (t == 0) d.cell_start[n] = d.nc;  // (the table has a word to spare)
+        static_assert(kSmallColliders * 4u <= 16u * kSmallThreads, "cells of the largest: next power of two of four a collider");
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < d.nc; i += kSmallThreads) scatter_at(i, sc);
+    __syncthreads();
+    for (uint32_t i = t; i < (d.nc + BG_WAVE - 1u) / BG_WAVE * BG_WAVE; i += kSmallThreads)
+        contact_lists<GROUPS, SENSORS>(d, a, lds[t / BG_WAVE], i, i / BG_WAVE);
+    __syncthreads();
+    for (uint32_t i = t; i < (d.nb * kMergeLanes + BG_WAVE - 1u) / BG_WAVE * BG_WAVE; i += kSmallThreads)
+        contact_merge(d, i);
+}
+
+__global__ __launch_bounds__(kSmallThreads) void k_small_integrate(DeviceWorld d, SubstepArgs a) {
+    __shared__ JointsLds lds;
+    __shared__ uint32_t s_box[4][kSmallThreads / BG_WAVE];
+    if (a.joint_rot)
+        for (uint32_t g = 0; g < d.n_jgroups; ++g) {
+            joint_group<kSmallThreads>(d, a.h, g, lds);
+            __syncthreads();
+        }
+    Box box;
+    for (uint32_t i = threadIdx.x; i < (d.nb * kBodyLanes + BG_WAVE - 1u) / BG_WAVE * BG_WAVE; i += kSmallThreads)
+        integrate_at(d, a, i, box);
+    box_flush<kSmallThreads>(d, a.parity, box, s_box);
 }
 
 }  // namespace
@@ -1004,9 +1148,8 @@ hipError_t launch_rebuild_sort_and_cells(DeviceWorld& d) {
     hipError_t e = exclusive_scan_u32(d.cell_count, d.cell_start, d.cells_cap + 1, d.sort, d.stream, last);
     if (e != hipSuccess) return e;
     const uint32_t n = d.nc > 0 ? d.nc : 1u;
-    k_cell_scatter<<<div_up(n, kThreads), kThreads, 0, d.stream>>>(d.keys, d.vals_tmp, d.nc, d.cell_start, d.vals,
-                                                                   d.cell_count, d.cells_cap + 1, d.c.abs,
-                                                                   d.c.radius, d.c.parent, d.crec, d.grid);
+    k_cell_scatter<<<div_up(n, kThreads), kThreads, 0, d.stream>>>(cell_scatter_of(d), d.cell_count, d.cells_cap + 1,
+                                                                   d.grid);
     return hipGetLastError();
 }
 
@@ -1014,6 +1157,38 @@ hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, bool gro
                                   const KeysArgs* rebuild) {
     if (d.nb == 0) return hipSuccess;
     const uint32_t blocks = div_up(d.nb, kThreads);
+    const bool small = rebuild && a.collisions && d.clist && d.nc > 0 && d.nc <= kSmallColliders && d.nb <= kSmallGeneral;
+    SubstepArgs ai = a;
+    ai.joint_rot = 0u;
+    if (d.n_jgroups > 0 && d.j_iters > 0) {
+        ai.joint_rot = 1u;
+        ai.joint_iters = d.j_iters;
+        ai.joint_count = d.nj;
+    }
+    if (small) {
+        const CellScatter sc = cell_scatter_of(d);
+        const uint32_t fb = std::min(div_up(d.nb, kContactThreads), 256u);
+#define BG_SMALL(G, S)                                                                  \
+    do {                                                                                \
+        k_small_contacts<G, S><<<1, kSmallThreads, 0, d.stream>>>(*rebuild, sc, d, a);  \
+        k_contacts<G, S><<<fb, kContactThreads, 0, d.stream>>>(d, a, d.cfb_list);       \
+    } while (0)
+        if (groups && sensors)
+            BG_SMALL(true, true);
+        else if (groups)
+            BG_SMALL(true, false);
+        else if (sensors)
+            BG_SMALL(false, true);
+        else
+            BG_SMALL(false, false);
+#undef BG_SMALL
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        e = launch_contacts_ordered(d, a, groups, sensors);
+        if (e != hipSuccess) return e;
+        k_small_integrate<<<1, kSmallThreads, 0, d.stream>>>(d, ai);
+        return hipGetLastError();
+    }
     // the rebuild's keys and the substep's forces in one launch, then the rest of the rebuild
     const uint32_t key_blocks = rebuild ? div_up(rebuild->nc > 0 ? rebuild->nc : 1u, kThreads) : 0u;
     const uint32_t force_blocks = a.has_springs ? blocks : 0u;
@@ -1054,14 +1229,7 @@ hipError_t launch_general_substep(DeviceWorld& d, const SubstepArgs& a, bool gro
         e = launch_contacts_ordered(d, a, groups, sensors);
         if (e != hipSuccess) return e;
     }
-    SubstepArgs ai = a;
-    ai.joint_rot = 0u;
-    if (d.n_jgroups > 0 && d.j_iters > 0) {
-        k_joints<<<d.n_jgroups, kJointThreads, 0, d.stream>>>(d, a.h);
-        ai.joint_rot = 1u;
-        ai.joint_iters = d.j_iters;
-        ai.joint_count = d.nj;
-    }
+    if (ai.joint_rot) k_joints<<<d.n_jgroups, kJointThreads, 0, d.stream>>>(d, a.h);
     k_integrate<<<div_up(d.nb, kThreads / kBodyLanes), kThreads, 0, d.stream>>>(d, ai);
     return hipGetLastError();
 }
