@@ -36,6 +36,7 @@ constexpr uint32_t kPushOutHold = 4;
 // more comes through pinned staging of two halves of at most kStageHalf bytes.
 constexpr size_t kExportDirect = 256 << 10;
 constexpr size_t kStageHalf = 4 << 20;
+constexpr size_t kStageLeast = 32 << 10;
 
 template <class T>
 hipError_t dmalloc(T** p, size_t n) {
@@ -507,7 +508,8 @@ int World::get_collider_positions(float* abs, uint32_t* count) {
 }
 
 int World::ensure_staging(size_t bytes) {
-    const size_t half = std::min<size_t>(kStageHalf, (bytes + 4095) & ~(size_t)4095);
+    // (pinned memory costs some 200 us an allocation: a small world's first one does for all its reads)
+    const size_t half = std::min<size_t>(kStageHalf, std::max<size_t>((bytes + 4095) & ~(size_t)4095, kStageLeast));
     for (hipEvent_t& e : stage_event_)
         if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (half <= stage_half_) return BG_OK;
