@@ -243,7 +243,15 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         return r;
     };
     int result = BG_OK;
-    const uint32_t todo = n_chunks - done;
+    // (a longer rebuild interval on trial: the last chunk, eagerly; chunks too short for that go over to it)
+    const bool trial = trial_due_ && n_chunks - done > 1u &&
+                       (uint64_t)chunk_steps * params_.substeps >= level_substeps(interval_level_ - 1u);
+    if (trial_due_ && !trial && !trial_ran_) {
+        trial_due_ = false;
+        --interval_level_;
+        interval_calm_ = 0;
+    }
+    const uint32_t todo = n_chunks - done - (trial ? 1u : 0u);
     bool cyclic = false;
     if (todo > 0) {
         const LaunchState s0 = state();
@@ -267,6 +275,12 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         // device stopped (todo % m graphs into the cycle)
         if (cyclic && result == BG_OK)
             for (uint32_t r = 0; r < todo % m && result == BG_OK; ++r) result = capture(false);
+    }
+    if (trial && result == BG_OK) {
+        trial_allowed_ = true;
+        result = launch_steps(delta, chunk_steps);
+        trial_allowed_ = false;
+        if (result == BG_OK) advance_time(delta, chunk_steps);
     }
     hipError_t e = hipStreamSynchronize(d.stream);
     release();

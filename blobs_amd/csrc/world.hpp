@@ -206,7 +206,10 @@ private:
     uint32_t rebuild_interval_ = 0;  // in steps; 0: adapted to the outliers (adapt_interval)
     uint32_t interval_level_ = kLevelUnset, interval_calm_ = 0, interval_backoff_ = 0;
     static constexpr uint32_t kLevelUnset = 0xFFu, kLevels = 5;
+    // the next longer interval is to be tried at the end of a call; this call has done so
+    bool trial_due_ = false, trial_allowed_ = false, trial_ran_ = false;
     uint32_t interval_substeps();
+    uint32_t level_substeps(uint32_t level) const;
     void adapt_interval(const StepAccum& acc, uint32_t n_steps);
     // world properties fixed at upload
     float rmax_ = 0.0f;
