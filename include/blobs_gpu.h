@@ -201,7 +201,8 @@ int bg_synchronize(bg_world *w);
 int bg_set_deferred_checks(bg_world *w, int enable);
 /* n_chunks x chunk_steps calls of Physics::step(delta) (physics.rs:78-82),
  * each chunk replayed from a hipGraph captured once (launch overhead paid
- * once per capture, not per kernel).  Same results as bg_step with
+ * once per capture, not per kernel; small worlds take one launch a chunk
+ * and no graph).  Same results as bg_step with
  * n_steps = chunk_steps * n_chunks.  The reference has no counterpart: it
  * is the multi-step driver the batched benchmark loop needs. */
 int bg_batch_run(bg_world *w, double delta, uint32_t chunk_steps, uint32_t n_chunks);
