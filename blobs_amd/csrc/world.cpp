@@ -780,6 +780,7 @@ int World::set_broadphase(float cell_scale, float skin, uint32_t rebuild_interva
     cell_scale_ = cell_scale;
     skin_scale_ = skin;
     rebuild_interval_ = rebuild_interval;
+    trial_due_ = trial_ran_ = check_trial_ = false;
     need_rebuild_ = true;
     return BG_OK;
 }
@@ -1807,7 +1808,7 @@ int World::finish_deferred_check(bool wait) {
         HIP_TRY(q);
     }
     check_pending_ = false;
-    adapt_interval(*host_acc_, check_steps_);
+    adapt_interval(*host_acc_, check_steps_, check_trial_);
     return process_flags(host_acc_->error_flags);
 }
 
@@ -1817,7 +1818,7 @@ int World::check_errors(uint32_t* flags_out, uint32_t n_steps) {
     HIP_TRY(hipMemcpyAsync(&acc, d.accum, sizeof(acc), hipMemcpyDeviceToHost, d.stream));
     HIP_TRY(hipStreamSynchronize(d.stream));
     if (flags_out) *flags_out = acc.error_flags;
-    adapt_interval(acc, n_steps);
+    adapt_interval(acc, n_steps, trial_ran_);
     if (acc.error_flags) {
         uint32_t zero = 0;
         HIP_TRY(hipMemcpyAsync(&d.accum->error_flags, &zero, 4, hipMemcpyHostToDevice, d.stream));
@@ -2079,15 +2080,16 @@ uint32_t World::level_substeps(uint32_t level) const {
 //
 // In a call of many steps the longer interval is first tried on the last of them only: a wrong one
 // for all of 30 steps took 5.8 and 8.1 ms instead of 3.2 at 50,021 bodies.
-void World::adapt_interval(const StepAccum& acc, uint32_t n_steps) {
+void World::adapt_interval(const StepAccum& acc, uint32_t n_steps, bool tried) {
     if (rebuild_interval_ || small_active() || path_ != StepPath::Sphere || !params_.collisions_enabled || n_steps == 0) return;
     (void)interval_substeps();
     static constexpr uint32_t kOutlierShare[kLevels] = {512, 200, 64, 32, 32};  // one body in so many
     // (A second rebuild within a step is another 40 us of launches however small the world, the
     // price of some 2,000 outliers: 2,360 bodies fallen on a pile take 346 us with it, 300 without.)
     auto limit_of = [&](uint32_t level) { return std::max(d_.nb / kOutlierShare[level], level >= 2 ? 2048u : 16u); };
-    if (trial_ran_) {
-        trial_due_ = trial_ran_ = false;
+    if (trial_ran_ && !tried) return;  // an older call's record: the trial's is on its way
+    if (tried) {
+        trial_due_ = trial_ran_ = check_trial_ = false;
         interval_calm_ = 0;
         if (acc.n_outliers <= limit_of(interval_level_ - 1u))
             --interval_level_;
@@ -2144,6 +2146,7 @@ int World::step(double delta, uint32_t n) {
         HIP_TRY(hipEventRecord(check_event_, d.stream));
         check_pending_ = true;
         check_steps_ = n;
+        check_trial_ = trial_ran_;
         return BG_OK;
     }
     uint32_t flags = 0;

@@ -208,9 +208,10 @@ private:
     static constexpr uint32_t kLevelUnset = 0xFFu, kLevels = 5;
     // the next longer interval is to be tried at the end of a call; this call has done so
     bool trial_due_ = false, trial_allowed_ = false, trial_ran_ = false;
+    bool check_trial_ = false;  // the pending deferred check is of a call that has tried it
     uint32_t interval_substeps();
     uint32_t level_substeps(uint32_t level) const;
-    void adapt_interval(const StepAccum& acc, uint32_t n_steps);
+    void adapt_interval(const StepAccum& acc, uint32_t n_steps, bool tried);
     // world properties fixed at upload
     float rmax_ = 0.0f;
     float mass_per_r_ = 0.0f;  // sphere path: every body's mass is exactly this times its radius (0: not so)

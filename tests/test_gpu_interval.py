@@ -59,3 +59,19 @@ def test_adapted_interval_of_a_batch_in_chunks():
         b.run_chunks(scs[0].dt, 2, 3)
         assert np.array_equal(bits(a.bodies()["position"]), bits(b.bodies()["position"]))
     assert a.contact_count() == b.contact_count() > 0
+
+
+@pytest.mark.parametrize("steps_per_call", [1, 40])
+def test_adapted_interval_with_deferred_checks(steps_per_call):
+    # one call's record is read while the next call, perhaps with a trial, is queued
+    sc = fast_scene(3000, 13)
+    a, b = sc.build_physics()[0], sc.build_physics()[0]
+    a.set_deferred_checks(True)
+    b.set_broadphase(1.25, 1, 0.25)
+    for _ in range(240 // steps_per_call):
+        a.step(sc.dt, steps_per_call)
+        b.step(sc.dt, steps_per_call)
+    a.synchronize()
+    sa, sb = a.bodies(), b.bodies()
+    for k in ("position", "position_old", "velocity"):
+        assert np.array_equal(bits(sa[k]), bits(sb[k])), k
