@@ -205,7 +205,12 @@ __device__ __forceinline__ GridParams grid_from_bbox(const uint32_t* bb, float c
         maxx = maxy = 0.0f;
     }
     if (!(cell > 0.0f) || !finitef(cell)) cell = 1.0f;
-    float ex = maxx - minx, ey = maxy - miny;
+    const float ex = fminf(maxx - minx, 3.0e38f), ey = fminf(maxy - miny, 3.0e38f);
+    // A box of more cells than there are takes the smallest cell that fits, not the next double:
+    // the crowded middle of a scene that flies apart pays for each needless half.  512 worlds of 1.5M
+    // bodies, 60 steps 51.1 -> 41.1 ms (fewer bodies are without a list), 50,021 bodies, 30 steps 3.82 ->
+    // 3.56 ms, 294,249 colliders, 8 steps 9.30 -> 8.95-9.02 ms (its scan covers more cells).
+    bool fitted = false;
     int32_t nx, ny;
     for (;;) {
         float fx = floorf(ex / cell) + 1.0f, fy = floorf(ey / cell) + 1.0f;
@@ -214,7 +219,13 @@ __device__ __forceinline__ GridParams grid_from_bbox(const uint32_t* bb, float c
             ny = (int32_t)fy;
             break;
         }
-        cell = cell * 2.0f;
+        if (fitted) {
+            cell = cell * 1.0625f;  // the partial cells at the edges
+        } else {
+            const float cap = (float)min(cells_cap, 1u << 30);
+            cell = fmaxf(cell, fmaxf(sqrtf(ex) * (sqrtf(ey) / sqrtf(cap)), fmaxf(ex, ey) / fminf(65536.0f, cap)));
+            fitted = true;
+        }
     }
     g.ox = minx;
     g.oy = miny;
