@@ -209,7 +209,7 @@ __device__ __forceinline__ GridParams grid_from_bbox(const uint32_t* bb, float c
     // A box of more cells than there are takes the smallest cell that fits, not the next double:
     // the crowded middle of a scene that flies apart pays for each needless half.  512 worlds of 1.5M
     // bodies, 60 steps 51.1 -> 41.1 ms (fewer bodies are without a list), 50,021 bodies, 30 steps 3.82 ->
-    // 3.56 ms, 294,249 colliders, 8 steps 9.30 -> 8.95-9.02 ms (its scan covers more cells).
+    // 3.56 ms, 294,249 colliders, 8 steps 9.30 -> 8.95-9.02 ms (its scan covers more cells; clipped 8.28).
     bool fitted = false;
     int32_t nx, ny;
     for (;;) {
