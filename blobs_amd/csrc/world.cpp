@@ -1214,7 +1214,7 @@ int World::upload() {
         for (uint32_t w = 0; w < W; ++w) {
             const uint32_t n_w = wstart[w + 1] - wstart[w];
             // cells of the world's grid: worlds spread (nothing bounds them), and a grid that
-            // outgrows its cells doubles its cell size, which crowds the partner walks; the
+            // outgrows its cells takes larger ones, which crowds the partner walks; the
             // rebuild scans only the cells a grid uses, so room is cheap
             const uint64_t cap = std::max<uint64_t>(8ull * n_w, 8192ull);
             const uint64_t base = (uint64_t)cell_base[w] + ((cap + 63ull) & ~63ull);
@@ -2047,8 +2047,8 @@ int World::launch_grid_steps(double delta, uint32_t n) {
             if (st) return st;
             fresh_ = false;
             stepped_since_upload_ = true;
-            // the general path widens every query by the largest displacement since its
-            // rebuild (one fast collider would slow every query): it re-sorts every substep
+            // the general path sorts every substep, on the substep's own positions (one fast
+            // collider would otherwise widen every query)
             if (path_ == StepPath::General || sub_since_rebuild_ >= interval) need_rebuild_ = true;
         }
     }
