@@ -112,7 +112,7 @@ def batched_leg(chunk_steps: int, n_chunks: int, n_worlds: int, autotune: bool, 
         cs, sk, iv = batch.autotune(dt, 4)
         tuned = {"cell_scale": cs, "skin": sk, "rebuild_interval": iv}
         log(f"batched: autotune -> {tuned} ({time.perf_counter() - t0:.1f} s)")
-    broadphase = tuned or {"cell_scale": 1.5, "skin": 0.25, "rebuild_interval": 3, "source": "the batch's defaults"}
+    broadphase = tuned or {"cell_scale": 1.5, "skin": 0.25, "rebuild_interval": "follows the outliers, from 3 steps", "source": "the batch's defaults"}
     def timed(n, segments=1):
         batch.run_chunks(dt, chunk_steps, 1)  # graph capture warm-up
         batch._lib.bg_synchronize(batch._w)
