@@ -201,9 +201,11 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         host_behind();
         return check_and_process(chunk_steps * n_chunks);
     }
-    // the first chunk after an upload runs eagerly (user inputs are consumed once)
+    // From here on the path is the grid's (or the persistent step's) whatever a capture finds: a tail
+    // captured to bring the host mirror up has to repeat what the replayed graphs ran.
+    // The first chunk after an upload runs eagerly (user inputs are consumed once).
     if (fresh_) {
-        st = launch_steps(delta, chunk_steps);
+        st = launch_large_steps(delta, chunk_steps);
         if (st) return st;
         advance_time(delta, chunk_steps);
         ++done;
@@ -223,7 +225,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         hipError_t e = hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal);
         int r = BG_OK;
         if (e == hipSuccess) {
-            r = launch_steps(delta, chunk_steps);
+            r = launch_large_steps(delta, chunk_steps);
             e = hipStreamEndCapture(d.stream, &g);
         }
         profiling_ = prof;
@@ -267,7 +269,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
                 hipError_t e = hipGraphLaunch(execs[c % m], d.stream);
                 if (e != hipSuccess) result = fail(BG_ERR_HIP, std::string("hipGraphLaunch: ") + hipGetErrorString(e));
             } else {
-                result = launch_steps(delta, chunk_steps);  // past a non-repeating capture: eager
+                result = launch_large_steps(delta, chunk_steps);  // past a non-repeating capture: eager
             }
             if (result == BG_OK) advance_time(delta, chunk_steps);
         }
@@ -278,7 +280,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
     }
     if (trial && result == BG_OK) {
         trial_allowed_ = true;
-        result = launch_steps(delta, chunk_steps);
+        result = launch_large_steps(delta, chunk_steps);
         trial_allowed_ = false;
         if (result == BG_OK) advance_time(delta, chunk_steps);
     }

@@ -166,7 +166,6 @@ enum : uint32_t {
     ERR_ORDERED_CAP = 1u << 4,  // a push-out cluster outgrew the ordered contact pass's buffers
     INFO_PUSH_OUT = 1u << 8,    // physics.rs:272-286: a pair's snapshots coincided
     INFO_PUSH_OUT_PAIRWISE = 1u << 9,  // ... on the fused sphere path, resolved pair by pair
-    INFO_LISTS_FULL = 1u << 10,  // small worlds: a body had more partners than a list holds
 };
 
 // Body flag bits (device SoA `bflags`).

@@ -407,7 +407,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
                 for (uint32_t j = 0; j < PER; ++j)
                     over |= t + j * NT < nb && n_list[o.id[j] & 0xFFFFu] > kListCap;
-                if (tries == kListTries && over) flags |= INFO_LISTS_FULL;
                 if (__syncthreads_or(over && tries < kListTries) == 0) break;
                 span *= 0.5f;
                 rest *= 0.5f;

@@ -1771,7 +1771,6 @@ int World::run_substep(float h, bool fresh, bool last) {
 // Panics and routing from the step record's error flags (physics.rs:293,
 // 447-448, 471-474).
 int World::process_flags(uint32_t flags) {
-    if (flags & INFO_LISTS_FULL) small_hold_ = kSmallHold;
     const uint32_t panic_bits = flags & (ERR_NAN_NORMAL | ERR_JOINT_MASS | ERR_JOINT_ROT | ERR_ORDERED_CAP);
     route_after_step(flags);
     if (panic_bits & ERR_NAN_NORMAL) return fail(BG_ERR_PANIC, "assertion failed: !n.is_nan() (physics.rs:293)");
@@ -1943,10 +1942,9 @@ int World::launch_persistent(double delta, uint32_t n, bool fresh, hipStream_t s
 }
 
 // Small worlds (small_kernels.hip).  A setting made with bg_set_broadphase, and stage timing,
-// are the grid path's; so is a world with more partners about a body than a list holds, for a while.
+// are the grid path's.
 bool World::small_active() const {
-    return small_ && path_ == StepPath::Sphere && rebuild_interval_ == 0 && !profiling_ && small_hold_ == 0 &&
-           !d_.gather_pending;
+    return small_ && path_ == StepPath::Sphere && rebuild_interval_ == 0 && !profiling_ && !d_.gather_pending;
 }
 
 int World::launch_small(double delta, uint32_t n) {
@@ -1988,8 +1986,10 @@ int World::launch_small(double delta, uint32_t n) {
 }
 
 int World::launch_steps(double delta, uint32_t n) {
-    if (small_active()) return launch_small(delta, n);
-    small_hold_ -= std::min(small_hold_, n);
+    return small_active() ? launch_small(delta, n) : launch_large_steps(delta, n);
+}
+
+int World::launch_large_steps(double delta, uint32_t n) {
     if (persist_ && path_ == StepPath::Sphere && n > 0) {
         DeviceWorld& d = d_;
         const bool fresh = fresh_;

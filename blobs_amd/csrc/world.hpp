@@ -147,6 +147,7 @@ private:
     int prepare_step();
     int ensure_joint_schedule();
     int launch_steps(double delta, uint32_t n);
+    int launch_large_steps(double delta, uint32_t n);  // never the small worlds' kernel
     int launch_grid_steps(double delta, uint32_t n);
     int launch_persistent(double delta, uint32_t n, bool fresh, hipStream_t stream);
     void advance_time(double delta, uint32_t n);
@@ -255,11 +256,9 @@ private:
     // constraints or events, worlds of at most kPersistMaxBodies bodies).  Off by default:
     // over long runs of spreading worlds the grid path alone is faster
     bool persist_enabled_ = false, persist_ = false;
-    // small worlds (small_kernels.hip): the uploaded worlds all fit, and the steps left on the
-    // grid path since a list overflowed
+    // small worlds (small_kernels.hip): the uploaded worlds all fit
     bool small_ = false;
-    uint32_t small_hold_ = 0;
-    static constexpr uint32_t kSmallHold = 256, kSmallSubsteps = 512;  // substeps of a launch
+    static constexpr uint32_t kSmallSubsteps = 512;  // substeps of a launch
     bool small_active() const;
     int launch_small(double delta, uint32_t n);
     SphereArrays p_src_{};  // where the last persistent launch (or the upload) left its worlds' records
