@@ -118,7 +118,7 @@ constexpr uint32_t kLdsBodies = kPersistPer * 1024;
 constexpr uint32_t kPersistMinBodies = 1025;
 
 // Worlds of at most kSmallBodies single centred spheres: every substep of a launch by one
-// workgroup a world (small_kernels.hip).
+// workgroup a world (small_kernels.hip).  Several only if they record no events.
 constexpr uint32_t kSmallClasses = 4;
 constexpr uint32_t kSmallClassThreads[kSmallClasses] = {1024, 1024, 512, 256};
 constexpr uint32_t kSmallClassBodies[kSmallClasses] = {2048, 1024, 512, 256};

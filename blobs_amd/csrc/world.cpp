@@ -1530,7 +1530,9 @@ int World::upload() {
         const std::vector<uint32_t>& wstart = small_worlds;
         uint32_t largest = 0;
         for (uint32_t w = 0; w < W; ++w) largest = std::max(largest, wstart[w + 1] - wstart[w]);
-        if (largest <= kSmallBodies) {
+        // (worlds run ahead of each other, so several would fill the events' buffer out of the substeps'
+        // order, by which collect_events keeps the same ones whatever the atomics' order)
+        if (largest <= kSmallBodies && (W == 1 || event_cap_ == 0)) {
             int cus = 0;
             if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d.device) != hipSuccess || cus < 1)
                 cus = 1;
