@@ -415,7 +415,7 @@ uint32_t Rollout::recompute_segments() {
     const uint64_t per_sub = (uint64_t)nb_ * (sizeof(float2) * (1u + (d_tape_v_ ? 1u : 0u)) + sizeof(uint16_t) * kDiffTapeNbr) +
                              (uint64_t)n_solves_ * sizeof(float2);
     uint64_t segs = std::min<uint64_t>(n_seg, cus_ / n_worlds_);
-    if (per_sub > 0) segs = std::min<uint64_t>(segs, kTapeBytes / (per_sub * seg_sub));
+    if (per_sub * seg_sub > 0) segs = std::min<uint64_t>(segs, kTapeBytes / (per_sub * seg_sub));
     segs = std::max<uint64_t>(segs, 1);
     if (segs > 1 && ensure_tape((uint32_t)segs * seg_sub) != BG_OK) {
         (void)hipGetLastError();  // no room: one at a time

@@ -1,0 +1,23 @@
+"""Rollouts at the edges of their parameters."""
+import numpy as np
+import pytest
+
+from blobs_amd import scenes
+from blobs_amd.rollout import Rollout
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("joints", [0, 5])
+def test_worlds_of_no_substeps(joints):
+    """Nothing moves, and no parameter has a gradient (a backward divided by the segment's substeps)."""
+    sc = scenes.rollout_world(40, 20, scenes.Rng(3), damping=1.0, n_joints=joints, anchor=0.2)
+    worlds = [sc.build_physics()[0] for _ in range(2)]
+    for w in worlds:
+        w.substeps = 0
+    r = Rollout(worlds, np.zeros((2, 2), np.float32), checkpoint_every=2)
+    loss = r.forward(sc.dt, 5)
+    assert np.isfinite(loss).all()
+    assert np.array_equal(r.final_positions(), np.concatenate([sc.pos, sc.pos]).astype(np.float32))
+    gv, gk = r.backward()
+    assert not gv.any() and not gk.any()
