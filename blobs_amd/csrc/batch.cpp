@@ -190,16 +190,21 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         return s;
     };
     const bool prof = profiling_;
+    const uint32_t steps = (uint32_t)std::min<uint64_t>((uint64_t)chunk_steps * n_chunks, 0xFFFFFFFFull);
     uint32_t done = 0;
     if (event_cap_ > 0 || small_active()) {
         // Events are stamped with the substep index the host passes: a replayed graph would
         // repeat the stamps, so a world that records events runs its chunks eagerly.  So do
         // small worlds, whose chunks are a launch or two.
-        st = launch_steps(delta, chunk_steps * n_chunks);
-        if (st) return st;
-        advance_time(delta, chunk_steps * n_chunks);
+        for (uint64_t left = (uint64_t)chunk_steps * n_chunks; left > 0;) {  // (may pass 2^32)
+            const uint32_t n = (uint32_t)std::min<uint64_t>(left, 1u << 30);
+            st = launch_steps(delta, n);
+            if (st) return st;
+            advance_time(delta, n);
+            left -= n;
+        }
         host_behind();
-        return check_and_process(chunk_steps * n_chunks);
+        return check_and_process(steps);
     }
     // From here on the path is the grid's (or the persistent step's) whatever a capture finds: a tail
     // captured to bring the host mirror up has to repeat what the replayed graphs ran.
@@ -289,7 +294,7 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
     if (e != hipSuccess && result == BG_OK) result = fail(BG_ERR_HIP, hipGetErrorString(e));
     host_behind();
     if (result != BG_OK) return result;
-    return check_and_process(chunk_steps * n_chunks);
+    return check_and_process(steps);
 }
 
 int World::set_persistent(bool enable) {

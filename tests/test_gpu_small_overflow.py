@@ -1,5 +1,7 @@
-"""Small worlds (small_kernels.hip) with bodies of more partners than a list holds:
-they stay on their path, through chunks of any length, with the grid path's bits.
+"""Small worlds (small_kernels.hip) past what their lists and counters hold: with
+bodies of more partners than a list they stay on their path, through chunks of
+any length, with the grid path's bits; and chunks of any number of steps run all
+of them.
 """
 import numpy as np
 import pytest
@@ -37,3 +39,11 @@ def test_chunks_of_overflowing_worlds(sizes, chunk, chunks):
         for k in ("position", "position_old", "velocity", "rotation"):
             assert np.array_equal(bits(sa[k]), bits(sb[k])), (k, call)
     assert a.contact_count() == b.contact_count() > 0
+
+
+def test_chunks_of_more_than_32_bits_of_steps():
+    """(Of no substeps each, so that only the clock moves.)"""
+    p = crowd(20).build_physics()[0]
+    p.substeps = 0
+    p.run_chunks(2.0 ** -20, 1 << 16, 1 << 16)
+    assert p.time == 2.0 ** 12
