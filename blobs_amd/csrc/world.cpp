@@ -411,6 +411,9 @@ int World::get_params(bg_params* p) {
 
 int World::set_params(const bg_params* p) {
     float old = params_.old_dt;
+    // An old_dt set after an export is the mirror's from then on: a later download would bring
+    // the device's, on the sphere path not the one set here.
+    if (host_stale_ && old_dt_known_ && __builtin_memcmp(&old, &p->old_dt, 4) != 0 && sync_host()) return BG_ERR_HIP;
     params_ = *p;
     if (d_.accum && !dev_dirty_ && __builtin_memcmp(&old, &p->old_dt, 4) != 0) {
         HIP_TRY(hipMemcpyAsync(&d_.accum->old_dt, &params_.old_dt, sizeof(float), hipMemcpyHostToDevice, d_.stream));
