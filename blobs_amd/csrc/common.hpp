@@ -196,4 +196,11 @@ __device__ __forceinline__ int32_t cell_coord(float x, float o, float inv, int32
     return (int32_t)fminf(fmaxf((x - o) * inv, 0.0f), (float)(n - 1));
 }
 
+// A cell size `factor` (> 1) times larger, and larger in any case: among the least floats the
+// product rounds back to what it was, and a fit that only multiplied would not end.
+__device__ __forceinline__ float larger_cell(float cell, float factor) {
+    const float grown = cell * factor;
+    return grown > cell ? grown : cell * 2.0f;
+}
+
 }  // namespace bg

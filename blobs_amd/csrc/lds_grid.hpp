@@ -181,7 +181,7 @@ __device__ __forceinline__ void lds_fit(const LdsFit& f, float cell, uint32_t ce
                     ny = (int32_t)fy;
                     break;
                 }
-                cell = cell * (fx > 65536.0f || fy > 65536.0f ? 16.0f : 1.25f);
+                cell = larger_cell(cell, fx > 65536.0f || fy > 65536.0f ? 16.0f : 1.25f);
                 if (!finitef(cell)) break;  // an infinite extent: one cell
             }
             grid->ox = minx;

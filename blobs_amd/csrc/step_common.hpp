@@ -220,7 +220,7 @@ __device__ __forceinline__ GridParams grid_from_bbox(const uint32_t* bb, float c
             break;
         }
         if (fitted) {
-            cell = cell * 1.0625f;  // the partial cells at the edges
+            cell = larger_cell(cell, 1.0625f);  // the partial cells at the edges
         } else {
             const float cap = (float)min(cells_cap, 1u << 30);
             cell = fmaxf(cell, fmaxf(sqrtf(ex) * (sqrtf(ey) / sqrtf(cap)), fmaxf(ex, ey) / fminf(65536.0f, cap)));
