@@ -111,7 +111,7 @@ __device__ void build_grid(const float4* SN, uint32_t* CNT, Idx* SRT, uint32_t n
         }
         float cell = 2.0f * rmax;
         if (!(cell > 0.0f) || !finitef(cell)) cell = 1.0f;
-        const float ex = maxx - minx, ey = maxy - miny;
+        const float ex = fminf(maxx - minx, 3.0e38f), ey = fminf(maxy - miny, 3.0e38f);  // (an infinite box fits no cells)
         int32_t nx = 1, ny = 1;
         for (;;) {
             const float fx = floorf(ex / cell) + 1.0f, fy = floorf(ey / cell) + 1.0f;

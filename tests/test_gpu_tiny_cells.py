@@ -1,6 +1,7 @@
 """Grids fitted to bodies whose radii and distances are a few of the least floats,
 where a cell size times a little more than one is the same cell size: the fit
-ends, and results are the oracle's and the same on every path.
+ends, and results are the oracle's and the same on every path.  So for a box too
+wide for the type.
 """
 import numpy as np
 import pytest
@@ -57,3 +58,22 @@ def test_tiny_worlds_of_a_batch_and_a_rollout(radius, width):
     r.forward(scs[0].dt, 2)
     assert np.array_equal(bits(a.bodies()["position"]), bits(b.bodies()["position"]))
     assert np.array_equal(bits(a.bodies()["position"]), bits(r.final_positions()))
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+def test_world_wider_than_the_type(persistent):
+    """Two bodies so far apart that their distance overflows: the box is cut to the type's range."""
+    scs = [scenes.plain_large_scene(n=n, seed=5) for n in (1100, 30)]
+    for sc in scs:
+        sc.pos[3], sc.pos[7] = (3e38, -3e38), (-3e38, 3e38)
+        sc.col_abs = sc.pos[sc.col_parent].copy()
+    b = Physics.batch([sc.build_physics()[0] for sc in scs])
+    b.set_persistent(persistent)
+    b.step(scs[0].dt, 2)
+    assert b.persistent_active() == persistent
+    got, at = b.bodies()["position"], 0
+    for sc in scs:
+        o = OracleWorld(sc, np.float32)
+        o.step(sc.dt, 2)
+        assert np.array_equal(bits(got[at:at + len(sc.pos)]), bits(o.pos))
+        at += len(sc.pos)
