@@ -64,6 +64,23 @@ hipError_t d2h(std::vector<T>& dst, const T* src, size_t n, hipStream_t s) {
     return hipMemcpyAsync(dst.data(), src, n * sizeof(T), hipMemcpyDeviceToHost, s);
 }
 
+// The caller's current device is `device` for as long as this lives.
+class OnDevice {
+public:
+    explicit OnDevice(int device) {
+        int now = -1;
+        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before_ = now;
+    }
+    ~OnDevice() {
+        if (before_ >= 0) (void)hipSetDevice(before_);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+
+private:
+    int before_ = -1;
+};
+
 uint32_t next_pow2(uint32_t v) {
     uint32_t p = 1;
     while (p < v) p <<= 1;
@@ -561,6 +578,7 @@ int World::copy_to_host(const CopyOut* c, uint32_t n) {
 // (the general path's arrays are in dense order already), which then comes over in pieces.
 int World::export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos) {
     DeviceWorld& d = d_;
+    const OnDevice on(d.device);  // a read allocates and launches there, whichever device is the caller's
     const bool sphere = path_ == StepPath::Sphere;
     const uint32_t id_mask = snap_flags_ ? kSnapIdMask : ~kSnapOutlier;
     const uint32_t n_old = sphere ? d.n_worlds : 1u;
