@@ -43,7 +43,7 @@ namespace bg {
 
 namespace {
 
-constexpr uint32_t kListCap = 16;      // partners of a list; a body with more tests every body
+constexpr uint32_t kListCap = 16;      // partners of a list; a body with more is tested against every body
 constexpr uint32_t kListGroups = kListCap / 4;
 constexpr float kSkinSubsteps = 8.0f;  // substeps a list is meant to last
 // Least and largest skin, in diameters of the largest body.  At 1,024 worlds of 64 to 1,024 a step
@@ -51,7 +51,12 @@ constexpr float kSkinSubsteps = 8.0f;  // substeps a list is meant to last
 // 1,288 bodies falling on a pile 225 then, instead of 142 (0.05 and 0.25: 211).
 constexpr float kSkinRest = 0.1f;
 constexpr float kSkinMax = 1.0f;
-constexpr uint32_t kListTries = 4;     // builds with skins halved while a list overflows
+constexpr uint32_t kListTries = 4;     // builds with skins halved while lists overflow
+// A list that overflows for one body in so many threads is left so: lists with smaller skins last
+// shorter, for everyone.  A step of 300, 1,000 and 2,000 bodies of ragged radii under one of 24
+// times their size takes 426, 956 and 2,137 us (929, 1,591, 3,546 with none left); of 2,000 pressed into a
+// circle 1,417 (1,406, and 1,456 with one in 64).
+constexpr uint32_t kListsOver = 256;
 constexpr uint32_t kFast = 0x10000u;   // record flag: more than the least skin
 constexpr float kMaxDrift = 16.0f;     // common motion a list is kept for (rounding of x - x0 - drift)
 
@@ -111,6 +116,10 @@ __device__ __forceinline__ void put(T (&v)[PER], uint32_t j, T x) {
         v[0] = j ? v[0] : x;
         v[1] = j ? x : v[1];
     }
+}
+
+__device__ __forceinline__ float lane_f32(float v, int lane) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
 }
 
 // Sorts the first n (at most N) partners of body li's list and fills up to N with li, by
@@ -251,6 +260,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const float2 a = xy[own], b = xy[other], ra = rm[own], rb = rm[other];
         return lds_correction(make_float4(a.x, a.y, ra.x, 0.0f), make_float4(b.x, b.y, rb.x, 0.0f), ra.y, rb.y,
                               own > other, false);
+    };
+    // whether they can be one
+    auto near = [&](uint32_t own, uint32_t other) -> uint32_t {
+        const float2 a = xy[own], b = xy[other];
+        const float dx = a.x - b.x, dy = a.y - b.y, r = rm[own].x, rs = r + (alike ? r : rm[other].x);
+        return dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f ? 0u : 1u;
     };
     auto append = [&](uint32_t to, uint32_t partner) {
         const uint32_t at = atomicAdd(&n_list[to], 1u);
@@ -407,7 +422,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
                 for (uint32_t j = 0; j < PER; ++j)
                     over |= t + j * NT < nb && n_list[o.id[j] & 0xFFFFu] > kListCap;
-                if (__syncthreads_or(over && tries < kListTries) == 0) break;
+                if (__syncthreads_count(over) <= (int)(NT / kListsOver) || tries == kListTries) break;
                 span *= 0.5f;
                 rest *= 0.5f;
             }
@@ -431,20 +446,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 if (t + j * NT < nb) {
                     li = pick(o.id, j) & 0xFFFFu;
                     const float2 own = xy[li];
-                    const float r = rm[li].x;
                     n = n_list[li];
                     const bool fin = finitef(own.x) && finitef(own.y);
                     all = fin && n > kListCap;
                     if (!fin || all) n = 0;
-                    auto near = [&](uint32_t lj) -> uint32_t {
-                        const float2 b = xy[lj];
-                        const float dx = own.x - b.x, dy = own.y - b.y, rs = r + (alike ? r : rm[lj].x);
-                        return dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f ? 0u : 1u;
-                    };
                     for (uint32_t f = 0; f < n; f += 4) {
                         const uint2 l = *(const uint2*)lists[f >> 2][li];
-                        marked |= (near(l.x & 0xFFFFu) | near(l.x >> 16) << 1 | near(l.y & 0xFFFFu) << 2 |
-                                   near(l.y >> 16) << 3) << f;
+                        marked |= (near(li, l.x & 0xFFFFu) | near(li, l.x >> 16) << 1 | near(li, l.y & 0xFFFFu) << 2 |
+                                   near(li, l.y >> 16) << 3) << f;
                     }
                     marked &= (1u << n) - 1u;
                     static_assert(kListCap < 32, "the mask");
@@ -472,23 +481,42 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
             }
             __syncthreads();
             if (s_direct[par]) {
-                // no room in the queue, or a list that overflowed: the body's thread works its
-                // contacts out itself, in ascending partner index
+                // No room in the queue: the body's thread works its contacts out itself.  A list that
+                // overflowed: the body's wave tests it against everyone, a partner a lane, one such body
+                // after the other.  Both in ascending partner index.
 #pragma unroll 1
                 for (uint32_t j = 0; j < per; ++j) {
-                    if (!(PER == 1 || j == 0 ? pr[0].direct : pr[PER - 1].direct)) continue;
-                    const uint32_t li = pick(o.id, j) & 0xFFFFu, n = n_list[li];
+                    const bool direct = t + j * NT < nb && (PER == 1 || j == 0 ? pr[0].direct : pr[PER - 1].direct);
+                    const uint32_t li = pick(o.id, j) & 0xFFFFu, n = direct ? n_list[li] : 0u;
                     float2 p = pick(o.p, j);
-                    for (uint32_t i = 0; i < (n > kListCap ? nb : n); ++i) {
-                        const uint32_t lj = n > kListCap ? i : (uint32_t)lists[i >> 2][li][i & 3u];
-                        if (lj == li) continue;
+                    uint32_t within = 0;
+                    for (uint32_t i = 0; i < (n > kListCap ? 0u : n); ++i) within |= near(li, lists[i >> 2][li][i & 3u]) << i;
+                    for (; within != 0; within &= within - 1) {
+                        const uint32_t i = (uint32_t)__builtin_ctz(within), lj = lists[i >> 2][li][i & 3u];
                         const LdsContact c = contact(li, lj);
                         if (!c.hit) continue;
                         tally(li, lj, c, sub);
                         p.x = p.x + c.c.x;
                         p.y = p.y + c.c.y;
                     }
-                    put(o.p, j, p);
+                    for (uint64_t left = __ballot(n > kListCap); left != 0; left &= left - 1) {
+                        const int of = __builtin_ctzll(left);
+                        const uint32_t own = (uint32_t)__builtin_amdgcn_readlane((int)li, of);
+                        float2 q = make_float2(lane_f32(p.x, of), lane_f32(p.y, of));
+                        for (uint32_t first = 0; first < nb; first += BG_WAVE) {
+                            const uint32_t lj = first + lane;
+                            LdsContact c = {make_float2(0.0f, 0.0f), false, false, false};
+                            if (lj < nb && lj != own) c = contact(own, lj);
+                            if (c.hit) tally(own, lj, c, sub);
+                            for (uint64_t hits = __ballot(c.hit); hits != 0; hits &= hits - 1) {
+                                const int h = __builtin_ctzll(hits);
+                                q.x = q.x + lane_f32(c.c.x, h);
+                                q.y = q.y + lane_f32(c.c.y, h);
+                            }
+                        }
+                        if ((int)lane == of) p = q;
+                    }
+                    if (direct) put(o.p, j, p);
                 }
                 __syncthreads();  // before anyone publishes
             }

@@ -1542,7 +1542,11 @@ int World::upload() {
     // Small path against the grid path at one rebuild a step, us a step, best of three runs:
     // 364 bodies 47 / 131 (and 55 / 139 as a settled pile), 1,288 62 / 131 (102 / 197), 2,000 free
     // 85 / 117; batches 128 worlds of 64-512 31 / 106, 1,024 of 512-1,024 163 / 296, 512 of
-    // 1,024-2,048 127 / 286, 4,096 of 64-256 123 / 311: never slower over the sizes it takes.
+    // 1,024-2,048 127 / 286, 4,096 of 64-256 123 / 311.  With lists that overflow: 1,000 about one of
+    // five times their size 400 / 6,900, 2,000 under one of 24 times theirs 2,137 / 3,036, 2,000 pressed
+    // into a circle 414-430 / 2,150-2,430.  Slower in one scene tried, while it is young: 2,000 and
+    // two of three times their size falling over each other in a bowl rebuild their lists every
+    // substep, 602-764 / 468-495 over the first 60 steps (and 299 / 582 over the next 20).
     small_ = false;
     std::vector<uint32_t> small_worlds;  // slot ranges [W + 1], then the worlds by class [W]
     if (sphere && !persist_ && zero_off_ && !groups_ && !sensors_) {

@@ -1,8 +1,10 @@
 """Small worlds (small_kernels.hip) past what their lists and counters hold: with
 bodies of more partners than a list they stay on their path, through chunks of
-any length, with the grid path's bits; and chunks of any number of steps run all
-of them.
+any length, with the grid path's bits and in less than its time; and chunks of
+any number of steps run all of them.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -24,6 +26,24 @@ def crowd(n, seed=5):
     return sc
 
 
+def pebbles(n, seed=5):
+    """A large body among small ones, in a round container."""
+    sc = scenes.plain_large_scene(n=n, seed=seed)
+    lo, hi = sc.pos.min(0), sc.pos.max(0)
+    sc.col_r[n // 2] = 4.0
+    sc.con_pos = ((lo + hi) / 2).astype(np.float32)[None, :]
+    sc.con_r = np.array([0.5 * float((hi - lo).max())], np.float32)
+    return sc
+
+
+def giant(n, seed=5):
+    """One body that covers many others, with ragged radii."""
+    sc = scenes.plain_large_scene(n=n, seed=seed)
+    sc.col_r = (0.1 + 0.4 * np.random.default_rng(seed + n).random(n)).astype(np.float32)
+    sc.col_r[n // 2] = 12.0
+    return sc
+
+
 @pytest.mark.parametrize("chunk,chunks", [(3, 3), (1, 5), (5, 2)])
 @pytest.mark.parametrize("sizes", [(300,), (90, 300, 40)])
 def test_chunks_of_overflowing_worlds(sizes, chunk, chunks):
@@ -39,6 +59,25 @@ def test_chunks_of_overflowing_worlds(sizes, chunk, chunks):
         for k in ("position", "position_old", "velocity", "rotation"):
             assert np.array_equal(bits(sa[k]), bits(sb[k])), (k, call)
     assert a.contact_count() == b.contact_count() > 0
+
+
+@pytest.mark.parametrize("make,n", [(pebbles, 300), (pebbles, 1000), (giant, 2000)])
+def test_overflowing_world_takes_less_than_the_grid_path(make, n):
+    # (in calls of thirty steps and in calls of one, after lists have overflowed)
+    sc = make(n)
+    a, b = sc.build_physics()[0], sc.build_physics()[0]
+    b.set_broadphase(*GRID)
+    took = {}
+    for w in (a, b):
+        w.step(sc.dt, 2)
+        t0 = time.perf_counter()
+        for _ in range(12):
+            w.step(sc.dt)
+        t1 = time.perf_counter()
+        w.step(sc.dt, 30)
+        took[w] = (t1 - t0, time.perf_counter() - t1)
+    assert took[a][0] < 0.9 * took[b][0] and took[a][1] < 0.9 * took[b][1], list(took.values())
+    assert np.array_equal(bits(a.bodies()["position"]), bits(b.bodies()["position"]))
 
 
 def test_chunks_of_more_than_32_bits_of_steps():
