@@ -13,7 +13,7 @@
 // leaves its world's cells, so pairs never cross worlds.
 //
 // Broadphase.  A rebuild fits each world's grid to the bounding box of its
-// snapshots over the previous period (clipped to the centroid +- 3 sigma;
+// snapshots over the previous period (clipped to the centroid +- 4 sigma;
 // bodies outside are clamped into border cells), counts bodies per cell with atomic
 // ranks, scans the counts into the cell table and scatters the snapshot
 // records and the permutation.  The first substep after it gathers the body
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(kThreads) void k_world_stats(const float4* __restri
 }
 
 // Grid of every world over its snapshots: their bounding box clipped to the
-// centroid +- 3 sigma so a few far-flung bodies (clamped into border cells)
+// centroid +- 4 sigma so a few far-flung bodies (clamped into border cells)
 // do not coarsen the cells of the rest; the mean velocity of its dynamic
 // bodies (drift model).
 // One wave per world (the replica sums are reduced across its lanes).
@@ -857,12 +857,12 @@ __global__ __launch_bounds__(BG_WAVE) void k_world_grids(uint32_t n_worlds, uint
         const float sx = sqrtf(fmaxf(st[5] / n - mx * mx, 0.0f)), sy = sqrtf(fmaxf(st[6] / n - my * my, 0.0f));
         const float mg = 2.0f * cell;
         if (finitef(mx) && finitef(sx)) {
-            bb[0] = max(bb[0], f2ord(mx - 3.0f * sx - mg));
-            bb[2] = min(bb[2], f2ord(mx + 3.0f * sx + mg));
+            bb[0] = max(bb[0], f2ord(mx - 4.0f * sx - mg));
+            bb[2] = min(bb[2], f2ord(mx + 4.0f * sx + mg));
         }
         if (finitef(my) && finitef(sy)) {
-            bb[1] = max(bb[1], f2ord(my - 3.0f * sy - mg));
-            bb[3] = min(bb[3], f2ord(my + 3.0f * sy + mg));
+            bb[1] = max(bb[1], f2ord(my - 4.0f * sy - mg));
+            bb[3] = min(bb[3], f2ord(my + 4.0f * sy + mg));
         }
         if (bb[0] > bb[2]) bb[0] = bb[2];
         if (bb[1] > bb[3]) bb[1] = bb[3];
