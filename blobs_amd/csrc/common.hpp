@@ -139,7 +139,7 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 // bounding box of collider snapshots (order-mapped floats) and the contact
 // count.  Block-reduced, then one atomic per block.
 struct StepAccum {
-    uint32_t pad0;
+    uint32_t clip_hold;  // general path: substeps for which the grid's box is not clipped
     uint32_t last_outliers;  // sphere path: n_outliers of the rebuild period before this one
     uint32_t bbox[2][4];  // [parity]{minx, miny, maxx, maxy} as f2ord
     uint32_t n_outliers;  // sphere path: bodies beyond the skin since the last rebuild

@@ -66,6 +66,7 @@ struct JointGroup {
     uint32_t l0, l1;  // levels
 };
 constexpr uint32_t kSmallColliders = 1152, kSmallGeneral = 256;  // general path: worlds in four launches a substep
+constexpr uint32_t kClipWait = 64;  // general path: substeps after an upload with the grid's whole box (clip_box)
 constexpr uint32_t kGroupJoints = 64;  // joints of a group (a larger component is a group by itself)
 
 // Ordered contact pass (general path).  A push-out (physics.rs:272-286)

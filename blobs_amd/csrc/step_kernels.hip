@@ -42,10 +42,19 @@ constexpr uint32_t kContactThreads = 64;  // block size of k_contacts (block_con
 // loads hit the cache, and a statistics pass or a barrier would cost more.  294,249 colliders over
 // their first 112 steps, as the box grows from 776 to 12,000 units: k_contact_lists 28.0 -> 16.8 us,
 // k_keys_forces, this included, 20.4 -> 17.6.
+//
+// What lies outside may be a group, and crowd a border cell where each of its colliders walks all of
+// it: a step of 147,000 colliders with 7% of them 5,000 units off took 12,457 us, against 1,030 with the
+// whole box.  So a border cell of more than kBorderCrowd (128 to walk take a wave some 11 us) keeps
+// the box whole for kClipHold substeps (one crowded one in 1,024 is about 1%), and so does an upload for
+// kClipWait.  A scene that flies apart on all sides comes to that now and then: eight steps of 65,536
+// bodies, over their first 200, 8.39 ms, 8.02 with no limit, 8.20 at 256 -- where groups of 3% and 7% to
+// one side took up to 18% more than with the whole box -- and 8.63 at 21.
+constexpr uint32_t kBorderCrowd = 128, kClipHold = 1024;  // (kClipWait: device_state.hpp)
 __device__ __forceinline__ void clip_box(uint32_t (&bb)[4], const KeysArgs& k) {
     constexpr uint32_t kSample = 4;  // a lane
     const float minx = ord2f(bb[0]), miny = ord2f(bb[1]), ex = ord2f(bb[2]) - minx, ey = ord2f(bb[3]) - miny;
-    if (k.nc < 16u * kSample * BG_WAVE || !finitef(ex) || !finitef(ey) ||
+    if (k.accum->clip_hold != 0u || k.nc < 16u * kSample * BG_WAVE || !finitef(ex) || !finitef(ey) ||
         !((ex / k.cell + 1.0f) * (ey / k.cell + 1.0f) > (float)k.cells_cap))
         return;
     const uint32_t lane = threadIdx.x & (BG_WAVE - 1), stride = k.nc / (kSample * BG_WAVE);
@@ -136,13 +145,19 @@ CellScatter cell_scatter_of(const DeviceWorld& d) {
     return {d.keys, d.vals_tmp, d.nc, d.cell_start, d.vals, d.c.abs, d.c.radius, d.c.parent, d.crec};
 }
 
-// The counts are cleared for the next rebuild.
+// The counts are cleared for the next rebuild; a crowded border cell is noted for clip_box.
 __global__ __launch_bounds__(kThreads) void k_cell_scatter(CellScatter k, uint32_t* cnt, uint32_t n_cnt,
-                                                           const GridParams* __restrict__ grid) {
+                                                           const GridParams* __restrict__ grid, StepAccum* accum) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // only the grid's cells were counted (and scanned): clear those
     const uint32_t n_used = grid->ncells + 1u < n_cnt ? grid->ncells + 1u : n_cnt;
     for (uint32_t c = i; c < n_used; c += gridDim.x * blockDim.x) cnt[c] = 0u;
+    if (i == 0 && accum->clip_hold != 0u) atomicSub(&accum->clip_hold, 1u);  // (read by the key pass only)
+    if (i < k.nc && k.rank[i] >= kBorderCrowd) {
+        const uint32_t nx = (uint32_t)grid->nx, cy = k.keys[i] / nx, cx = k.keys[i] - cy * nx;
+        if (cx == 0u || cx == nx - 1u || cy == 0u || cy == (uint32_t)grid->ny - 1u)
+            atomic_max_if_greater(&accum->clip_hold, kClipHold);
+    }
     scatter_at(i, k);
 }
 
@@ -1197,7 +1212,7 @@ hipError_t launch_rebuild_sort_and_cells(DeviceWorld& d) {
     if (e != hipSuccess) return e;
     const uint32_t n = d.nc > 0 ? d.nc : 1u;
     k_cell_scatter<<<div_up(n, kThreads), kThreads, 0, d.stream>>>(cell_scatter_of(d), d.cell_count, d.cells_cap + 1,
-                                                                   d.grid);
+                                                                   d.grid, d.accum);
     return hipGetLastError();
 }
 

@@ -1604,6 +1604,7 @@ int World::upload() {
     acc0.bbox[0][3] = f2ord_host(maxy);
     acc0.bbox[1][0] = acc0.bbox[1][1] = 0xFFFFFFFFu;
     acc0.old_dt = params_.old_dt;
+    acc0.clip_hold = kClipWait;
     HIP_TRY(hipMemcpyAsync(d.accum, &acc0, sizeof(acc0), hipMemcpyHostToDevice, s));
     HIP_TRY(hipStreamSynchronize(s));  // host vectors die at return
 
