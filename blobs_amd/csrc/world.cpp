@@ -33,10 +33,8 @@ float col_inertia(const bg_collider& c) {
 constexpr uint32_t kPushOutHold = 4;
 
 // Exports: state up to kExportDirect bytes is stored to pinned memory by the kernel;
-// more comes through pinned staging of two halves of at most kStageHalf bytes.
+// more comes through the staging's two halves.
 constexpr size_t kExportDirect = 256 << 10;
-constexpr size_t kStageHalf = 4 << 20;
-constexpr size_t kStageLeast = 32 << 10;
 
 template <class T>
 hipError_t dmalloc(T** p, size_t n) {
@@ -96,6 +94,7 @@ uint32_t next_pow2(uint32_t v) {
 }  // namespace
 
 World::World(float gx, float gy, bool use_spatial_hash) {
+    Staging::world_begins();
     // Physics::new defaults, physics.rs:42-68
     params_.gravity[0] = gx;
     params_.gravity[1] = gy;
@@ -112,9 +111,6 @@ World::~World() {
     if (d_.stream) (void)hipStreamSynchronize(d_.stream);
     if (check_event_) (void)hipEventDestroy(check_event_);
     if (host_acc_) (void)hipHostFree(host_acc_);
-    if (stage_) (void)hipHostFree(stage_);
-    for (hipEvent_t e : stage_event_)
-        if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : event_pool_) (void)hipEventDestroy(e);
     for (auto& v : pending_)
         for (auto& pr : v) {
@@ -122,6 +118,7 @@ World::~World() {
             (void)hipEventDestroy(pr.second);
         }
     free_device();
+    Staging::world_ends();
 }
 
 int World::set_profiling(bool enable) {
@@ -480,8 +477,12 @@ int World::get_col(bg_handle h, bg_collider* out) {
 
 int World::get_bodies(float* pos, float* pos_old, float* vel, float* rot, float* omega, bg_handle* handles) {
     if (host_stale_ && d_.allocated) {
-        if (handles) std::copy(body_handle_of_dense_.begin(), body_handle_of_dense_.end(), handles);
-        return export_state(pos, pos_old, vel, rot, omega, nullptr);
+        bool room = false;
+        const int st = export_state(pos, pos_old, vel, rot, omega, nullptr, &room);
+        if (room) {
+            if (handles) std::copy(body_handle_of_dense_.begin(), body_handle_of_dense_.end(), handles);
+            return st;
+        }
     }
     if (sync_host()) return BG_ERR_HIP;
     uint32_t k = 0;
@@ -510,8 +511,12 @@ int World::get_bodies(float* pos, float* pos_old, float* vel, float* rot, float*
 
 int World::get_collider_positions(float* abs, uint32_t* count) {
     if (host_stale_ && d_.allocated) {
-        if (count) *count = d_.nc;
-        return abs ? export_state(nullptr, nullptr, nullptr, nullptr, nullptr, abs) : BG_OK;
+        bool room = true;
+        const int st = abs ? export_state(nullptr, nullptr, nullptr, nullptr, nullptr, abs, &room) : BG_OK;
+        if (room) {
+            if (count) *count = d_.nc;
+            return st;
+        }
     }
     if (sync_host()) return BG_ERR_HIP;
     uint32_t k = 0;
@@ -527,57 +532,41 @@ int World::get_collider_positions(float* abs, uint32_t* count) {
     return BG_OK;
 }
 
-int World::ensure_staging(size_t bytes) {
-    // (pinned memory costs some 200 us an allocation: a small world's first one does for all its reads)
-    const size_t half = std::min<size_t>(kStageHalf, std::max<size_t>((bytes + 4095) & ~(size_t)4095, kStageLeast));
-    for (hipEvent_t& e : stage_event_)
-        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (half <= stage_half_) return BG_OK;
-    if (stage_) (void)hipHostFree(stage_);
-    stage_ = nullptr;
-    stage_half_ = 0;
-    HIP_TRY(hipHostMalloc((void**)&stage_, 2 * half, hipHostMallocDefault));
-    stage_half_ = half;
-    return BG_OK;
-}
-
 // Device arrays to pageable host memory, a piece through one half of the staging while the
 // previous piece is copied out of the other.
-int World::copy_to_host(const CopyOut* c, uint32_t n) {
-    size_t most = 0;
-    for (uint32_t i = 0; i < n; ++i) most = std::max(most, c[i].bytes);
-    if (most == 0) return BG_OK;
-    if (int st = ensure_staging(most)) return st;
+int World::copy_to_host(const Staging& stage, const CopyOut* c, uint32_t n) {
     struct Piece {
         char* dst = nullptr;
         size_t bytes = 0;
     } prev;
     uint32_t k = 0;
     auto finish = [&](const Piece& p, uint32_t half) -> int {
-        HIP_TRY(hipEventSynchronize(stage_event_[half]));
-        memcpy(p.dst, stage_ + half * stage_half_, p.bytes);
+        HIP_TRY(hipEventSynchronize(stage.event(half)));
+        memcpy(p.dst, stage.half(half), p.bytes);
         return BG_OK;
     };
     for (uint32_t i = 0; i < n; ++i)
-        for (size_t at = 0; at < c[i].bytes; at += stage_half_, ++k) {
+        for (size_t at = 0; at < c[i].bytes; at += stage.half_bytes(), ++k) {
             Piece p;
             p.dst = (char*)c[i].dst + at;
-            p.bytes = std::min(stage_half_, c[i].bytes - at);
-            HIP_TRY(hipMemcpyAsync(stage_ + (k & 1u) * stage_half_, (const char*)c[i].src + at, p.bytes,
-                                   hipMemcpyDeviceToHost, d_.stream));
-            HIP_TRY(hipEventRecord(stage_event_[k & 1u], d_.stream));
+            p.bytes = std::min(stage.half_bytes(), c[i].bytes - at);
+            HIP_TRY(hipMemcpyAsync(stage.half(k & 1u), (const char*)c[i].src + at, p.bytes, hipMemcpyDeviceToHost,
+                                   d_.stream));
+            HIP_TRY(hipEventRecord(stage.event(k & 1u), d_.stream));
             if (prev.dst)
                 if (int st = finish(prev, (k & 1u) ^ 1u)) return st;
             prev = p;
         }
-    return finish(prev, (k & 1u) ^ 1u);
+    return prev.dst ? finish(prev, (k & 1u) ^ 1u) : BG_OK;
 }
 
 // The state the caller asked for (null: not wanted), in dense order, from the device.  A small
 // world's kernel stores straight into pinned memory; a large one's gathers into device memory
 // (the general path's arrays are in dense order already), which then comes over in pieces.
-int World::export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos) {
+int World::export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos,
+                        bool* room) {
     DeviceWorld& d = d_;
+    *room = true;
     const OnDevice on(d.device);  // a read allocates and launches there, whichever device is the caller's
     const bool sphere = path_ == StepPath::Sphere;
     const uint32_t id_mask = snap_flags_ ? kSnapIdMask : ~kSnapOutlier;
@@ -596,19 +585,28 @@ int World::export_state(float* pos, float* pos_old, float* vel, float* rot, floa
         auto f1 = [&](int i) { return dst[i] ? (float*)(base + at[i]) : nullptr; };
         return ExportOut{f2(kPos), f2(kPosOld), f2(kVel), f1(kRot), f1(kOmega), f1(kOldDt), f2(kCol)};
     };
+    size_t largest = 0;
+    for (int i = 0; i < kParts; ++i)
+        if (dst[i]) largest = std::max(largest, size[i]);
+    auto no_room = [&]() {
+        (void)hipGetLastError();
+        *room = false;
+        return BG_OK;
+    };
+    Staging stage;
+    if (stage.take(total <= kExportDirect ? total : largest, d.device) != hipSuccess) return no_room();
     if (total <= kExportDirect) {
-        if (int st = ensure_staging(total)) return st;
-        HIP_TRY(launch_export(d, sphere, id_mask, outputs(stage_)));
+        HIP_TRY(launch_export(d, sphere, id_mask, outputs(stage.half(0))));
         HIP_TRY(hipStreamSynchronize(d.stream));
         for (int i = 0; i < kParts; ++i)
-            if (dst[i]) memcpy(dst[i], stage_ + at[i], size[i]);
+            if (dst[i]) memcpy(dst[i], stage.half(0) + at[i], size[i]);
     } else {
         const void* src[kParts] = {d.b.pos, d.b.pos_old, d.b.vel, d.b.rot, d.b.omega, &d.accum->old_dt, d.c.abs};
         if (sphere) {
             if (total > d.export_size) {
                 dfree(d.export_buf);
                 d.export_size = 0;
-                HIP_TRY(dmalloc(&d.export_buf, total));
+                if (dmalloc(&d.export_buf, total) != hipSuccess) return no_room();
                 d.export_size = total;
             }
             HIP_TRY(launch_export(d, sphere, id_mask, outputs(d.export_buf)));
@@ -618,7 +616,10 @@ int World::export_state(float* pos, float* pos_old, float* vel, float* rot, floa
         uint32_t n = 0;
         for (int i = 0; i < kParts; ++i)
             if (dst[i]) c[n++] = {dst[i], src[i], size[i]};
-        if (int st = copy_to_host(c, n)) return st;
+        if (int st = copy_to_host(stage, c, n)) {
+            (void)hipStreamSynchronize(d.stream);  // the staging goes back
+            return st;
+        }
     }
     if (sphere && !batch_start_.empty())
         batch_old_dt_ = old_dt;

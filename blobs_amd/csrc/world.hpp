@@ -15,6 +15,7 @@
 #include "../../include/blobs_gpu.h"
 #include "arena.hpp"
 #include "device_state.hpp"
+#include "staging.hpp"
 
 namespace bg {
 
@@ -138,9 +139,9 @@ private:
         const void* src;
         size_t bytes;
     };
-    int ensure_staging(size_t bytes);
-    int copy_to_host(const CopyOut* c, uint32_t n);
-    int export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos);
+    int copy_to_host(const Staging& stage, const CopyOut* c, uint32_t n);
+    // (*room: false if there is no memory for it, and nothing was read)
+    int export_state(float* pos, float* pos_old, float* vel, float* rot, float* omega, float* col_pos, bool* room);
     void mark_dirty() { dev_dirty_ = true; }
     int rebuild();
     int run_substep(float h, bool fresh, bool last);
@@ -184,11 +185,6 @@ private:
     bool dev_dirty_ = true;
     bool host_stale_ = false;
     bool old_dt_known_ = false;  // host_stale_, but an export brought the worlds' old_dt
-    // pinned staging of exports: two halves of stage_half_ bytes (allocated by the first
-    // export, at most 2 x kStageHalf), an event each
-    char* stage_ = nullptr;
-    size_t stage_half_ = 0;
-    hipEvent_t stage_event_[2] = {nullptr, nullptr};
     std::vector<bg_handle> body_handle_of_dense_;
     bool stepped_since_upload_ = false;
     bool fresh_ = true;
