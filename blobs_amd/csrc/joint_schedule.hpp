@@ -31,24 +31,38 @@ struct JointSchedule {
     // n_bodies), numbered `ids`, swept `iterations` times.  `last` is scratch, all zero.
     void add_group(const std::vector<std::pair<uint32_t, uint32_t>>& joints, const std::vector<uint32_t>& ids,
                    uint32_t iterations, std::vector<uint32_t>& last, uint32_t width) {
-        std::vector<std::vector<std::pair<uint32_t, uint32_t>>> levels;
+        std::vector<uint32_t> filled;  // solves of each level
+        std::vector<uint32_t> room;    // of each level: itself, or where to look on for one with room
+        std::vector<uint32_t> at;      // each solve's level, in the order of the sweep
+        at.reserve(joints.size() * iterations);
         for (uint32_t it = 0; it < iterations; ++it)
-            for (size_t k = 0; k < joints.size(); ++k) {
-                uint32_t& la = last[joints[k].first];
-                uint32_t& lb = last[joints[k].second];
+            for (const auto& j : joints) {
+                uint32_t& la = last[j.first];
+                uint32_t& lb = last[j.second];
                 uint32_t l = std::max(la, lb);
-                while (l < levels.size() && levels[l].size() >= width) ++l;
-                if (l >= levels.size()) levels.resize(l + 1);
-                levels[l].push_back({ids[k], it});
+                while (l < room.size() && room[l] != l) {  // (halving the path, or a wide component walks all its levels)
+                    if (room[l] < room.size()) room[l] = room[room[l]];
+                    l = room[l];
+                }
+                for (; l >= room.size(); filled.push_back(0)) room.push_back((uint32_t)room.size());
+                if (++filled[l] == width) room[l] = l + 1;
+                at.push_back(l);
                 la = lb = l + 1;
             }
         for (const auto& j : joints) last[j.first] = last[j.second] = 0;
-        for (const auto& l : levels) {
-            for (const auto& e : l) {
-                entry.push_back(e.first);
-                iteration.push_back(e.second);
-            }
-            level_start.push_back((uint32_t)entry.size());
+        const size_t first = entry.size();
+        std::vector<uint32_t> next(filled.size());
+        for (size_t l = 0, n = first; l < filled.size(); ++l) {
+            next[l] = (uint32_t)n;
+            n += filled[l];
+            level_start.push_back((uint32_t)n);
+        }
+        entry.resize(first + at.size());
+        iteration.resize(first + at.size());
+        for (size_t s = 0; s < at.size(); ++s) {
+            const uint32_t to = next[at[s]]++;
+            entry[to] = ids[s % joints.size()];
+            iteration[to] = (uint32_t)(s / joints.size());
         }
         group_level.push_back((uint32_t)level_start.size() - 1);
     }

@@ -1879,20 +1879,48 @@ int World::ensure_joint_schedule() {
     if (iters == 0) return BG_OK;
     const uint32_t nj = (uint32_t)joint_bodies_.size();
     if ((uint64_t)nj * iters > 0xFFFFFFFFull) return fail(BG_ERR_CAPACITY, "joint solves of a substep exceed 2^32");
+    JointPlan& p = joint_plan_;
+    if (p.iters != iters || p.joints != joint_bodies_ || p.comp_start != joint_comp_start_ || p.statics != joint_static_)
+        make_joint_plan(iters);
+    hipStream_t s = d.stream;
+    HIP_TRY(dmalloc(&d.jg, p.groups.size()));
+    HIP_TRY(dmalloc(&d.jl_start, p.level_start.size()));
+    HIP_TRY(dmalloc(&d.j_entry, p.entry.size()));
+    HIP_TRY(dmalloc(&d.jg_body, p.bodies.size()));
+    HIP_TRY(dmalloc(&d.jq_ab, p.ab.size()));
+    HIP_TRY(dmalloc(&d.jrot, (size_t)iters * nj));
+    HIP_TRY(h2d(d.jg, p.groups, s));
+    HIP_TRY(h2d(d.jl_start, p.level_start, s));
+    HIP_TRY(h2d(d.j_entry, p.entry, s));
+    HIP_TRY(h2d(d.jg_body, p.bodies, s));
+    HIP_TRY(h2d(d.jq_ab, p.ab, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    d.n_jgroups = (uint32_t)p.groups.size();
+    d.j_iters = iters;
+    return BG_OK;
+}
+
+void World::make_joint_plan(uint32_t iters) {
+    JointPlan& p = joint_plan_;
+    p = JointPlan{};
+    p.joints = joint_bodies_;
+    p.comp_start = joint_comp_start_;
+    p.statics = joint_static_;
+    p.iters = iters;
+    const uint32_t nj = (uint32_t)joint_bodies_.size(), n_comp = (uint32_t)joint_comp_start_.size() - 1;
     JointSchedule sched;
-    std::vector<JointGroup> groups;
-    std::vector<int32_t> bodies, local(d.nb, -1);
-    std::vector<uint2> ab(nj);
+    std::vector<int32_t> local(joint_static_.size(), -1);
+    p.ab.resize(nj);
     std::vector<std::pair<uint32_t, uint32_t>> joints;
     std::vector<uint32_t> ids, last;
-    for (uint32_t c = 0; c < d.n_jcomp;) {
+    for (uint32_t c = 0; c < n_comp;) {
         JointGroup g;
         g.q0 = joint_comp_start_[c];
-        g.b0 = (uint32_t)bodies.size();
+        g.b0 = (uint32_t)p.bodies.size();
         g.l0 = (uint32_t)sched.level_start.size() - 1;
         do
             ++c;
-        while (c < d.n_jcomp && joint_comp_start_[c + 1] - g.q0 <= kGroupJoints);
+        while (c < n_comp && joint_comp_start_[c + 1] - g.q0 <= kGroupJoints);
         g.q1 = joint_comp_start_[c];
         joints.clear();
         ids.clear();
@@ -1901,45 +1929,29 @@ int World::ensure_joint_schedule() {
             for (int e = 0; e < 2; ++e) {
                 const int32_t b = e ? joint_bodies_[q].second : joint_bodies_[q].first;
                 if (local[b] < 0) {
-                    local[b] = (int32_t)(bodies.size() - g.b0);
-                    bodies.push_back(b);
+                    local[b] = (int32_t)(p.bodies.size() - g.b0);
+                    p.bodies.push_back(b);
                 }
                 l[e] = (uint32_t)local[b];
             }
-            ab[q].x = l[0] | (uint32_t)joint_static_[joint_bodies_[q].first] << 31;
-            ab[q].y = l[1] | (uint32_t)joint_static_[joint_bodies_[q].second] << 31;
+            p.ab[q].x = l[0] | (uint32_t)joint_static_[joint_bodies_[q].first] << 31;
+            p.ab[q].y = l[1] | (uint32_t)joint_static_[joint_bodies_[q].second] << 31;
             joints.push_back({l[0], l[1]});
             ids.push_back(q - g.q0);
         }
-        g.b1 = (uint32_t)bodies.size();
+        g.b1 = (uint32_t)p.bodies.size();
         last.assign(g.b1 - g.b0, 0);
         sched.add_group(joints, ids, iters, last, BG_WAVE);
         g.l1 = (uint32_t)sched.level_start.size() - 1;
-        groups.push_back(g);
+        p.groups.push_back(g);
     }
-    std::vector<uint2> entry(sched.entry.size());
-    for (const JointGroup& g : groups)
+    p.entry.resize(sched.entry.size());
+    for (const JointGroup& g : p.groups)
         for (uint32_t e = sched.level_start[g.l0]; e < sched.level_start[g.l1]; ++e)
-            entry[e] = make_uint2(sched.entry[e], sched.iteration[e] * nj + g.q0 + sched.entry[e]);
-    hipStream_t s = d.stream;
-    HIP_TRY(dmalloc(&d.jg, groups.size()));
-    HIP_TRY(dmalloc(&d.jl_start, sched.level_start.size()));
-    HIP_TRY(dmalloc(&d.j_entry, entry.size()));
-    HIP_TRY(dmalloc(&d.jg_body, bodies.size()));
-    HIP_TRY(dmalloc(&d.jq_ab, ab.size()));
-    HIP_TRY(dmalloc(&d.jrot, (size_t)iters * nj));
-    HIP_TRY(h2d(d.jg, groups, s));
-    HIP_TRY(h2d(d.jl_start, sched.level_start, s));
-    HIP_TRY(h2d(d.j_entry, entry, s));
-    HIP_TRY(h2d(d.jg_body, bodies, s));
-    HIP_TRY(h2d(d.jq_ab, ab, s));
-    HIP_TRY(hipStreamSynchronize(s));  // host vectors die at return
-    d.n_jgroups = (uint32_t)groups.size();
-    d.j_iters = iters;
-    return BG_OK;
+            p.entry[e] = make_uint2(sched.entry[e], sched.iteration[e] * nj + g.q0 + sched.entry[e]);
+    p.level_start = std::move(sched.level_start);
 }
 
-// Enqueues n steps (no host synchronisation; safe under stream capture).
 // The persistent batched step: every substep of the n steps for the worlds
 // it runs, in one launch per size class (batch_kernels.hip).  `fresh`: the
 // first of these substeps consumes the one-off user inputs.
@@ -2014,10 +2026,12 @@ int World::launch_small(double delta, uint32_t n) {
     return BG_OK;
 }
 
+// Enqueues n steps (no host synchronisation).
 int World::launch_steps(double delta, uint32_t n) {
     return small_active() ? launch_small(delta, n) : launch_large_steps(delta, n);
 }
 
+// The same, safe under stream capture.
 int World::launch_large_steps(double delta, uint32_t n) {
     if (persist_ && path_ == StepPath::Sphere && n > 0) {
         DeviceWorld& d = d_;

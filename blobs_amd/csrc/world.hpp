@@ -236,6 +236,20 @@ private:
     std::vector<std::pair<int32_t, int32_t>> joint_bodies_;
     std::vector<uint32_t> joint_comp_start_;
     std::vector<uint8_t> joint_static_;
+    // the schedule of the sweep, and what it was made from: an upload that changes none of it
+    // takes it as it is
+    struct JointPlan {
+        std::vector<std::pair<int32_t, int32_t>> joints;
+        std::vector<uint32_t> comp_start;
+        std::vector<uint8_t> statics;
+        uint32_t iters = 0;
+        std::vector<JointGroup> groups;
+        std::vector<uint32_t> level_start;
+        std::vector<uint2> entry, ab;
+        std::vector<int32_t> bodies;
+    };
+    JointPlan joint_plan_;
+    void make_joint_plan(uint32_t iters);
     // broadphase drift of the current rebuild period
     double drift_x_ = 0, drift_y_ = 0, vdrift_x_ = 0, vdrift_y_ = 0, h_prev_ = 0;
     uint64_t contact_base_ = 0;
