@@ -26,7 +26,9 @@ namespace bg {
 
 namespace {
 
-constexpr uint64_t kTapeBytes = 2ull << 30;  // tape memory beyond which segments are recomputed one at a time
+// Tape memory beyond which segments are recomputed one at a time: checkpoint_every is the caller's
+// bound on it, which several segments at once may not pass by much.
+constexpr uint64_t kTapeBytes = 64ull << 20;
 
 template <class T>
 hipError_t dalloc(T** p, size_t n) {

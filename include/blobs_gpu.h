@@ -332,7 +332,8 @@ int bg_autotune(bg_world *w, double delta, uint32_t steps_per_trial, float *cell
  * adjoint differentiates every stage of the step (gravity, springs with
  * their damping, contacts, joint positions, Verlet) with every substep's
  * contact pair set held fixed, recomputing each segment from its
- * checkpoint.  Body rotations are not tracked: with centred colliders and
+ * checkpoint (several at once as long as their tapes take at most 64 MiB
+ * together).  Body rotations are not tracked: with centred colliders and
  * unrotated joint anchors (physics.rs:434-435) no position depends on them. */
 typedef struct bg_rollout bg_rollout;
 int bg_rollout_create(bg_world *const *worlds, uint32_t n_worlds, const float *targets_xy, uint32_t checkpoint_every,

@@ -21,3 +21,17 @@ def test_worlds_of_no_substeps(joints):
     assert np.array_equal(r.final_positions(), np.concatenate([sc.pos, sc.pos]).astype(np.float32))
     gv, gk = r.backward()
     assert not gv.any() and not gk.any()
+
+
+@pytest.mark.parametrize("every", [1, 2])
+def test_memory_of_a_backward(every):
+    """A backward takes at most 64 MiB beside the segment of tape that checkpoint_every stands for."""
+    torch = pytest.importorskip("torch")
+    rng = scenes.Rng(4)
+    scs = [scenes.rollout_world(2048, 0, rng) for _ in range(48)]
+    r = Rollout([sc.build_physics()[0] for sc in scs], np.zeros((48, 2), np.float32), checkpoint_every=every)
+    r.forward(scs[0].dt, 8)
+    before = torch.cuda.mem_get_info()[0]
+    gv, _ = r.backward()
+    assert before - torch.cuda.mem_get_info()[0] <= 64 << 20
+    assert np.isfinite(gv).all() and gv.any()
