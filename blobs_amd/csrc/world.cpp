@@ -187,12 +187,12 @@ int World::stage_begin(uint32_t stage) {
     return BG_OK;
 }
 
-int World::stage_end(uint32_t stage) {
+int World::stage_end(uint32_t stage, uint32_t count) {
     if (!profiling_ || !open_[stage]) return BG_OK;
     hipEvent_t e;
     HIP_TRY(pooled_event(&e));
     HIP_TRY(hipEventRecord(e, d_.stream));
-    pending_[stage].push_back({open_[stage], e});
+    pending_[stage].push_back({open_[stage], e, count});
     open_[stage] = nullptr;
     return BG_OK;
 }
@@ -204,7 +204,7 @@ int World::collect_stage_times() {
             float ms = 0.0f;
             HIP_TRY(hipEventElapsedTime(&ms, pr.first, pr.second));
             stage_ms_[k] += ms;
-            stage_launches_[k] += 1;
+            stage_launches_[k] += pr.count;
             event_pool_.push_back(pr.first);
             event_pool_.push_back(pr.second);
         }
@@ -1787,7 +1787,7 @@ int World::run_substep(float h, bool fresh, bool last) {
         const hipError_t e = launch_sphere_substep(d, a, groups_, sensors_, zero_off_, d.nk > 0);
         d.prof_start = d.prof_stop = nullptr;
         HIP_TRY(e);
-        if (profiling_) pending_[BG_STAGE_SUBSTEP].push_back({e0, e1});
+        if (profiling_) pending_[BG_STAGE_SUBSTEP].push_back({e0, e1, 1});
         return BG_OK;
     }
     if (int st = stage_begin(BG_STAGE_SUBSTEP)) return st;
@@ -1982,10 +1982,9 @@ int World::launch_persistent(double delta, uint32_t n, bool fresh, hipStream_t s
     return BG_OK;
 }
 
-// Small worlds (small_kernels.hip).  A setting made with bg_set_broadphase, and stage timing,
-// are the grid path's.
+// Small worlds (small_kernels.hip).  A setting made with bg_set_broadphase is the grid path's.
 bool World::small_active() const {
-    return small_ && path_ == StepPath::Sphere && rebuild_interval_ == 0 && !profiling_ && !d_.gather_pending;
+    return small_ && path_ == StepPath::Sphere && rebuild_interval_ == 0 && !d_.gather_pending;
 }
 
 int World::launch_small(double delta, uint32_t n) {
@@ -2016,7 +2015,9 @@ int World::launch_small(double delta, uint32_t n) {
         k.nsub = (uint32_t)std::min<uint64_t>(left, kSmallSubsteps);
         k.fresh = fresh_ ? 1u : 0u;
         k.sub_global = substep_seq_;
+        if (int st = stage_begin(BG_STAGE_SUBSTEP)) return st;
         HIP_TRY(launch_small_step(k, d.stream));
+        if (int st = stage_end(BG_STAGE_SUBSTEP, k.nsub)) return st;
         substep_seq_ += k.nsub;
         left -= k.nsub;
         fresh_ = false;

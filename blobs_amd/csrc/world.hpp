@@ -168,7 +168,7 @@ private:
     void free_arrays();
     hipError_t pooled_event(hipEvent_t* out);
     int stage_begin(uint32_t stage);
-    int stage_end(uint32_t stage);
+    int stage_end(uint32_t stage, uint32_t count = 1);
     int collect_stage_times();
     int collect_events();
 
@@ -277,7 +277,11 @@ private:
     // profiling: event pairs recorded since the last collection, per stage
     bool profiling_ = false;
     std::vector<hipEvent_t> event_pool_;
-    std::vector<std::pair<hipEvent_t, hipEvent_t>> pending_[BG_STAGE_COUNT];
+    struct Timed {
+        hipEvent_t first, second;
+        uint32_t count;  // launches it stands for
+    };
+    std::vector<Timed> pending_[BG_STAGE_COUNT];
     hipEvent_t open_[BG_STAGE_COUNT] = {nullptr, nullptr};
     uint64_t stage_launches_[BG_STAGE_COUNT] = {0, 0};
     double stage_ms_[BG_STAGE_COUNT] = {0.0, 0.0};

@@ -424,7 +424,9 @@ int bg_spatial_hash_query_noalloc(float cell_size, const bg_spatial_point *point
 /* Per-stage timing with HIP events on the world's stream, the analogue of
  * the reference's tracy spans around `substep` and the contact pass
  * (lib.rs:195-209, physics.rs:402,242).  Stages: BG_STAGE_SUBSTEP (all
- * kernels of one substep), BG_STAGE_REBUILD (broadphase rebuild). */
+ * kernels of one substep), BG_STAGE_REBUILD (broadphase rebuild).  A small
+ * world's launch covers many substeps, its partner lists included: its time
+ * is the substep stage's, counted as that many launches. */
 enum { BG_STAGE_SUBSTEP = 0, BG_STAGE_REBUILD = 1, BG_STAGE_COUNT = 2 };
 int bg_set_profiling(bg_world *w, int enable);
 /* Launch count and summed event time (ms) of a stage since profiling was
