@@ -441,7 +441,7 @@ constexpr uint32_t kColList = 16;   // corrections a collider keeps (the smalles
 constexpr uint32_t kFlatRows = 3;   // rows of cells walked as one flat list of candidates
 constexpr uint32_t kFlatMax = 64;   // candidates of a flat list (one 64-bit mask)
 constexpr uint32_t kPairCap = 320;  // pairs a wave queues
-constexpr int kDirectRegs = 4;      // corrections of a collider outside the queue sorted in registers a pass
+constexpr int kDirectRegs = 4;      // corrections of a collider outside the queue sorted in registers
 
 // Contacts, first half of the two-kernel form: every collider walks its own
 // stencil (physics.rs:248-300 for the pairs it is in), counts the pairs it is
@@ -468,6 +468,10 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
+__device__ __forceinline__ uint64_t merge_key(float4 v) {
+    return ((uint64_t)__float_as_uint(v.x) << 32) | __float_as_uint(v.y);
+}
+
 template <bool GROUPS, bool SENSORS>
 __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const SubstepArgs& a, ListsLds& lds, uint32_t slot,
                                               uint32_t count_slot) {
@@ -495,7 +499,7 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
     // record rb, collider j, mass mp: put(x, y) with the correction, if it is a contact that has
     // one.  axis = A - B with A the higher collider index; b - a == -(a - b) up to the sign of a
     // zero, so the unoriented difference decides.  A push-out only records its row (as k_contacts).
-    auto contact = [&](bool once, uint32_t cc, int32_t body, const float4& o, const float4& rb, uint32_t j, float mp,
+    auto contact = [&](uint32_t cc, int32_t body, const float4& o, const float4& rb, uint32_t j, float mp,
                        auto&& put) {
         float ax = o.x - rb.x, ay = o.y - rb.y;
         const float rs = o.z + rb.z;
@@ -508,7 +512,7 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
             if (!((ga.x & gb.y) != 0u && (gb.x & ga.y) != 0u)) return;
         }
         const bool isA = cc > j;
-        if (once && isA) {
+        if (isA) {
             ++count;
             if (d.events) {  // physics.rs:288-311
                 const unsigned long long e = atomicAdd(&d.accum->event_count, 1ull);
@@ -533,12 +537,10 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
             dist = vlen(ax, ay);
             px = isA ? 0.01f : -0.01f;
             py = isA ? 0.0f : -0.0f;
-            if (once) {
-                flags |= INFO_PUSH_OUT;
-                if (isA) {
-                    const uint32_t bit = 1u << (cc & 31u);
-                    if (!(atomicOr(&d.ord_mark[cc >> 5], bit) & bit)) d.ord_rows[atomicAdd(d.ord_n, 1u)] = cc;
-                }
+            flags |= INFO_PUSH_OUT;
+            if (isA) {
+                const uint32_t bit = 1u << (cc & 31u);
+                if (!(atomicOr(&d.ord_mark[cc >> 5], bit) & bit)) d.ord_rows[atomicAdd(d.ord_n, 1u)] = cc;
             }
         }
         if (SENSORS && ((d.c.cflags[cc] | d.c.cflags[j]) & 1u)) {
@@ -548,7 +550,7 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
         const float mA = isA ? o.w : mp, mB = isA ? mp : o.w;
         const float ratio = 1.0f - mA / (mA + mB);
         const float nx = ax / dist, ny = ay / dist;
-        if (once && (nx != nx || ny != ny)) flags |= ERR_NAN_NORMAL;
+        if (nx != nx || ny != ny) flags |= ERR_NAN_NORMAL;
         const float delta = rs - dist;
         const float k = isA ? ratio * delta : (1.0f - ratio) * delta;
         float cx = isA ? k * nx : -(k * nx), cy = isA ? k * ny : -(k * ny);
@@ -640,7 +642,7 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
         const uint32_t j = d.vals[pr.y];
         const uint2 id = s_id[pr.x];
         s_pair[e].x = kNil;
-        contact(true, id.x, (int32_t)id.y, s_own[pr.x], rb, j, d.b.mass[__float_as_int(rb.w)], [&](float x, float y) {
+        contact(id.x, (int32_t)id.y, s_own[pr.x], rb, j, d.b.mass[__float_as_int(rb.w)], [&](float x, float y) {
             s_pair[e].x = j;
             s_res[e] = make_float2(x, y);
         });
@@ -662,32 +664,53 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
         next = best + 1u;
     }
     if (direct) {  // more candidates than a flat list, or no room in the queue
+        // The first few contacts are sorted in registers; all go to the list as they are found, and
+        // are sorted there if they are more.  (One large collider sends everyone here: a step of 5,000
+        // bodies with one of 12 units 2,747 us, 5,559 with a record a load and a pass for every four
+        // contacts; 50,000 bodies 3,646 and 7,246.)
         ContactList<kDirectRegs, uint32_t> L;
-        uint32_t last = 0;
-        for (bool once = true;; once = false) {
-            L.init();
-            for (int32_t cy = cy0; cy <= cy1; ++cy) {
-                const uint32_t row = (uint32_t)cy * nx;
-                const uint32_t t1 = min(d.cell_start[row + (uint32_t)cx1 + 1u], d.nc);
-                for (uint32_t t = d.cell_start[row + (uint32_t)cx0]; t < t1; ++t) {
-                    const float4 rb = d.crec[t];
-                    if (!near(rb)) continue;
-                    const uint32_t j = d.vals[t];
-                    if (!once && j <= last) continue;
-                    contact(once, c, b, own, rb, j, d.b.mass[__float_as_int(rb.w)],
-                            [&](float x, float y) { L.add(j, x, y); });
+        L.init();
+        for (int32_t cy = cy0; cy <= cy1; ++cy) {
+            const uint32_t row = (uint32_t)cy * nx;
+            const uint32_t t1 = min(d.cell_start[row + (uint32_t)cx1 + 1u], d.nc);
+            for (uint32_t t = d.cell_start[row + (uint32_t)cx0]; t < t1; t += 4) {
+                // (four records load together: a walk of hundreds waits for each of its loads)
+                float4 four[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) four[u] = d.crec[min(t + u, t1 - 1u)];
+                uint32_t bits = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) bits |= t + u < t1 && near(four[u]) ? 1u << u : 0u;
+                for (; bits != 0; bits &= bits - 1) {
+                    const uint32_t slot_b = t + (uint32_t)__builtin_ctz(bits);
+                    const float4 rb = d.crec[slot_b];
+                    const uint32_t j = d.vals[slot_b];
+                    contact(c, b, own, rb, j, d.b.mass[__float_as_int(rb.w)], [&](float x, float y) {
+                        store(L.n, j, x, y);
+                        L.add(j, x, y);
+                    });
                 }
             }
+        }
+        n_put = L.n;
+        if (n_put <= (uint32_t)kDirectRegs) {
 #pragma unroll
             for (int i = 0; i < kDirectRegs; ++i)
-                if ((uint32_t)i < L.n) store(n_put + (uint32_t)i, L.key[i], L.cx[i], L.cy[i]);
-            if (once && L.n > kColList) {  // (the count alone matters then)
-                n_put = L.n;
-                break;
+                if ((uint32_t)i < n_put) store((uint32_t)i, L.key[i], L.cx[i], L.cy[i]);
+        } else if (n_put <= kColList) {  // (the count alone matters past that)
+            float4* list = d.clist + c;
+            for (uint32_t i = 0; i + 1 < n_put; ++i) {
+                uint32_t least = i;
+                uint64_t key = merge_key(list[(size_t)i * d.nc]);
+                for (uint32_t k = i + 1; k < n_put; ++k) {
+                    const uint64_t other = merge_key(list[(size_t)k * d.nc]);
+                    least = other < key ? k : least;
+                    key = other < key ? other : key;
+                }
+                const float4 v = list[(size_t)i * d.nc];
+                list[(size_t)i * d.nc] = list[(size_t)least * d.nc];
+                list[(size_t)least * d.nc] = v;
             }
-            n_put += min(L.n, (uint32_t)kDirectRegs);
-            if (L.n <= (uint32_t)kDirectRegs) break;
-            last = L.key[kDirectRegs - 1];
         }
     }
     if (slot < d.nc) d.ccnt[c] = n_put;
@@ -719,10 +742,6 @@ __global__ __launch_bounds__(kContactThreads) void k_contact_lists(DeviceWorld d
 constexpr uint32_t kMergeLanes = 8;
 constexpr uint32_t kMergeAhead = 2;  // corrections a lane loads before its count is known
 constexpr int kMergeRegs = 6;
-
-__device__ __forceinline__ uint64_t merge_key(float4 v) {
-    return ((uint64_t)__float_as_uint(v.x) << 32) | __float_as_uint(v.y);
-}
 
 // (whole waves: thread t of the pass)
 __device__ __forceinline__ void contact_merge(const DeviceWorld& d, uint32_t t) {
