@@ -252,7 +252,8 @@ int Rollout::create(World* const* worlds, uint32_t n, const float* targets, uint
                     const float ratio = inv_a / ims;
                     joints.push_back({(uint32_t)h.ja[q], (uint32_t)h.jb[q]});
                     ids.push_back((uint32_t)j_ab.size() - d.jq0);
-                    j_ab.push_back((uint32_t)h.ja[q] | ((uint32_t)h.jb[q] << 16));
+                    j_ab.push_back((uint32_t)h.ja[q] | (h.flags[h.ja[q]] & BF_STATIC ? 1u << 15 : 0u) |
+                                   (uint32_t)h.jb[q] << 16 | (h.flags[h.jb[q]] & BF_STATIC ? 1u << 31 : 0u));
                     j_anchor.push_back(make_float4(h.jan_a[q].x, h.jan_a[q].y, h.jan_b[q].x, h.jan_b[q].y));
                     j_dist.push_back(h.jdist[q]);
                     j_mass.push_back(make_float4(ims, ratio, 1.0f - ratio, 1.0f));

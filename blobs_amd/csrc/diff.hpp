@@ -65,7 +65,7 @@ struct DiffArgs {
     const uint32_t* jg_level;
     const uint32_t* jl_start;
     const uint32_t* j_entry;
-    const uint32_t* j_ab;      // local body a | local body b << 16
+    const uint32_t* j_ab;      // local a | a is static << 15 | local b << 16 | b is static << 31
     const float4* j_anchor;    // anchor a (x, y), anchor b (z, w)
     const float* j_dist;
     const float4* j_mass;  // 1/m_a + 1/m_b, ratio, 1 - ratio, unused

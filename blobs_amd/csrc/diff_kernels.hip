@@ -197,8 +197,6 @@ static __device__ __forceinline__ JointRec joint_rec(const Ctx& c, const DiffArg
         r.mass = a.j_mass[W.jq0 + q];
         r.mass.w = a.j_dist[W.jq0 + q];
         r.ab = a.j_ab[W.jq0 + q];
-        if (a.flags[W.b0 + (r.ab & 0x7FFFu)] & BF_STATIC) r.ab |= 1u << 15;
-        if (a.flags[W.b0 + ((r.ab >> 16) & 0x7FFFu)] & BF_STATIC) r.ab |= 1u << 31;
     }
     return r;
 }

@@ -7,6 +7,7 @@ import pytest
 from blobs_amd import _lib as L
 from blobs_amd import scenes
 from blobs_amd.rollout import Rollout
+from oracle.oracle import OracleWorld
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +45,22 @@ def test_memory_of_a_backward(every):
     gv, _ = r.backward()
     assert before - free_memory() <= 64 << 20
     assert np.isfinite(gv).all() and gv.any()
+
+
+@pytest.mark.parametrize("joints", [4, 256, 257])  # staged in LDS, and one more than it holds
+def test_joints_of_static_bodies(joints):
+    """Every second joint holds its body a or b, or both, in place (the records carry the flags)."""
+    sc = scenes.rollout_world(300, 20, scenes.Rng(9), damping=1.0, n_joints=joints, anchor=0.2)
+    sc.body_type = sc.body_type.copy()
+    sc.body_type[sc.joint_a[::4]] = 1
+    sc.body_type[sc.joint_b[2::4]] = 1
+    got = []
+    for every in (1, 3):
+        r = Rollout([sc.build_physics()[0]], np.zeros((1, 2), np.float32), checkpoint_every=every)
+        r.forward(sc.dt, 4)
+        got.append((r.final_positions(), *r.backward()))
+    o = OracleWorld(sc, np.float32)
+    o.step(sc.dt, 4)
+    assert np.array_equal(got[0][0].view(np.uint32), np.ascontiguousarray(o.pos, np.float32).view(np.uint32))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
