@@ -56,3 +56,30 @@ def test_lists_change_no_result(n, kind):
         b0 += sc.n_bodies
     for a, b in zip(*got):
         assert np.array_equal(bits(a), bits(b))
+
+
+@pytest.mark.parametrize("partners", [1, 2, 15, 16, 17, 18, 33])
+@pytest.mark.parametrize("n", [256, 700, 2048])
+def test_bodies_of_many_partners_in_rounds(n, partners):
+    """Hubs with so many bodies touching them and no others, in random index order; more pairs than the
+    queue holds at once, where a body's last 16 partners are kept from the walk that counts them."""
+    rng = np.random.default_rng(n + partners)
+    sc = scenes.rollout_world(n, 8, scenes.Rng(42), damping=1.0)
+    size = partners + 1
+    k = np.arange(n)
+    hub, member = k // size, k % size
+    wide = int(np.ceil(np.sqrt(n / size)))
+    at = np.stack([hub % wide, hub // wide], 1) * 12.0 - 6.0 * wide
+    angle = 2.0 * np.pi * member / max(partners, 1)
+    at += np.where(member[:, None] > 0, 4.0 * np.stack([np.cos(angle), np.sin(angle)], 1), 0.0)
+    order = rng.permutation(n)
+    sc.pos, sc.col_r = np.zeros((n, 2), np.float32), np.zeros(n, np.float32)
+    sc.pos[order] = at + rng.uniform(-0.02, 0.02, (n, 2))
+    sc.col_r[order] = np.where(member > 0, 0.33, 3.75)
+    sc.col_abs = sc.pos.copy()
+    got = [run([sc], 3, ck) for ck in (1, 2)]
+    o = OracleWorld(sc, np.float32)
+    o.step(sc.dt, 3)
+    assert np.array_equal(bits(got[0][0]), bits(o.pos))
+    for a, b in zip(*got):
+        assert np.array_equal(bits(a), bits(b))
