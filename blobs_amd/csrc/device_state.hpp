@@ -65,7 +65,8 @@ struct JointGroup {
     uint32_t b0, b1;  // body list
     uint32_t l0, l1;  // levels
 };
-constexpr uint32_t kSmallColliders = 1152, kSmallGeneral = 256;  // general path: worlds in four launches a substep
+// General path: worlds in four launches a substep (the limits' reasons: step_kernels.hip).
+constexpr uint32_t kSmallColliders = 1152, kSmallGeneral = 256;
 constexpr uint32_t kClipWait = 64;  // general path: substeps after an upload with the grid's whole box (clip_box)
 constexpr uint32_t kGroupJoints = 64;  // joints of a group (a larger component is a group by itself)
 
@@ -106,12 +107,13 @@ constexpr uint32_t kOrdTerms = 8192;  // addends of one body's position sum
 // Persistent batched step (batch_kernels.hip): the worlds of a batch with
 // kPersistMinBodies to kLdsBodies bodies, each run by ONE workgroup of
 // kPersistClassThreads threads for every substep of a launch, bodies in
-// registers (kPersistPer per thread), snapshot and grid in LDS.  Smaller
-// worlds are cheaper on the grid path: a world of a few hundred bodies is
-// too little parallel work for a workgroup's serial chain of grid-build
-// phases per substep (measured on the 4,096-world batch: 0.45 vs 0.20 ms per
-// step for its worlds up to 256 bodies, 0.59 vs 0.41 up to 1,024, 0.73 vs
-// 1.12 from 1,025 to 4,096).
+// registers (kPersistPer per thread), snapshot and grid in LDS.  It builds the
+// grid anew every substep, and the smaller worlds of a batch of all sizes are too
+// little parallel work for that chain of phases: they stay on the grid path
+// (ms a step of the 4,096-world batch: 0.45 against 0.20 there for its worlds up
+// to 256 bodies, 0.59 against 0.41 up to 1,024, 0.73 against 1.12 from 1,025 to
+// 4,096).  A batch of nothing but small worlds takes small_kernels.hip, which
+// keeps partner lists instead.
 constexpr uint32_t kPersistPer = 4;
 constexpr uint32_t kPersistClasses = 1;
 constexpr uint32_t kPersistClassThreads[kPersistClasses] = {1024};

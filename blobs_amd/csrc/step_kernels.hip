@@ -1141,10 +1141,16 @@ __global__ __launch_bounds__(kThreads) void k_integrate(DeviceWorld d, SubstepAr
 // launches instead of ten: one workgroup sorts and works out the contacts, one solves the
 // joints and integrates (the fallback and the ordered pass in between, which have nothing to do
 // in most substeps).  A pass of such a world is a launch's few microseconds whatever it does, and
-// a barrier a tenth of one; but one workgroup has one CU's latency to hide its loads in, so a
-// second round over the colliders costs what the launches did.  A step: 48 bodies 251 us against
-// 319 in ten launches, 120 285 against 359, 250 (1,115 colliders) 359 against 379, but 300
-// 460 against 395.
+// a barrier a tenth of one; but one workgroup has one CU's latency to hide its loads in, and each
+// further round over the colliders (1,024 a round) or the bodies (256, at four lanes each) costs part
+// of what the launches did.  A step in one workgroup against ten launches, us:
+//   48 bodies 273 / 330, 120 301 / 360, 200 329 / 371;
+//   256 bodies of  256 colliders 292 / 344,   512 303 / 352,   817 322 / 364, 1,024 354 / 450,
+//              1,152 386 / 464, 1,216 408 / 471, 1,280 445 / 492, 1,408 575 / 569, 1,536 734 / 658;
+//   128 bodies of 1,000 746 / 777, 1,100 906 / 896, 1,152 1,027 / 995, 1,280 1,305 / 1,238;
+//   past 256 bodies: 262 of 1,152 406 / 382, 300 442 / 389, 320 of 320 359 / 361, 512 of 512 411 / 366.
+// So the bodies stop at one round.  The colliders' second round still pays up to some 1,400 where a body
+// has few of them, and from 1,100 on no longer at nine a body: the limit lies between the two.
 constexpr uint32_t kSmallThreads = 1024;
 
 template <bool GROUPS, bool SENSORS>
