@@ -315,7 +315,7 @@ int bg_step_path(bg_world* w, uint32_t* out) {
 }
 
 // Internal diagnostic hook (bgx_: not part of the Physics ABI): the world's
-// step record {n_outliers, dmax bits, push_outs, error_flags}.
+// step record {n_outliers, 0, push_outs, error_flags}.
 int bgx_world_accum(bg_world* w, uint32_t* out4) {
     return guarded(w, [&](bg::World& x) { return x.debug_accum(out4); });
 }

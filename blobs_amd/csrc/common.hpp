@@ -135,9 +135,10 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     return (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 }
 
-// Per-step reduction record: max displacement since the last rebuild, the
-// bounding box of collider snapshots (order-mapped floats) and the contact
-// count.  Block-reduced, then one atomic per block.
+// The step's record, which every call reads: the bounding box of the collider
+// snapshots (order-mapped floats; reduced in a block, then an atomic each),
+// counters of outliers, events and push-outs, error flags, and what the next
+// steps' choices go by.
 struct StepAccum {
     uint32_t clip_hold;  // general path: substeps for which the grid's box is not clipped
     uint32_t last_outliers;  // sphere path: n_outliers of the rebuild period before this one
