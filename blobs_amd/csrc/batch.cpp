@@ -160,7 +160,7 @@ namespace {
 // only from the state it was captured in.
 struct LaunchState {
     const void* p[8];
-    uint32_t u[5];
+    uint32_t u[4];
     bool operator==(const LaunchState& o) const { return memcmp(this, &o, sizeof(*this)) == 0; }
 };
 
@@ -183,10 +183,9 @@ int World::step_chunks(double delta, uint32_t chunk_steps, uint32_t n_chunks) {
         s.p[6] = p_src_.pp;  // the persistent launch reads its worlds from here
         s.p[7] = p_src_.snap;
         s.u[0] = bbox_parity_;
-        s.u[1] = 0;
-        s.u[2] = (need_rebuild_ ? 1u : 0u) | (d.gather_pending ? 2u : 0u) | (fresh_ ? 4u : 0u);
-        s.u[3] = sub_since_rebuild_;
-        s.u[4] = interval_substeps();
+        s.u[1] = (need_rebuild_ ? 1u : 0u) | (d.gather_pending ? 2u : 0u) | (fresh_ ? 4u : 0u);
+        s.u[2] = sub_since_rebuild_;
+        s.u[3] = interval_substeps();
         return s;
     };
     const bool prof = profiling_;
