@@ -136,38 +136,6 @@ struct Own {
 };
 static constexpr uint32_t kIncMany = 0xFFFFFFu;
 static_assert(PER == 1 || PER == 2, "the picks");
-template <class T>
-static __device__ __forceinline__ T pick(const T (&v)[PER], uint32_t j) {
-    if constexpr (PER == 1)
-        return v[0];
-    else
-        return j ? v[1] : v[0];
-}
-static __device__ __forceinline__ float2 pick(const float2 (&v)[PER], uint32_t j) {
-    if constexpr (PER == 1)
-        return v[0];
-    else
-        return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
-}
-template <class T>
-static __device__ __forceinline__ void put(T (&v)[PER], uint32_t j, T x) {
-    if constexpr (PER == 1) {
-        v[0] = x;
-    } else {
-        v[0] = j ? v[0] : x;
-        v[1] = j ? x : v[1];
-    }
-}
-static __device__ __forceinline__ void put(float2 (&v)[PER], uint32_t j, float2 x) {
-    if constexpr (PER == 1) {
-        v[0] = x;
-    } else {
-        v[0].x = j ? v[0].x : x.x;
-        v[0].y = j ? v[0].y : x.y;
-        v[1].x = j ? x.x : v[1].x;
-        v[1].y = j ? x.y : v[1].y;
-    }
-}
 static __device__ __forceinline__ uint32_t per_thread(const DiffWorld& W) { return PER == 1 || W.nb <= NT ? 1u : 2u; }
 
 // The thread's index, opaque to the compiler: the phases of a substep recompute what they

@@ -1,14 +1,17 @@
 // lds_grid.hpp -- contacts of one world inside one workgroup: its bodies'
-// snapshot filed by cell in LDS every substep, and the contact pass of one
-// body over it (physics.rs:241-317).  Shared by the differentiable rollouts
-// and the persistent step.
+// snapshot filed by cell in LDS, from which partner lists are filled (or, in a
+// rollout too dense for lists, each substep's candidates taken), and the queue
+// that their contacts are worked out from (physics.rs:241-317).  Shared by the
+// differentiable rollouts and the small worlds' step; the general path takes
+// the wave scans and the flat rows of cells.
 //
 // What bounds such a substep is VALU issue and the chain of phases between
-// barriers, not memory.  So the grid is fitted once every kFitEvery substeps
-// (bodies outside it clamp into border cells; any grid gives the same pairs),
-// the scans and reductions are DPP chains in registers (a ds_bpermute per
-// step costs the LDS latency six times over), and contacts are worked out by
-// all threads from a queue of the pairs within reach.
+// barriers, not memory.  So the grid is fitted when the lists are built and, by
+// a world filed every substep, every kFitEvery of them (bodies outside it clamp
+// into border cells; any grid gives the same pairs), the scans and reductions
+// are DPP chains in registers (a ds_bpermute per step costs the LDS latency six
+// times over), and contacts are worked out by all threads from a queue of the
+// pairs within reach.
 #pragma once
 
 #include "step_common.hpp"
@@ -80,9 +83,49 @@ __device__ __forceinline__ void lds_scan(uint32_t* cnt, uint32_t n, uint32_t* re
     __syncthreads();
 }
 
+// ---- a thread's one or two bodies --------------------------------------------
+//
+// By selects: an index known only at run time would put the arrays into scratch memory.
+
+template <class T, uint32_t N>
+__device__ __forceinline__ T pick(const T (&v)[N], uint32_t j) {
+    static_assert(N <= 2, "one select");
+    if constexpr (N == 1)
+        return v[0];
+    else
+        return j ? v[1] : v[0];
+}
+template <uint32_t N>
+__device__ __forceinline__ float2 pick(const float2 (&v)[N], uint32_t j) {
+    if constexpr (N == 1)
+        return v[0];
+    else
+        return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
+}
+template <uint32_t N>
+__device__ __forceinline__ void put(float2 (&v)[N], uint32_t j, float2 x) {
+    if constexpr (N == 1) {
+        v[0] = x;
+    } else {
+        v[0].x = j ? v[0].x : x.x;
+        v[0].y = j ? v[0].y : x.y;
+        v[1].x = j ? x.x : v[1].x;
+        v[1].y = j ? x.y : v[1].y;
+    }
+}
+template <class T, uint32_t N>
+__device__ __forceinline__ void put(T (&v)[N], uint32_t j, T x) {
+    if constexpr (N == 1) {
+        v[0] = x;
+    } else {
+        v[0] = j ? v[0] : x;
+        v[1] = j ? x : v[1];
+    }
+}
+
 // ---- the grid -------------------------------------------------------------
 
-constexpr uint32_t kFitEvery = 32;  // substeps between fits of the grid to the bodies
+constexpr uint32_t kFitEvery = 32;  // substeps between fits of a grid that is filed every substep
 
 struct LdsGrid {
     float ox, oy, inv_cell;
@@ -248,8 +291,8 @@ __device__ __forceinline__ LdsRect lds_rect(const LdsGrid& g, float x, float y, 
     return c;
 }
 
-// A body's pairs in the queue: `n` entries from `first`, or its contacts are left to
-// lds_contacts_direct (too many candidates, or no room).
+// A body's pairs in the queue: `n` entries from `first`, or (direct: no room for them) its
+// contacts are left to the caller.
 struct LdsPairs {
     uint32_t first, n;
     bool direct;
@@ -295,27 +338,29 @@ struct LdsRows {
         return (i >= end0 ? step1 : 0u) + (i >= end1 ? step2 : 0u) + (base + i);
     }
 };
+// The cells of `c` in a grid of nx columns (neither past 65,536) whose records start at start[cell].
+__device__ __forceinline__ LdsRows flat_rows(const uint32_t* start, uint32_t nx, const LdsRect& c) {
+    LdsRows l;
+    const uint32_t row0 = __umul24((uint32_t)c.cy0, nx), last = __umul24((uint32_t)c.cy1, nx);
+    const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
+    const uint32_t* s0 = start + c.cx0;
+    const uint32_t* s1 = start + c.cx1 + 1;
+    const uint32_t lo0 = s0[row0], hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
+    const int32_t rows = c.cy1 - c.cy0 + 1;
+    l.base = lo0;
+    l.end0 = hi0 - lo0;
+    l.step1 = lo1 - hi0;
+    l.end1 = l.end0 + (rows > 1 ? hi1 - lo1 : 0u);
+    l.step2 = (lo2 - l.end1) - (lo1 - l.end0);
+    l.n = l.end1 + (rows > 2 ? hi2 - lo2 : 0u);
+    l.flat = rows <= kLdsRows && l.n <= kLdsFlat;
+    if (!l.flat) l.n = 0;
+    static_assert(kLdsRows == 3, "the rows above");
+    return l;
+}
 __device__ __forceinline__ LdsRows lds_rows(const LdsGrid& g, const uint32_t* start, bool active, float2 xy, float Q) {
     LdsRows l = {0, 0, 0, 0, 0, 0, false};
-    if (active) {
-        const LdsRect c = lds_rect(g, xy.x, xy.y, Q);
-        const uint32_t nx = (uint32_t)g.nx;
-        const uint32_t row0 = __umul24((uint32_t)c.cy0, nx), last = __umul24((uint32_t)c.cy1, nx);
-        const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
-        const uint32_t* s0 = start + c.cx0;
-        const uint32_t* s1 = start + c.cx1 + 1;
-        const uint32_t lo0 = s0[row0], hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
-        const int32_t rows = c.cy1 - c.cy0 + 1;
-        l.base = lo0;
-        l.end0 = hi0 - lo0;
-        l.step1 = lo1 - hi0;
-        l.end1 = l.end0 + (rows > 1 ? hi1 - lo1 : 0u);
-        l.step2 = (lo2 - l.end1) - (lo1 - l.end0);
-        l.n = l.end1 + (rows > 2 ? hi2 - lo2 : 0u);
-        l.flat = rows <= kLdsRows && l.n <= kLdsFlat;
-        if (!l.flat) l.n = 0;
-    }
-    static_assert(kLdsRows == 3, "the rows above");
+    if (active) l = flat_rows(start, (uint32_t)g.nx, lds_rect(g, xy.x, xy.y, Q));
     return l;
 }
 

@@ -83,41 +83,6 @@ struct Own {
     float gm[PER], skin[PER];
     uint32_t id[PER];  // local index | body flags << 16
 };
-template <class T, uint32_t PER>
-__device__ __forceinline__ T pick(const T (&v)[PER], uint32_t j) {
-    if constexpr (PER == 1)
-        return v[0];
-    else
-        return j ? v[1] : v[0];
-}
-template <uint32_t PER>
-__device__ __forceinline__ float2 pick(const float2 (&v)[PER], uint32_t j) {
-    if constexpr (PER == 1)
-        return v[0];
-    else
-        return make_float2(j ? v[1].x : v[0].x, j ? v[1].y : v[0].y);
-}
-template <uint32_t PER>
-__device__ __forceinline__ void put(float2 (&v)[PER], uint32_t j, float2 x) {
-    if constexpr (PER == 1) {
-        v[0] = x;
-    } else {
-        v[0].x = j ? v[0].x : x.x;
-        v[0].y = j ? v[0].y : x.y;
-        v[1].x = j ? x.x : v[1].x;
-        v[1].y = j ? x.y : v[1].y;
-    }
-}
-template <class T, uint32_t PER>
-__device__ __forceinline__ void put(T (&v)[PER], uint32_t j, T x) {
-    if constexpr (PER == 1) {
-        v[0] = x;
-    } else {
-        v[0] = j ? v[0] : x;
-        v[1] = j ? x : v[1];
-    }
-}
-
 __device__ __forceinline__ float lane_f32(float v, int lane) {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
 }

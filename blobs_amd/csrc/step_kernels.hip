@@ -438,8 +438,6 @@ __global__ __launch_bounds__(kContactThreads) void k_contacts(DeviceWorld d, Sub
 }
 
 constexpr uint32_t kColList = 16;   // corrections a collider keeps (the smallest keys)
-constexpr uint32_t kFlatRows = 3;   // rows of cells walked as one flat list of candidates
-constexpr uint32_t kFlatMax = 64;   // candidates of a flat list (one 64-bit mask)
 constexpr uint32_t kPairCap = 320;  // pairs a wave queues
 constexpr int kDirectRegs = 4;      // corrections of a collider outside the queue sorted in registers
 
@@ -567,11 +565,10 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
     };
 
     // ---- mark
-    int32_t cx0 = 0, cx1 = 0, cy0 = 0, cy1 = 0;
+    LdsRect cells = {0, 0, 0, 0};
+    LdsRows rows = {0, 0, 0, 0, 0, 0, false};
     uint64_t marked = 0;
-    uint32_t lo0 = 0, step1 = 0, step2 = 0, end0 = 0, end1 = 0;
     const uint32_t nx = (uint32_t)d.grid->nx;
-    auto flat_slot = [&](uint32_t i) { return (i >= end0 ? step1 : 0u) + (i >= end1 ? step2 : 0u) + (lo0 + i); };
     auto near = [&](const float4& rb) {
         const float dx = own.x - rb.x, dy = own.y - rb.y, rs = own.z + rb.z;
         const int32_t pj = __float_as_int(rb.w);
@@ -583,35 +580,22 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
         const float2 q = make_float2(own.x - a.drift_prev_x, own.y - a.drift_prev_y);
         const float R = stencil_reach(q, own.z + a.rmax);
         own.w = d.b.mass[b];
-        cx1 = g.nx - 1;
-        cy1 = g.ny - 1;
+        cells.cx1 = g.nx - 1;
+        cells.cy1 = g.ny - 1;
         if (R < 1e30f && finitef(q.x) && finitef(q.y)) {
-            cx0 = cell_coord(q.x - R, g.ox, g.inv_cell, g.nx);
-            cx1 = cell_coord(q.x + R, g.ox, g.inv_cell, g.nx);
-            cy0 = cell_coord(q.y - R, g.oy, g.inv_cell, g.ny);
-            cy1 = cell_coord(q.y + R, g.oy, g.inv_cell, g.ny);
+            cells.cx0 = cell_coord(q.x - R, g.ox, g.inv_cell, g.nx);
+            cells.cx1 = cell_coord(q.x + R, g.ox, g.inv_cell, g.nx);
+            cells.cy0 = cell_coord(q.y - R, g.oy, g.inv_cell, g.ny);
+            cells.cy1 = cell_coord(q.y + R, g.oy, g.inv_cell, g.ny);
         }
-        // candidates as one flat list: entry i is slot lo0 + i, plus step1 from end0 on (the
-        // second row), plus step2 from end1 on (modulo 2^32)
-        const uint32_t* s0 = d.cell_start + (uint32_t)cx0;
-        const uint32_t* s1 = d.cell_start + (uint32_t)cx1 + 1u;
-        const uint32_t row0 = (uint32_t)cy0 * nx, last = (uint32_t)cy1 * nx;
-        const uint32_t row1 = min(row0 + nx, last), row2 = min(row1 + nx, last);
-        lo0 = s0[row0];
-        const uint32_t hi0 = s1[row0], lo1 = s0[row1], hi1 = s1[row1], lo2 = s0[row2], hi2 = s1[row2];
-        const int32_t rows = cy1 - cy0 + 1;
-        end0 = hi0 - lo0;
-        step1 = lo1 - hi0;
-        end1 = end0 + (rows > 1 ? hi1 - lo1 : 0u);
-        step2 = (lo2 - end1) - (lo1 - end0);
-        const uint32_t total = end1 + (rows > 2 ? hi2 - lo2 : 0u);
-        static_assert(kFlatRows == 3, "the rows above");
-        direct = rows > (int32_t)kFlatRows || total > kFlatMax;
-        const uint32_t n_flat = direct ? 0u : total;
+        rows = flat_rows(d.cell_start, nx, cells);
+        static_assert(kLdsFlat <= 64, "one mask");
+        direct = !rows.flat;
+        const uint32_t n_flat = rows.n;
         for (uint32_t f = 0; f < n_flat; f += 4) {
             float4 rb[4];
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) rb[u] = d.crec[min(flat_slot(min(f + u, n_flat - 1u)), d.nc - 1u)];
+            for (uint32_t u = 0; u < 4; ++u) rb[u] = d.crec[min(rows.slot(min(f + u, n_flat - 1u)), d.nc - 1u)];
             uint32_t bits = 0;
 #pragma unroll
             for (uint32_t u = 0; u < 4; ++u) bits |= (f + u < n_flat) && near(rb[u]) ? 1u << u : 0u;
@@ -633,7 +617,7 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
     }
     if (fits)
         for (uint32_t e = first; marked != 0; ++e, marked &= marked - 1)
-            s_pair[e] = make_uint2(lane, flat_slot((uint32_t)__builtin_ctzll(marked)));
+            s_pair[e] = make_uint2(lane, rows.slot((uint32_t)__builtin_ctzll(marked)));
     wave_sync();
     // ---- correct: a pair a lane
     for (uint32_t e = lane; e < queued; e += BG_WAVE) {
@@ -670,10 +654,10 @@ __device__ __forceinline__ void contact_lists(const DeviceWorld& d, const Subste
         // contacts; 50,000 bodies 3,646 and 7,246.)
         ContactList<kDirectRegs, uint32_t> L;
         L.init();
-        for (int32_t cy = cy0; cy <= cy1; ++cy) {
+        for (int32_t cy = cells.cy0; cy <= cells.cy1; ++cy) {
             const uint32_t row = (uint32_t)cy * nx;
-            const uint32_t t1 = min(d.cell_start[row + (uint32_t)cx1 + 1u], d.nc);
-            for (uint32_t t = d.cell_start[row + (uint32_t)cx0]; t < t1; t += 4) {
+            const uint32_t t1 = min(d.cell_start[row + (uint32_t)cells.cx1 + 1u], d.nc);
+            for (uint32_t t = d.cell_start[row + (uint32_t)cells.cx0]; t < t1; t += 4) {
                 // (four records load together: a walk of hundreds waits for each of its loads)
                 float4 four[4];
 #pragma unroll
