@@ -576,10 +576,10 @@ static __device__ __forceinline__ void mark_lists(Ctx& c, const Own& o, const Di
 // thrown on eight times their area's worth, 10 steps: 28.6 ms, 88.0 that way.)
 //
 // Bound by the walks over the candidates, so one walk both counts a body's partners and keeps the
-// last kKept of them, and only a body of more is walked again to enter them.  Against two walks of
-// every body, forward: 8 worlds of 700 at 0.4 of their area's side 1.6x faster, of 1,500 1.5x, of
-// 2,048 1.6x.  A thread's two bodies are done one after the other: with both in flight the state
-// spilled 7 VGPRs.
+// last kKept of them, and only a body of more is walked again to enter them.  A thread's two bodies
+// are done one after the other, written out twice (in a loop the state in flight costs 10%).  Against
+// two walks of every body and a loop, forward, us: 8 worlds of 700 with their positions scaled by
+// 0.4 1,850 -> 1,160, of 1,500 5,420 -> 3,260, of 2,048 7,310 -> 3,790; by 0.15, of 2,048 29,900 -> 24,400.
 template <class Contact, class Finish>
 static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const DiffWorld& W, bool lists, uint32_t nout,
                                                     uint32_t pending, Contact&& contact, Finish&& finish) {
@@ -626,8 +626,9 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
             }
         }
     };
-#pragma unroll 1
-    for (uint32_t j = 0; j < per; ++j) {
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) {
+        if (j >= per) break;
         bool todo = ((pending >> j) & 1u) != 0u;
         const uint32_t own = (tid + j * kDiffThreads) << 16;
         uint32_t need = 0;
@@ -639,22 +640,19 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
                 for (uint32_t k = kKept / 2 - 1; k > 0; --k) kept[k] = kept[k] << 16 | kept[k - 1] >> 16;
                 kept[0] = kept[0] << 16 | lj;
             });
-        if (need > kPairs) {  // never fits
-            finish(j, 0u, kNoRoom, false);
-            todo = false;
-        }
+        const bool never = need > kPairs;  // fits the queue
         for (;;) {  // (the first body in line fits, so every round does some)
             __syncthreads();
             if (tid == 0) c.out->round = c.out->more = 0;
             __syncthreads();
-            const uint32_t n = todo ? need : 0u;
+            const uint32_t n = todo && !never ? need : 0u;
             const uint32_t incl = wave_prefix(n, 0u, AddU32());
             const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, BG_WAVE - 1);
             uint32_t first = 0;
             if (total > 0 && (tid & (BG_WAVE - 1)) == 0) first = atomicAdd(&c.out->round, total);
             first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + incl - n;
-            const bool placed = todo && first + n <= kPairs;
-            if (placed) {
+            const bool placed = todo && (never || first + n <= kPairs);
+            if (placed && !never) {
                 uint32_t e = first;
                 const float2 range = make_float2(__uint_as_float(first), __uint_as_float(first + n));
                 auto enter = [&](uint32_t lj) {
@@ -671,7 +669,7 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
                 } else {
                     partners(j, enter);
                 }
-            } else if (todo) {
+            } else if (todo && !never) {
                 for (uint32_t e = first; e < kPairs; ++e) c.entries[e] = kNoPair;
             }
             __syncthreads();
@@ -703,7 +701,7 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
                     c.res[to[i]] = k[i];
                 }
             __syncthreads();
-            if (placed) finish(j, first, need, true);
+            if (placed) finish(j, first, never ? kNoRoom : need, !never);
             todo = todo && !placed;
             if (todo) c.out->more = 1;
             __syncthreads();
@@ -842,7 +840,10 @@ static __device__ __forceinline__ void substep_forward(Ctx& c, Own& o, Walk& w, 
         else
             finish(j, first, count, false);
     }
-    if (crowd) queue_rounds(c, o, W, lists, nout, pending, contact, finish);
+    // (The hint keeps the rounds' state from taking registers that two bodies a thread need in every
+    // substep: 256 worlds of 2,048 over 50 steps 4.83 ms without it, 4.76 with.  With one body a thread
+    // it costs 96 worlds of 700 a hundredth.)
+    if (PER == 1 ? crowd : __builtin_expect(crowd, 0)) queue_rounds(c, o, W, lists, nout, pending, contact, finish);
     if (tid == 0) c.out->pairs[par ^ 1u] = 0;
     if (tid < kOutMax) c.out->count[par ^ 1u][tid] = 0;
     // From here to the end of the substep a thread touches the positions and velocities of its

@@ -58,11 +58,12 @@ def test_lists_change_no_result(n, kind):
         assert np.array_equal(bits(a), bits(b))
 
 
-@pytest.mark.parametrize("partners", [1, 2, 15, 16, 17, 18, 33])
+@pytest.mark.parametrize("partners", [1, 2, 15, 16, 17, 18, 33, 1500])
 @pytest.mark.parametrize("n", [256, 700, 2048])
 def test_bodies_of_many_partners_in_rounds(n, partners):
     """Hubs with so many bodies touching them and no others, in random index order; more pairs than the
-    queue holds at once, where a body's last 16 partners are kept from the walk that counts them."""
+    queue holds at once, where a body's last 16 partners are kept from the walk that counts them, and
+    a hub of more than the queue ever holds (1,200 pairs, worlds past 1,024 bodies)."""
     rng = np.random.default_rng(n + partners)
     sc = scenes.rollout_world(n, 8, scenes.Rng(42), damping=1.0)
     size = partners + 1
