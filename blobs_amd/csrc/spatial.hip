@@ -244,15 +244,23 @@ constexpr uint32_t table_size(uint32_t n) {
 
 constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Bytes of scratch for n records and nq queries, and the views into it.
-constexpr size_t scratch_bytes(uint32_t n, uint32_t nq) {
+// Bytes of scratch for n records and nq queries: the table with the scan's sums, and the records.
+constexpr size_t table_bytes(uint32_t n, uint32_t nq) {
     const uint32_t T = table_size(n);
     const uint32_t m = T + 2 > nq + 1 ? T + 2 : nq + 1;
     const uint32_t tiles = (m + kScanTile - 1) / kScanTile;
     return align256(sizeof(unsigned long long) * T) + align256(sizeof(uint32_t) * (T + 2)) +
-           3 * align256(sizeof(uint32_t) * (n > 1u ? n : 1u)) + align256(sizeof(float4) * (n > 1u ? n : 1u)) +
            align256(sizeof(uint32_t) * tiles);
 }
+constexpr size_t record_bytes(uint32_t n) {
+    return 3 * align256(sizeof(uint32_t) * (n > 1u ? n : 1u)) + align256(sizeof(float4) * (n > 1u ? n : 1u));
+}
+constexpr size_t scratch_bytes(uint32_t n, uint32_t nq) { return table_bytes(n, nq) + record_bytes(n); }
+
+// hipMalloc and hipFree of one block of at most 2 MiB take some 10 us, of a larger one some 50.  So
+// where the two parts are within that limit and their sum is not (32,769 to 65,536 records), each
+// has a block of its own: 40,000 points and queries 172 us a call with one block, 133 with two.
+constexpr size_t kCheapBlock = 2u << 20;
 
 // The no-allocation entry point's scratch: one array per GPU, held until the
 // process ends, large enough for kNoAllocMaxPoints records and
@@ -283,15 +291,18 @@ int scratch_on_current_device(char** out) {
     return BG_OK;
 }
 
-SpatialScratch carve(char* base, uint32_t n, uint32_t nq) {
+// The views into a table's and the records' bytes.
+SpatialScratch carve(char* table, char* records, uint32_t n, uint32_t nq) {
     SpatialScratch s;
     s.T = table_size(n);
     const uint32_t tiles = div_up(std::max(s.T + 2, nq + 1), kScanTile);
-    char* p = base;
+    char* p = table;
     s.keys = (unsigned long long*)p;
     p += align256(sizeof(unsigned long long) * s.T);
     s.start = (uint32_t*)p;
     p += align256(sizeof(uint32_t) * (s.T + 2));
+    s.scan.tile_sums = (uint32_t*)p;
+    p = records;
     s.slot = (uint32_t*)p;
     p += align256(sizeof(uint32_t) * std::max(n, 1u));
     s.rank = (uint32_t*)p;
@@ -299,9 +310,7 @@ SpatialScratch carve(char* base, uint32_t n, uint32_t nq) {
     s.order = (uint32_t*)p;
     p += align256(sizeof(uint32_t) * std::max(n, 1u));
     s.rec = (float4*)p;
-    p += align256(sizeof(float4) * std::max(n, 1u));
     s.kept = nq <= n ? nq : 0u;
-    s.scan.tile_sums = (uint32_t*)p;
     s.scan.max_scan_tiles = tiles;
     s.scan.hist = nullptr;
     s.scan.max_items = 0;
@@ -358,15 +367,19 @@ int bg_spatial_hash_query(float cell_size, const bg_spatial_point* points, uint3
                      uint32_t hit_cap, uint64_t* total_hits) {
     using namespace bg;
     if (int st = check_args(cell_size, points, n_points, queries, n_queries, offsets, hits, hit_cap)) return st;
-    char* mem = nullptr;
-    const hipError_t ea = hipMalloc((void**)&mem, scratch_bytes(n_points, n_queries));
+    const size_t bt = table_bytes(n_points, n_queries), br = record_bytes(n_points);
+    const bool apart = bt + br > kCheapBlock && bt <= kCheapBlock && br <= kCheapBlock;
+    char *mem = nullptr, *records = nullptr;
+    hipError_t ea = hipMalloc((void**)&mem, apart ? bt : bt + br);
+    if (ea == hipSuccess && apart && (ea = hipMalloc((void**)&records, br)) != hipSuccess) (void)hipFree(mem);
     if (ea != hipSuccess) return fail(BG_ERR_HIP, std::string("spatial query: scratch: ") + hipGetErrorString(ea));
-    const SpatialScratch s = carve(mem, n_points, n_queries);
+    const SpatialScratch s = carve(mem, apart ? records : mem + bt, n_points, n_queries);
     hipError_t e = spatial_query_on(s, cell_size, points, n_points, queries, n_queries, offsets, hits, hit_cap,
                                     nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     const int st = finish(e, offsets, n_queries, hit_cap, total_hits);
     (void)hipFree(mem);
+    if (apart) (void)hipFree(records);
     return st;
 }
 
@@ -427,7 +440,7 @@ int bg_spatial_hash_query_noalloc(float cell_size, const bg_spatial_point* point
     char* mem = nullptr;
     if (int st = scratch_on_current_device(&mem)) return st;
     // every table word the call reads is cleared by its first kernel (k_sh_clear)
-    const SpatialScratch s = carve(mem, n_points, n_queries);
+    const SpatialScratch s = carve(mem, mem + table_bytes(n_points, n_queries), n_points, n_queries);
     hipError_t e = spatial_query_on(s, cell_size, points, n_points, queries, n_queries, offsets, hits, hit_cap,
                                     nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
