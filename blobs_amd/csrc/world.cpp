@@ -2128,9 +2128,10 @@ void World::adapt_interval(const StepAccum& acc, uint32_t n_steps, bool tried) {
     if (rebuild_interval_ || small_active() || path_ != StepPath::Sphere || !params_.collisions_enabled || n_steps == 0) return;
     (void)interval_substeps();
     static constexpr uint32_t kOutlierShare[kLevels] = {512, 200, 64, 32, 32};  // one body in so many
-    // (A second rebuild within a step is another 40 us of launches however small the world, the
-    // price of some 2,000 outliers: 2,360 bodies fallen on a pile take 346 us with it, 300 without.)
-    auto limit_of = [&](uint32_t level) { return std::max(d_.nb / kOutlierShare[level], level >= 2 ? 2048u : 16u); };
+    // (A second rebuild within a step is another 40 us of launches however small the world: 2,360
+    // bodies fallen on a pile take 346 us with it, 300 without; 18,984 with 2,300 outliers and
+    // 21,997 with 3,700, a part of them falling and a part not, 155 and 145 us, 125 and 113 without.)
+    auto limit_of = [&](uint32_t level) { return std::max(d_.nb / kOutlierShare[level], level >= 2 ? 4096u : 16u); };
     if (trial_ran_ && !tried) return;  // an older call's record: the trial's is on its way
     if (tried) {
         trial_due_ = trial_ran_ = check_trial_ = false;
