@@ -611,8 +611,6 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
                 }
             }
             static_assert(kLdsRecPad >= 3, "reads past the last record");
-        } else if (n == kOut) {
-            for (uint32_t lj = 0; lj < W.nb; ++lj) test(lj, c.xy[lj], c.rad[lj]);
         } else {
             for (uint32_t i = 0; i < n; ++i) {
                 const uint32_t lj = c.lists[i >> 2][li][i & 3u];
@@ -626,14 +624,40 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
             }
         }
     };
+    // The same by the whole wave for a body outside the lists, which tests everyone: f(hit, lj, the hits'
+    // lanes) for 64 candidates at a time.  (Its lane alone took some 50 us a substep of a world of 700: 8 of
+    // them scaled by 0.55, a little too dense for lists, 1,190 us forward for 4 steps, 745 so.)
+    const uint32_t lane = tid & (BG_WAVE - 1);
+    auto everyone = [&](uint32_t li, auto&& f) {
+        const float2 p = c.xy[li];
+        const float r = c.rad[li];
+        for (uint32_t base = 0; base < W.nb; base += BG_WAVE) {
+            const uint32_t lj = base + lane;
+            bool hit = false;
+            if (lj < W.nb) {
+                const float2 b = c.xy[lj];
+                const float dx = p.x - b.x, dy = p.y - b.y, rs = r + c.rad[lj];
+                hit = (lj != li) & !(dx * dx + dy * dy > (rs * rs) * 1.00000095367431640625f);
+            }
+            f(hit, lj, __ballot(hit));
+        }
+    };
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) {
         if (j >= per) break;
         bool todo = ((pending >> j) & 1u) != 0u;
         const uint32_t own = (tid + j * kDiffThreads) << 16;
+        const bool all = todo && lists && ((o.nl >> (4u * j)) & 15u) == kOut;
         uint32_t need = 0;
         uint32_t kept[kKept / 2] = {};  // the last kKept partners found, 16 bits each
-        if (todo)
+        for (uint64_t m = __ballot(all); m; m &= m - 1) {
+            const int l = __builtin_ctzll(m);
+            uint32_t n = 0;
+            everyone((uint32_t)__builtin_amdgcn_readlane((int)own, l) >> 16,
+                     [&](bool, uint32_t, uint64_t hits) { n += (uint32_t)__popcll(hits); });
+            if (lane == (uint32_t)l) need = n;
+        }
+        if (todo && !all)
             partners(j, [&](uint32_t lj) {
                 ++need;
 #pragma unroll
@@ -652,7 +676,22 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
             if (total > 0 && (tid & (BG_WAVE - 1)) == 0) first = atomicAdd(&c.out->round, total);
             first = (uint32_t)__builtin_amdgcn_readfirstlane((int)first) + incl - n;
             const bool placed = todo && (never || first + n <= kPairs);
-            if (placed && !never) {
+            for (uint64_t m = __ballot(all && placed && !never); m; m &= m - 1) {
+                const int l = __builtin_ctzll(m);
+                const uint32_t body = (uint32_t)__builtin_amdgcn_readlane((int)own, l);
+                uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)first, l);
+                const uint32_t e1 = e + (uint32_t)__builtin_amdgcn_readlane((int)need, l);
+                const float2 range = make_float2(__uint_as_float(e), __uint_as_float(e1));
+                everyone(body >> 16, [&](bool hit, uint32_t lj, uint64_t hits) {
+                    if (hit) {
+                        const uint32_t at = e + (uint32_t)__popcll(hits & lanemask_lt());
+                        c.entries[at] = body | lj;
+                        c.res[at] = range;
+                    }
+                    e += (uint32_t)__popcll(hits);
+                });
+            }
+            if (placed && !never && !all) {
                 uint32_t e = first;
                 const float2 range = make_float2(__uint_as_float(first), __uint_as_float(first + n));
                 auto enter = [&](uint32_t lj) {
@@ -669,7 +708,7 @@ static __device__ __forceinline__ void queue_rounds(Ctx& c, const Own& o, const 
                 } else {
                     partners(j, enter);
                 }
-            } else if (todo && !never) {
+            } else if (todo && !placed) {
                 for (uint32_t e = first; e < kPairs; ++e) c.entries[e] = kNoPair;
             }
             __syncthreads();

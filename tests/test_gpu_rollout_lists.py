@@ -84,3 +84,26 @@ def test_bodies_of_many_partners_in_rounds(n, partners):
     assert np.array_equal(bits(got[0][0]), bits(o.pos))
     for a, b in zip(*got):
         assert np.array_equal(bits(a), bits(b))
+
+
+@pytest.mark.parametrize("n", [200, 321, 700, 1300, 2048])
+def test_a_body_over_all_others(n):
+    """One body outside the lists and in contact with everyone, who touch nobody else: as many pairs as the
+    queue still holds, and more than it ever does (past 1,200)."""
+    rng = np.random.default_rng(n)
+    sc = scenes.rollout_world(n, 8, scenes.Rng(43), damping=1.0)
+    wide = int(np.ceil(np.sqrt(n)))
+    k = np.arange(n)
+    at = np.stack([k % wide, k // wide], 1) * 2.5 - 1.25 * wide + rng.uniform(-0.2, 0.2, (n, 2))
+    order = rng.permutation(n)
+    sc.pos, sc.col_r = np.zeros((n, 2), np.float32), np.zeros(n, np.float32)
+    sc.pos[order] = at
+    sc.col_r[order] = 0.5
+    sc.pos[n // 3], sc.col_r[n // 3] = (0.3, -0.2), 2.0 * wide
+    sc.col_abs = sc.pos.copy()
+    got = [run([sc], 3, ck) for ck in (1, 2)]
+    o = OracleWorld(sc, np.float32)
+    o.step(sc.dt, 3)
+    assert np.array_equal(bits(got[0][0]), bits(o.pos))
+    for a, b in zip(*got):
+        assert np.array_equal(bits(a), bits(b))
