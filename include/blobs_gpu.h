@@ -252,7 +252,10 @@ int bg_get_joint(bg_world *w, bg_handle h, bg_fixed_joint *out);
 /* physics.springs.get(h) (pub arena, physics.rs:14). */
 int bg_get_spring(bg_world *w, bg_handle h, bg_spring *out);
 /* Bulk read of body state in arena (iteration) order: each pointer may be
- * NULL; arrays hold rbd_count entries (x,y interleaved for Vec2 fields). */
+ * NULL; arrays hold rbd_count entries (x,y interleaved for Vec2 fields).
+ * After a step it comes over pinned memory from a pool that worlds share: a
+ * process's first read (and each further one running at once) allocates some,
+ * about 200 us; where none is to be had, the read is slower but the same. */
 int bg_get_bodies(bg_world *w, float *position, float *position_old, float *velocity, float *rotation,
                   float *angular_velocity, bg_handle *handles);
 /* Bulk read of collider absolute translations in arena order. */
